@@ -36,7 +36,7 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contr
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument",
              f"-I{INC}", f"-I{CSRC}"]
 # per-file contraction override (kernels whose arithmetic is not pinned bit-for-bit)
-FAST_CONTRACT = {"mixed.hip"}
+FAST_CONTRACT = {"mixed.hip", "vcycle.hip"}
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", f"-I{INC}", f"-I{CSRC}",
              "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]
 

@@ -225,14 +225,29 @@ hipError_t launch_cg_step23(const Grid &g, double *x, double *r, double *z, doub
 hipError_t launch_axpy(int n, double a, const double *x, double *y, hipStream_t st);
 hipError_t launch_copy(int n, const double *x, double *y, hipStream_t st);
 
+// ---------------- launchers (vcycle.hip) ----------------
+// The FP32 operator of an all-elastic RVE as a stencil dictionary: a 16-bit
+// code per node (the phases of its eight elements) and the table of stencils.
+struct StencilOp {
+  const uint16_t *code = nullptr;  // stencil_code_len(g) entries
+  const float *tab = nullptr;      // stencil_table_len() floats
+};
+size_t stencil_code_len(const Grid &g);
+size_t stencil_table_len();
+int stencil_blocks(const Grid &g);
+// ke: the FP64 element stiffness per phase (3 x 576)
+hipError_t launch_d_setup(const Grid &g, const int *et, const double *ke, uint16_t *code, float *tab, hipStream_t st);
+// AP = A P and the (p, Ap) partials part1[field * stencil_blocks(g) + block]
+hipError_t launch_d_spmv(const Grid &g, int K, const StencilOp &op, const float *P, float *AP, double *part1,
+                         const void *state, hipStream_t st);
+
 // ---------------- launchers (mixed.hip): K right-hand sides, K in {4,8,12,16} ----------------
 size_t mixed_matrix_floats(const Grid &g);
 size_t mixed_vector_len(const Grid &g, int K);
 size_t mixed_partials(const Grid &g, int K);
 size_t mixed_state_bytes();
-// FP32 matrix A D^-1 and the Jacobi weights (scratch64: 3 NP doubles)
-hipError_t launch_m_asm32(const Grid &g, const int *et, const double *ke, int phase_mode, double *scratch64, float *A,
-                          float *kinv, hipStream_t st);
+// the FP32 Jacobi weights of an all-elastic RVE (zero off the interior)
+hipError_t launch_m_kinv(const Grid &g, const int *et, const double *ke, float *kinv, hipStream_t st);
 hipError_t launch_m_setbc(const Grid &g, int K, const double *eps, double *U, hipStream_t st);
 // F: adjoint sources (FP64, the layout of U) or null
 hipError_t launch_m_resid(const Grid &g, int K, const int *et, const double *ke, const double *U, const double *F,
@@ -262,13 +277,13 @@ hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float 
                           void *state, hipStream_t st);
 // the full symmetric FP32 copy of the lower triangle (column-major) of the
 // FP64 inverse a64 (n x n): ainv[i * n + j]
-hipError_t launch_m_iter(const Grid &g, int K, const float *A, const float *kinv, float *R, float *X, float *P,
+// (the operator: the stored FP32 matrix A, K = 4 only, or, when A is null, the
+// stencil dictionary op)
+hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                          float *AP, double *part, void *state, int parity, hipStream_t st,
                          const CoarseDev *coarse = nullptr);
 // blocks per component of the vector kernels (the partial tables' stride)
 size_t coarse_vec_blocks(const Grid &g);
-hipError_t launch_m_spmv_only(const Grid &g, int K, const float *A, const float *P, float *AP, double *part,
-                              const void *state, hipStream_t st);
 hipError_t launch_m_accum(const Grid &g, int K, const float *X, double *U, hipStream_t st);
 // mixed-precision solves of an assembled FP64 ELL system (field 0 of K = 4):
 // FP32 node-block copy of the interior block + Jacobi weights; FP64 residual

@@ -37,174 +37,24 @@
 // k of the inner CG reads state[k & 1] and writes state[(k+1) & 1].  The
 // SpMV maps slices to XCDs so that each XCD's L2 holds a contiguous slab of
 // nodes.
-#include "internal.hpp"
-#include "kernels.hpp"
-#include "physics.hpp"
-#include "reduce.hpp"
+#include "mixed.hpp"
 
 namespace mpp {
 
-constexpr int kMaxRhs = 16;
-constexpr int kRowQuads = 7, kRows = 9;         // stencil rows (dz, dy) of 27 floats + 1 pad
-constexpr int kNodeQuads = kRowQuads * kRows;  // 63 float4 per node
-__host__ __device__ constexpr int mslot(int nb, int fi, int fj) { return (nb / 3) * 28 + (nb % 3) * 9 + fi * 3 + fj; }
-constexpr int kRedThreads = 256;  // threads of the one-block reducers
-constexpr int kVecNodes = 2048;   // nodes per block of the vector kernels
-
-// inner CG scalars per field: rz = (r, z), alpha / beta of the iteration, pn
-// the current ||z||, pn0 the start value, tau the relative stop
-struct MState {
-  double rz[kMaxRhs], alpha[kMaxRhs], beta[kMaxRhs], pn[kMaxRhs], pn0[kMaxRhs], tau[kMaxRhs];
-  int done[kMaxRhs];
-  int its, max_its, all_done, pad;
-};
-
-// outer (defect-correction) test per field: pn = ||kinv r|| (the reference
-// CG's metric), rn = ||r||_2 over the interior DOFs (assembly_rhs's norm:
-// its Dirichlet rows are zero), and their values at the last `first` call
-struct MOuter {
-  double pn[kMaxRhs], pn0[kMaxRhs], target[kMaxRhs], rn[kMaxRhs], rn0[kMaxRhs];
-  int conv[kMaxRhs];
-  int all_conv, pad[3];
-};
-
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ bool node_on_boundary(const Grid &g, int i, int j, int k) {
-  return i == 0 || j == 0 || k == 0 || i == g.nx - 1 || j == g.ny - 1 || k == g.nz - 1;
-}
-
-// Blocks are dispatched round-robin over the 8 XCDs; launch 8 * per blocks and
-// give XCD x the logical blocks [x * per, (x + 1) * per).
-__device__ __forceinline__ int xcd_block(int per) {
-  const int b = blockIdx.x;
-  return (b & 7) * per + (b >> 3);
-}
-
-// Row sums of a partial table part[row * stride + j], j < n, rows < NR, by
-// one block of kRedThreads: every thread accumulates its entries j = t,
-// t + kRedThreads, ... of all rows (independent loads, all in flight), each
-// wave adds its lanes with DPP moves, and thread t < NR adds the waves' sums
-// of row t.  Fixed order throughout.  Thread t < NR returns the sum of row t
-// (others return 0).
-// The two halves of rows_sum, for callers that issue other loads in between
-// (vector-memory loads complete in issue order, so loads issued after the
-// partials' do not delay their sum): rows_load adds this thread's entries of
-// each row in index order, rows_finish combines the threads.
-template <int NR, int UNROLL = 1>
-__device__ __forceinline__ void rows_load(const double *part, size_t stride, int n, double (&s)[NR]) {
-#pragma unroll
-  for (int q = 0; q < NR; ++q) s[q] = 0.0;
-  // UNROLL > 1 keeps several rounds of loads in flight (long rows)
-#pragma unroll UNROLL
-  for (int j = threadIdx.x; j < n; j += kRedThreads)
-#pragma unroll
-    for (int q = 0; q < NR; ++q) s[q] += part[(size_t)q * stride + j];
-}
-template <int NR>
-__device__ __forceinline__ double rows_finish(double (&s)[NR]) {
-  static_assert(NR <= kRedThreads, "one row per thread at the end");
-  constexpr int kW = kRedThreads / 64;
-  __shared__ double lds[kW][NR];
-  const int t = threadIdx.x, w = t >> 6;
-  __syncthreads();  // lds may still be read by a previous call
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double v = wave_sum_dpp(s[q]);
-    if ((t & 63) == 0) lds[w][q] = v;
-  }
-  __syncthreads();
-  double r = 0.0;
-  if (t < NR)
-    for (int i = 0; i < kW; ++i) r += lds[i][t];
-  return r;
-}
-template <int NR, int UNROLL = 1>
-__device__ __forceinline__ double rows_sum(const double *part, size_t stride, int n) {
-  double s[NR];
-  rows_load<NR, UNROLL>(part, stride, n, s);
-  return rows_finish<NR>(s);
-}
-
-// ---------------------------------------------------------------------------
-// The element blocks (phase table or per element) around interior node n:
-// blk[q] the 24x24 block of element q = (a*2+b)*2+c, la[q] the node's local
-// index in it.  Entry (fi, fj) of the node block towards neighbour nb is the
-// FP64 sum of the element contributions in the reference element order.
-// ---------------------------------------------------------------------------
-struct NodeBlocks {
-  const double *blk[8];
-  int la[8];
-  __device__ NodeBlocks(const Grid &g, int i, int j, int k, const int *et, const double *ke, int phase_mode) {
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b)
-        for (int c = 0; c < 2; ++c) {
-          const int q = (a * 2 + b) * 2 + c;
-          const int e = ((k - 1 + c) * g.ney + (j - 1 + b)) * g.nex + (i - 1 + a);
-          blk[q] = ke + (size_t)(phase_mode ? et[e] : e) * 576;
-          la[q] = local_node(1 - a, 1 - b, 1 - c);
-        }
-  }
-  __device__ double entry(int nb, int fi, int fj) const {
-    const int dz = nb / 9 - 1, dy = (nb / 3) % 3 - 1, dx = nb % 3 - 1;
-    double acc = 0.0;
-    for (int a = 0; a < 2; ++a) {
-      const int px = 1 - a + dx;
-      if (px < 0 || px > 1) continue;
-      for (int b = 0; b < 2; ++b) {
-        const int py = 1 - b + dy;
-        if (py < 0 || py > 1) continue;
-        for (int c = 0; c < 2; ++c) {
-          const int pz = 1 - c + dz;
-          if (pz < 0 || pz > 1) continue;
-          const int q = (a * 2 + b) * 2 + c;
-          acc += blk[q][(la[q] * 3 + fi) * 24 + local_node(px, py, pz) * 3 + fj];
-        }
-      }
-    }
-    return acc;
-  }
-};
-
-// Jacobi weights: kinv64[d * NP + n] = 1 / A_nn(d, d) (FP64, zero on
-// Dirichlet DOFs and padding) and its FP32 copy kinv
-__global__ void __launch_bounds__(256) k_m_kinv(Grid g, int NP, const int *et, const double *ke, int phase_mode,
-                                                double *kinv64, float *kinv) {
+// Jacobi weights: kinv[d * NP + n] = 1 / A_nn(d, d), formed in FP64 and
+// rounded once (zero on Dirichlet DOFs and padding)
+__global__ void __launch_bounds__(256) k_m_kinv(Grid g, int NP, const int *et, const double *ke, float *kinv) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= NP) return;
   double w[3] = {0.0, 0.0, 0.0};
   if (n < g.nn) {
     const int i = n % g.nx, j = (n / g.nx) % g.ny, k = n / (g.nx * g.ny);
     if (!node_on_boundary(g, i, j, k)) {
-      const NodeBlocks B(g, i, j, k, et, ke, phase_mode);
+      const NodeBlocks B(g, i, j, k, et, ke, 1);
       for (int d = 0; d < 3; ++d) w[d] = 1.0 / B.entry(13, d, d);
     }
   }
-  for (int d = 0; d < 3; ++d) {
-    kinv64[(size_t)d * NP + n] = w[d];
-    kinv[(size_t)d * NP + n] = (float)w[d];
-  }
-}
-
-// FP32 matrix: slot (nb, fi, fj) of node n = A(n fi, m fj) for neighbour m,
-// rounded once; rows and columns of Dirichlet DOFs are zero
-__global__ void __launch_bounds__(256) k_m_asm32(Grid g, int NP, const int *et, const double *ke, int phase_mode,
-                                                 float *A) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= NP) return;
-  float *base = A + ((size_t)(n >> 6) * kNodeQuads * 64 + (n & 63)) * 4;
-  auto put = [&](int s, float v) { base[(size_t)(s >> 2) * 256 + (s & 3)] = v; };
-  for (int s = 0; s < kNodeQuads * 4; ++s) put(s, 0.0f);
-  if (n >= g.nn) return;
-  const int i = n % g.nx, j = (n / g.nx) % g.ny, k = n / (g.nx * g.ny);
-  if (node_on_boundary(g, i, j, k)) return;
-  const NodeBlocks B(g, i, j, k, et, ke, phase_mode);
-  for (int nb = 0; nb < 27; ++nb) {
-    const int dz = nb / 9 - 1, dy = (nb / 3) % 3 - 1, dx = nb % 3 - 1;
-    if (node_on_boundary(g, i + dx, j + dy, k + dz)) continue;  // column of a Dirichlet DOF: dropped
-    for (int fi = 0; fi < 3; ++fi)
-      for (int fj = 0; fj < 3; ++fj) put(mslot(nb, fi, fj), (float)B.entry(nb, fi, fj));
-  }
+  for (int d = 0; d < 3; ++d) kinv[(size_t)d * NP + n] = (float)w[d];
 }
 
 // ---------------------------------------------------------------------------
@@ -558,21 +408,6 @@ __device__ __forceinline__ void read_stage(const float4 *stage, float a[28]) {
     a[q * 4 + 2] = m[q].z;
     a[q * 4 + 3] = m[q].w;
   }
-}
-
-// DPP wave shifts: lane i takes lane i - 1's value (lane 0 keeps `old`), or
-// lane i + 1's (lane 63 keeps `old`)
-__device__ __forceinline__ float4 from_left(const float4 &v, const float4 &old) {
-  auto f = [](float x, float o) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(o), __float_as_int(x), 0x138, 0xf, 0xf, false));
-  };
-  return make_float4(f(v.x, old.x), f(v.y, old.y), f(v.z, old.z), f(v.w, old.w));
-}
-__device__ __forceinline__ float4 from_right(const float4 &v, const float4 &old) {
-  auto f = [](float x, float o) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(o), __float_as_int(x), 0x130, 0xf, 0xf, false));
-  };
-  return make_float4(f(v.x, old.x), f(v.y, old.y), f(v.z, old.z), f(v.w, old.w));
 }
 
 template <int K>
@@ -1697,26 +1532,6 @@ __global__ void __launch_bounds__(256) k_m_accum_ell(Grid g, int NP, const float
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-static unsigned nblk(size_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-
-struct MLaunch {
-  int NP;         // nodes rounded up to 256
-  int per, nb;    // node blocks of 256 per XCD, blocks launched (8 * per)
-  int nsl, pers;  // slices of 64 nodes, slices per XCD (8 * pers launched)
-  int nbx;        // blocks of 256 float4 per component
-};
-
-static MLaunch mshape(const Grid &g) {
-  MLaunch s;
-  s.NP = (int)round_up((size_t)g.nn, 256);
-  s.per = (s.NP / 256 + 7) / 8;
-  s.nb = s.per * 8;
-  s.nsl = s.NP / 64;
-  s.pers = (s.nsl + 7) / 8;
-  s.nbx = (int)nblk((size_t)s.NP / 4, 256);
-  return s;
-}
-
 size_t mixed_matrix_floats(const Grid &g) { return (size_t)mshape(g).NP * kNodeQuads * 4; }
 size_t mixed_vector_len(const Grid &g, int K) { return (size_t)mshape(g).NP * 3 * K; }
 size_t mixed_partials(const Grid &g, int K) {
@@ -1726,37 +1541,12 @@ size_t mixed_partials(const Grid &g, int K) {
   const size_t iter = (size_t)K * s.nsl + 2 * (size_t)3 * K * (s.NP / 256);
   return std::max(std::max(resid, ave), iter);
 }
-size_t mixed_state_bytes() { return 2 * sizeof(MState) + sizeof(MOuter); }
-
-hipError_t launch_m_asm32(const Grid &g, const int *et, const double *ke, int phase_mode, double *scratch64, float *A,
-                          float *kinv, hipStream_t st) {
+hipError_t launch_m_kinv(const Grid &g, const int *et, const double *ke, float *kinv, hipStream_t st) {
   const MLaunch s = mshape(g);
-  hipLaunchKernelGGL(k_m_kinv, dim3(s.NP / 256), dim3(256), 0, st, g, s.NP, et, ke, phase_mode, scratch64, kinv);
-  hipLaunchKernelGGL(k_m_asm32, dim3(s.NP / 256), dim3(256), 0, st, g, s.NP, et, ke, phase_mode, A);
+  hipLaunchKernelGGL(k_m_kinv, dim3(s.NP / 256), dim3(256), 0, st, g, s.NP, et, ke, kinv);
   return hipGetLastError();
 }
-
-#define MPP_K_DISPATCH(K, CALL)                     \
-  switch (K) {                                      \
-    case 4: {                                       \
-      constexpr int KK = 4;                         \
-      CALL;                                         \
-    } break;                                        \
-    case 8: {                                       \
-      constexpr int KK = 8;                         \
-      CALL;                                         \
-    } break;                                        \
-    case 12: {                                      \
-      constexpr int KK = 12;                        \
-      CALL;                                         \
-    } break;                                        \
-    case 16: {                                      \
-      constexpr int KK = 16;                        \
-      CALL;                                         \
-    } break;                                        \
-    default:                                        \
-      return hipErrorInvalidValue;                  \
-  }
+size_t mixed_state_bytes() { return 2 * sizeof(MState) + sizeof(MOuter); }
 
 hipError_t launch_m_setbc(const Grid &g, int K, const double *eps, double *U, hipStream_t st) {
   const MLaunch s = mshape(g);
@@ -1812,7 +1602,7 @@ static void coarse_solve(const Grid &g, const MLaunch &s, const CoarseDev &c, co
                      cur);
 }
 
-hipError_t launch_m_iter(const Grid &g, int K, const float *A, const float *kinv, float *R, float *X, float *P,
+hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                          float *AP, double *part, void *state, int parity, hipStream_t st, const CoarseDev *coarse) {
   const MLaunch s = mshape(g);
   MState *ms = static_cast<MState *>(state);
@@ -1822,20 +1612,27 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const float *kinv
   // with a coarse level k_m_upd runs on blocks of whole x-lines (lpb a block, nbu blocks)
   const int lpb = coarse ? kVecNodes / g.nx : 0;
   const int nbu = coarse ? (g.ny * g.nz + lpb - 1) / lpb : nbx;
-  double *part1 = part;                                   // K x nsl
-  double *pz = part + (size_t)K * s.nsl;                  // 3K x nbu: (z, z)
+  const int np1 = A ? s.nsl : stencil_blocks(g);          // (p, Ap) partials per field
+  double *part1 = part;                                   // K x np1
+  double *pz = part + (size_t)K * np1;                    // 3K x nbu: (z, z)
   double *pr = pz + (size_t)3 * K * std::max(nbx, nbu);   // 3K x nbx: (r, z)
   const dim3 vgrid(nbx, 3 * K / 4);
   const CGrid cg = coarse ? coarse->cg : CGrid{};
-  MPP_K_DISPATCH(K, {
-    hipLaunchKernelGGL(k_m_spmv<KK>, dim3(8 * s.pers), dim3(16 * KK), 0, st, g, s.NP, s.nsl, s.pers,
+  if (A) {
+    if (K != 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_m_spmv<4>, dim3(8 * s.pers), dim3(64), 0, st, g, s.NP, s.nsl, s.pers,
                        reinterpret_cast<const float4 *>(A), reinterpret_cast<const float4 *>(P),
                        reinterpret_cast<float4 *>(AP), part1, cur);
+  } else {
+    const hipError_t e = launch_d_spmv(g, K, op, P, AP, part1, cur, st);
+    if (e != hipSuccess) return e;
+  }
+  MPP_K_DISPATCH(K, {
     if (coarse) {
       // R -= alpha AP with the x-restriction of the new R; then the coarse
       // solve, z and (r, z) with the coarse correction (its partials in
       // place of the Jacobi (r, z) ones), and the p-update from z
-      hipLaunchKernelGGL((k_m_upd<KK, true>), dim3(nbu, 3 * K / 4), dim3(kRedThreads), 0, st, s.NP, s.nsl, part1,
+      hipLaunchKernelGGL((k_m_upd<KK, true>), dim3(nbu, 3 * K / 4), dim3(kRedThreads), 0, st, s.NP, np1, part1,
                          kinv, reinterpret_cast<const float4 *>(AP), reinterpret_cast<float4 *>(R), pz, pr, cur, g,
                          cg, lpb, reinterpret_cast<float4 *>(coarse->t1));
       coarse_solve<KK>(g, s, *coarse, R, cur, st, false);
@@ -1846,7 +1643,7 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const float *kinv
                          reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(coarse->z),
                          reinterpret_cast<float4 *>(P), reinterpret_cast<float4 *>(X), pz, nbu, pr, cur, nxt);
     } else {
-      hipLaunchKernelGGL((k_m_upd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, s.nsl, part1, kinv,
+      hipLaunchKernelGGL((k_m_upd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv,
                          reinterpret_cast<const float4 *>(AP), reinterpret_cast<float4 *>(R), pz, pr, cur, g, cg,
                          0, nullptr);
       hipLaunchKernelGGL((k_m_pupd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv,
@@ -1874,16 +1671,6 @@ hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float 
 }
 
 size_t coarse_vec_blocks(const Grid &g) { return nblk(mshape(g).NP, kVecNodes); }
-
-hipError_t launch_m_spmv_only(const Grid &g, int K, const float *A, const float *P, float *AP, double *part,
-                              const void *state, hipStream_t st) {
-  const MLaunch s = mshape(g);
-  const MState *cur = static_cast<const MState *>(state);
-  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_spmv<KK>, dim3(8 * s.pers), dim3(16 * KK), 0, st, g, s.NP, s.nsl, s.pers,
-                                       reinterpret_cast<const float4 *>(A), reinterpret_cast<const float4 *>(P),
-                                       reinterpret_cast<float4 *>(AP), part, cur));
-  return hipGetLastError();
-}
 
 hipError_t launch_m_from_ell(const Grid &g, const double *vals, float *A, double *kinv64, float *kinv,
                              hipStream_t st) {

@@ -717,7 +717,8 @@ struct mppd_msolver {
   hipStream_t st = nullptr;
   double *ke = nullptr;         // phase table 3 x 576 (FP64)
   material_base *mats_d = nullptr;
-  float *A = nullptr, *kinv = nullptr;
+  StencilOp op;                 // the FP32 operator
+  float *kinv = nullptr;
   float *X = nullptr, *R = nullptr, *P = nullptr, *AP = nullptr;  // 4-field-group layout
   double *U = nullptr, *eps_d = nullptr, *part = nullptr, *sig_d = nullptr;
   void *state = nullptr, *state_h = nullptr;
@@ -748,11 +749,11 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
       break;
     }
     const size_t nv = mixed_vector_len(g, nrhs);
-    // The device buffers in one allocation, 256-byte aligned parts, the FP32
-    // matrix last: everything before it is zero-filled on m->st in one fill
-    // (ordered before the set-up kernels; mats_d is then written by a
-    // blocking copy), the matrix is written whole by the assembly.  The
-    // pinned staging in one host allocation.
+    // The device buffers in one allocation, 256-byte aligned parts, the
+    // operator's codes and stencils last: everything before them is
+    // zero-filled on m->st in one fill (ordered before the set-up kernels;
+    // mats_d is then written by a blocking copy), they are written whole by
+    // the set-up.  The pinned staging in one host allocation.
     hipStream_t st = m->st;
     size_t off = 0;
     auto carve = [&off](size_t bytes) {
@@ -766,7 +767,8 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
     const size_t o_U = carve(nv * sizeof(double)), o_eps = carve(16 * 6 * sizeof(double)),
                  o_sig = carve(16 * 6 * sizeof(double)), o_part = carve(mixed_partials(g, nrhs) * sizeof(double));
     const size_t o_state = carve(mixed_state_bytes()), o_act = carve(kMaxRhsFields * sizeof(int));
-    const size_t zeroed = off, o_A = carve(mixed_matrix_floats(g) * sizeof(float));
+    const size_t zeroed = off, o_code = carve(stencil_code_len(g) * sizeof(uint16_t)),
+                 o_tab = carve(stencil_table_len() * sizeof(float));
     e = hipMalloc(&m->arena, off);
     if (e == hipSuccess) e = hipMemsetAsync(m->arena, 0, zeroed, st);
     if (e != hipSuccess) {
@@ -787,7 +789,10 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
     m->part = reinterpret_cast<double *>(base + o_part);
     m->state = base + o_state;
     m->act_d = reinterpret_cast<int *>(base + o_act);
-    m->A = reinterpret_cast<float *>(base + o_A);
+    uint16_t *code = reinterpret_cast<uint16_t *>(base + o_code);
+    float *tab = reinterpret_cast<float *>(base + o_tab);
+    m->op.code = code;
+    m->op.tab = tab;
     off = 0;
     const size_t h_state = carve(mixed_state_bytes()), h_act = carve(kMaxRhsFields * sizeof(int)),
                  h_eps = carve(16 * 6 * sizeof(double)), h_sig = carve(16 * 6 * sizeof(double));
@@ -801,10 +806,10 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
       e = hipStreamSynchronize(st);  // the fill, before the blocking copy into mats_d
     }
     if (e == hipSuccess) e = hipMemcpy(m->mats_d, r->mats, 3 * sizeof(material_base), hipMemcpyHostToDevice);
-    // element stiffness per phase (FP64, the plain path's kernel), then the FP32 node-block matrix
+    // element stiffness per phase (FP64, the plain path's kernel), then the FP32 operator and Jacobi weights
     if (e == hipSuccess) e = launch_elem_ke(g, r->bmat, r->mats_d, r->et, nullptr, nullptr, 1, m->ke, m->st);
-    // (U serves as FP64 scratch for the Jacobi weights: 3 NP <= 3 K NP doubles)
-    if (e == hipSuccess) e = launch_m_asm32(g, r->et, m->ke, 1, m->U, m->A, m->kinv, m->st);
+    if (e == hipSuccess) e = launch_d_setup(g, r->et, m->ke, code, tab, m->st);
+    if (e == hipSuccess) e = launch_m_kinv(g, r->et, m->ke, m->kinv, m->st);
     if (e == hipSuccess) e = hipStreamSynchronize(m->st);
     if (e != hipSuccess) {
       rc = hip_fail(e, "msolver set-up");
@@ -842,7 +847,7 @@ int mppd_msolver_destroy(mppd_msolver *m) {
 // convergence rate (iterations still needed, + 2), so few iterations are
 // queued past the end.  *its = iterations run; *finite (may be NULL) = every
 // field's ||z|| is finite at the end (no breakdown).
-static int mixed_inner(const Grid &g, int K, const float *A, const float *kinv, float *R, float *X, float *P,
+static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                        float *AP, double *part, void *state, void *state_h, int max_inner, hipStream_t st,
                        int *its_out, bool *finite = nullptr, bool stop_on_stall = false,
                        const CoarseDev *coarse = nullptr) {
@@ -857,7 +862,7 @@ static int mixed_inner(const Grid &g, int K, const float *A, const float *kinv, 
     const int nq = std::min(chunk, max_inner - queued);
     if (nq <= 0) break;
     for (int i = 0; i < nq; ++i)
-      MPP_HIP(launch_m_iter(g, K, A, kinv, R, X, P, AP, part, state, queued + i, st, coarse));
+      MPP_HIP(launch_m_iter(g, K, A, op, kinv, R, X, P, AP, part, state, queued + i, st, coarse));
     queued += nq;
     MPP_HIP(hipMemcpyAsync(state_h, state, mixed_state_bytes(), hipMemcpyDeviceToHost, st));
     MPP_HIP(hipStreamSynchronize(st));
@@ -925,7 +930,7 @@ static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, co
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
     if (all_conv || outer >= p->max_outer) break;
-    int its = 0, rc = mixed_inner(g, K, m->A, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
+    int its = 0, rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
                                   p->max_inner_its, m->st, &its, nullptr, false, m->coarse);
     if (rc) return rc;
     inner_total += its;
@@ -1095,7 +1100,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
       mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
       if (all_conv || outer >= max_outer) break;
       int inner = 0;
-      if ((rc = mixed_inner(g, K, m->A, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
+      if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
                             m->st, &inner, nullptr, false, m->coarse)))
         return rc;
       inner_total += inner;
@@ -1246,7 +1251,7 @@ int mppd_newton_mixed(mppd_solver *s, const mppd_solver *A0, const double eps[6]
       }
       int inner = 0;
       bool finite = true;
-      if ((rc = mixed_inner(g, K, ml->A, ml->kinv, ml->R, ml->X, ml->P, ml->AP, ml->part, ml->state, ml->state_h,
+      if ((rc = mixed_inner(g, K, ml->A, StencilOp{}, ml->kinv, ml->R, ml->X, ml->P, ml->AP, ml->part, ml->state, ml->state_h,
                             max_inner, s->st, &inner, &finite, true, ml->coarse)))
         return rc;
       solver_its += inner;
@@ -1362,10 +1367,10 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
   for (auto &x : ev) MPP_HIP(hipEventCreate(&x));
   hipError_t e = hipEventRecord(ev[0], m->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_m_spmv_only(g, K, m->A, m->P, m->AP, m->part, m->state, m->st);
+    e = launch_d_spmv(g, K, m->op, m->P, m->AP, m->part, m->state, m->st);
   if (e == hipSuccess) e = hipEventRecord(ev[1], m->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_m_iter(g, K, m->A, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, i, m->st, m->coarse);
+    e = launch_m_iter(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, i, m->st, m->coarse);
   if (e == hipSuccess) e = hipEventRecord(ev[2], m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
   float ms1 = 0.f, ms2 = 0.f;
