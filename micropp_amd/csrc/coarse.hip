@@ -32,6 +32,11 @@ int pick_side(int ne, int dmax) {
   return 0;
 }
 
+// positions of a fine element along a side (see k_cs_table)
+__host__ __device__ inline int npos(int h, int l) { return l == h ? h : h + l; }
+// first fine element of coarse element E of d along a side of ne
+__device__ __forceinline__ int cnode(int E, int ne, int d) { return E * ne / d; }
+
 // corner A of a hexahedron (the element's local node order: (0,0,0), (1,0,0),
 // (1,1,0), (0,1,0), then the same at z + 1) and its inverse
 __device__ __forceinline__ int hex_ox(int A) { return ((A + 1) >> 1) & 1; }
@@ -40,18 +45,21 @@ __device__ __forceinline__ int hex_oz(int A) { return A >> 2; }
 __device__ __forceinline__ int hex_corner(int ox, int oy, int oz) { return oz * 4 + (oy ? 3 - ox : ox); }
 
 // C[(pos * 3 + phase) * 576 + r * 24 + c] = (P_e^T Ke_phase P_e)[r][c] for the
-// fine element at position pos = (pz hy + py) hx + px: block (pos, phase),
-// one thread per entry
+// fine element at position pos = (pz ny + py) nx + px, nx = npos(hx, lx) ...
+// (p < h: the position in an element h wide; h + p: in one l wide):
+// block (pos, phase), one thread per entry
 __global__ void __launch_bounds__(576) k_cs_table(CGrid cg, const double *ke, double *C) {
   __shared__ double N[8][8];  // N[a][A]: coarse corner A's hat at the fine element's node a
   __shared__ double K[576];
   const int pos = blockIdx.x, ph = blockIdx.y, t = threadIdx.x;
-  const int px = pos % cg.hx, py = (pos / cg.hx) % cg.hy, pz = pos / (cg.hx * cg.hy);
+  const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
+  const int px = pos % nx, py = (pos / nx) % ny, pz = pos / (nx * ny);
   K[t] = ke[(size_t)ph * 576 + t];
   if (t < 64) {
     const int a = t >> 3, A = t & 7;
-    const double xi = (double)(px + hex_ox(a)) / cg.hx, yi = (double)(py + hex_oy(a)) / cg.hy,
-                 zi = (double)(pz + hex_oz(a)) / cg.hz;
+    const double xi = px < cg.hx ? (double)(px + hex_ox(a)) / cg.hx : (double)(px - cg.hx + hex_ox(a)) / cg.lx,
+                 yi = py < cg.hy ? (double)(py + hex_oy(a)) / cg.hy : (double)(py - cg.hy + hex_oy(a)) / cg.ly,
+                 zi = pz < cg.hz ? (double)(pz + hex_oz(a)) / cg.hz : (double)(pz - cg.hz + hex_oz(a)) / cg.lz;
     N[a][A] = (hex_ox(A) ? xi : 1.0 - xi) * (hex_oy(A) ? yi : 1.0 - yi) * (hex_oz(A) ? zi : 1.0 - zi);
   }
   __syncthreads();
@@ -71,12 +79,17 @@ __global__ void __launch_bounds__(576) k_cs_elem(Grid g, CGrid cg, int dx, int d
                                                  double *KE) {
   const int E = blockIdx.x, t = threadIdx.x;
   const int Ex = E % dx, Ey = (E / dx) % dy, Ez = E / (dx * dy);
+  const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
+  const int x0 = cnode(Ex, g.nex, cg.mx + 1), y0 = cnode(Ey, g.ney, cg.my + 1), z0 = cnode(Ez, g.nez, cg.mz + 1);
+  const int wx = cnode(Ex + 1, g.nex, cg.mx + 1) - x0, wy = cnode(Ey + 1, g.ney, cg.my + 1) - y0,
+            wz = cnode(Ez + 1, g.nez, cg.mz + 1) - z0;
+  const int ox = wx != cg.hx ? cg.hx : 0, oy = wy != cg.hy ? cg.hy : 0, oz = wz != cg.hz ? cg.hz : 0;
   double s = 0.0;
-  for (int pz = 0; pz < cg.hz; ++pz)
-    for (int py = 0; py < cg.hy; ++py)
-      for (int px = 0; px < cg.hx; ++px) {
-        const int e = ((Ez * cg.hz + pz) * g.ney + (Ey * cg.hy + py)) * g.nex + Ex * cg.hx + px;
-        const int pos = (pz * cg.hy + py) * cg.hx + px;
+  for (int pz = 0; pz < wz; ++pz)
+    for (int py = 0; py < wy; ++py)
+      for (int px = 0; px < wx; ++px) {
+        const int e = ((z0 + pz) * g.ney + y0 + py) * g.nex + x0 + px;
+        const int pos = ((oz + pz) * ny + oy + py) * nx + ox + px;
         s += C[((size_t)pos * 3 + et[e]) * 576 + t];
       }
   KE[(size_t)E * 576 + t] = s;
@@ -449,6 +462,24 @@ bool coarse_enabled() {
   return !(env && std::atoi(env) == 0);
 }
 
+// the coarse grid of hx, hy, hz (lx, ly, lz) fine elements per coarse element
+// and mx, my, mz interior nodes
+static CGrid make_grid(int hx, int hy, int hz, int lx, int ly, int lz, int mx, int my, int mz) {
+  CGrid cg;
+  cg.hx = hx;
+  cg.hy = hy;
+  cg.hz = hz;
+  cg.lx = lx;
+  cg.ly = ly;
+  cg.lz = lz;
+  cg.mx = mx;
+  cg.my = my;
+  cg.mz = mz;
+  cg.nq = mx * my * mz;
+  cg.nc = 3 * cg.nq;
+  return cg;
+}
+
 // The coarsest-first search: the largest coarse grid aligned with g (a
 // divisor of each side's element count, at least 2 coarse elements a side)
 // with at most max_dofs coarse DOFs and at most kCoarseMaxPos fine elements
@@ -464,31 +495,67 @@ bool coarse_grid(const Grid &g, int max_dofs, CGrid *out) {
     dx = dy = dz = 0;
   }
   if (!dx) return false;
-  CGrid cg;
-  cg.hx = g.nex / dx;
-  cg.hy = g.ney / dy;
-  cg.hz = g.nez / dz;
-  cg.mx = dx - 1;
-  cg.my = dy - 1;
-  cg.mz = dz - 1;
-  cg.nq = cg.mx * cg.my * cg.mz;
-  cg.nc = 3 * cg.nq;
+  const int hx = g.nex / dx, hy = g.ney / dy, hz = g.nez / dz;
+  const CGrid cg = make_grid(hx, hy, hz, hx, hy, hz, dx - 1, dy - 1, dz - 1);
   if (cg.hx * cg.hy * cg.hz > kCoarseMaxPos) return false;
   *out = cg;
   return true;
 }
 
+bool coarse_grid_by_two(const Grid &g, CGrid *out) {
+  if (g.nex < 4 || g.ney < 4 || g.nez < 4) return false;
+  *out = make_grid(2, 2, 2, 2 - g.nex % 2, 2 - g.ney % 2, 2 - g.nez % 2, (g.nex - 1) / 2, (g.ney - 1) / 2,
+                   (g.nez - 1) / 2);
+  return true;
+}
+
+// At h = 4 to 5 the second level's smoother covers what lies between the grids
+// (50^3, contrast 10: 21 iterations at h = 5, 26 at h = 7; 30^3: 17 at h = 3, 19
+// at h = 5), while the dense inverse stays small: 375 coarse DOFs at 30^3
+// against 2187 at h = 3, whose inverse (19 MB read an iteration) and
+// factorisation (1.2 ms) cost more than the two iterations.
+bool coarse_grid_cycle(const Grid &g, CGrid *out) {
+  if (g.nex < 4 || g.ney < 4 || g.nez < 4) return false;
+  if (g.nx > kCoarseMaxLine || g.ny > kCoarseMaxLine || g.nz > kCoarseMaxLine) return false;
+  const int ne[3] = {g.nex, g.ney, g.nez};
+  for (int most = 5; most <= kCoarseMaxLine; ++most) {  // the widest coarse element looked at
+    int h[3], l[3], m[3];
+    for (int d = 0; d < 3; ++d) {
+      const int n = std::max(2, (ne[d] + most - 1) / most);
+      h[d] = ne[d] / n;
+      l[d] = h[d] + (ne[d] % n != 0);
+      m[d] = n - 1;
+    }
+    if (3 * m[0] * m[1] * m[2] > kCoarseMaxDofs) continue;
+    const CGrid cg = make_grid(h[0], h[1], h[2], l[0], l[1], l[2], m[0], m[1], m[2]);
+    // the set-up's table holds every position along a side (h, and l of the wider elements)
+    if (coarse_table_len(cg) / (3 * 576) > (size_t)kCoarseMaxPos * 4) return false;
+    *out = cg;
+    return true;
+  }
+  return false;
+}
+
+size_t coarse_table_len(const CGrid &cg) {
+  return (size_t)npos(cg.hx, cg.lx) * npos(cg.hy, cg.ly) * npos(cg.hz, cg.lz) * 3 * 576;
+}
+
+hipError_t launch_cs_table(const CGrid &cg, const double *ke, double *C, hipStream_t st) {
+  hipLaunchKernelGGL(k_cs_table, dim3((unsigned)(coarse_table_len(cg) / (3 * 576)), 3), dim3(576), 0, st, cg, ke, C);
+  return hipGetLastError();
+}
+
 int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double *ke_d, float *ainv, hipStream_t st,
                    bool *ok) {
   *ok = false;
-  const int nc = cg.nc, npos = cg.hx * cg.hy * cg.hz;
+  const int nc = cg.nc;
   const int dx = cg.mx + 1, dy = cg.my + 1, ncel = dx * dy * (cg.mz + 1);
   Band b;
   b.n = nc;
   b.nt = (nc + kChT - 1) / kChT;
   b.bt = (3 * (cg.mx * cg.my + cg.mx + 1) + 2 + kChT - 1) / kChT;
   const size_t nband = (size_t)b.nt * (b.bt + 1) * kChTT, nw = tri_slot(b.nt, 0) * kChTT;
-  const size_t nC = (size_t)npos * 3 * 576, nKE = (size_t)ncel * 576;
+  const size_t nC = coarse_table_len(cg), nKE = (size_t)ncel * 576;
   double *buf = nullptr;
   int *info_d = nullptr;
   int rc = MPPD_OK;
@@ -502,7 +569,7 @@ int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double
       rc = hip_fail(e, "coarse factor status");
       break;
     }
-    hipLaunchKernelGGL(k_cs_table, dim3(npos, 3), dim3(576), 0, st, cg, ke_d, C);
+    (void)launch_cs_table(cg, ke_d, C, st);
     hipLaunchKernelGGL(k_cs_elem, dim3(ncel), dim3(576), 0, st, g, cg, dx, dy, et_d, C, KE);
     hipLaunchKernelGGL(k_cs_band, dim3((unsigned)((nband + 255) / 256)), dim3(256), 0, st, cg, dx, dy, b, KE, Ab);
     for (int k = -1; k < b.nt; ++k) {

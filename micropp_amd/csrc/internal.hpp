@@ -116,6 +116,7 @@ inline bool alloc_fault_injected() {
 // (cy - 1)) mx + (cx - 1).
 struct CGrid {
   int hx, hy, hz;  // fine elements per coarse element
+  int lx, ly, lz;  // = h where all are h wide; else some are l wide (multilevel preconditioner only)
   int mx, my, mz;  // interior coarse nodes per side
   int nq, nc;      // interior coarse nodes, coarse DOFs (3 nq)
 };
@@ -135,11 +136,38 @@ constexpr int kCoarseSplit = 16;    // column splits of the coarse solve (one pa
 constexpr int kCoarseMaxLine = 256;  // nodes per side a coarse level allows
 constexpr int kCoarseMaxDofs = 2200;  // coarse DOFs of a multi-RHS solver (3 x 9^3 = 2187: 10^3 coarse elements)
 constexpr int kCoarseMaxPos = 4096;   // fine elements per coarse element (the set-up's table size)
+// Multilevel (V-cycle) preconditioner of the multi-RHS inner CG on a stencil
+// dictionary (vcycle.hip): Jacobi smoothing on the fine grid and on the grid of
+// twice its spacing (its Galerkin operator stored as FP32 node blocks), and the
+// dense inverse of a coarse Galerkin matrix.
+struct VCycleDev {
+  CGrid mid, cg;     // second level (h = 2), coarse grid (hats on the fine grid's indices)
+  Grid g1;           // the second level as a grid: m + 2 nodes a side, the boundary among them
+  const float *ainv;          // nc x nc
+  float *rc, *ecp;            // restricted residual (nc x K), split partials of the coarse solve (nsplit x nc x K)
+  int nsplit;
+  float *A1, *kinv1;          // second level: node blocks (63 float4 a node, A1[quad * NP1 + node]) and Jacobi weights
+  float *R1, *E0, *T1, *E;    // second level: residual, Jacobi part, smoothed residual, correction
+  float *z;                   // fine work vector, in R's layout
+  double *prz;                // partials of (r, z) at the inner CG's start: K x stencil_blocks
+  float w0, w1;               // damping of the two Jacobi smoothers
+  void *arena;
+};
 // MPPD_COARSE=0 in the environment turns the coarse levels off
 bool coarse_enabled();
 // the largest coarse grid aligned with g with at most max_dofs coarse DOFs
 // (false: none)
 bool coarse_grid(const Grid &g, int max_dofs, CGrid *out);
+// the grid of twice the spacing (an odd side's last element 1 wide; false: a side of fewer than 4 elements)
+bool coarse_grid_by_two(const Grid &g, CGrid *out);
+// the coarse grid of the multilevel preconditioner: about 5 fine elements per coarse element and side, coarse node q
+// of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
+// divide the side, l = h + 1); false: none
+bool coarse_grid_cycle(const Grid &g, CGrid *out);
+// C (device, coarse_table_len(cg) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position
+// (position px of a side: px < h in a regular element, h + px in a last element of another width)
+size_t coarse_table_len(const CGrid &cg);
+hipError_t launch_cs_table(const CGrid &cg, const double *ke, double *C, hipStream_t st);
 // ainv (nc x nc floats, device) = the FP32 inverse of the Galerkin coarse
 // matrix of the RVE (phase map et_d, per-phase element stiffness ke_d) on cg;
 // *ok = false when that matrix is not positive definite
@@ -227,19 +255,37 @@ hipError_t launch_copy(int n, const double *x, double *y, hipStream_t st);
 
 // ---------------- launchers (vcycle.hip) ----------------
 // The FP32 operator of an all-elastic RVE as a stencil dictionary: a 16-bit
-// code per node (the phases of its eight elements) and the table of stencils.
+// code per node (the phases of its eight elements), the table of stencils, the
+// nodes whose elements differ in phase (nif of them, ascending) and the
+// symmetric stencils of the others.
 struct StencilOp {
-  const uint16_t *code = nullptr;  // stencil_code_len(g) entries
-  const float *tab = nullptr;      // stencil_table_len() floats
+  const uint16_t *code = nullptr;
+  const int *list = nullptr;
+  const float *tab = nullptr, *hom = nullptr;
+  int nif = 0;
 };
-size_t stencil_code_len(const Grid &g);
-size_t stencil_table_len();
-int stencil_blocks(const Grid &g);
-// ke: the FP64 element stiffness per phase (3 x 576)
-hipError_t launch_d_setup(const Grid &g, const int *et, const double *ke, uint16_t *code, float *tab, hipStream_t st);
-// AP = A P and the (p, Ap) partials part1[field * stencil_blocks(g) + block]
+size_t stencil_bytes(const Grid &g);  // device bytes of an operator
+// partials per field of a stencil kernel (at most ..._max, whatever the phases)
+int stencil_blocks(const Grid &g, const StencilOp &op);
+int stencil_blocks_max(const Grid &g);
+// fills buf (stencil_bytes) and *op; ke: the FP64 element stiffness per phase (3 x 576); synchronizes st
+hipError_t launch_d_setup(const Grid &g, const int *et, const double *ke, void *buf, StencilOp *op, hipStream_t st);
+// AP = A P and the (p, Ap) partials part1[field * stencil_blocks + block]
 hipError_t launch_d_spmv(const Grid &g, int K, const StencilOp &op, const float *P, float *AP, double *part1,
                          const void *state, hipStream_t st);
+// the multilevel preconditioner of a K-field system (*out = nullptr: no
+// coarse grid, or MPPD_COARSE=0); P and AP are its scratch during the set-up
+int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
+                 float *P, float *AP, hipStream_t st, VCycleDev **out);
+void vcycle_free(VCycleDev *v);
+// OUT = M R with Z = D^-1 R given (Z may be v.z), T a work vector, and the (r, OUT) partials
+// pr[field * stencil_blocks + block]; OUT may be Z or T, not v.z
+hipError_t launch_vcycle(const Grid &g, int K, const VCycleDev &v, const StencilOp &op, const float *kinv,
+                         const float *R, const float *Z, float *T, float *OUT, double *pr, const void *cur,
+                         hipStream_t st);
+// after launch_m_resid: the inner CG's start direction P = M R and the state's (r, z)
+hipError_t launch_v_start(const Grid &g, int K, const VCycleDev &v, const StencilOp &op, const float *kinv,
+                          const float *R, float *P, float *AP, void *state, hipStream_t st);
 
 // ---------------- launchers (mixed.hip): K right-hand sides, K in {4,8,12,16} ----------------
 size_t mixed_matrix_floats(const Grid &g);
@@ -281,7 +327,9 @@ hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float 
 // stencil dictionary op)
 hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                          float *AP, double *part, void *state, int parity, hipStream_t st,
-                         const CoarseDev *coarse = nullptr);
+                         const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr);
+// s0's (r, z) from partials prz[field * row + i]
+hipError_t launch_c_rzfix(int K, int row, const double *prz, void *state, hipStream_t st);
 // blocks per component of the vector kernels (the partial tables' stride)
 size_t coarse_vec_blocks(const Grid &g);
 hipError_t launch_m_accum(const Grid &g, int K, const float *X, double *U, hipStream_t st);

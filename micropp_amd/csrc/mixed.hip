@@ -519,14 +519,9 @@ __global__ void __launch_bounds__(256) k_m_spmv(Grid g, int NP, int nsl, int per
   // registers from row 4
   double pap[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const float4 pc = pg[(size_t)d * KG * NP + n];
-    AP[(size_t)(d * KG + grp) * NP + n] = make_float4(acc[d][0], acc[d][1], acc[d][2], acc[d][3]);
-    pap[0] += (double)pc.x * acc[d][0];
-    pap[1] += (double)pc.y * acc[d][1];
-    pap[2] += (double)pc.z * acc[d][2];
-    pap[3] += (double)pc.w * acc[d][3];
-  }
+  for (int d = 0; d < 3; ++d)
+    apply_out<kApplyCg>(pg[(size_t)d * KG * NP + n], make_float4(acc[d][0], acc[d][1], acc[d][2], acc[d][3]), nullptr,
+                        nullptr, 0.0f, AP, (size_t)(d * KG + grp) * NP + n, 0, pap);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const double s = wave_sum_dpp(pap[r]);
@@ -543,15 +538,18 @@ __global__ void __launch_bounds__(256) k_m_spmv(Grid g, int NP, int nsl, int per
 // [(field * 3 + d) * gridDim.x + block] (the 3 gridDim.x partials of a field
 // contiguous; pr = pz + 3 K gridDim.x).  X is advanced in k_m_pupd, which
 // reads P anyway.
-// COARSE (two-level preconditioner): the block holds whole x-lines, lpb of
-// them (lpb nx <= kVecNodes nodes), so that it can also restrict its new r
+// PC: kPcCoarse (two-level preconditioner): the block holds whole x-lines, lpb
+// of them (lpb nx <= kVecNodes nodes), so that it can also restrict its new r
 // along x from LDS: T1 as k_c_rx writes it, the same sums in the same order.
 // Its partials then number ceil(ny nz / lpb) per (field, d) (gridDim.x).
-template <int K, bool COARSE>
+// kPcCycle (multilevel preconditioner): z = kinv r goes to T1 (R's layout).
+enum { kPcJacobi = 0, kPcCoarse = 1, kPcCycle = 2 };
+template <int K, int PC>
 __global__ void __launch_bounds__(kRedThreads) k_m_upd(int NP, int nsl, const double *part1, const float *kinv,
                                                        const float4 *AP, float4 *R, double *pz, double *pr,
                                                        MState *cur, Grid g, CGrid cg, int lpb, float4 *T1) {
   __shared__ double lds[4 * 8];
+  constexpr bool COARSE = PC == kPcCoarse;
   __shared__ double al_s[4];
   __shared__ float4 rl[COARSE ? kVecNodes : 1];
   __shared__ float wt[COARSE ? kCoarseMaxLine : 1];
@@ -612,6 +610,7 @@ __global__ void __launch_bounds__(kRedThreads) k_m_upd(int NP, int nsl, const do
     r.w -= al.w * ap.w;
     R[o] = r;
     if constexpr (COARSE) rl[n - nbeg] = r;
+    if constexpr (PC == kPcCycle) T1[o] = make_float4(kv * r.x, kv * r.y, kv * r.z, kv * r.w);
     const float rv[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -633,7 +632,7 @@ __global__ void __launch_bounds__(kRedThreads) k_m_upd(int NP, int nsl, const do
     const size_t o = ((size_t)(r0 + (q & 3)) * 3 + d) * gridDim.x + blockIdx.x;
     if (q < 4)
       pz[o] = t;
-    else if (!COARSE)  // the coarse variant's (r, z) partials come from k_c_zdot
+    else if (PC == kPcJacobi)  // else the (r, z) partials come from the kernel that forms z
       pr[o] = t;
   }
   if constexpr (COARSE) {
@@ -959,11 +958,11 @@ __global__ void __launch_bounds__(kZdotThreads) k_c_zdot(Grid g, CGrid cg, int N
   }
 }
 
-// start: the state's (r, z) of every field from k_c_zdot<K, true>'s partials
+// start: the state's (r, z) of every field from the partials (row per field)
+// of the kernel that formed z
 template <int K>
-__global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int nbx, const double *prz, MState *s0) {
-  const size_t row = (size_t)3 * nbx;
-  const double rz = rows_sum<K>(prz, row, (int)row);
+__global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int row, const double *prz, MState *s0) {
+  const double rz = rows_sum<K>(prz, row, row);
   if (threadIdx.x < K) s0->rz[threadIdx.x] = rz;
 }
 
@@ -972,12 +971,12 @@ __global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int nbx, const double *
 // its four fields in the same fixed order (so all blocks agree bit for bit),
 // and block (0, 0) sums all fields and writes the state of the next iteration
 // (beta, ||z||, stop flags, iteration count).  Grid as k_m_upd.
-// COARSE (two-level preconditioner): z is read from Z (k_c_zdot) instead of
-// being formed from kinv and R.
+// COARSE (two-level and multilevel preconditioners): z is read from Z instead
+// of being formed from kinv and R.  rowz, row: partials per field of pz, pr.
 template <int K, bool COARSE>
 __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kinv, const float4 *R, const float4 *Z,
-                                                        float4 *P, float4 *X, const double *pz, int nbz,
-                                                        const double *pr, const MState *cur,
+                                                        float4 *P, float4 *X, const double *pz, int rowz,
+                                                        const double *pr, int row, const MState *cur,
                                                         MState *nxt) {
   constexpr int KG = K / 4;
   __shared__ double beta_s[kMaxRhs];
@@ -992,15 +991,14 @@ __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kin
     }
     return;
   }
-  const size_t row = (size_t)3 * gridDim.x, rowz = (size_t)3 * nbz;  // (r, z) / (z, z) partials per field
   // The block's (z, z) / (r, z) partials are loaded first (block (0, 0) sums
   // every field's after its vectors), then this block's vectors (rows
   // clamped; the update skips n >= NP), which stay in flight while the
   // partials are summed.
   double szz[4] = {}, srz[4] = {};
   if (!head) {
-    rows_load<4>(pz + r0 * rowz, rowz, (int)rowz, szz);
-    rows_load<4>(pr + r0 * row, row, (int)row, srz);
+    rows_load<4>(pz + (size_t)r0 * rowz, rowz, rowz, szz);
+    rows_load<4>(pr + (size_t)r0 * row, row, row, srz);
   }
   asm volatile("" ::: "memory");
   constexpr int J = kVecNodes / 256;
@@ -1023,8 +1021,8 @@ __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kin
   }
   const int its = cur->its + 1;
   if (head) {
-    const double zz = rows_sum<K>(pz, rowz, (int)rowz);
-    const double rz = rows_sum<K>(pr, row, (int)row);
+    const double zz = rows_sum<K>(pz, rowz, rowz);
+    const double rz = rows_sum<K>(pr, row, row);
     const int r = threadIdx.x;
     if (r < K) {
       const MStep o = m_step(cur, r, zz, rz);
@@ -1538,7 +1536,8 @@ size_t mixed_partials(const Grid &g, int K) {
   const MLaunch s = mshape(g);
   const size_t resid = std::max((size_t)s.nb, (size_t)g.nrow_pad / 256) * 3 * K;  // k_m_resid / k_m_resid_ell
   const size_t ave = (size_t)nblk(g.nelem, 256) * 6 * K;
-  const size_t iter = (size_t)K * s.nsl + 2 * (size_t)3 * K * (s.NP / 256);
+  // (p, Ap), (z, z) and (r, z) of an iteration
+  const size_t iter = 2 * (size_t)K * std::max(s.nsl, stencil_blocks_max(g)) + 2 * (size_t)3 * K * (s.NP / 256);
   return std::max(std::max(resid, ave), iter);
 }
 hipError_t launch_m_kinv(const Grid &g, const int *et, const double *ke, float *kinv, hipStream_t st) {
@@ -1602,53 +1601,60 @@ static void coarse_solve(const Grid &g, const MLaunch &s, const CoarseDev &c, co
                      cur);
 }
 
-hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
-                         float *AP, double *part, void *state, int parity, hipStream_t st, const CoarseDev *coarse) {
+hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R,
+                         float *X, float *P, float *AP, double *part, void *state, int parity, hipStream_t st,
+                         const CoarseDev *coarse, const VCycleDev *vc) {
   const MLaunch s = mshape(g);
   MState *ms = static_cast<MState *>(state);
   MState *cur = ms + (parity & 1);
   MState *nxt = ms + ((parity + 1) & 1);
+  if (A ? K != 4 || vc : coarse != nullptr) return hipErrorInvalidValue;
   const int nbx = (int)nblk(s.NP, kVecNodes);
   // with a coarse level k_m_upd runs on blocks of whole x-lines (lpb a block, nbu blocks)
   const int lpb = coarse ? kVecNodes / g.nx : 0;
   const int nbu = coarse ? (g.ny * g.nz + lpb - 1) / lpb : nbx;
-  const int np1 = A ? s.nsl : stencil_blocks(g);          // (p, Ap) partials per field
+  const int np1 = A ? s.nsl : stencil_blocks(g, op);          // (p, Ap) partials per field
   double *part1 = part;                                   // K x np1
   double *pz = part + (size_t)K * np1;                    // 3K x nbu: (z, z)
-  double *pr = pz + (size_t)3 * K * std::max(nbx, nbu);   // 3K x nbx: (r, z)
+  double *pr = pz + (size_t)3 * K * std::max(nbx, nbu);   // 3K x nbx (multilevel: K x stencil_blocks): (r, z)
   const dim3 vgrid(nbx, 3 * K / 4);
-  const CGrid cg = coarse ? coarse->cg : CGrid{};
-  if (A) {
-    if (K != 4) return hipErrorInvalidValue;
+  const float4 *r4 = reinterpret_cast<const float4 *>(R), *ap4 = reinterpret_cast<const float4 *>(AP);
+  float4 *x4 = reinterpret_cast<float4 *>(X), *p4 = reinterpret_cast<float4 *>(P);
+  hipError_t e = hipSuccess;
+  if (A)
     hipLaunchKernelGGL(k_m_spmv<4>, dim3(8 * s.pers), dim3(64), 0, st, g, s.NP, s.nsl, s.pers,
-                       reinterpret_cast<const float4 *>(A), reinterpret_cast<const float4 *>(P),
-                       reinterpret_cast<float4 *>(AP), part1, cur);
-  } else {
-    const hipError_t e = launch_d_spmv(g, K, op, P, AP, part1, cur, st);
-    if (e != hipSuccess) return e;
+                       reinterpret_cast<const float4 *>(A), p4, reinterpret_cast<float4 *>(AP), part1, cur);
+  else
+    e = launch_d_spmv(g, K, op, P, AP, part1, cur, st);
+  if (e != hipSuccess) return e;
+  if (coarse) {
+    // R -= alpha AP with the x-restriction of the new R; then the coarse
+    // solve, z and (r, z) with the coarse correction (its partials in
+    // place of the Jacobi (r, z) ones), and the p-update from z
+    const CGrid cg = coarse->cg;
+    hipLaunchKernelGGL((k_m_upd<4, kPcCoarse>), dim3(nbu, 3), dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
+                       reinterpret_cast<float4 *>(R), pz, pr, cur, g, cg, lpb, reinterpret_cast<float4 *>(coarse->t1));
+    coarse_solve<4>(g, s, *coarse, R, cur, st, false);
+    hipLaunchKernelGGL((k_c_zdot<4, false>), vgrid, dim3(kZdotThreads), 0, st, g, cg, s.NP, kinv, r4,
+                       reinterpret_cast<const float4 *>(coarse->ec), reinterpret_cast<float4 *>(coarse->z), pr, cur);
+    hipLaunchKernelGGL((k_m_pupd<4, true>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4,
+                       reinterpret_cast<const float4 *>(coarse->z), p4, x4, pz, 3 * nbu, pr, 3 * nbx, cur, nxt);
+    return hipGetLastError();
   }
   MPP_K_DISPATCH(K, {
-    if (coarse) {
-      // R -= alpha AP with the x-restriction of the new R; then the coarse
-      // solve, z and (r, z) with the coarse correction (its partials in
-      // place of the Jacobi (r, z) ones), and the p-update from z
-      hipLaunchKernelGGL((k_m_upd<KK, true>), dim3(nbu, 3 * K / 4), dim3(kRedThreads), 0, st, s.NP, np1, part1,
-                         kinv, reinterpret_cast<const float4 *>(AP), reinterpret_cast<float4 *>(R), pz, pr, cur, g,
-                         cg, lpb, reinterpret_cast<float4 *>(coarse->t1));
-      coarse_solve<KK>(g, s, *coarse, R, cur, st, false);
-      hipLaunchKernelGGL((k_c_zdot<KK, false>), vgrid, dim3(kZdotThreads), 0, st, g, cg, s.NP, kinv,
-                         reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(coarse->ec),
-                         reinterpret_cast<float4 *>(coarse->z), pr, cur);
-      hipLaunchKernelGGL((k_m_pupd<KK, true>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv,
-                         reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(coarse->z),
-                         reinterpret_cast<float4 *>(P), reinterpret_cast<float4 *>(X), pz, nbu, pr, cur, nxt);
+    if (vc) {
+      // R -= alpha AP and D^-1 R, then z = M R into AP (with the (r, z)
+      // partials), and the p-update from it
+      hipLaunchKernelGGL((k_m_upd<KK, kPcCycle>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
+                         reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, reinterpret_cast<float4 *>(vc->z));
+      if ((e = launch_vcycle(g, K, *vc, op, kinv, R, vc->z, AP, AP, pr, cur, st)) != hipSuccess) return e;
+      hipLaunchKernelGGL((k_m_pupd<KK, true>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, ap4, p4, x4, pz,
+                         3 * nbx, pr, np1, cur, nxt);
     } else {
-      hipLaunchKernelGGL((k_m_upd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv,
-                         reinterpret_cast<const float4 *>(AP), reinterpret_cast<float4 *>(R), pz, pr, cur, g, cg,
-                         0, nullptr);
-      hipLaunchKernelGGL((k_m_pupd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv,
-                         reinterpret_cast<const float4 *>(R), nullptr, reinterpret_cast<float4 *>(P),
-                         reinterpret_cast<float4 *>(X), pz, nbx, pr, cur, nxt);
+      hipLaunchKernelGGL((k_m_upd<KK, kPcJacobi>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
+                         reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, nullptr);
+      hipLaunchKernelGGL((k_m_pupd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, nullptr, p4, x4, pz,
+                         3 * nbx, pr, 3 * nbx, cur, nxt);
     }
   });
   return hipGetLastError();
@@ -1656,17 +1662,20 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &
 
 hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float *kinv, const float *R, float *P,
                           void *state, hipStream_t st) {
+  if (K != 4) return hipErrorInvalidValue;
   const MLaunch s = mshape(g);
   MState *s0 = static_cast<MState *>(state);
   const int nbx = (int)nblk(s.NP, kVecNodes);
-  const dim3 vgrid(nbx, 3 * K / 4);
-  MPP_K_DISPATCH(K, {
-    coarse_solve<KK>(g, s, c, R, s0, st);
-    hipLaunchKernelGGL((k_c_zdot<KK, true>), vgrid, dim3(kZdotThreads), 0, st, g, c.cg, s.NP, kinv,
-                       reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(c.ec),
-                       reinterpret_cast<float4 *>(P), c.prz, s0);
-    hipLaunchKernelGGL(k_c_rzfix<KK>, dim3(1), dim3(kRedThreads), 0, st, nbx, c.prz, s0);
-  });
+  coarse_solve<4>(g, s, c, R, s0, st);
+  hipLaunchKernelGGL((k_c_zdot<4, true>), dim3(nbx, 3), dim3(kZdotThreads), 0, st, g, c.cg, s.NP, kinv,
+                     reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(c.ec),
+                     reinterpret_cast<float4 *>(P), c.prz, s0);
+  return launch_c_rzfix(K, 3 * nbx, c.prz, state, st);
+}
+
+hipError_t launch_c_rzfix(int K, int row, const double *prz, void *state, hipStream_t st) {
+  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_c_rzfix<KK>, dim3(1), dim3(kRedThreads), 0, st, row, prz,
+                                       static_cast<MState *>(state)));
   return hipGetLastError();
 }
 

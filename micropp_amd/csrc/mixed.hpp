@@ -102,6 +102,43 @@ __device__ __forceinline__ double rows_sum(const double *part, size_t stride, in
 }
 
 // ---------------------------------------------------------------------------
+// What an operator kernel does with y = A P at a node (one direction, four
+// fields; pc = P there): see k_m_spmv and k_d_apply.
+// ---------------------------------------------------------------------------
+enum ApplyMode { kApplyCg, kApplyRes, kApplyPost, kApplyPow };
+template <int MODE>
+__device__ __forceinline__ void apply_out(const float4 &pc, const float4 &y, const float4 *R, const float *kinv,
+                                          float omega, float4 *OUT, size_t o, size_t ok, double (&s)[4]) {
+  float4 v = y;
+  if constexpr (MODE == kApplyRes || MODE == kApplyPost) {
+    const float4 r = R[o];
+    if constexpr (MODE == kApplyRes) {
+      v = make_float4(r.x - omega * y.x, r.y - omega * y.y, r.z - omega * y.z, r.w - omega * y.w);
+    } else {
+      const float w = omega * kinv[ok];
+      v = make_float4(pc.x + w * (r.x - y.x), pc.y + w * (r.y - y.y), pc.z + w * (r.z - y.z), pc.w + w * (r.w - y.w));
+      s[0] += (double)r.x * v.x;
+      s[1] += (double)r.y * v.y;
+      s[2] += (double)r.z * v.z;
+      s[3] += (double)r.w * v.w;
+    }
+  } else if constexpr (MODE == kApplyCg) {
+    s[0] += (double)pc.x * y.x;
+    s[1] += (double)pc.y * y.y;
+    s[2] += (double)pc.z * y.z;
+    s[3] += (double)pc.w * y.w;
+  } else {  // kApplyPow
+    const float w = kinv[ok];
+    v = make_float4(w * y.x, w * y.y, w * y.z, w * y.w);
+    s[0] += (double)v.x * y.x;
+    s[1] += (double)v.y * y.y;
+    s[2] += (double)v.z * y.z;
+    s[3] += (double)v.w * y.w;
+  }
+  OUT[o] = v;
+}
+
+// ---------------------------------------------------------------------------
 // The element blocks (phase table or per element) around interior node n:
 // blk[q] the 24x24 block of element q = (a*2+b)*2+c, la[q] the node's local
 // index in it.  Entry (fi, fj) of the node block towards neighbour nb is the

@@ -713,7 +713,7 @@ constexpr int kMaxRhsFields = 16;  // largest K of an msolver
 struct mppd_msolver {
   mppd_rve *r = nullptr;
   int K = 0;
-  CoarseDev *coarse = nullptr;  // two-level preconditioner of the inner CG (null: Jacobi alone)
+  VCycleDev *vc = nullptr;  // multilevel preconditioner of the inner CG (null: Jacobi alone)
   hipStream_t st = nullptr;
   double *ke = nullptr;         // phase table 3 x 576 (FP64)
   material_base *mats_d = nullptr;
@@ -767,8 +767,7 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
     const size_t o_U = carve(nv * sizeof(double)), o_eps = carve(16 * 6 * sizeof(double)),
                  o_sig = carve(16 * 6 * sizeof(double)), o_part = carve(mixed_partials(g, nrhs) * sizeof(double));
     const size_t o_state = carve(mixed_state_bytes()), o_act = carve(kMaxRhsFields * sizeof(int));
-    const size_t zeroed = off, o_code = carve(stencil_code_len(g) * sizeof(uint16_t)),
-                 o_tab = carve(stencil_table_len() * sizeof(float));
+    const size_t zeroed = off, o_op = carve(stencil_bytes(g));
     e = hipMalloc(&m->arena, off);
     if (e == hipSuccess) e = hipMemsetAsync(m->arena, 0, zeroed, st);
     if (e != hipSuccess) {
@@ -789,10 +788,6 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
     m->part = reinterpret_cast<double *>(base + o_part);
     m->state = base + o_state;
     m->act_d = reinterpret_cast<int *>(base + o_act);
-    uint16_t *code = reinterpret_cast<uint16_t *>(base + o_code);
-    float *tab = reinterpret_cast<float *>(base + o_tab);
-    m->op.code = code;
-    m->op.tab = tab;
     off = 0;
     const size_t h_state = carve(mixed_state_bytes()), h_act = carve(kMaxRhsFields * sizeof(int)),
                  h_eps = carve(16 * 6 * sizeof(double)), h_sig = carve(16 * 6 * sizeof(double));
@@ -808,14 +803,14 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
     if (e == hipSuccess) e = hipMemcpy(m->mats_d, r->mats, 3 * sizeof(material_base), hipMemcpyHostToDevice);
     // element stiffness per phase (FP64, the plain path's kernel), then the FP32 operator and Jacobi weights
     if (e == hipSuccess) e = launch_elem_ke(g, r->bmat, r->mats_d, r->et, nullptr, nullptr, 1, m->ke, m->st);
-    if (e == hipSuccess) e = launch_d_setup(g, r->et, m->ke, code, tab, m->st);
+    if (e == hipSuccess) e = launch_d_setup(g, r->et, m->ke, base + o_op, &m->op, m->st);
     if (e == hipSuccess) e = launch_m_kinv(g, r->et, m->ke, m->kinv, m->st);
     if (e == hipSuccess) e = hipStreamSynchronize(m->st);
     if (e != hipSuccess) {
       rc = hip_fail(e, "msolver set-up");
       break;
     }
-    rc = coarse_setup(g, r->et, m->ke, nrhs, m->st, &m->coarse);
+    rc = vcycle_setup(g, nrhs, r->et, m->ke, m->op, m->kinv, m->P, m->AP, m->st, &m->vc);
   } while (0);
   if (rc) {
     mppd_msolver_destroy(m);
@@ -831,7 +826,7 @@ int mppd_msolver_destroy(mppd_msolver *m) {
   for (void *p : {m->arena, (void *)m->F, (void *)m->G, (void *)m->apart, (void *)m->adj_d}) dfree(p);
   for (void *p : {m->harena, (void *)m->adj_h})
     if (p) (void)hipHostFree(p);
-  coarse_free(m->coarse);
+  vcycle_free(m->vc);
   if (m->st) (void)hipStreamDestroy(m->st);
   delete m;
   return MPPD_OK;
@@ -850,9 +845,12 @@ int mppd_msolver_destroy(mppd_msolver *m) {
 static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                        float *AP, double *part, void *state, void *state_h, int max_inner, hipStream_t st,
                        int *its_out, bool *finite = nullptr, bool stop_on_stall = false,
-                       const CoarseDev *coarse = nullptr) {
+                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr) {
   int queued = 0, its = 0, done = 0, its_prev = 0;
-  int chunk = 32;
+  // (with the multilevel preconditioner a solve takes about 10 iterations of
+  // up to 13 launches each, so few are queued past the end)
+  int chunk = vc ? 8 : 32;
+  const int slack = vc ? 0 : 2, least = vc ? 1 : 4;
   std::vector<double> pn_prev(K, 0.0);
   for (int k = 0; k < K; ++k) {
     double target;
@@ -862,7 +860,7 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
     const int nq = std::min(chunk, max_inner - queued);
     if (nq <= 0) break;
     for (int i = 0; i < nq; ++i)
-      MPP_HIP(launch_m_iter(g, K, A, op, kinv, R, X, P, AP, part, state, queued + i, st, coarse));
+      MPP_HIP(launch_m_iter(g, K, A, op, kinv, R, X, P, AP, part, state, queued + i, st, coarse, vc));
     queued += nq;
     MPP_HIP(hipMemcpyAsync(state_h, state, mixed_state_bytes(), hipMemcpyDeviceToHost, st));
     MPP_HIP(hipStreamSynchronize(st));
@@ -879,13 +877,13 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
       if (dit > 0 && pn_prev[k] > 0 && pnk > 0 && pnk < pn_prev[k]) {
         const double rate = std::log(pnk / pn_prev[k]) / dit;
         const double est = std::log(target / pnk) / rate;
-        if (std::isfinite(est)) need = (int)std::ceil(est) + 2;
+        if (std::isfinite(est)) need = (int)std::ceil(est) + slack;
       }
       next = std::max(next, need);
       pn_prev[k] = pnk;
     }
     its_prev = its;
-    chunk = std::max(4, std::min(256, next));
+    chunk = std::max(least, std::min(256, next));
     // FP32 CG that no longer reduces ||z|| by 10% over a chunk of >= 32
     // iterations (rounding, or a nonsymmetric Newton tangent) is stopped: the
     // caller's FP64 defect correction restarts it from the true residual
@@ -925,13 +923,13 @@ static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, co
   for (;;) {
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, F, m->kinv, m->R, m->X, m->P, m->part, outer == 0,
                            p->rel_tol, p->abs_tol, p->inner_tol, p->max_inner_its, m->state, m->st));
-    if (m->coarse) MPP_HIP(launch_c_start(g, K, *m->coarse, m->kinv, m->R, m->P, m->state, m->st));
+    if (m->vc) MPP_HIP(launch_v_start(g, K, *m->vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
     if (all_conv || outer >= p->max_outer) break;
     int its = 0, rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
-                                  p->max_inner_its, m->st, &its, nullptr, false, m->coarse);
+                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, m->vc);
     if (rc) return rc;
     inner_total += its;
     MPP_HIP(launch_m_accum(g, K, m->X, m->U, m->st));
@@ -1063,7 +1061,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
     MPP_HIP(hipMemcpyAsync(m->act_d, m->act_h, K * sizeof(int), hipMemcpyHostToDevice, m->st));
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, nullptr, m->kinv, m->R, m->X, m->P, m->part, first,
                            p->cg_rel_tol, p->cg_abs_tol, inner_tol, max_inner, m->state, m->st, m->act_d));
-    if (m->coarse) MPP_HIP(launch_c_start(g, K, *m->coarse, m->kinv, m->R, m->P, m->state, m->st));
+    if (m->vc) MPP_HIP(launch_v_start(g, K, *m->vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_norms(m->state_h, K, cflag.data(), rn.data(), rn0.data());
@@ -1101,7 +1099,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
       if (all_conv || outer >= max_outer) break;
       int inner = 0;
       if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
-                            m->st, &inner, nullptr, false, m->coarse)))
+                            m->st, &inner, nullptr, false, nullptr, m->vc)))
         return rc;
       inner_total += inner;
       ++outer_total;
@@ -1362,7 +1360,7 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
   MPP_HIP(launch_m_setbc(g, K, m->eps_d, m->U, m->st));
   MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, nullptr, m->kinv, m->R, m->X, m->P, m->part, 1, 0.0, 0.0, 0.0,
                          iters + 1, m->state, m->st));
-  if (m->coarse) MPP_HIP(launch_c_start(g, K, *m->coarse, m->kinv, m->R, m->P, m->state, m->st));
+  if (m->vc) MPP_HIP(launch_v_start(g, K, *m->vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
   hipEvent_t ev[3];
   for (auto &x : ev) MPP_HIP(hipEventCreate(&x));
   hipError_t e = hipEventRecord(ev[0], m->st);
@@ -1370,7 +1368,7 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
     e = launch_d_spmv(g, K, m->op, m->P, m->AP, m->part, m->state, m->st);
   if (e == hipSuccess) e = hipEventRecord(ev[1], m->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_m_iter(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, i, m->st, m->coarse);
+    e = launch_m_iter(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, i, m->st, nullptr, m->vc);
   if (e == hipSuccess) e = hipEventRecord(ev[2], m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
   float ms1 = 0.f, ms2 = 0.f;
@@ -1385,7 +1383,7 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
 
 int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h) {
   if (!m || !dims) return fail(MPPD_ERR_ARG, "bad msolver_coarse arguments");
-  const CoarseDev *c = m->coarse;
+  const VCycleDev *c = m->vc;
   const CGrid cg = c ? c->cg : CGrid{};
   const int v[7] = {cg.nc, cg.hx, cg.hy, cg.hz, cg.mx, cg.my, cg.mz};
   for (int i = 0; i < 7; ++i) dims[i] = v[i];
