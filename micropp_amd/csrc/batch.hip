@@ -140,7 +140,7 @@ __device__ __forceinline__ const double *cg_matrix(const BRve &R, const int *a0o
 __global__ void __launch_bounds__(256) kb_cg_init(const BRve *rv, const int *map, const int *act, const int *blk0,
                                                   const int *a0on) {
   MPP_BATCH_PROLOGUE(map)
-  cg_init_body(R.g, blockIdx.x - blk0[rid], cg_matrix(R, a0on, rid), R.b, R.x, R.r, R.z, R.p, R.kinv, R.part);
+  cg_init_body(R.g, blockIdx.x - blk0[rid], cg_matrix(R, a0on, rid), R.b, R.x, R.r, R.kinv, R.part);
 }
 
 // one block per RVE; an inactive RVE's CG starts (and stays) done
@@ -171,23 +171,24 @@ __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int *ma
   if (b >= nb) return;
   const int rid = map[b];
   const BRve &R = rv[rid];
-  // both matrices are assembled here: the stencil columns follow from the grid
-  cg_step1_body<CH, true>(R.g, b - blk0[rid], nullptr, cg_matrix(R, a0on, rid), R.p, R.Ap, R.part,
-                          R.cg + (parity & 1));
+  // vals and a0 are assembled here: the stencil columns follow from the grid
+  const int k = parity & 1;
+  const double *A = cg_matrix(R, a0on, rid);
+  cg_step1_body64<CH>(R.g, b - blk0[rid], R.nb_row, A, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap, R.part, R.cg + k,
+                      R.cg + (k ^ 1));
 }
 
 __global__ void __launch_bounds__(256) kb_cg_step2(const BRve *rv, const int *map, const int *blk0, int parity) {
   const int rid = map[blockIdx.x];
   const BRve &R = rv[rid];
-  cg_step2_body(blockIdx.x - blk0[rid], R.nb_row, R.x, R.r, R.z, R.p, R.Ap, R.kinv, R.part, R.part + R.nb_row,
-                R.cg + (parity & 1));
+  const int n = (parity & 1) ^ 1;
+  cg_step2_body64(blockIdx.x - blk0[rid], R.nb_row, R.x, R.r, R.p[n], R.Ap, R.kinv, R.part, R.cg + n);
 }
 
-__global__ void __launch_bounds__(256) kb_cg_step3(const BRve *rv, const int *map, const int *blk0, int parity) {
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  cg_step3_body(blockIdx.x - blk0[rid], R.nb_row, R.z, R.p, R.part, R.part + R.nb_row, R.cg + (parity & 1),
-                R.cg + ((parity + 1) & 1));
+// one block per RVE
+__global__ void __launch_bounds__(256) kb_cg_tail(const BRve *rv) {
+  const BRve &R = rv[blockIdx.x];
+  cg_tail_body(R.part + R.nb_row, R.nb_row, R.cg);
 }
 
 // uw += x
@@ -366,8 +367,8 @@ __global__ void __launch_bounds__(256) kb_m_step1(const BRve *rv, const int *map
   if (b >= nb) return;
   const int rid = map[b];
   const BRve &R = rv[rid];
-  cg_step1_body<CH, true>(R.g, b - blk0[rid], nullptr, (const float *)R.vals32, (const float *)R.p32, R.Ap32,
-                          R.part, R.cg + (parity & 1));
+  cg_step1_body<CH>(R.g, b - blk0[rid], (const float *)R.vals32, (const float *)R.p32, R.Ap32, R.part,
+                    R.cg + (parity & 1));
 }
 
 __global__ void __launch_bounds__(256) kb_m_step2(const BRve *rv, const int *map, const int *blk0, int parity) {
@@ -611,7 +612,10 @@ hipError_t launch_b_cg_iter(const BLaunch &L, int parity, hipStream_t st) {
   hipError_t e = launch_b_spmv(L, L.spmv_shape, parity, st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kb_cg_step2, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, parity);
-  hipLaunchKernelGGL(kb_cg_step3, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, parity);
+  return hipGetLastError();
+}
+hipError_t launch_b_cg_tail(const BLaunch &L, hipStream_t st) {
+  hipLaunchKernelGGL(kb_cg_tail, dim3(L.nrve), dim3(256), 0, st, L.rv);
   return hipGetLastError();
 }
 hipError_t launch_b_axpy(const BLaunch &L, hipStream_t st) {

@@ -22,7 +22,7 @@ struct BRve {
   double *ke;                  // 576 per element, or per phase in phase mode
   double *be;                  // 24 per element
   double *uw, *u_n, *u_k;      // working / converged / current displacements
-  double *x, *r, *z, *p, *Ap, *kinv, *b;
+  double *x, *r, *p[2], *Ap, *kinv, *b;
   double *vars_n, *vars_k, *vars_aux;
   double *part;                // partials: max(3 nb_row, 6 nb_elem)
   CgState *cg;                 // ping-pong pair
@@ -108,6 +108,8 @@ hipError_t launch_b_vars_new(const BLaunch &L, int *flags, hipStream_t st);
 hipError_t launch_b_cg_init(const BLaunch &L, double min_err, double rel_err, int max_its, hipStream_t st);
 // one CG iteration of every RVE (inactive / converged RVEs return at once)
 hipError_t launch_b_cg_iter(const BLaunch &L, int parity, hipStream_t st);
+// the sums of the last of an even number of iterations into cg[0]
+hipError_t launch_b_cg_tail(const BLaunch &L, hipStream_t st);
 // the CG SpMV alone in one of kSpmvShapes shapes: shape = 3 * xcd + c, with
 // c = 0, 1, 2 for 9, 27, 81 slots in flight and xcd = 1 for the XCD-grouped
 // block order (timing of the autotuner; same results in every shape)
@@ -126,7 +128,7 @@ hipError_t launch_b_nt_start(const BLaunch &L, const int *on, const double *norm
 // initial matrix while its < its_with_A0 when has_a0); applied = pend = 0
 hipError_t launch_b_nt_prepare(const BLaunch &L, BNewton *nst, int has_a0, int its_with_A0, int *act, int *ke,
                                int *gather, int *a0on, int *pend, hipStream_t st);
-// finish the RVEs whose CG has stopped (state cg[0]: the host queues an even
+// (after launch_b_cg_tail) finish the RVEs whose CG has stopped (state cg[0]: the host queues an even
 // number of iterations) and whose correction is not yet applied: uw += x
 // (rows), then applied = pend = 1 and sits += CG iterations, then (with
 // L.act = pend) the residual b and its norm, then its += 1 and the test of

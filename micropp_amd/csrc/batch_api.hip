@@ -246,6 +246,7 @@ int cg_batch(mppd_batch *B, const std::vector<int> &on, std::vector<int> &its) {
     queued += reps * G;
     B->cg_queued += reps * G;
     B->graph_launches += reps;
+    MPP_HIP(launch_b_cg_tail(B->launch(M_MAIN), B->st));
     if ((rc = read_cg(B))) return rc;
     all = true;
     int next = 0;
@@ -505,7 +506,8 @@ int capture_newton_graphs(mppd_batch *B) {
       if (e == hipSuccess) e = launch_b_mat(L, B->mask_d[M_KE], B->mask_d[M_GATHER], B->st);
       if (e == hipSuccess) e = launch_b_cg_init(L, p.cg_abs_tol, p.cg_rel_tol, p.cg_max_its, B->st);
     } else {
-      e = launch_b_nt_finish(L, newton_test(B), B->nst_d, B->pend_d, B->norms_d, B->st);
+      e = launch_b_cg_tail(L, B->st);
+      if (e == hipSuccess) e = launch_b_nt_finish(L, newton_test(B), B->nst_d, B->pend_d, B->norms_d, B->st);
     }
     hipGraph_t graph = nullptr;
     const hipError_t e2 = hipStreamEndCapture(B->st, &graph);
@@ -684,6 +686,7 @@ int tune_spmv(mppd_batch *B, bool fp32 = false) {
   for (auto &c : live) {
     c = CgState{};
     c.max_its = 1;
+    c.fresh = 1;
   }
   MPP_HIP(hipMemcpy(B->cg, live.data(), sizeof(CgState) * live.size(), hipMemcpyHostToDevice));
   hipEvent_t e0, e1;
@@ -945,7 +948,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     MPP_HIP(hipMemcpy(B->map_d[k], map[k].data(), sizeof(int) * map[k].size(), hipMemcpyHostToDevice));
     MPP_HIP(hipMemcpy(B->blk0_d[k], blk0[k].data(), sizeof(int) * n, hipMemcpyHostToDevice));
   }
-  constexpr int kRowVecs = 10;  // uw u_n u_k x r z p Ap kinv b
+  constexpr int kRowVecs = 10;  // uw u_n u_k x r p[2] Ap kinv b
   if ((rc = dalloc(&B->vec, rows * kRowVecs))) return rc;
   if ((rc = dalloc(&B->vals, slots))) return rc;
   if ((rc = dalloc(&B->ke, kes, false))) return rc;
@@ -973,7 +976,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     R.vals = B->vals + o_slot;
     R.ke = B->ke + o_ke;
     R.be = B->be + o_be;
-    double **vecs[kRowVecs] = {&R.uw, &R.u_n, &R.u_k, &R.x, &R.r, &R.z, &R.p, &R.Ap, &R.kinv, &R.b};
+    double **vecs[kRowVecs] = {&R.uw, &R.u_n, &R.u_k, &R.x, &R.r, &R.p[0], &R.p[1], &R.Ap, &R.kinv, &R.b};
     for (int q = 0; q < kRowVecs; ++q) *vecs[q] = B->vec + rows * q + o_row;
     if (!v->all_elastic) {
       const size_t nv = (size_t)g.nelem * 8 * NVAR;
@@ -1321,6 +1324,7 @@ int mppd_batch_spmv_profile(mppd_batch *b, int fp32, int iters, double *ms, doub
   for (auto &c : live) {
     c = CgState{};
     c.max_its = 1;
+    c.fresh = 1;
   }
   MPP_HIP(hipMemcpy(b->cg, live.data(), sizeof(CgState) * live.size(), hipMemcpyHostToDevice));
   const BLaunch L = b->launch(M_MAIN);

@@ -40,7 +40,8 @@ struct Grid {
 // Jacobi-PCG scalars of one system (device resident).
 struct CgState {
   double rz, pn0, pn, alpha, beta, min_err, rel_err, pAp;
-  int its, max_its, done, pad;
+  int its, max_its, done;
+  int fresh;  // FP64 CG: the scalars hold the last step2's sums (kernels.hpp)
   unsigned cnt;
   unsigned pad2[3];
 };
@@ -238,18 +239,26 @@ hipError_t launch_elem_fields(const Grid &g, const double *bmat, const material_
 
 // ---------------- launchers (solver.hip) ----------------
 // CG state is a pair: iteration k reads state[k & 1] and writes
-// state[(k + 1) & 1] (parity = k).  part needs 3 * (nrow_pad / 256) doubles.
+// state[(k + 1) & 1] (parity = k); so are the search directions p[0], p[1].
+// part needs 3 * (nrow_pad / 256) doubles.  Before state[q & 1] is read after
+// q iterations, launch_cg_tail(.., q, ..) takes in the last one's sums.
 hipError_t launch_spmv(const Grid &g, const int *cols, const double *vals, const double *x, double *y, hipStream_t st);
-hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, double *x, double *r, double *z,
-                          double *p, double *kinv, double *part, double min_err, double rel_err, int max_its,
-                          CgState *state, hipStream_t st);
-hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, double *x, double *r, double *z,
-                          double *p, double *Ap, const double *kinv, double *part, CgState *state, int parity,
+// The working set of one Jacobi-PCG: vectors of nrow_pad doubles, the partial
+// table and the state pair.
+struct CgVecs {
+  double *x, *r, *p[2], *Ap, *kinv, *part;
+  CgState *state;
+};
+hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, const CgVecs &w, double min_err,
+                          double rel_err, int max_its, hipStream_t st);
+// step1 of an iteration; cols == nullptr: the matrix was assembled here and
+// the stencil columns are computed.  dir = false leaves out the kernel that
+// forms p where step1 does not (timing of the SpMV alone, after one call with it)
+hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
+                           hipStream_t st, bool dir = true);
+hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
                           hipStream_t st);
-hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const double *p, double *Ap,
-                           double *part, CgState *state, int parity, hipStream_t st);
-hipError_t launch_cg_step23(const Grid &g, double *x, double *r, double *z, double *p, const double *Ap,
-                            const double *kinv, double *part, CgState *state, int parity, hipStream_t st);
+hipError_t launch_cg_tail(const Grid &g, const CgVecs &w, int queued, hipStream_t st);
 hipError_t launch_axpy(int n, double a, const double *x, double *y, hipStream_t st);
 hipError_t launch_copy(int n, const double *x, double *y, hipStream_t st);
 

@@ -546,30 +546,37 @@ __device__ __forceinline__ T row_dot_grid_seg(const T *vals, const T (*seg)[kSeg
 }
 
 // ---------------------------------------------------------------------------
-// ell_solve_cgpd (src/ell.cpp:66-122), the reference recurrence in three
-// kernels per iteration:
-//   step1  Ap = A p and the per-block partials of p.Ap
+// ell_solve_cgpd (src/ell.cpp:66-122), the reference recurrence in two
+// kernels per iteration (FP64):
+//   step1  the scalars that the previous iteration's sums give (beta, the
+//          stopping test), p = z + beta p with z = k r, Ap = A p and the
+//          per-block partials of p.Ap
 //   step2  alpha = r.z / sum(partials); x += alpha p; r -= alpha Ap; z = k r;
 //          per-block partials of z.z and r.z
-//   step3  beta = sum(r.z) / r.z_old; p = z + beta p; the new scalars
-// Every block of step2/step3 re-sums all partials of its RVE in the same
-// fixed order, so every block holds identical scalars.  The scalars of
-// iteration k are read from state[k & 1] and written (by block 0 of step3)
-// to state[(k+1) & 1].  Once the stopping test holds, later iterations
-// return at once and step3 only carries the final state forward.
-// Partials: part1 = part[0 .. nb), part2 = part[nb .. 3 nb).  The steps take
-// vectors (and, in step 1, the matrix) of type T: double for the FP64 CG,
-// float for the inner CG of the mixed-precision batch, whose products and
-// partials are still formed in FP64.
+// The new p has to be read by every row's neighbours, so each block of step1
+// forms it, from k, r and the old p, for all nodes on its 9 stencil runs while
+// it stages them in LDS (about 9 times each value, the same products each
+// time), and stores its own rows' share: p lives in two vectors, read from
+// p[i & 1] and written to p[(i + 1) & 1] in iteration i.  z is not stored.
+// Every block re-sums all partials of its RVE in the same fixed order, so
+// every block holds identical scalars.  Iteration i reads state[i & 1] and
+// block 0 of its step1 writes state[(i + 1) & 1], which step2 reads.  The
+// sums of the last step2 queued are taken in by cg_tail (before the host
+// reads the state), which marks the state fresh: the next step1 then only
+// applies its beta.  Once the stopping test holds, later iterations return at
+// once and step1 only carries the final state forward.
+// Partials: part1 = part[0 .. nb), part2 = part[nb .. 3 nb).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int cg_done(const CgState &c) {
+template <typename C>
+__device__ __forceinline__ int cg_done(const C &c) {
   const bool conv = (c.pn < c.min_err) || (c.pn < c.pn0 * c.rel_err);
   return (c.its >= c.max_its || conv) ? 1 : 0;
 }
 
-// k = 1/diag; x = 0; r = b - A*0 = b; z = k r; p = z; partials of r.z, z.z
+// k = 1/diag; x = 0; r = b - A*0 = b; partials of r.z, z.z with z = k r (the
+// first step1 takes p = z)
 __device__ __forceinline__ void cg_init_body(const Grid &g, int lb, const double *vals, const double *b, double *x,
-                                             double *r, double *z, double *p, double *kinv, double *part) {
+                                             double *r, double *kinv, double *part) {
 #pragma clang fp contract(off)
   __shared__ double lds[4 * 2];
   const int row = lb * 256 + threadIdx.x;
@@ -583,8 +590,6 @@ __device__ __forceinline__ void cg_init_body(const Grid &g, int lb, const double
   kinv[row] = k;
   x[row] = 0.0;
   r[row] = rv;
-  z[row] = zv;
-  p[row] = zv;
   double v[2] = {rv * zv, zv * zv};
   block_sum<2, 256>(v, lds);
   if (threadIdx.x == 0) {
@@ -607,28 +612,203 @@ __device__ __forceinline__ void cg_init_state_body(const double *part, int npart
     c.pn0 = sqrt(t[1]);
     c.pn = c.pn0;
     c.its = 0;
+    c.fresh = 1;
     c.done = cg_done(c);
     state[0] = c;
   }
 }
 
-// STENCIL: the matrix has nonzeros only on in-grid stencil slots (assembled
-// here), so the columns are computed (row_dot_grid); otherwise they are read.
-template <int CH = kChunk, bool STENCIL = true, typename T>
-__device__ __forceinline__ void cg_step1_body(const Grid &g, int lb, const int *cols, const T *vals, const T *p,
-                                              T *Ap, double *part1, const CgState *cur) {
+// a CgState in registers: only the fields that the CG reads.  (A copy of the
+// whole struct goes through LDS, whose addresses take the block size from the
+// dispatch packet: a read of host memory by every wave, 11 us at 1555 blocks.)
+struct CgRegs {
+  double rz, pn0, pn, beta, min_err, rel_err;
+  int its, max_its, done, fresh;
+};
+
+__device__ __forceinline__ CgRegs cg_load(const CgState *s) {
+  return CgRegs{s->rz, s->pn0, s->pn, s->beta, s->min_err, s->rel_err, s->its, s->max_its, s->done, s->fresh};
+}
+
+__device__ __forceinline__ void cg_store(const CgRegs &c, int fresh, CgState *s) {
+  s->rz = c.rz;
+  s->pn0 = c.pn0;
+  s->pn = c.pn;
+  s->beta = c.beta;
+  s->min_err = c.min_err;
+  s->rel_err = c.rel_err;
+  s->its = c.its;
+  s->max_its = c.max_its;
+  s->done = c.done;
+  s->fresh = fresh;
+}
+
+// the scalars of the iteration that c's last step2 belongs to, from the sums
+// of its partials (no-op on a fresh state)
+__device__ __forceinline__ void cg_scalars(CgRegs &c, const double *part2, int nb) {
+#pragma clang fp contract(off)
+  if (c.fresh) return;
+  double t[2];
+  seg_sum<2>(part2, nb, t);
+  c.beta = t[1] / c.rz;
+  c.pn = sqrt(t[0]);
+  c.rz = t[1];
+  c.its += 1;
+  c.done = cg_done(c);
+}
+
+// the state entering an iteration: true if the CG goes on.  part2 holds the
+// previous iteration's sums; block 0 writes the state that step2 and the next
+// step1 read.
+__device__ __forceinline__ bool cg_enter(CgRegs &c, int lb, int nb, const double *part2, CgState *nxt) {
+  if (!c.done) cg_scalars(c, part2, nb);
+  if (lb == 0 && threadIdx.x == 0) cg_store(c, c.done, nxt);  // a stopped state has no sums to come
+  return !c.done;
+}
+
+// p of the iteration at one row: p = z + beta p, and p = z in the first
+__device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, double p) {
+#pragma clang fp contract(off)
+  const double z = k * r;
+  return c.its == 0 ? z : z + c.beta * p;
+}
+
+// step1 of a matrix assembled here (computed stencil columns).  What bounds
+// it: at 50^3 nodes the 648 bytes of values per row from HBM; on RVEs of a few
+// thousand rows the chain of waits (state, sums, stage, values).  The first
+// chunk of the row's values does not depend on any of the others, so it is
+// loaded before them, and each later chunk before the previous one's products;
+// the barriers in between wait for LDS alone.
+template <int CH>
+__device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, const double *vals, const double *kinv,
+                                                const double *r, const double *p, double *pn, double *Ap,
+                                                double *part1, const CgState *cur, CgState *nxt) {
+#pragma clang fp contract(off)
+  static_assert(kSlots % CH == 0 && CH % 3 == 0, "chunks tile the row in whole neighbours");
+  __shared__ double seg[9 * kSegNodes * 3];
+  __shared__ double lds[4];
+  CgRegs c = cg_load(cur);
+  const int row0 = lb * 256, row = row0 + threadIdx.x;
+  const double *v = vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
+  double vi[2][CH];
+  if (!c.done)
+#pragma unroll
+    for (int k = 0; k < CH; ++k) vi[0][k] = __builtin_nontemporal_load(&v[k * 64]);
+  if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
+  // the block's 86 nodes (wherever its 256 rows start) and their stencil
+  // neighbours: one contiguous run of 88 nodes per (dz, dy), or, while those of
+  // one dz overlap, one run per dz
+  const bool joined = g.nx <= kSegNodes;
+  const int ly = joined ? g.nx : kSegNodes, ny = joined ? 1 : 3;  // LDS pitch of dy; runs per dz
+  const int len = joined ? kSegNodes + 2 * g.nx : kSegNodes, lz = joined ? len : 3 * kSegNodes;
+  const int n_lo = row0 / 3, nxny = g.nx * g.ny, hi = g.nn - 1;
+  for (int dz = -1; dz <= 1; ++dz)
+    for (int y = 0; y < ny; ++y) {
+      const int n0 = n_lo - 1 + dz * nxny + (y - 1) * g.nx;
+      double *out = seg + ((dz + 1) * lz + y * kSegNodes) * 3;
+#pragma unroll 2
+      for (int e3 = threadIdx.x; e3 < 3 * len; e3 += 256) {
+        const int q = 3 * min(max(n0 + e3 / 3, 0), hi) + e3 % 3;
+        out[e3] = cg_dir(c, kinv[q], r[q], p[q]);
+      }
+    }
+  lds_barrier();
+  const double *own = seg + (row / 3 - n_lo + 1 + ly + lz) * 3;  // the row's node
+  // rows past the last node lie on its run's clamped end; p is zero there
+  const double pv = row < g.nrow ? own[row % 3] : 0.0;
+  double acc = 0;
+#pragma unroll
+  for (int ch = 0; ch < kSlots / CH; ++ch) {
+    if (ch + 1 < kSlots / CH)
+#pragma unroll
+      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = __builtin_nontemporal_load(&v[((ch + 1) * CH + k) * 64]);
+#pragma unroll
+    for (int k = 0; k < CH; k += 3) {
+      const int n = (ch * CH + k) / 3;
+      const double *sv = own + ((n / 9 - 1) * lz + ((n / 3) % 3 - 1) * ly + n % 3 - 1) * 3;
+#pragma unroll
+      for (int fj = 0; fj < 3; ++fj) acc += vi[ch & 1][k + fj] * sv[fj];
+    }
+  }
+  pn[row] = pv;
+  Ap[row] = acc;
+  double t[1] = {pv * acc};
+  block_sum<1, 256>(t, lds);
+  if (threadIdx.x == 0) part1[lb] = t[0];
+}
+
+// p = z + beta p and the state of the iteration alone, ahead of the SpMV of an
+// uploaded matrix: its columns are read, so its gathers are not staged
+__device__ __forceinline__ void cg_dir_body(int lb, int nb, const double *kinv, const double *r, const double *p,
+                                            double *pn, const double *part2, const CgState *cur, CgState *nxt) {
+  CgRegs c = cg_load(cur);
+  if (!cg_enter(c, lb, nb, part2, nxt)) return;
+  const int row = lb * 256 + threadIdx.x;
+  pn[row] = cg_dir(c, kinv[row], r[row], p[row]);
+}
+
+__device__ __forceinline__ void cg_spmv_cols_body(int lb, const int *cols, const double *vals, const double *p,
+                                                  double *Ap, double *part1, const CgState *cur) {
 #pragma clang fp contract(off)
   __shared__ double lds[4];
   if (cur->done) return;
   const int row = lb * 256 + threadIdx.x;
-  T y;
-  if constexpr (STENCIL) {
-    __shared__ T seg[9][kSegNodes * 3];
-    stage_grid_runs(g, lb * 256, p, seg);
-    y = row_dot_grid_seg<CH>(vals, seg, lb * 256, row);
-  } else {
-    y = row_dot<CH>(cols, vals, p, row);
+  const double y = row_dot(cols, vals, p, row);
+  Ap[row] = y;
+  double t[1] = {p[row] * y};
+  block_sum<1, 256>(t, lds);
+  if (threadIdx.x == 0) part1[lb] = t[0];
+}
+
+// step2; its vectors are loaded before the sums that alpha waits for
+__device__ __forceinline__ void cg_step2_body64(int lb, int nb, double *x, double *r, const double *p,
+                                                const double *Ap, const double *kinv, double *part,
+                                                const CgState *cur) {
+#pragma clang fp contract(off)
+  __shared__ double lds[4 * 2];
+  if (cur->done) return;
+  const int row = lb * 256 + threadIdx.x;
+  const double xo = x[row], ro = r[row], po = p[row], ao = Ap[row], ko = kinv[row];
+  double pap[1];
+  seg_sum<1>(part, nb, pap);
+  const double alpha = cur->rz / pap[0];
+  x[row] = xo + alpha * po;
+  const double rv = ro - alpha * ao;
+  r[row] = rv;
+  const double zv = ko * rv;
+  double v[2] = {zv * zv, rv * zv};
+  block_sum<2, 256>(v, lds);
+  if (threadIdx.x == 0) {
+    part[nb + (size_t)lb * 2 + 0] = v[0];
+    part[nb + (size_t)lb * 2 + 1] = v[1];
   }
+}
+
+// one block: the sums of the last step2 queued into the state, in place
+__device__ __forceinline__ void cg_tail_body(const double *part2, int nb, CgState *state) {
+  CgRegs c = cg_load(state);
+  if (c.done || c.fresh) return;
+  cg_scalars(c, part2, nb);
+  if (threadIdx.x == 0) cg_store(c, 1, state);
+}
+
+// ---------------------------------------------------------------------------
+// The FP32 inner CG of the mixed-precision batch, three kernels per iteration
+// (its preconditioner runs between the second and the third): step1 Ap = A p,
+// step2 alpha, x, r, z = k r, step3 beta, p = z + beta p and the new scalars,
+// read from state[k & 1] and written to state[(k+1) & 1].  Products and
+// partials are formed in FP64.
+// ---------------------------------------------------------------------------
+template <int CH = kChunk, typename T>
+__device__ __forceinline__ void cg_step1_body(const Grid &g, int lb, const T *vals, const T *p, T *Ap, double *part1,
+                                              const CgState *cur) {
+#pragma clang fp contract(off)
+  __shared__ double lds[4];
+  if (cur->done) return;
+  const int row = lb * 256 + threadIdx.x;
+  __shared__ T seg[9][kSegNodes * 3];
+  stage_grid_runs(g, lb * 256, p, seg);
+  const T y = row_dot_grid_seg<CH>(vals, seg, lb * 256, row);
   Ap[row] = y;
   double v[1] = {(double)p[row] * (double)y};
   block_sum<1, 256>(v, lds);

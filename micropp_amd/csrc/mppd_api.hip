@@ -63,7 +63,7 @@ struct mppd_solver {
   int phase_mode = 0;
   int ke_phase_ready = 0;
   double *be = nullptr;
-  double *x = nullptr, *rr = nullptr, *z = nullptr, *p = nullptr, *Ap = nullptr, *kinv = nullptr;
+  double *x = nullptr, *rr = nullptr, *p = nullptr, *p2 = nullptr, *Ap = nullptr, *kinv = nullptr;
   double *b = nullptr, *du = nullptr;
   double *partials = nullptr;
   CgState *cg = nullptr, *cg_h = nullptr;
@@ -318,7 +318,7 @@ int mppd_solver_create(mppd_solver **out, mppd_rve *r) {
     if ((rc = dalloc(&s->vals, np * kSlots, st))) break;
     if ((rc = dalloc(&s->ke, (s->phase_mode ? 3 : (size_t)g.nelem) * 576, false))) break;
     if ((rc = dalloc(&s->be, (size_t)g.nelem * 24, false))) break;
-    double **vecs[] = {&s->x, &s->rr, &s->z, &s->p, &s->Ap, &s->kinv, &s->b, &s->du};
+    double **vecs[] = {&s->x, &s->rr, &s->p, &s->p2, &s->Ap, &s->kinv, &s->b, &s->du};
     for (double **v : vecs)
       if ((rc = dalloc(v, np, st))) break;
     if (rc) break;
@@ -344,7 +344,7 @@ int mppd_solver_destroy(mppd_solver *s) {
   if (!s) return MPPD_OK;
   if (s->st) (void)hipStreamSynchronize(s->st);
   for (void *p : {(void *)s->cols, (void *)s->vals, (void *)s->ke, (void *)s->be, (void *)s->x, (void *)s->rr,
-                  (void *)s->z, (void *)s->p, (void *)s->Ap, (void *)s->kinv, (void *)s->b, (void *)s->du,
+                  (void *)s->p, (void *)s->p2, (void *)s->Ap, (void *)s->kinv, (void *)s->b, (void *)s->du,
                   (void *)s->partials, (void *)s->cg, (void *)s->red})
     dfree(p);
   if (s->cg_h) (void)hipHostFree(s->cg_h);
@@ -459,23 +459,26 @@ int mppd_ell_mvp(mppd_solver *s, const double *x_d, double *y_d) {
   return MPPD_OK;
 }
 
-// The working set of one Jacobi-PCG: vectors of nrow_pad doubles, the
-// partial table (3 * nrow_pad / 256 doubles), the ping-pong state pair on the
-// device and one host (pinned) state for the reads between chunks.
+// One Jacobi-PCG: its working set and one host (pinned) state for the reads
+// between chunks.
 struct CgWork {
-  double *x, *r, *z, *p, *Ap, *kinv, *part;
-  CgState *state, *state_h;
+  CgVecs v;
+  CgState *state_h;
 };
+
+static CgVecs cg_vecs(const mppd_solver *s) {
+  return CgVecs{s->x, s->rr, {s->p, s->p2}, s->Ap, s->kinv, s->partials, s->cg};
+}
 
 // CG on the device; the host queues iterations in chunks sized from the
 // observed convergence rate and reads the 64-byte state between chunks.
 // After `queued` iterations the current state is state[queued & 1].
 static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipStream_t st, const double *b_d,
                      double min_err, double rel_err, int max_its, int *its_out, double *err_out) {
-  MPP_HIP(launch_cg_init(g, A->vals, b_d, w.x, w.r, w.z, w.p, w.kinv, w.part, min_err, rel_err, max_its, w.state,
-                         st));
+  const CgVecs &v = w.v;
+  MPP_HIP(launch_cg_init(g, A->vals, b_d, v, min_err, rel_err, max_its, st));
   int queued = 0;
-  MPP_HIP(hipMemcpyAsync(w.state_h, w.state, sizeof(CgState), hipMemcpyDeviceToHost, st));
+  MPP_HIP(hipMemcpyAsync(w.state_h, v.state, sizeof(CgState), hipMemcpyDeviceToHost, st));
   MPP_HIP(hipStreamSynchronize(st));
   double pn_prev = w.state_h->pn;
   int its_prev = 0;
@@ -484,10 +487,10 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
     const int n = std::min(chunk, max_its - queued);
     if (n <= 0) break;
     for (int i = 0; i < n; ++i)
-      MPP_HIP(launch_cg_iter(g, A->vals_stencil ? nullptr : A->cols, A->vals, w.x, w.r, w.z, w.p, w.Ap, w.kinv,
-                             w.part, w.state, queued + i, st));
+      MPP_HIP(launch_cg_iter(g, A->vals_stencil ? nullptr : A->cols, A->vals, v, queued + i, st));
     queued += n;
-    MPP_HIP(hipMemcpyAsync(w.state_h, w.state + (queued & 1), sizeof(CgState), hipMemcpyDeviceToHost, st));
+    MPP_HIP(launch_cg_tail(g, v, queued, st));
+    MPP_HIP(hipMemcpyAsync(w.state_h, v.state + (queued & 1), sizeof(CgState), hipMemcpyDeviceToHost, st));
     MPP_HIP(hipStreamSynchronize(st));
     const CgState &c = *w.state_h;
     if (c.done) break;
@@ -511,8 +514,7 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
 
 static int cg_run(mppd_solver *s, const mppd_solver *A, const double *b_d, double min_err, double rel_err,
                   int max_its, int *its_out, double *err_out) {
-  const CgWork w{s->x, s->rr, s->z, s->p, s->Ap, s->kinv, s->partials, s->cg, s->cg_h};
-  return cg_run_on(s->r->g, A, w, s->st, b_d, min_err, rel_err, max_its, its_out, err_out);
+  return cg_run_on(s->r->g, A, CgWork{cg_vecs(s), s->cg_h}, s->st, b_d, min_err, rel_err, max_its, its_out, err_out);
 }
 
 // A0's matrix is read with s's row layout: it must be a solver of an RVE grid
@@ -536,7 +538,7 @@ int mppd_cg(mppd_solver *s, const mppd_solver *A0, const double *b_d, double *x_
   return MPPD_OK;
 }
 
-// mppd_cg_noalloc: the working set of the CG (x, r, z, p, Ap, D^-1, the
+// mppd_cg_noalloc: the working set of the CG (x, r, the two p, Ap, D^-1, the
 // partial table and the state pair) lives in `scratch`, a fixed device array
 // of this file, instead of the solver's own buffers.  Layout (doubles): the
 // state pair in the first 256 bytes, then 6 vectors of kNoAllocRows, then the
@@ -587,17 +589,11 @@ int mppd_cg_noalloc(mppd_solver *s, const mppd_solver *A0, const double *b_d, do
   // rows of the vectors, every partial, state[0]) or by an earlier kernel of
   // the same solve, so nothing left by the previous call needs clearing
   double *v = ptr + kNoAllocHead;
-  const CgWork w{v,
-                 v + kNoAllocRows,
-                 v + 2 * kNoAllocRows,
-                 v + 3 * kNoAllocRows,
-                 v + 4 * kNoAllocRows,
-                 v + 5 * kNoAllocRows,
-                 v + 6 * kNoAllocRows,
-                 reinterpret_cast<CgState *>(ptr),
-                 s->cg_h};
+  const auto vec = [v](int i) { return v + i * kNoAllocRows; };
+  const CgWork w{
+      CgVecs{vec(0), vec(1), {vec(2), vec(3)}, vec(4), vec(5), vec(6), reinterpret_cast<CgState *>(ptr)}, s->cg_h};
   if (int rc = cg_run_on(g, A0 ? A0 : s, w, s->st, b_d, min_err, rel_err, max_its, its, err)) return rc;
-  MPP_HIP(launch_copy(g.nrow, w.x, x_d, s->st));
+  MPP_HIP(launch_copy(g.nrow, w.v.x, x_d, s->st));
   MPP_HIP(hipStreamSynchronize(s->st));
   return MPPD_OK;
 }
@@ -677,20 +673,21 @@ int mppd_cg_profile(mppd_solver *s, const double *b_d, int iters, double *spmv_m
   if (!s || !b_d || iters <= 0) return fail(MPPD_ERR_ARG, "bad cg_profile arguments");
   const Grid &g = s->r->g;
   // min_err = rel_err = 0: the stopping test never holds within iters + 1
-  MPP_HIP(launch_cg_init(g, s->vals, b_d, s->x, s->rr, s->z, s->p, s->kinv, s->partials, 0.0, 0.0, iters + 1, s->cg,
-                         s->st));
+  const CgVecs v = cg_vecs(s);
+  const int *cols = s->vals_stencil ? nullptr : s->cols;
+  MPP_HIP(launch_cg_init(g, s->vals, b_d, v, 0.0, 0.0, iters + 1, s->st));
   hipEvent_t ev[3];
   for (auto &x : ev) MPP_HIP(hipEventCreate(&x));
-  // (1) the SpMV kernel back to back: it reads p and state[0], writes Ap and
-  // its partials, so repeating it leaves the CG state unchanged
-  hipError_t e = hipEventRecord(ev[0], s->st);
+  // (1) step1 back to back: it reads p[0], r and state[0] and writes p[1], Ap,
+  // its partials and state[1], so repeating it changes nothing
+  hipError_t e = launch_cg_step1(g, cols, s->vals, v, 0, s->st);
+  if (e == hipSuccess) e = hipEventRecord(ev[0], s->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_cg_step1(g, s->vals_stencil ? nullptr : s->cols, s->vals, s->p, s->Ap, s->partials, s->cg, 0, s->st);
+    e = launch_cg_step1(g, cols, s->vals, v, 0, s->st, false);
   // (2) whole iterations
   if (e == hipSuccess) e = hipEventRecord(ev[1], s->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_cg_iter(g, s->vals_stencil ? nullptr : s->cols, s->vals, s->x, s->rr, s->z, s->p, s->Ap, s->kinv,
-                       s->partials, s->cg, i, s->st);
+    e = launch_cg_iter(g, cols, s->vals, v, i, s->st);
   if (e == hipSuccess) e = hipEventRecord(ev[2], s->st);
   if (e == hipSuccess) e = hipStreamSynchronize(s->st);
   float ms1 = 0.f, ms2 = 0.f;

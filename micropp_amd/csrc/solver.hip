@@ -9,19 +9,17 @@
 // 16 bytes per row.
 //
 // ell_solve_cgpd (src/ell.cpp:66-122): the reference recurrence, one
-// iteration = three kernels:
-//   step1  Ap = A p and the per-block partials of p.Ap
-//   step2  alpha = r.z / sum(partials); x += alpha p; r -= alpha Ap; z = k r;
-//          per-block partials of z.z and r.z
-//   step3  beta = sum(r.z) / r.z_old; p = z + beta p; the new scalars
-// No kernel uses atomics or fences: each block writes its partial, and every
-// block of the next kernel re-sums all partials in the same fixed order, so
-// every block holds identical scalars.  The scalars of iteration k are read
-// from state[k & 1] and written (by block 0 of step3) to state[(k+1) & 1]; the
-// parity is a kernel argument, so a run of iterations can be queued or
-// captured in a graph ahead of time.  Once the stopping test holds, the
-// kernels of later iterations return at once and step3 only carries the
-// final state forward.
+// iteration = two kernels (kernels.hpp: step1 forms p and Ap, step2 x and r),
+// or three for an uploaded matrix, where k_cg_dir forms p ahead of the SpMV.  No kernel uses
+// atomics or fences: each block writes its partial, and every block of the
+// next kernel re-sums all partials in the same fixed order, so every block
+// holds identical scalars.  The parity is a kernel argument, so a run of
+// iterations can be queued or captured in a graph ahead of time.
+// Time per iteration (us) in two kernels, and as three (SpMV, x and r, p) with
+// shuffled block sums: 6^3 nodes 9.3 / 14.1, 11^3 10.0 / 15.6, 21^3 10.7 /
+// 16.2, 31^3 17.7 / 23.0, 41^3 33.0 / 37.8, 51^3 58.0 / 60.4.  Small RVEs wait
+// for launches and block sums (kernels of about 6 and 3 us), 51^3 for 259 MB of
+// values a pass (5.5 TB/s).
 #include "kernels.hpp"
 
 namespace mpp {
@@ -34,8 +32,8 @@ __global__ void __launch_bounds__(256) k_spmv(Grid g, const int *cols, const dou
 }
 
 __global__ void __launch_bounds__(256) k_cg_init(Grid g, const double *vals, const double *b, double *x, double *r,
-                                                 double *z, double *p, double *kinv, double *part) {
-  cg_init_body(g, blockIdx.x, vals, b, x, r, z, p, kinv, part);
+                                                 double *kinv, double *part) {
+  cg_init_body(g, blockIdx.x, vals, b, x, r, kinv, part);
 }
 
 __global__ void __launch_bounds__(256) k_cg_init_state(const double *part, int nparts, double min_err,
@@ -46,23 +44,34 @@ __global__ void __launch_bounds__(256) k_cg_init_state(const double *part, int n
 // Blocks are dispatched round-robin over the 8 XCDs: the 8 * per launched
 // blocks give XCD x the row blocks [x * per, (x + 1) * per), so each XCD's
 // L2 holds a contiguous slab of the gathered vector (2-5% faster SpMV).
-template <bool STENCIL>
-__global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const int *cols, const double *vals,
-                                                  const double *p, double *Ap, double *part1, const CgState *cur) {
+__global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const double *vals, const double *kinv,
+                                                  const double *r, const double *p, double *pn, double *Ap,
+                                                  double *part, const CgState *cur, CgState *nxt) {
   const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (lb >= nb) return;
-  cg_step1_body<kChunk, STENCIL>(g, lb, cols, vals, p, Ap, part1, cur);
+  cg_step1_body64<kChunk>(g, lb, nb, vals, kinv, r, p, pn, Ap, part, cur, nxt);
 }
 
-__global__ void __launch_bounds__(256) k_cg_step2(double *x, double *r, double *z, const double *p, const double *Ap,
-                                                  const double *kinv, const double *part1, double *part2,
-                                                  const CgState *cur) {
-  cg_step2_body(blockIdx.x, gridDim.x, x, r, z, p, Ap, kinv, part1, part2, cur);
+__global__ void __launch_bounds__(256) k_cg_dir(const double *kinv, const double *r, const double *p, double *pn,
+                                                const double *part2, const CgState *cur, CgState *nxt) {
+  cg_dir_body(blockIdx.x, gridDim.x, kinv, r, p, pn, part2, cur, nxt);
 }
 
-__global__ void __launch_bounds__(256) k_cg_step3(const double *z, double *p, const double *part1,
-                                                  const double *part2, const CgState *cur, CgState *nxt) {
-  cg_step3_body(blockIdx.x, gridDim.x, z, p, part1, part2, cur, nxt);
+__global__ void __launch_bounds__(256) k_cg_spmv_cols(int nb, int per, const int *cols, const double *vals,
+                                                      const double *p, double *Ap, double *part1,
+                                                      const CgState *cur) {
+  const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (lb >= nb) return;
+  cg_spmv_cols_body(lb, cols, vals, p, Ap, part1, cur);
+}
+
+__global__ void __launch_bounds__(256) k_cg_step2(double *x, double *r, const double *p, const double *Ap,
+                                                  const double *kinv, double *part, const CgState *cur) {
+  cg_step2_body64(blockIdx.x, gridDim.x, x, r, p, Ap, kinv, part, cur);
+}
+
+__global__ void __launch_bounds__(256) k_cg_tail(const double *part2, int nb, CgState *state) {
+  cg_tail_body(part2, nb, state);
 }
 
 __global__ void k_axpy(int n, double a, const double *x, double *y) {
@@ -84,44 +93,44 @@ hipError_t launch_spmv(const Grid &g, const int *cols, const double *vals, const
   return hipGetLastError();
 }
 
-hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, double *x, double *r, double *z,
-                          double *p, double *kinv, double *part, double min_err, double rel_err, int max_its,
-                          CgState *state, hipStream_t st) {
+hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, const CgVecs &w, double min_err,
+                          double rel_err, int max_its, hipStream_t st) {
   const unsigned nb = nblk(g.nrow_pad, 256);
-  hipLaunchKernelGGL(k_cg_init, dim3(nb), dim3(256), 0, st, g, vals, b, x, r, z, p, kinv, part);
-  hipLaunchKernelGGL(k_cg_init_state, dim3(1), dim3(256), 0, st, part, (int)nb, min_err, rel_err, max_its, state);
+  hipLaunchKernelGGL(k_cg_init, dim3(nb), dim3(256), 0, st, g, vals, b, w.x, w.r, w.kinv, w.part);
+  hipLaunchKernelGGL(k_cg_init_state, dim3(1), dim3(256), 0, st, w.part, (int)nb, min_err, rel_err, max_its, w.state);
   return hipGetLastError();
 }
 
-hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const double *p, double *Ap,
-                           double *part, CgState *state, int parity, hipStream_t st) {
-  const int nb = (int)nblk(g.nrow_pad, 256), per = (nb + 7) / 8;
-  // cols == nullptr: the matrix was assembled here and the stencil columns are computed
-  if (cols)
-    hipLaunchKernelGGL(k_cg_step1<false>, dim3(8 * per), dim3(256), 0, st, g, nb, per, cols, vals, p, Ap, part,
-                       state + (parity & 1));
-  else
-    hipLaunchKernelGGL(k_cg_step1<true>, dim3(8 * per), dim3(256), 0, st, g, nb, per, cols, vals, p, Ap, part,
-                       state + (parity & 1));
+hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
+                           hipStream_t st, bool dir) {
+  const int nb = (int)nblk(g.nrow_pad, 256), per = (nb + 7) / 8, k = parity & 1;
+  CgState *cur = w.state + k, *nxt = w.state + (k ^ 1);
+  if (cols) {
+    if (dir)
+      hipLaunchKernelGGL(k_cg_dir, dim3(nb), dim3(256), 0, st, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.part + nb, cur, nxt);
+    hipLaunchKernelGGL(k_cg_spmv_cols, dim3(8 * per), dim3(256), 0, st, nb, per, cols, vals, w.p[k ^ 1], w.Ap, w.part,
+                       nxt);
+  } else {
+    hipLaunchKernelGGL(k_cg_step1, dim3(8 * per), dim3(256), 0, st, g, nb, per, vals, w.kinv, w.r, w.p[k], w.p[k ^ 1],
+                       w.Ap, w.part, cur, nxt);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_cg_step23(const Grid &g, double *x, double *r, double *z, double *p, const double *Ap,
-                            const double *kinv, double *part, CgState *state, int parity, hipStream_t st) {
-  const unsigned nb = nblk(g.nrow_pad, 256);
-  double *part1 = part, *part2 = part + nb;
-  CgState *cur = state + (parity & 1), *nxt = state + ((parity + 1) & 1);
-  hipLaunchKernelGGL(k_cg_step2, dim3(nb), dim3(256), 0, st, x, r, z, p, Ap, kinv, part1, part2, cur);
-  hipLaunchKernelGGL(k_cg_step3, dim3(nb), dim3(256), 0, st, z, p, part1, part2, cur, nxt);
-  return hipGetLastError();
-}
-
-hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, double *x, double *r, double *z,
-                          double *p, double *Ap, const double *kinv, double *part, CgState *state, int parity,
+hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
                           hipStream_t st) {
-  hipError_t e = launch_cg_step1(g, cols, vals, p, Ap, part, state, parity, st);
-  if (e == hipSuccess) e = launch_cg_step23(g, x, r, z, p, Ap, kinv, part, state, parity, st);
-  return e;
+  const hipError_t e = launch_cg_step1(g, cols, vals, w, parity, st);
+  if (e != hipSuccess) return e;
+  const int n = (parity & 1) ^ 1;
+  hipLaunchKernelGGL(k_cg_step2, dim3(nblk(g.nrow_pad, 256)), dim3(256), 0, st, w.x, w.r, w.p[n], w.Ap, w.kinv, w.part,
+                     w.state + n);
+  return hipGetLastError();
+}
+
+hipError_t launch_cg_tail(const Grid &g, const CgVecs &w, int queued, hipStream_t st) {
+  const unsigned nb = nblk(g.nrow_pad, 256);
+  hipLaunchKernelGGL(k_cg_tail, dim3(1), dim3(256), 0, st, w.part + nb, (int)nb, w.state + (queued & 1));
+  return hipGetLastError();
 }
 
 hipError_t launch_axpy(int n, double a, const double *x, double *y, hipStream_t st) {

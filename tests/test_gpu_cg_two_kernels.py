@@ -1,0 +1,48 @@
+"""GPU: the FP64 Jacobi-CG at the edges of its kernels.
+
+step1 forms p and Ap of 256 rows in one kernel: its LDS runs are one per z plane up to 88 nodes a line and nine
+beyond; for an uploaded matrix p is formed ahead of it.  Every form does the oracle's
+arithmetic except for the order of the inner products, so a solve to 1e-6 stops within an iteration of it and
+agrees to ten times that; the forms among each other differ in nothing, so they agree bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mp():
+    import micropp_amd
+
+    micropp_amd.load()
+    if not micropp_amd.gpu_available():
+        pytest.skip("no HIP device")
+    return micropp_amd
+
+
+# lines of 87, 88 and 89 nodes, fewer rows than a block, whole blocks and a remainder
+SIZES = [(2, 2, 2), (3, 3, 2), (5, 4, 6), (87, 3, 4), (88, 4, 3), (89, 3, 4), (17, 30, 9), (32, 16, 8), (23, 31, 50)]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_solve_by_computed_and_by_uploaded_columns(mp, oracle, size):
+    """An assembled matrix against the same values uploaded, and both against the oracle: chunks of 32 iterations
+    end inside the solve (40 of them), so the scalars pass through the state read by the host too."""
+    r = mp.Rve(size, mp.MIC3D_RANDOM_SPHERES, (7.0, 5.0, 0.1, 0.3), [mp.material(0, 1e6, 0.3), mp.material(0, 1e7, 0.25),
+                                                                   mp.material(0, 1e7, 0.25)])
+    s, up = mp.Solver(r), mp.Solver(r)
+    u, b = mp.DeviceArray(r.nrow), mp.DeviceArray(r.nrow)
+    s.set_displ_bc([5e-3, -1e-3, 2e-3, 1e-3, 0.0, -2e-3], u)
+    s.assembly_mat(u)
+    s.assembly_rhs(u, None, b)
+    cols, vals = s.ell()
+    up.upload_vals(vals)
+    x, xu = mp.DeviceArray(r.nrow), mp.DeviceArray(r.nrow)
+    its, err = s.cg(b, x, 1e-50, 1e-300, 40)
+    its_u, err_u = up.cg(b, xu, 1e-50, 1e-300, 40)
+    assert (its, err) == (its_u, err_u) or (np.isnan(err) and np.isnan(err_u))
+    assert np.array_equal(x.numpy(), xu.numpy(), equal_nan=True)
+    if min(size) > 2:  # an interior: the solution is not zero
+        xo, io, _ = oracle.ell_cg(r.nrow // 3, 3, 81, 13, cols, vals, b.numpy(), 1e-50, 1e-6, 40)
+        it6, _ = s.cg(b, x, 1e-50, 1e-6, 40)
+        assert abs(it6 - io) <= 1 and np.abs(x.numpy() - xo).max() <= 1e-5 * np.abs(xo).max()
