@@ -165,24 +165,22 @@ __global__ void __launch_bounds__(256) kb_cg_init_state(const BRve *rv, const in
 // (blocks are dispatched round-robin over the 8 XCDs).  The arithmetic is
 // the same in every shape.
 template <int CH, bool XCD>
-__global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int *map, const int *blk0, const int *a0on,
+__global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *at, CgState *cg, const int *a0on,
                                                    int nb, int per, int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
   if (b >= nb) return;
-  const int rid = map[b];
+  const int rid = at[b].x, k = parity & 1;
   const BRve &R = rv[rid];
   // vals and a0 are assembled here: the stencil columns follow from the grid
-  const int k = parity & 1;
   const double *A = cg_matrix(R, a0on, rid);
-  cg_step1_body64<CH>(R.g, b - blk0[rid], R.nb_row, A, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap, R.part, R.cg + k,
-                      R.cg + (k ^ 1));
+  cg_step1_body64<CH>(R.g, at[b].y, R.nb_row, A, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap, R.part, cg + 2 * rid + k,
+                      cg + 2 * rid + (k ^ 1));
 }
 
-__global__ void __launch_bounds__(256) kb_cg_step2(const BRve *rv, const int *map, const int *blk0, int parity) {
-  const int rid = map[blockIdx.x];
+__global__ void __launch_bounds__(256) kb_cg_step2(const BRve *rv, const int2 *at, const CgState *cg, int parity) {
+  const int rid = at[blockIdx.x].x, n = (parity & 1) ^ 1;
   const BRve &R = rv[rid];
-  const int n = (parity & 1) ^ 1;
-  cg_step2_body64(blockIdx.x - blk0[rid], R.nb_row, R.x, R.r, R.p[n], R.Ap, R.kinv, R.part, R.cg + n);
+  cg_step2_body64(at[blockIdx.x].y, R.nb_row, R.x, R.r, R.p[n], R.Ap, R.kinv, R.part, cg + 2 * rid + n);
 }
 
 // one block per RVE
@@ -306,15 +304,16 @@ __global__ void __launch_bounds__(256) kb_m_resid(const BRve *rv, const int *map
   const float r32 = (float)rr;
   const float z32 = R.kinv32[row] * r32;
   R.r[row] = rr;
-  R.r32[row] = r32;
-  R.z32[row] = z32;
-  R.p32[row] = z32;
+  R.r32[0][row] = r32;
   R.x32[row] = 0.0f;
   double v[3] = {zr * zr, (double)r32 * z32, (double)z32 * z32};
   block_sum<3, 256>(v, lds);
   if (threadIdx.x == 0)
     for (int q = 0; q < 3; ++q) R.part[(size_t)lb * 3 + q] = v[q];
 }
+
+// the coarse solve's blocks of one RVE (none without a coarse level)
+__device__ __forceinline__ int coarse_blocks(const BRve &R) { return (R.cgrid.nc + kGemvRows - 1) / kGemvRows; }
 
 // one block per RVE: the outer test and the inner CG's start state (an
 // inactive or converged RVE's inner CG starts done)
@@ -332,8 +331,9 @@ __global__ void __launch_bounds__(256) kb_m_outer(const BRve *rv, const int *act
     }
     return;
   }
-  double t[3];
+  double t[3], cz[1];
   seg_sum<3>(R.part, R.nb_row, t);
+  seg_sum<1>(R.cpart, coarse_blocks(R), cz);
   if (threadIdx.x == 0) {
     BOuter &o = out[rid];
     const double pn = sqrt(t[0]);
@@ -346,7 +346,8 @@ __global__ void __launch_bounds__(256) kb_m_outer(const BRve *rv, const int *act
     o.pn = pn;
     o.conv = conv;
     CgState c{};
-    c.rz = t[1];
+    c.fresh = 1;
+    c.rz = t[1] + cz[0];
     c.pn0 = sqrt(t[2]);
     c.pn = c.pn0;
     c.min_err = 0.0;
@@ -359,30 +360,193 @@ __global__ void __launch_bounds__(256) kb_m_outer(const BRve *rv, const int *act
   }
 }
 
-// shapes as kb_cg_step1
+// ---------------------------------------------------------------------------
+// The inner FP32 CG, four kernels per iteration:
+//   dir    the scalars that the previous iteration's sums give (beta, the
+//          stopping test), z = D^-1 r + P_c e and p = z + beta p
+//   spmv   Ap = A p, partials of p.Ap (shapes as kb_cg_step1)
+//   upd    alpha, x, r, partials of r.D^-1 r and of the stopping test's
+//          ||D^-1 r||^2 on the row blocks; r_c = P_c^T r on the coarse ones
+//   gemv   e = A_c^-1 r_c and partials of r_c.e
+// with e the coarse correction of the two-level preconditioner: trilinear
+// hats of the RVE's coarse grid (R.cgrid) and the inverse of the Galerkin
+// coarse matrix of its initial (elastic) tangent.  (r, z) is r.D^-1 r +
+// r_c.e, so z needs no kernel (nor vector) of its own.  The coarse blocks of
+// upd form r - alpha Ap from the old r, beside the row blocks that store it:
+// r lives in two vectors, read from r[k & 1] and written to r[(k + 1) & 1].
+// States as in the FP64 CG (kernels.hpp).  FP32 residual rows: row = node * 3
+// + d; sums run in fixed orders, those over the rows in FP64.
+// What bounds it: the SpMV streams 324 bytes per row (5.8 TB/s with eight
+// RVEs of 25..31 nodes a side live); the other kernels, and the SpMV once most
+// RVEs have stopped, wait for their launch, the state and the partial sums
+// (4 to 6 us each), hence as few of them as the data allow.
+// Eight J2 RVEs of 25..31 nodes a side, all live, us: SpMV 30, dir 4.4, upd
+// 11.3, gemv 4.8 (eight kernels before, of 4 to 7 beside the SpMV); two live:
+// 10, 3.4, 5.3, 3.5.  With a coarse level on every side (not only those with a
+// suitable divisor) the slowest of them takes 392 iterations a load step
+// instead of 1233, and the step 33 ms instead of 75.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void m_scalars(CgRegs &c, const BRve &R) {
+#pragma clang fp contract(off)
+  if (c.done || c.fresh) return;
+  double t[2], cz[1];
+  seg_sum<2>(R.part + R.nb_row, R.nb_row, t);
+  seg_sum<1>(R.cpart, coarse_blocks(R), cz);
+  const double rz = t[1] + cz[0];
+  c.beta = rz / c.rz;
+  c.pn = sqrt(t[0]);
+  c.rz = rz;
+  c.its += 1;
+  c.done = cg_done(c);
+}
+
+// one thread per node: the weights of the 8 coarse nodes around it (zero
+// outside) serve its three rows
+__global__ void __launch_bounds__(256) kb_m_dir(const BRve *rv, const int2 *at, CgState *cg, int parity) {
+  const int rid = at[blockIdx.x].x, lb = at[blockIdx.x].y, k = parity & 1;
+  const BRve &R = rv[rid];
+  CgRegs c = cg_load(cg + 2 * rid + k);
+  const Grid &g = R.g;
+  const CGrid &cgd = R.cgrid;
+  const int node = lb * 256 + threadIdx.x;
+  const bool in = node < g.nn;
+  float z[3] = {}, p[3] = {};
+  if (in && !c.done) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      z[d] = R.kinv32[node * 3 + d] * R.r32[k][node * 3 + d];
+      p[d] = R.p32[node * 3 + d];
+    }
+    if (cgd.nc) {
+      const int i = node % g.nx, j = (node / g.nx) % g.ny, l = node / (g.nx * g.ny);
+      const HatEntry hx = R.hat[0][i], hy = R.hat[1][j], hz = R.hat[2][l];
+      float acc[3] = {};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const float w = (t & 1 ? hx.w1 : hx.w0) * ((t & 2 ? hy.w1 : hy.w0) * (t & 4 ? hz.w1 : hz.w0));
+        const float *e = R.cec + ((t & 1 ? hx.q1 : hx.q0) + (t & 2 ? hy.q1 : hy.q0) + (t & 4 ? hz.q1 : hz.q0));
+#pragma unroll
+        for (int d = 0; d < 3; ++d) acc[d] += w * e[d];
+      }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) z[d] += acc[d];
+    }
+  }
+  m_scalars(c, R);
+  if (lb == 0 && threadIdx.x == 0) cg_store(c, c.done, cg + 2 * rid + (k ^ 1));
+  if (c.done || !in) return;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) R.p32[node * 3 + d] = c.its == 0 ? z[d] : (float)(z[d] + c.beta * p[d]);
+}
+
 template <int CH, bool XCD>
-__global__ void __launch_bounds__(256) kb_m_step1(const BRve *rv, const int *map, const int *blk0, int nb, int per,
-                                                  int parity) {
+__global__ void __launch_bounds__(256) kb_m_spmv(const BRve *rv, const int2 *at, const CgState *cg, int nb, int per,
+                                                 int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
   if (b >= nb) return;
-  const int rid = map[b];
+  const int rid = at[b].x;
   const BRve &R = rv[rid];
-  cg_step1_body<CH>(R.g, b - blk0[rid], (const float *)R.vals32, (const float *)R.p32, R.Ap32, R.part,
-                    R.cg + (parity & 1));
+  cg_spmv_body32<CH>(R.g, at[b].y, R.vals32, R.p32, R.Ap32, R.part, cg + 2 * rid + ((parity & 1) ^ 1));
 }
 
-__global__ void __launch_bounds__(256) kb_m_step2(const BRve *rv, const int *map, const int *blk0, int parity) {
-  const int rid = map[blockIdx.x];
+// START: r_c of the residual kb_m_resid has stored (RVEs in act); the row
+// blocks have nothing to do
+template <bool START>
+__global__ void __launch_bounds__(256) kb_m_upd(const BRve *rv, const int2 *at, const int *act, const CgState *cg,
+                                                int parity) {
+#pragma clang fp contract(off)
+  __shared__ double lds[4 * 2];
+  const int rid = at[blockIdx.x].x, lb = at[blockIdx.x].y, k = START ? 0 : parity & 1;
   const BRve &R = rv[rid];
-  cg_step2_body(blockIdx.x - blk0[rid], R.nb_row, R.x32, R.r32, R.z32, (const float *)R.p32, (const float *)R.Ap32,
-                (const float *)R.kinv32, R.part, R.part + R.nb_row, R.cg + (parity & 1));
+  const CgState *cur = cg + 2 * rid + (k ^ 1);
+  if (START ? !act[rid] || lb < R.nb_row : cur->done != 0) return;
+  double alpha = 0.0;
+  const float *r = R.r32[k], *Ap = R.Ap32;
+  if (lb < R.nb_row) {
+    const int row = lb * 256 + threadIdx.x;
+    const float xo = R.x32[row], ro = r[row], po = R.p32[row], ao = Ap[row], ko = R.kinv32[row];
+    double pap[1];
+    seg_sum<1>(R.part, R.nb_row, pap);
+    alpha = cur->rz / pap[0];
+    R.x32[row] = xo + alpha * po;
+    const float rv2 = ro - alpha * ao;
+    R.r32[k ^ 1][row] = rv2;
+    const float zv = ko * rv2;
+    double v[2] = {(double)zv * zv, (double)rv2 * zv};
+    block_sum<2, 256>(v, lds);
+    if (threadIdx.x == 0) {
+      R.part[R.nb_row + (size_t)lb * 2 + 0] = v[0];
+      R.part[R.nb_row + (size_t)lb * 2 + 1] = v[1];
+    }
+    return;
+  }
+  const CGrid &cgd = R.cgrid;
+  const int q = lb - R.nb_row;
+  if (q >= cgd.nq) return;
+  if (!START) {
+    double pap[1];
+    seg_sum<1>(R.part, R.nb_row, pap);
+    alpha = cur->rz / pap[0];
+  }
+  // the nodes under the hat of coarse node (cx, cy, cz), between its neighbours
+  const int dx = cgd.mx + 1, dy = cgd.my + 1, dz = cgd.mz + 1;
+  const int cx = q % cgd.mx, cy = (q / cgd.mx) % cgd.my, cz = q / (cgd.mx * cgd.my);  // interior index, 0-based
+  const int i0 = cx * R.g.nex / dx + 1, j0 = cy * R.g.ney / dy + 1, l0 = cz * R.g.nez / dz + 1;
+  const int wx = (cx + 2) * R.g.nex / dx - i0, wy = (cy + 2) * R.g.ney / dy - j0;
+  const int n = wx * wy * ((cz + 2) * R.g.nez / dz - l0);
+  const int ox = 3 * cx, oy = 3 * cgd.mx * cy, oz = 3 * cgd.mx * cgd.my * cz;
+  const auto weight = [](const HatEntry &h, int o) { return (h.q0 == o ? h.w0 : 0.0f) + (h.q1 == o ? h.w1 : 0.0f); };
+  float acc[3] = {};
+#pragma unroll 2
+  for (int s = threadIdx.x; s < n; s += 256) {
+    const int i = i0 + s % wx, j = j0 + (s / wx) % wy, l = l0 + s / (wx * wy);
+    const float w = weight(R.hat[0][i], ox) * (weight(R.hat[1][j], oy) * weight(R.hat[2][l], oz));
+    const int e = ((l * R.g.ny + j) * R.g.nx + i) * 3;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) acc[d] += w * (START ? r[e + d] : (float)(r[e + d] - alpha * Ap[e + d]));
+  }
+  __shared__ float ldf[4 * 3];
+  block_sum<3, 256>(acc, ldf);
+  if (threadIdx.x < 3) R.crc[q * 3 + threadIdx.x] = acc[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(256) kb_m_step3(const BRve *rv, const int *map, const int *blk0, int parity) {
-  const int rid = map[blockIdx.x];
+// e = A_c^-1 r_c: a wave per two coarse rows (the inverse's rows read along
+// their length); act: at the start, else the RVEs whose CG goes on
+__global__ void __launch_bounds__(256) kb_c_gemv(const BRve *rv, const int2 *at, const int *act, const CgState *cg,
+                                                 int parity) {
+  __shared__ double lds[4];
+  const int rid = at[blockIdx.x].x, lb = at[blockIdx.x].y, nc = rv[rid].cgrid.nc;
   const BRve &R = rv[rid];
-  cg_step3_body(blockIdx.x - blk0[rid], R.nb_row, (const float *)R.z32, R.p32, R.part, R.part + R.nb_row,
-                R.cg + (parity & 1), R.cg + ((parity + 1) & 1));
+  if (lb * kGemvRows >= nc || (act ? !act[rid] : cg[2 * rid + ((parity & 1) ^ 1)].done != 0)) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, row = lb * kGemvRows + 2 * w;
+  const float *rc = R.crc;
+  const float *a0 = R.cainv + (size_t)min(row, nc - 1) * nc, *a1 = R.cainv + (size_t)min(row + 1, nc - 1) * nc;
+  float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll 8
+  for (int c = lane; c < nc; c += 64) {
+    const float v = rc[c];
+    s0 = fmaf(a0[c], v, s0);
+    s1 = fmaf(a1[c], v, s1);
+  }
+  s0 = wave_sum_dpp(s0);
+  s1 = wave_sum_dpp(s1);
+  if (lane == 0) {
+    double z = 0.0;
+    if (row < nc) R.cec[row] = s0, z += (double)rc[row] * s0;
+    if (row + 1 < nc) R.cec[row + 1] = s1, z += (double)rc[row + 1] * s1;
+    lds[w] = z;
+  }
+  lds_barrier();
+  if (threadIdx.x == 0) R.cpart[lb] = ((lds[0] + lds[1]) + lds[2]) + lds[3];
+}
+
+// one block per RVE
+__global__ void __launch_bounds__(256) kb_m_tail(const BRve *rv, CgState *cg) {
+  CgState *state = cg + 2 * blockIdx.x;
+  CgRegs c = cg_load(state);
+  if (c.done || c.fresh) return;
+  m_scalars(c, rv[blockIdx.x]);
+  if (threadIdx.x == 0) cg_store(c, 1, state);
 }
 
 __global__ void __launch_bounds__(256) kb_m_accum(const BRve *rv, const int *map, const int *act, const int *blk0) {
@@ -392,169 +556,8 @@ __global__ void __launch_bounds__(256) kb_m_accum(const BRve *rv, const int *map
 }
 
 // ---------------------------------------------------------------------------
-// Two-level preconditioner of the inner FP32 CG (mixed precision): z = D^-1 r
-// + P_c A_c^-1 P_c^T r per RVE, with the trilinear hats of the RVE's coarse
-// grid (R.cgrid) and the inverse of the Galerkin coarse matrix of its initial
-// (elastic) tangent.  It runs at the inner CG's start, after kb_m_resid (act
-// != nullptr: the RVEs in act), and in every iteration between kb_m_step2 and
-// kb_m_step3 (act == nullptr: the RVEs whose CG state `parity` is running).
-// FP32 residual rows: row = node * 3 + d.  The stopping test keeps the
-// Jacobi ||D^-1 r|| of kb_m_step2; only (r, z) and z change.  Sums run in
-// fixed orders.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ bool kb_c_skip(const BRve &R, const int *act, int rid, int parity) {
-  return R.cgrid.nc == 0 || (act ? !act[rid] : R.cg[parity & 1].done != 0);
-}
-
-// restriction along x: one thread per (direction d, interior x-line (j, k),
-// interior coarse x node cx), over the 2 hx - 1 nodes of the hat
-__global__ void __launch_bounds__(256) kb_c_rx(const BRve *rv, const int *map, const int *blk0, const int *act,
-                                               int parity) {
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  if (kb_c_skip(R, act, rid, parity)) return;
-  const Grid &g = R.g;
-  const CGrid &cg = R.cgrid;
-  const int ly = g.ny - 2, lz = g.nz - 2;
-  const int t = (blockIdx.x - blk0[rid]) * 256 + threadIdx.x;
-  if (t >= 3 * ly * lz * cg.mx) return;
-  const int cx = t % cg.mx + 1;
-  int rest = t / cg.mx;
-  const int j = rest % ly + 1;
-  rest /= ly;
-  const int k = rest % lz + 1, d = rest / lz;
-  const float *line = R.r32 + ((size_t)k * g.ny + j) * g.nx * 3 + d;
-  const int i0 = (cx - 1) * cg.hx + 1, n = 2 * cg.hx - 1;
-  float acc = 0.0f;
-#pragma unroll 8
-  for (int s = 0; s < n; ++s) acc += hat(i0 + s, cx, cg.hx) * line[(size_t)(i0 + s) * 3];
-  R.ct1[((size_t)(d * g.nz + k) * g.ny + j) * cg.mx + (cx - 1)] = acc;
-}
-
-// restriction along y and z: one wave per coarse DOF q * 3 + d, its lanes over
-// the x-restricted lines under q's hats, then a wave sum
-__global__ void __launch_bounds__(256) kb_c_ryz(const BRve *rv, const int *map, const int *blk0, const int *act,
-                                                int parity) {
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  if (kb_c_skip(R, act, rid, parity)) return;
-  const Grid &g = R.g;
-  const CGrid &cg = R.cgrid;
-  const int wave = (blockIdx.x - blk0[rid]) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (wave >= cg.nc) return;  // whole wave
-  const int q = wave / 3, d = wave % 3;
-  const int cx = q % cg.mx + 1, cy = (q / cg.mx) % cg.my + 1, cz = q / (cg.mx * cg.my) + 1;
-  const int wy = 2 * cg.hy - 1, npair = wy * (2 * cg.hz - 1);
-  const int j0 = (cy - 1) * cg.hy + 1, k0 = (cz - 1) * cg.hz + 1;
-  float acc = 0.0f;
-  for (int s = lane; s < npair; s += 64) {
-    const int j = j0 + s % wy, k = k0 + s / wy;
-    acc += hat(j, cy, cg.hy) * hat(k, cz, cg.hz) * R.ct1[((size_t)(d * g.nz + k) * g.ny + j) * cg.mx + (cx - 1)];
-  }
-  const float sum = wave_sum_dpp(acc);
-  if (lane == 0) R.crc[wave] = sum;
-}
-
-// the coarse solve e = A_c^-1 r_c: block (64 coarse rows, column split s of
-// R.csplit), each wave a quarter of the split's columns (the symmetric
-// inverse read by column), the waves added in order; into cec directly with
-// one split, else into the split's partial row of cecp
-__global__ void __launch_bounds__(256) kb_c_gemv(const BRve *rv, const int *map, const int *blk0, const int *act,
-                                                 int parity) {
-  __shared__ float red[3][64];
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  if (kb_c_skip(R, act, rid, parity)) return;
-  const int nc = R.cgrid.nc, lane = threadIdx.x & 63, ns = R.csplit;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lb = blockIdx.x - blk0[rid], tile = lb / ns, split = lb % ns;
-  const int chunk = (nc + ns - 1) / ns, c0 = split * chunk, c1 = min(nc, c0 + chunk);
-  const int row = tile * 64 + lane, rowc = min(row, nc - 1);
-  const float *ainv = R.cainv, *rc = R.crc;
-  float acc = 0.0f;
-#pragma unroll 4
-  for (int col = c0 + w; col < c1; col += 4) acc += ainv[(size_t)col * nc + rowc] * rc[col];
-  if (w > 0) red[w - 1][lane] = acc;
-  __syncthreads();
-  if (w == 0 && row < nc) {
-    const float v = acc + red[0][lane] + red[1][lane] + red[2][lane];
-    if (ns == 1)
-      R.cec[row] = v;
-    else
-      R.cecp[(size_t)split * nc + row] = v;
-  }
-}
-
-// the splits' sum in order (RVEs with csplit > 1)
-__global__ void __launch_bounds__(256) kb_c_gsum(const BRve *rv, const int *map, const int *blk0, const int *act,
-                                                 int parity) {
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  if (kb_c_skip(R, act, rid, parity)) return;
-  const int nc = R.cgrid.nc, row = (blockIdx.x - blk0[rid]) * 256 + threadIdx.x;
-  if (row >= nc) return;
-  float v = 0.0f;
-  for (int s = 0; s < R.csplit; ++s) v += R.cecp[(size_t)s * nc + row];
-  R.cec[row] = v;
-}
-
-// z += P_c e on the RVE's rows (the 8 coarse nodes around a node, zero
-// weights outside) and the block's (r, z) partial in place of the Jacobi one:
-// part[lb * 3 + 1] at the start (where p = z as well), else the (r, z) slot
-// of kb_m_step2's partials
-__global__ void __launch_bounds__(256) kb_c_zfix(const BRve *rv, const int *map, const int *blk0, const int *act,
-                                                 int parity) {
-  __shared__ double lds[4];
-  const int rid = map[blockIdx.x];
-  const BRve &R = rv[rid];
-  if (kb_c_skip(R, act, rid, parity)) return;
-  const Grid &g = R.g;
-  const CGrid &cg = R.cgrid;
-  const int lb = blockIdx.x - blk0[rid], row = lb * 256 + threadIdx.x;  // < nrow_pad
-  float z = R.z32[row];
-  const float r = R.r32[row];
-  if (row < g.nrow) {
-    const int node = row / 3, d = row % 3;
-    const int i = node % g.nx, j = (node / g.nx) % g.ny, k = node / (g.nx * g.ny);
-    float wx[2], wy[2], wz[2];
-    int qx[2], qy[2], qz[2];
-    hat_pair(i, cg.hx, cg.mx, wx, qx);
-    hat_pair(j, cg.hy, cg.my, wy, qy);
-    hat_pair(k, cg.hz, cg.mz, wz, qz);
-    float e[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-      e[t] = R.cec[((qz[t >> 2] * cg.my + qy[(t >> 1) & 1]) * cg.mx + qx[t & 1]) * 3 + d];
-    float acc = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) acc += wx[t & 1] * (wy[(t >> 1) & 1] * wz[t >> 2]) * e[t];
-    z += acc;
-  }
-  R.z32[row] = z;
-  if (act) R.p32[row] = z;
-  double v[1] = {(double)r * z};
-  block_sum<1, 256>(v, lds);
-  if (threadIdx.x == 0) {
-    if (act)
-      R.part[(size_t)lb * 3 + 1] = v[0];
-    else
-      R.part[R.nb_row + (size_t)lb * 2 + 1] = v[0];
-  }
-}
-
-// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-static hipError_t launch_bc(const BLaunch &L, const int *act, int parity, hipStream_t st) {
-  hipLaunchKernelGGL(kb_c_rx, dim3(L.crx.nb), dim3(256), 0, st, L.rv, L.crx.map, L.crx.blk0, act, parity);
-  hipLaunchKernelGGL(kb_c_ryz, dim3(L.cryz.nb), dim3(256), 0, st, L.rv, L.cryz.map, L.cryz.blk0, act, parity);
-  hipLaunchKernelGGL(kb_c_gemv, dim3(L.cgemv.nb), dim3(256), 0, st, L.rv, L.cgemv.map, L.cgemv.blk0, act, parity);
-  if (L.cgsum.nb)
-    hipLaunchKernelGGL(kb_c_gsum, dim3(L.cgsum.nb), dim3(256), 0, st, L.rv, L.cgsum.map, L.cgsum.blk0, act, parity);
-  hipLaunchKernelGGL(kb_c_zfix, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, act, parity);
-  return hipGetLastError();
-}
-
 hipError_t launch_b_set_bc(const BLaunch &L, const double *eps, hipStream_t st) {
   hipLaunchKernelGGL(kb_set_bc, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.act, L.row.blk0, eps);
   return hipGetLastError();
@@ -597,12 +600,12 @@ hipError_t launch_b_spmv(const BLaunch &L, int shape, int parity, hipStream_t st
   const int nb = L.row.nb, per = (nb + 7) / 8;
   const dim3 plain(nb), xcd(8 * per);
   switch (shape) {
-    case 0: hipLaunchKernelGGL((kb_cg_step1<9, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
-    case 1: hipLaunchKernelGGL((kb_cg_step1<27, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
-    case 2: hipLaunchKernelGGL((kb_cg_step1<81, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
-    case 3: hipLaunchKernelGGL((kb_cg_step1<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
-    case 4: hipLaunchKernelGGL((kb_cg_step1<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
-    case 5: hipLaunchKernelGGL((kb_cg_step1<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, L.a0on, nb, per, parity); break;
+    case 0: hipLaunchKernelGGL((kb_cg_step1<9, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 1: hipLaunchKernelGGL((kb_cg_step1<27, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 2: hipLaunchKernelGGL((kb_cg_step1<81, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 3: hipLaunchKernelGGL((kb_cg_step1<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 4: hipLaunchKernelGGL((kb_cg_step1<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 5: hipLaunchKernelGGL((kb_cg_step1<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -611,7 +614,7 @@ hipError_t launch_b_spmv(const BLaunch &L, int shape, int parity, hipStream_t st
 hipError_t launch_b_cg_iter(const BLaunch &L, int parity, hipStream_t st) {
   hipError_t e = launch_b_spmv(L, L.spmv_shape, parity, st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kb_cg_step2, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, parity);
+  hipLaunchKernelGGL(kb_cg_step2, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.at, L.cg, parity);
   return hipGetLastError();
 }
 hipError_t launch_b_cg_tail(const BLaunch &L, hipStream_t st) {
@@ -656,8 +659,8 @@ hipError_t launch_bm_resid(const BLaunch &L, int first, double rel, double abs_t
                            const int *tight, double tight_factor, BOuter *out, hipStream_t st) {
   hipLaunchKernelGGL(kb_m_resid, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.act, L.row.blk0, L.a0on);
   if (L.coarse) {
-    const hipError_t e = launch_bc(L, L.act, 0, st);
-    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kb_m_upd<true>, dim3(L.upd.nb), dim3(256), 0, st, L.rv, L.upd.at, L.act, L.cg, 0);
+    hipLaunchKernelGGL(kb_c_gemv, dim3(L.gemv.nb), dim3(256), 0, st, L.rv, L.gemv.at, L.act, L.cg, 0);
   }
   hipLaunchKernelGGL(kb_m_outer, dim3(L.nrve), dim3(256), 0, st, L.rv, L.act, first, rel, abs_tol, tau_min,
                      max_inner, tight, tight_factor, out);
@@ -667,25 +670,28 @@ hipError_t launch_bm_spmv(const BLaunch &L, int shape, int parity, hipStream_t s
   const int nb = L.row.nb, per = (nb + 7) / 8;
   const dim3 plain(nb), xcd(8 * per);
   switch (shape) {
-    case 0: hipLaunchKernelGGL((kb_m_step1<9, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
-    case 1: hipLaunchKernelGGL((kb_m_step1<27, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
-    case 2: hipLaunchKernelGGL((kb_m_step1<81, false>), plain, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
-    case 3: hipLaunchKernelGGL((kb_m_step1<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
-    case 4: hipLaunchKernelGGL((kb_m_step1<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
-    case 5: hipLaunchKernelGGL((kb_m_step1<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, nb, per, parity); break;
+    case 0: hipLaunchKernelGGL((kb_m_spmv<9, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 1: hipLaunchKernelGGL((kb_m_spmv<27, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 2: hipLaunchKernelGGL((kb_m_spmv<81, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 3: hipLaunchKernelGGL((kb_m_spmv<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 4: hipLaunchKernelGGL((kb_m_spmv<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 5: hipLaunchKernelGGL((kb_m_spmv<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 hipError_t launch_bm_iter(const BLaunch &L, int parity, hipStream_t st) {
+  hipLaunchKernelGGL(kb_m_dir, dim3(L.node.nb), dim3(256), 0, st, L.rv, L.node.at, L.cg, parity);
   const hipError_t e = launch_bm_spmv(L, L.spmv_shape32, parity, st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kb_m_step2, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, parity);
-  if (L.coarse) {
-    const hipError_t e2 = launch_bc(L, nullptr, parity, st);
-    if (e2 != hipSuccess) return e2;
-  }
-  hipLaunchKernelGGL(kb_m_step3, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.row.blk0, parity);
+  hipLaunchKernelGGL(kb_m_upd<false>, dim3(L.upd.nb), dim3(256), 0, st, L.rv, L.upd.at, L.act, L.cg, parity);
+  if (L.coarse)
+    hipLaunchKernelGGL(kb_c_gemv, dim3(L.gemv.nb), dim3(256), 0, st, L.rv, L.gemv.at, (const int *)nullptr, L.cg,
+                       parity);
+  return hipGetLastError();
+}
+hipError_t launch_bm_tail(const BLaunch &L, hipStream_t st) {
+  hipLaunchKernelGGL(kb_m_tail, dim3(L.nrve), dim3(256), 0, st, L.rv, L.cg);
   return hipGetLastError();
 }
 hipError_t launch_bm_accum(const BLaunch &L, hipStream_t st) {

@@ -6,7 +6,16 @@
 
 namespace mpp {
 
+constexpr int kGemvRows = 8;  // coarse rows per block of the coarse solve (two per wave)
 constexpr int kSpmvShapes = 6, kSpmvDefault = 4;  // default: 27 slots, XCD-grouped blocks
+
+// Trilinear hats along one side at one fine index: the interior coarse nodes
+// below and above it, as offsets into the coarse vectors, and their weights
+// (0 for a node on the boundary, with a valid offset).
+struct HatEntry {
+  float w0, w1;
+  int q0, q1;
+};
 
 // One RVE of a batch: its geometry and every device array the FP64 path
 // touches.  Row-space arrays hold nrow_pad entries, element arrays nelem
@@ -29,27 +38,30 @@ struct BRve {
   // mixed precision (nullptr without): the FP32 copy of the matrix being
   // solved (vals' layout), the inner CG's FP32 vectors and Jacobi weights;
   // x holds the FP64 correction du, r the FP64 residual, kinv the FP64 D^-1
-  float *vals32, *x32, *r32, *z32, *p32, *Ap32, *kinv32;
+  float *vals32, *x32, *r32[2], *p32, *Ap32, *kinv32;
   // mixed precision, two-level preconditioner of the inner CG (cgrid.nc = 0:
   // Jacobi alone): the inverse of the Galerkin coarse matrix of the RVE's
-  // initial (elastic) tangent, the x-restricted residual (3 nz ny mx), the
-  // restricted residual and the coarse correction (nc each)
+  // initial (elastic) tangent, the restricted residual and the coarse
+  // correction (nc each), the coarse solve's partials of their product, and
+  // the hats along x, y and z
   CGrid cgrid;
+  const HatEntry *hat[3];
   const float *cainv;
-  float *ct1, *crc, *cec;
-  int csplit;    // column splits of the coarse solve
-  float *cecp;   // their partial products (csplit > 1), csplit x nc
+  float *crc, *cec;
+  double *cpart;
   int phase_mode;              // all phases elastic: one Ke per phase
   int use_vars;                // the RVE has history (vars_n / vars_k in use)
   int nb_row, nb_elem;
 };
 
 // One launch shape: nb blocks in all; map[block] = RVE; blk0[rve] = the
-// RVE's first block.
+// RVE's first block; at[block] = {RVE, block within it}, one load instead of
+// two in a row.
 struct BShape {
   int nb;
   const int *map;
   const int *blk0;
+  const int2 *at;
 };
 
 // Outer (defect-correction) test of one RVE: pn = ||D^-1 (b - A du)||, pn0
@@ -81,12 +93,10 @@ struct BLaunch {
   const int *act;  // per-RVE activity mask of this launch
   const int *a0on;  // per RVE: the CG solves with a0 instead of vals
   BShape row, elem, ke;
-  // the two-level preconditioner's shapes: x-restriction (threads per
-  // (direction, interior x-line, coarse x node)), y/z-restriction (a wave per
-  // coarse DOF), coarse solve (64 coarse rows x one column split per block),
-  // the splits' sum (RVEs with more than one split); coarse = some RVE has a
-  // coarse level
-  BShape crx, cryz, cgemv, cgsum;
+  CgState *cg;  // the RVEs' state pairs
+  // the inner CG's shapes: nodes, rows and then coarse nodes, coarse rows
+  // (kGemvRows a block); coarse = some RVE has a coarse level
+  BShape node, upd, gemv;
   int coarse = 0;
   int spmv_shape = kSpmvDefault;    // see launch_b_spmv
   int spmv_shape32 = kSpmvDefault;  // the same choice for the inner FP32 SpMV (launch_bm_spmv)
@@ -150,6 +160,8 @@ hipError_t launch_bm_resid(const BLaunch &L, int first, double rel, double abs_t
 // one inner CG iteration of every RVE (done RVEs return at once); with a
 // coarse level, z = D^-1 r + P_c A_c^-1 P_c^T r
 hipError_t launch_bm_iter(const BLaunch &L, int parity, hipStream_t st);
+// the sums of the last of an even number of inner iterations into cg[0]
+hipError_t launch_bm_tail(const BLaunch &L, hipStream_t st);
 // the inner FP32 SpMV alone in one of kSpmvShapes shapes, as launch_b_spmv
 hipError_t launch_bm_spmv(const BLaunch &L, int shape, int parity, hipStream_t st);
 // du += x32

@@ -26,10 +26,7 @@ constexpr double kDEpsCtanAve = 1e-8;  // D_EPS_CTAN_AVE (include/params.hpp:32)
 // coarse DOFs per RVE of a mixed-precision batch: every inner iteration
 // reads the nc^2 FP32 inverse beside the RVE's 324 B/row FP32 matrix, so nc
 // is held to max(400, 4 sqrt(rows)), an inverse of at most 64 B per row
-// (30^3: 6 coarse elements a side, 375 DOFs; 40^3: 8, 1029; 50^3: 10, 2187)
-// columns per split of the coarse solve (kb_c_gemv); more than one split is
-// summed by kb_c_gsum
-constexpr int kBatchCoarseSplitCols = 512;
+// (24^3 to 30^3 elements: 375 to 1029 DOFs; 40^3: 1029; 50^3: 2187)
 int batch_coarse_max_dofs(const Grid &g) { return std::max(400, (int)(4.0 * std::sqrt((double)g.nrow))); }
 
 struct BState {
@@ -55,13 +52,16 @@ struct mppd_batch {
   std::vector<BState> s;
   BRve *rv = nullptr;
   // launch shapes
-  // launch shapes: rows, elements, element stiffness, then the coarse
-  // level's x-restriction, y/z-restriction and coarse solve
-  static constexpr int kShapes = 7;
+  // launch shapes: rows, elements, element stiffness, then the inner CG's
+  // nodes, rows and coarse nodes, coarse rows
+  static constexpr int kShapes = 6;
   int *map_d[kShapes] = {}, *blk0_d[kShapes] = {};
+  int2 *at_d[kShapes] = {};
   int nb[kShapes] = {};
   int coarse_any = 0;    // mixed precision: some RVE has a coarse level
   float *c32 = nullptr;  // coarse arena: inverses, restriction and correction vectors
+  double *cpart = nullptr;  // partials of the coarse solves
+  HatEntry *hat_d = nullptr;  // hats of the coarse grids
   // arenas
   double *vec = nullptr, *vals = nullptr, *ke = nullptr, *be = nullptr, *vars = nullptr, *part = nullptr;
   double *a0 = nullptr;  // initial matrices (use_A0), one per distinct RVE
@@ -112,13 +112,9 @@ struct mppd_batch {
     L.rv = rv;
     L.act = mask_d[mask];
     L.a0on = mask_d[M_A0];
-    L.row = {nb[0], map_d[0], blk0_d[0]};
-    L.elem = {nb[1], map_d[1], blk0_d[1]};
-    L.ke = {nb[2], map_d[2], blk0_d[2]};
-    L.crx = {nb[3], map_d[3], blk0_d[3]};
-    L.cryz = {nb[4], map_d[4], blk0_d[4]};
-    L.cgemv = {nb[5], map_d[5], blk0_d[5]};
-    L.cgsum = {nb[6], map_d[6], blk0_d[6]};
+    L.cg = cg;
+    BShape *const shapes[kShapes] = {&L.row, &L.elem, &L.ke, &L.node, &L.upd, &L.gemv};
+    for (int k = 0; k < kShapes; ++k) *shapes[k] = {nb[k], map_d[k], blk0_d[k], at_d[k]};
     L.coarse = coarse_any;
     L.spmv_shape = spmv_shape;
     L.spmv_shape32 = spmv_shape32;
@@ -346,6 +342,7 @@ int cg_batch_mixed(mppd_batch *B, const std::vector<int> &on, const std::vector<
       queued += reps * G;
       B->cg_queued += reps * G;
       B->graph_launches += reps;
+      MPP_HIP(launch_bm_tail(L, B->st));
       if ((rc = read_cg(B))) return rc;
       all = true;
       int next = 0;
@@ -752,9 +749,10 @@ void destroy(mppd_batch *B) {
   for (int k = 0; k < mppd_batch::kShapes; ++k) {
     dfree(B->map_d[k]);
     dfree(B->blk0_d[k]);
+    dfree(B->at_d[k]);
   }
   for (void *p : {(void *)B->rv, (void *)B->vec, (void *)B->vals, (void *)B->a0, (void *)B->f32, (void *)B->c32,
-                  (void *)B->outer_d, (void *)B->ke, (void *)B->be, (void *)B->vars, (void *)B->part, (void *)B->cg,
+                  (void *)B->cpart, (void *)B->hat_d, (void *)B->outer_d, (void *)B->ke, (void *)B->be, (void *)B->vars, (void *)B->part, (void *)B->cg,
                   (void *)B->flags_d, (void *)B->eps_d, (void *)B->norms_d, (void *)B->sig_d, (void *)B->nst_d,
                   (void *)B->pend_d})
     dfree(p);
@@ -832,6 +830,17 @@ int setup_a0(mppd_batch *B, const mppd_batch_rve *in) {
   return upload_table(B);
 }
 
+// the hats along a side of ne fine and d coarse elements: coarse node q (0 .. d)
+// at fine index floor(q ne / d), an interior one at offset (q - 1) stride
+void add_hats(std::vector<HatEntry> &out, int ne, int d, int stride) {
+  for (int i = 0; i <= ne; ++i) {
+    const int e = std::min(((i + 1) * d - 1) / ne, d - 1), a = e * ne / d, b = (e + 1) * ne / d;  // coarse element
+    const float f = (float)(i - a) / (float)(b - a);
+    out.push_back({e >= 1 ? 1.0f - f : 0.0f, e + 1 < d ? f : 0.0f, (std::max(e, 1) - 1) * stride,
+                   (std::min(e + 1, d - 1) - 1) * stride});
+  }
+}
+
 // The coarse levels of a mixed-precision batch: per RVE with a coarse grid,
 // the FP32 inverse of the Galerkin coarse matrix of its initial tangent
 // (per-phase element stiffness at u = 0 without history: the elastic one),
@@ -841,6 +850,11 @@ int setup_coarse(mppd_batch *B, const mppd_batch_rve *in, size_t c32) {
   const int n = B->n;
   int rc = dalloc(&B->c32, c32, false);
   if (rc) return rc;
+  size_t nparts = 0, nhat = 0;
+  for (const BRve &R : B->h) nhat += R.cgrid.nc ? R.g.nx + R.g.ny + R.g.nz : 0;
+  std::vector<HatEntry> hats;
+  if ((rc = dalloc(&B->hat_d, nhat, false))) return rc;
+  if ((rc = dalloc(&B->cpart, (size_t)B->nb[5], false))) return rc;
   double *ke = nullptr;
   if ((rc = dalloc(&ke, 3 * 576, false))) return rc;
   std::vector<int> owner(n, -1);
@@ -872,18 +886,20 @@ int setup_coarse(mppd_batch *B, const mppd_batch_rve *in, size_t c32) {
       owner[r] = r;
       R.cainv = ainv;
     }
-    R.ct1 = B->c32 + off;
-    off += (size_t)3 * g.nz * g.ny * cg.mx;
     R.crc = B->c32 + off;
     R.cec = B->c32 + off + cg.nc;
     off += 2 * (size_t)cg.nc;
-    if (R.csplit > 1) {
-      R.cecp = B->c32 + off;
-      off += (size_t)R.csplit * cg.nc;
+    const int ne[3] = {g.nex, g.ney, g.nez}, m[3] = {cg.mx, cg.my, cg.mz};
+    for (int a = 0, stride = 3; a < 3; stride *= m[a++]) {
+      R.hat[a] = B->hat_d + hats.size();
+      add_hats(hats, ne[a], m[a] + 1, stride);
     }
+    R.cpart = B->cpart + nparts;
+    nparts += (size_t)(cg.nc + kGemvRows - 1) / kGemvRows;
   }
   (void)hipStreamSynchronize(B->st);
   dfree(ke);
+  if (!rc) MPP_HIP(hipMemcpy(B->hat_d, hats.data(), sizeof(HatEntry) * hats.size(), hipMemcpyHostToDevice));
   return rc;
 }
 
@@ -906,6 +922,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
   // coarse grid (a small one: its inverse is read by every inner iteration)
   constexpr int kS = mppd_batch::kShapes;
   std::vector<int> map[kS], blk0[kS];
+  std::vector<int2> at[kS];
   size_t rows = 0, slots = 0, kes = 0, bes = 0, nvars = 0, parts = 0, c32 = 0;
   for (int k = 0; k < kS; ++k) blk0[k].assign(n, 0);
   const bool coarse = B->prm.mixed_precision && coarse_enabled();
@@ -919,20 +936,22 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     R.nb_elem = (g.nelem + 255) / 256;
     const int nb_ke = ((R.phase_mode ? 3 : g.nelem) + kKeWaves - 1) / kKeWaves;
     R.cgrid = CGrid{};
-    if (coarse && !coarse_grid(g, batch_coarse_max_dofs(g), &R.cgrid)) R.cgrid = CGrid{};
+    if (coarse && !coarse_grid_wide(g, 2, batch_coarse_max_dofs(g), &R.cgrid)) R.cgrid = CGrid{};
     const CGrid &cg = R.cgrid;
-    const int nrx = cg.nc ? (3 * (g.ny - 2) * (g.nz - 2) * cg.mx + 255) / 256 : 0;
-    R.csplit = (cg.nc + kBatchCoarseSplitCols - 1) / kBatchCoarseSplitCols;
-    const int ngsum = R.csplit > 1 ? (cg.nc + 255) / 256 : 0;
-    const int counts[kS] = {R.nb_row, R.nb_elem, nb_ke, nrx, (cg.nc + 3) / 4, (cg.nc + 63) / 64 * R.csplit, ngsum};
+    const int counts[kS] = {R.nb_row,
+                            R.nb_elem,
+                            nb_ke,
+                            (g.nn + 255) / 256,
+                            R.nb_row + cg.nq,
+                            (cg.nc + kGemvRows - 1) / kGemvRows};
     if (cg.nc) {
       B->coarse_any = 1;
-      c32 += (size_t)cg.nc * cg.nc + (size_t)3 * g.nz * g.ny * cg.mx + 2 * (size_t)cg.nc;
-      if (R.csplit > 1) c32 += (size_t)R.csplit * cg.nc;
+      c32 += (size_t)cg.nc * cg.nc + 2 * (size_t)cg.nc;
     }
     for (int k = 0; k < kS; ++k) {
       blk0[k][r] = (int)map[k].size();
       map[k].insert(map[k].end(), counts[k], r);
+      for (int b = 0; b < counts[k]; ++b) at[k].push_back(make_int2(r, b));
     }
     rows += g.nrow_pad;
     slots += (size_t)g.nrow_pad * kSlots;
@@ -941,10 +960,14 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     if (!v->all_elastic) nvars += (size_t)g.nelem * 8 * NVAR;
     parts += std::max<size_t>(3 * (size_t)R.nb_row, 6 * (size_t)R.nb_elem);
   }
+  // the coarse nodes' blocks, which take longest, start first
+  std::stable_partition(at[4].begin(), at[4].end(), [&](const int2 &b) { return b.y >= B->h[b.x].nb_row; });
   for (int k = 0; k < kS; ++k) {
     B->nb[k] = (int)map[k].size();
     if ((rc = dalloc(&B->map_d[k], map[k].size(), false))) return rc;
     if ((rc = dalloc(&B->blk0_d[k], n, false))) return rc;
+    if ((rc = dalloc(&B->at_d[k], at[k].size(), false))) return rc;
+    MPP_HIP(hipMemcpy(B->at_d[k], at[k].data(), sizeof(int2) * at[k].size(), hipMemcpyHostToDevice));
     MPP_HIP(hipMemcpy(B->map_d[k], map[k].data(), sizeof(int) * map[k].size(), hipMemcpyHostToDevice));
     MPP_HIP(hipMemcpy(B->blk0_d[k], blk0[k].data(), sizeof(int) * n, hipMemcpyHostToDevice));
   }
@@ -995,13 +1018,13 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     o_part += std::max<size_t>(3 * (size_t)R.nb_row, 6 * (size_t)R.nb_elem);
   }
   if (B->prm.mixed_precision) {
-    constexpr int kVecs32 = 6;  // x32 r32 z32 p32 Ap32 kinv32
+    constexpr int kVecs32 = 6;  // x32 r32[2] p32 Ap32 kinv32
     if ((rc = dalloc(&B->f32, slots + rows * kVecs32))) return rc;
     size_t os = 0, orow = 0;
     for (int r = 0; r < n; ++r) {
       BRve &R = B->h[r];
       R.vals32 = B->f32 + os;
-      float **v[kVecs32] = {&R.x32, &R.r32, &R.z32, &R.p32, &R.Ap32, &R.kinv32};
+      float **v[kVecs32] = {&R.x32, &R.r32[0], &R.r32[1], &R.p32, &R.Ap32, &R.kinv32};
       for (int q = 0; q < kVecs32; ++q) *v[q] = B->f32 + slots + rows * q + orow;
       os += (size_t)R.g.nrow_pad * kSlots;
       orow += R.g.nrow_pad;

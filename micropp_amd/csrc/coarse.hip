@@ -514,11 +514,13 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out) {
 // at h = 5), while the dense inverse stays small: 375 coarse DOFs at 30^3
 // against 2187 at h = 3, whose inverse (19 MB read an iteration) and
 // factorisation (1.2 ms) cost more than the two iterations.
-bool coarse_grid_cycle(const Grid &g, CGrid *out) {
+bool coarse_grid_cycle(const Grid &g, CGrid *out) { return coarse_grid_wide(g, 5, kCoarseMaxDofs, out); }
+
+bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
   if (g.nex < 4 || g.ney < 4 || g.nez < 4) return false;
   if (g.nx > kCoarseMaxLine || g.ny > kCoarseMaxLine || g.nz > kCoarseMaxLine) return false;
   const int ne[3] = {g.nex, g.ney, g.nez};
-  for (int most = 5; most <= kCoarseMaxLine; ++most) {  // the widest coarse element looked at
+  for (int most = least; most <= kCoarseMaxLine; ++most) {  // the widest coarse element looked at
     int h[3], l[3], m[3];
     for (int d = 0; d < 3; ++d) {
       const int n = std::max(2, (ne[d] + most - 1) / most);
@@ -526,7 +528,7 @@ bool coarse_grid_cycle(const Grid &g, CGrid *out) {
       l[d] = h[d] + (ne[d] % n != 0);
       m[d] = n - 1;
     }
-    if (3 * m[0] * m[1] * m[2] > kCoarseMaxDofs) continue;
+    if (3 * m[0] * m[1] * m[2] > max_dofs) continue;
     const CGrid cg = make_grid(h[0], h[1], h[2], l[0], l[1], l[2], m[0], m[1], m[2]);
     // the set-up's table holds every position along a side (h, and l of the wider elements)
     if (coarse_table_len(cg) / (3 * 576) > (size_t)kCoarseMaxPos * 4) return false;

@@ -117,7 +117,7 @@ inline bool alloc_fault_injected() {
 // (cy - 1)) mx + (cx - 1).
 struct CGrid {
   int hx, hy, hz;  // fine elements per coarse element
-  int lx, ly, lz;  // = h where all are h wide; else some are l wide (multilevel preconditioner only)
+  int lx, ly, lz;  // = h where all are h wide; else some are l wide
   int mx, my, mz;  // interior coarse nodes per side
   int nq, nc;      // interior coarse nodes, coarse DOFs (3 nq)
 };
@@ -165,6 +165,8 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out);
 // of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
 // divide the side, l = h + 1); false: none
 bool coarse_grid_cycle(const Grid &g, CGrid *out);
+// the same with the narrowest coarse elements of at least `least` fine ones a side and at most max_dofs coarse DOFs
+bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out);
 // C (device, coarse_table_len(cg) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position
 // (position px of a side: px < h in a regular element, h + px in a last element of another width)
 size_t coarse_table_len(const CGrid &cg);

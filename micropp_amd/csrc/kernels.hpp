@@ -498,49 +498,57 @@ __device__ __forceinline__ T row_dot_grid(const Grid &g, const T *vals, const T 
 }
 
 // The gathers of row_dot_grid for a block of 256 consecutive rows, staged in
-// LDS: the block's rows belong to nodes n_lo .. n_hi (at most 86), whose
-// stencil neighbours lie on 9 runs of consecutive nodes (one per (dz, dy)),
-// each n_hi - n_lo + 3 <= kSegNodes long.  The block copies those runs
-// (clamped node indices, as row_dot_grid clamps each neighbour) into seg once,
-// coalesced, and every row reads its 81 values there instead of gathering
-// them from L1/L2: the same values in the same slot order, so the result is
-// bit-identical to row_dot_grid.  Every thread of the block must call it.
+// LDS.  The rows belong to 86 nodes from n_lo = row0 / 3 on (wherever the
+// block starts), whose stencil neighbours lie on runs of consecutive nodes:
+// one of 88 nodes per (dz, dy), or, while those of one dz overlap (a line of
+// at most 88 nodes), one run per dz.  The block writes f(entry) of every node
+// on the runs (clamped node indices, as row_dot_grid clamps each neighbour)
+// once, coalesced, and every row reads its 81 values there instead of
+// gathering them from L1/L2: the same values in the same slot order, so the
+// result is bit-identical to row_dot_grid.  ly and lz are the LDS distances,
+// in nodes, of a line and of a plane.  Every thread of the block must call it.
 constexpr int kSegNodes = 88;
-template <typename T>
-__device__ __forceinline__ void stage_grid_runs(const Grid &g, int row0, const T *x, T (*seg)[kSegNodes * 3]) {
-  const int n_lo = row0 / 3, n_hi = (row0 + 255) / 3, len = (n_hi - n_lo + 3) * 3;
-  const int nxny = g.nx * g.ny, hi = g.nn - 1;
-  for (int idx = threadIdx.x; idx < 9 * len; idx += 256) {
-    const int sgi = idx / len, e3 = idx - sgi * len;
-    const int base = n_lo - 1 + (sgi / 3 - 1) * nxny + (sgi % 3 - 1) * g.nx;
-    const int m = min(max(base + e3 / 3, 0), hi);
-    seg[sgi][e3] = x[3 * m + e3 % 3];
-  }
-  __syncthreads();
+struct SegPitch {
+  int ly, lz;
+};
+template <typename T, typename F>
+__device__ __forceinline__ SegPitch stage_runs(const Grid &g, int row0, T *seg /* [9 * kSegNodes * 3] */, F f) {
+  const bool joined = g.nx <= kSegNodes;
+  const int len = joined ? kSegNodes + 2 * g.nx : kSegNodes;
+  const SegPitch pt{joined ? g.nx : kSegNodes, joined ? len : 3 * kSegNodes};
+  const int n_lo = row0 / 3, nxny = g.nx * g.ny, hi = g.nn - 1, runs = joined ? 1 : 3;
+  for (int dz = -1; dz <= 1; ++dz)
+    for (int y = 0; y < runs; ++y) {
+      const int n0 = n_lo - 1 + dz * nxny + (y - 1) * g.nx;
+      T *out = seg + ((dz + 1) * pt.lz + y * kSegNodes) * 3;
+#pragma unroll 2
+      for (int e3 = threadIdx.x; e3 < 3 * len; e3 += 256)
+        out[e3] = f(3 * min(max(n0 + e3 / 3, 0), hi) + e3 % 3);
+    }
+  lds_barrier();
+  return pt;
 }
 
-template <int CH = kChunk, typename T>
-__device__ __forceinline__ T row_dot_grid_seg(const T *vals, const T (*seg)[kSegNodes * 3], int row0, int row) {
+// One row's products with the staged runs (own: its node there), in slot
+// order: the first chunk's values are loaded by the caller, each later chunk's
+// before the products of the one in front.
+template <int CH, typename T>
+__device__ __forceinline__ T dot_runs(const T *v, T (&vi)[2][CH], const T *own, SegPitch pt) {
 #pragma clang fp contract(off)
   static_assert(kSlots % CH == 0 && CH % 3 == 0, "chunks tile the row in whole neighbours");
-  const size_t base = (size_t)(row >> 6) * kSlots * 64 + (row & 63);
-  const T *v = vals + base;
-  const int e0 = row / 3 - row0 / 3;  // the row's node within the runs, less 1
   T acc = 0;
 #pragma unroll
   for (int ch = 0; ch < kSlots / CH; ++ch) {
-    T vi[CH], xv[CH];
+    if (ch + 1 < kSlots / CH)
 #pragma unroll
-    for (int k = 0; k < CH; ++k) vi[k] = __builtin_nontemporal_load(&v[(ch * CH + k) * 64]);
+      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = __builtin_nontemporal_load(&v[((ch + 1) * CH + k) * 64]);
 #pragma unroll
     for (int k = 0; k < CH; k += 3) {
-      const int nb = (ch * CH + k) / 3;
-      const T *sv = &seg[nb / 3][(e0 + nb % 3) * 3];
+      const int n = (ch * CH + k) / 3;
+      const T *sv = own + ((n / 9 - 1) * pt.lz + ((n / 3) % 3 - 1) * pt.ly + n % 3 - 1) * 3;
 #pragma unroll
-      for (int fj = 0; fj < 3; ++fj) xv[k + fj] = sv[fj];
+      for (int fj = 0; fj < 3; ++fj) acc += vi[ch & 1][k + fj] * sv[fj];
     }
-#pragma unroll
-    for (int k = 0; k < CH; ++k) acc += vi[k] * xv[k];
   }
   return acc;
 }
@@ -684,7 +692,6 @@ __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, c
                                                 const double *r, const double *p, double *pn, double *Ap,
                                                 double *part1, const CgState *cur, CgState *nxt) {
 #pragma clang fp contract(off)
-  static_assert(kSlots % CH == 0 && CH % 3 == 0, "chunks tile the row in whole neighbours");
   __shared__ double seg[9 * kSegNodes * 3];
   __shared__ double lds[4];
   CgRegs c = cg_load(cur);
@@ -695,41 +702,11 @@ __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, c
 #pragma unroll
     for (int k = 0; k < CH; ++k) vi[0][k] = __builtin_nontemporal_load(&v[k * 64]);
   if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
-  // the block's 86 nodes (wherever its 256 rows start) and their stencil
-  // neighbours: one contiguous run of 88 nodes per (dz, dy), or, while those of
-  // one dz overlap, one run per dz
-  const bool joined = g.nx <= kSegNodes;
-  const int ly = joined ? g.nx : kSegNodes, ny = joined ? 1 : 3;  // LDS pitch of dy; runs per dz
-  const int len = joined ? kSegNodes + 2 * g.nx : kSegNodes, lz = joined ? len : 3 * kSegNodes;
-  const int n_lo = row0 / 3, nxny = g.nx * g.ny, hi = g.nn - 1;
-  for (int dz = -1; dz <= 1; ++dz)
-    for (int y = 0; y < ny; ++y) {
-      const int n0 = n_lo - 1 + dz * nxny + (y - 1) * g.nx;
-      double *out = seg + ((dz + 1) * lz + y * kSegNodes) * 3;
-#pragma unroll 2
-      for (int e3 = threadIdx.x; e3 < 3 * len; e3 += 256) {
-        const int q = 3 * min(max(n0 + e3 / 3, 0), hi) + e3 % 3;
-        out[e3] = cg_dir(c, kinv[q], r[q], p[q]);
-      }
-    }
-  lds_barrier();
-  const double *own = seg + (row / 3 - n_lo + 1 + ly + lz) * 3;  // the row's node
+  const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return cg_dir(c, kinv[q], r[q], p[q]); });
+  const double *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
   // rows past the last node lie on its run's clamped end; p is zero there
   const double pv = row < g.nrow ? own[row % 3] : 0.0;
-  double acc = 0;
-#pragma unroll
-  for (int ch = 0; ch < kSlots / CH; ++ch) {
-    if (ch + 1 < kSlots / CH)
-#pragma unroll
-      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = __builtin_nontemporal_load(&v[((ch + 1) * CH + k) * 64]);
-#pragma unroll
-    for (int k = 0; k < CH; k += 3) {
-      const int n = (ch * CH + k) / 3;
-      const double *sv = own + ((n / 9 - 1) * lz + ((n / 3) % 3 - 1) * ly + n % 3 - 1) * 3;
-#pragma unroll
-      for (int fj = 0; fj < 3; ++fj) acc += vi[ch & 1][k + fj] * sv[fj];
-    }
-  }
+  const double acc = dot_runs<CH>(v, vi, own, pt);
   pn[row] = pv;
   Ap[row] = acc;
   double t[1] = {pv * acc};
@@ -792,82 +769,28 @@ __device__ __forceinline__ void cg_tail_body(const double *part2, int nb, CgStat
   if (threadIdx.x == 0) cg_store(c, 1, state);
 }
 
-// ---------------------------------------------------------------------------
-// The FP32 inner CG of the mixed-precision batch, three kernels per iteration
-// (its preconditioner runs between the second and the third): step1 Ap = A p,
-// step2 alpha, x, r, z = k r, step3 beta, p = z + beta p and the new scalars,
-// read from state[k & 1] and written to state[(k+1) & 1].  Products and
-// partials are formed in FP64.
-// ---------------------------------------------------------------------------
-template <int CH = kChunk, typename T>
-__device__ __forceinline__ void cg_step1_body(const Grid &g, int lb, const T *vals, const T *p, T *Ap, double *part1,
-                                              const CgState *cur) {
+// Ap = A p and the partials of p.Ap of the FP32 inner CG (mixed-precision
+// batch), p in memory; products of p and Ap are formed in FP64
+template <int CH>
+__device__ __forceinline__ void cg_spmv_body32(const Grid &g, int lb, const float *vals, const float *p, float *Ap,
+                                               double *part1, const CgState *cur) {
 #pragma clang fp contract(off)
+  __shared__ float seg[9 * kSegNodes * 3];
   __shared__ double lds[4];
+  const int row0 = lb * 256, row = row0 + threadIdx.x;
+  const float *v = vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
   if (cur->done) return;
-  const int row = lb * 256 + threadIdx.x;
-  __shared__ T seg[9][kSegNodes * 3];
-  stage_grid_runs(g, lb * 256, p, seg);
-  const T y = row_dot_grid_seg<CH>(vals, seg, lb * 256, row);
+  float vi[2][CH];
+#pragma unroll
+  for (int k = 0; k < CH; ++k) vi[0][k] = __builtin_nontemporal_load(&v[k * 64]);
+  const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return p[q]; });
+  const float *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
+  const float pv = row < g.nrow ? own[row % 3] : 0.0f;
+  const float y = dot_runs<CH>(v, vi, own, pt);
   Ap[row] = y;
-  double v[1] = {(double)p[row] * (double)y};
-  block_sum<1, 256>(v, lds);
-  if (threadIdx.x == 0) part1[lb] = v[0];
-}
-
-template <typename T>
-__device__ __forceinline__ void cg_step2_body(int lb, int nb, T *x, T *r, T *z, const T *p, const T *Ap,
-                                              const T *kinv, const double *part1, double *part2,
-                                              const CgState *cur) {
-#pragma clang fp contract(off)
-  __shared__ double lds[4 * 2];
-  if (cur->done) return;
-  double pap[1];
-  seg_sum<1>(part1, nb, pap);
-  const double alpha = cur->rz / pap[0];
-  const int row = lb * 256 + threadIdx.x;
-  x[row] += alpha * p[row];
-  const T rv = r[row] - alpha * Ap[row];
-  r[row] = rv;
-  const T zv = kinv[row] * rv;
-  z[row] = zv;
-  double v[2] = {(double)zv * zv, (double)rv * zv};
-  block_sum<2, 256>(v, lds);
-  if (threadIdx.x == 0) {
-    part2[(size_t)lb * 2 + 0] = v[0];
-    part2[(size_t)lb * 2 + 1] = v[1];
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void cg_step3_body(int lb, int nb, const T *z, T *p, const double *part1,
-                                              const double *part2, const CgState *cur, CgState *nxt) {
-#pragma clang fp contract(off)
-  if (cur->done) {
-    if (lb == 0 && threadIdx.x == 0) *nxt = *cur;
-    return;
-  }
-  double t[2];
-  seg_sum<2>(part2, nb, t);
-  const double rz_old = cur->rz;
-  const double beta = t[1] / rz_old;
-  const int row = lb * 256 + threadIdx.x;
-  p[row] = z[row] + beta * p[row];
-  if (lb == 0) {
-    double pap[1];
-    seg_sum<1>(part1, nb, pap);
-    if (threadIdx.x == 0) {
-      CgState c = *cur;
-      c.pAp = pap[0];
-      c.alpha = rz_old / pap[0];
-      c.pn = sqrt(t[0]);
-      c.beta = beta;
-      c.rz = t[1];
-      c.its = cur->its + 1;
-      c.done = cg_done(c);
-      *nxt = c;
-    }
-  }
+  double t[1] = {(double)pv * (double)y};
+  block_sum<1, 256>(t, lds);
+  if (threadIdx.x == 0) part1[lb] = t[0];
 }
 
 // ---------------------------------------------------------------------------
