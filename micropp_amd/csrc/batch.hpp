@@ -9,14 +9,6 @@ namespace mpp {
 constexpr int kGemvRows = 8;  // coarse rows per block of the coarse solve (two per wave)
 constexpr int kSpmvShapes = 6, kSpmvDefault = 4;  // default: 27 slots, XCD-grouped blocks
 
-// Trilinear hats along one side at one fine index: the interior coarse nodes
-// below and above it, as offsets into the coarse vectors, and their weights
-// (0 for a node on the boundary, with a valid offset).
-struct HatEntry {
-  float w0, w1;
-  int q0, q1;
-};
-
 // One RVE of a batch: its geometry and every device array the FP64 path
 // touches.  Row-space arrays hold nrow_pad entries, element arrays nelem
 // entries; the history arrays are null for an all-elastic RVE.

@@ -137,16 +137,25 @@ constexpr int kCoarseSplit = 16;    // column splits of the coarse solve (one pa
 constexpr int kCoarseMaxLine = 256;  // nodes per side a coarse level allows
 constexpr int kCoarseMaxDofs = 2200;  // coarse DOFs of a multi-RHS solver (3 x 9^3 = 2187: 10^3 coarse elements)
 constexpr int kCoarseMaxPos = 4096;   // fine elements per coarse element (the set-up's table size)
+// Trilinear hats along one side at one fine index: the interior coarse nodes
+// below and above it, as offsets into the coarse vectors, and their weights
+// (0 for a node on the boundary, with a valid offset).
+struct HatEntry {
+  float w0, w1;
+  int q0, q1;
+};
+
 // Multilevel (V-cycle) preconditioner of the multi-RHS inner CG on a stencil
 // dictionary (vcycle.hip): Jacobi smoothing on the fine grid and on the grid of
 // twice its spacing (its Galerkin operator stored as FP32 node blocks), and the
-// dense inverse of a coarse Galerkin matrix.
+// dense inverse of a coarse Galerkin matrix.  Small RVEs have no second level
+// (mid.nq = 0): their coarse grid is that fine itself.
 struct VCycleDev {
   CGrid mid, cg;     // second level (h = 2), coarse grid (hats on the fine grid's indices)
+  HatEntry *hat[3];  // the coarse hats along x, y, z
   Grid g1;           // the second level as a grid: m + 2 nodes a side, the boundary among them
   const float *ainv;          // nc x nc
-  float *rc, *ecp;            // restricted residual (nc x K), split partials of the coarse solve (nsplit x nc x K)
-  int nsplit;
+  float *rc, *ec;             // restricted residual and coarse correction (nc x K)
   float *A1, *kinv1;          // second level: node blocks (63 float4 a node, A1[quad * NP1 + node]) and Jacobi weights
   float *R1, *E0, *T1, *E;    // second level: residual, Jacobi part, smoothed residual, correction
   float *z;                   // fine work vector, in R's layout

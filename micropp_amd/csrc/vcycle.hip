@@ -392,7 +392,8 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 //   OUT = Z1 + w0 D^-1 (R - A Z1),
 // P1 the trilinear interpolation from the grid of twice the spacing (an odd
 // side's last element is 1 wide, so every side of at least 4 elements has one).  M1 is the
-// same cycle on that grid with its Galerkin operator A1 = P1^T A P1 and the
+// same cycle on that grid (small RVEs, vcycle_setup: P1 the coarse hats and M1
+// the dense inverse, nothing in between) with its Galerkin operator A1 = P1^T A P1 and the
 // dense inverse of the coarse Galerkin matrix as its correction (P2: the coarse
 // hats at the second level's nodes).  M is symmetric positive definite while w0 and w1 stay
 // below 2 / lambda_max(D^-1 A) of their levels (estimated at set-up by a power
@@ -404,25 +405,26 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 // application an iteration instead of three), 160 us an iteration against 85:
 // sigma and ctan of six strains to 1e-10 in 4.8 ms against 7.5 ms.  Sides
 // without a common divisor (29 x 37 x 23 elements) had no coarse level before:
-// 38 iterations against 250, 2.6 ms against 5.9 ms.
+// 38 iterations against 250, 2.4 ms against 5.9 ms.
 // ---------------------------------------------------------------------------
 
-// the coarse hats of a side of ne fine elements and d coarse ones, node q at
-// fine index c_q = floor(q ne / d): hat q at fine index i, and the interior
-// coarse nodes (0-based) below and above i with their weights (a boundary node:
-// weight 0, a valid index)
-__device__ __forceinline__ float hat_at(int i, int q, int ne, int d) {
-  const int c = q * ne / d, a = (q - 1) * ne / d, b = (q + 1) * ne / d;
-  return i <= a || i >= b ? 0.0f : i <= c ? (float)(i - a) / (float)(c - a) : (float)(b - i) / (float)(b - c);
-}
-__device__ __forceinline__ void hat_pair_at(int i, int ne, int d, float (&w)[2], int (&q)[2]) {
-  const int e = ((i + 1) * d - 1) / ne, a = e * ne / d, b = (e + 1) * ne / d;  // the coarse element [a, b) of i < ne
+// the coarse hats along a side of ne fine elements and d coarse ones, node q at
+// fine index floor(q ne / d) (HatEntry, at every fine index), offsets of stride
+// per interior coarse node
+__global__ void __launch_bounds__(256) k_v_hats(int ne, int d, int stride, HatEntry *out) {
+  const int i = threadIdx.x;  // sides have at most kCoarseMaxLine = 256 nodes
+  if (i > ne) return;
+  const int e = min(((i + 1) * d - 1) / ne, d - 1), a = e * ne / d, b = (e + 1) * ne / d;  // the coarse element
   const float f = (float)(i - a) / (float)(b - a);
-  w[0] = e >= 1 ? 1.0f - f : 0.0f;
-  w[1] = e + 1 < d ? f : 0.0f;
-  q[0] = max(e, 1) - 1;
-  q[1] = min(e + 1, d - 1) - 1;
+  out[i] = {e >= 1 ? 1.0f - f : 0.0f, e + 1 < d ? f : 0.0f, (max(e, 1) - 1) * stride, (min(e + 1, d - 1) - 1) * stride};
 }
+// a hat's weight at an index with entry h, the hat's node at offset o
+__device__ __forceinline__ float hat_weight(const HatEntry &h, int o) {
+  return (h.q0 == o ? h.w0 : 0.0f) + (h.q1 == o ? h.w1 : 0.0f);
+}
+struct Hats {
+  const HatEntry *x, *y, *z;
+};
 
 // R1 = P1^T T and E0 = D1^-1 R1.  One thread per second-level node (boundary
 // ones write zero) and component c = d KG + grp.
@@ -524,121 +526,116 @@ __global__ void __launch_bounds__(MODE == kApplyPow ? 192 : 48 * K)
   }
 }
 
-// rc = P2^T T1: a wave per coarse node and component, its lanes over the
-// second-level nodes under the node's hat, 8 x 8 of a plane at a time
-template <int K>
-__global__ void __launch_bounds__(256) k_v_coarse_rhs(Grid g, Grid g1, CGrid cg, int NP1, const float4 *T1,
+// rc = P^T T for the coarse hats at the nodes of grid gt, node i at fine index
+// S i (the second level, S = 2, or the fine grid itself): a wave per coarse node
+// and component, its lanes over the nodes under the node's hat
+template <int K, int S>
+__global__ void __launch_bounds__(256) k_v_coarse_rhs(Grid g, Grid gt, CGrid cg, Hats hats, int NPt, const float4 *T,
                                                       float4 *rc4, const MState *cur) {
   constexpr int KG = K / 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int id = blockIdx.x * 4 + wv, c = blockIdx.y, d = c / KG, grp = c % KG;
   if (id >= cg.nq || group_stopped(cur, grp * 4)) return;
-  const int cx = id % cg.mx + 1, cy = (id / cg.mx) % cg.my + 1, cz = id / (cg.mx * cg.my) + 1;
-  const int nx = cg.mx + 1, ny = cg.my + 1, nz = cg.mz + 1;
-  // second-level indices with a non-zero hat: fine indices 2 q strictly between the neighbouring coarse nodes
-  const int x0 = (cx - 1) * g.nex / nx / 2 + 1, y0 = (cy - 1) * g.ney / ny / 2 + 1, z0 = (cz - 1) * g.nez / nz / 2 + 1;
-  const int x1 = ((cx + 1) * g.nex / nx - 1) / 2, y1 = ((cy + 1) * g.ney / ny - 1) / 2, z1 = ((cz + 1) * g.nez / nz - 1) / 2;
+  const int cx = id % cg.mx, cy = (id / cg.mx) % cg.my, cz = id / (cg.mx * cg.my);  // interior index, 0-based
+  const int dx = cg.mx + 1, dy = cg.my + 1, dz = cg.mz + 1;
+  // nodes with a non-zero hat: fine indices S i strictly between the neighbouring coarse nodes
+  const int x0 = cx * g.nex / dx / S + 1, y0 = cy * g.ney / dy / S + 1, z0 = cz * g.nez / dz / S + 1;
+  const int wx = ((cx + 2) * g.nex / dx - 1) / S + 1 - x0, wy = ((cy + 2) * g.ney / dy - 1) / S + 1 - y0;
+  const int n = wx * wy * (((cz + 2) * g.nez / dz - 1) / S + 1 - z0);
+  const int ox = 3 * cx, oy = 3 * cg.mx * cy, oz = 3 * cg.mx * cg.my * cz;
+  const float4 *t = T + (size_t)c * NPt;
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int y = y0 + (lane >> 3); y <= y1; y += 8)
-    for (int x = x0 + (lane & 7); x <= x1; x += 8) {
-      const float wxy = hat_at(2 * x, cx, g.nex, nx) * hat_at(2 * y, cy, g.ney, ny);
-      const float4 *t = T1 + (size_t)c * NP1 + (size_t)y * g1.nx + x;
-#pragma unroll 5
-      for (int z = z0; z <= z1; ++z) fma4(acc, wxy * hat_at(2 * z, cz, g.nez, nz), t[(size_t)z * g1.ny * g1.nx]);
-    }
+#pragma unroll 2
+  for (int s = lane; s < n; s += 64) {
+    const int r = s / wx, x = x0 + s % wx, y = y0 + r % wy, z = z0 + r / wy;
+    const float w = hat_weight(hats.x[S * x], ox) * (hat_weight(hats.y[S * y], oy) * hat_weight(hats.z[S * z], oz));
+    fma4(acc, w, t[((size_t)z * gt.ny + y) * gt.nx + x]);
+  }
   acc = make_float4(wave_sum_dpp(acc.x), wave_sum_dpp(acc.y), wave_sum_dpp(acc.z), wave_sum_dpp(acc.w));
   if (lane == 0) rc4[(size_t)(id * 3 + d) * KG + grp] = acc;
 }
 
-// Split partials of ec = A_c^-1 rc: block (64 rows, split of at most kSplitCols
-// columns), the columns over the waves (lane = row; the symmetric inverse is
-// read by column, one coalesced line per column).  A wave's entries of the
-// inverse are all loaded before the split's rows of rc are staged in LDS, where
-// every lane reads the same address.  The waves are added in order;
-// k_v_coarse_add sums the splits.
+// ec = A_c^-1 rc, FP32 matrix instructions.  Block: 16 rows, its waves each a
+// share of the columns, 16 at a time: lane (r = l % 16, k = l / 16) loads the
+// four columns 4 k .. 4 k + 3 of row r (one 16-byte load; four lanes a 64-byte
+// line) and of rc the field r of the same four, so the step t of four 16x16x4
+// products takes column 4 k + t of both operands.  The waves' tiles are added
+// in LDS in order.  What bounds it is two memory latencies, and from about 2000
+// DOFs the inverse (19 MB at 2187, out of L2 and MALL); hence AHEAD steps of a
+// wave are loaded together, all of them up to 1280 columns.  12 fields, us: 375
+// DOFs 4, 2187 DOFs 8.6 (14.4 with one step at a time; a wave per 64 rows and
+// split columns, summed by the next kernel: 10 and 10).
 constexpr int kGemvWaves = 16;
-constexpr int kSplitCols = 512;
-template <int K>
+constexpr int kGemvRowsV = 16;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any multiple of 4 bytes
+template <int K, int AHEAD>
 __global__ void __launch_bounds__(64 * kGemvWaves) k_v_gemv(int nc, const float *__restrict__ ainv,
-                                                            const float4 *__restrict__ rc4,
-                                                            float *__restrict__ ecp, const MState *cur) {
-  constexpr int kW = kGemvWaves, KG = K / 4, kPer = kSplitCols / kW;
-  __shared__ float4 x[kSplitCols * KG];
-  __shared__ float red[kW - 1][64][K + 1];
+                                                            const float *__restrict__ rc, float *__restrict__ ec,
+                                                            const MState *cur) {
+  __shared__ float tile[kGemvWaves][256];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = blockIdx.x * 64 + lane, chunk = (nc + gridDim.y - 1) / gridDim.y;  // <= kSplitCols
-  const int c0 = blockIdx.y * chunk, n = min(nc, c0 + chunk) - c0;
-  const int rowc = min(row, nc - 1);  // loads of rows past nc are clamped, their sums not stored
-  float a[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i)
-    if (w + i * kW < n) a[i] = ainv[(size_t)(c0 + w + i * kW) * nc + rowc];
-  for (int t = threadIdx.x; t < n * KG; t += 64 * kW) x[t] = rc4[(size_t)c0 * KG + t];
+  const int r = lane & 15, k = lane >> 4, row0 = blockIdx.x * kGemvRowsV;
+  // rows past nc are clamped (not stored); columns past nc read on (into the
+  // next row, or the zeros behind the inverse) or, a whole step past it, the
+  // row's start, and meet zeros in place of rc
+  const float *a = ainv + (size_t)min(row0 + r, nc - 1) * nc + 4 * k;
   if (cur->all_done) return;  // whole grid
-  __syncthreads();
-  float4 acc[KG];
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c0 = 16 * w; c0 < nc; c0 += 16 * kGemvWaves * AHEAD) {
+    f32x4u av[AHEAD];
+    float b[AHEAD][4];
 #pragma unroll
-  for (int f = 0; f < KG; ++f) acc[f] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int s = 0; s < AHEAD; ++s) {
+      const int c = c0 + 16 * kGemvWaves * s;
+      av[s] = *reinterpret_cast<const f32x4u *>(a + (c < nc ? c : 0));
 #pragma unroll
-  for (int i = 0; i < kPer; ++i)
-    if (w + i * kW < n)
-#pragma unroll
-      for (int f = 0; f < KG; ++f) fma4(acc[f], a[i], x[(w + i * kW) * KG + f]);
-  if (w > 0)
-#pragma unroll
-    for (int f = 0; f < KG; ++f) {
-      red[w - 1][lane][4 * f] = acc[f].x;
-      red[w - 1][lane][4 * f + 1] = acc[f].y;
-      red[w - 1][lane][4 * f + 2] = acc[f].z;
-      red[w - 1][lane][4 * f + 3] = acc[f].w;
-    }
-  __syncthreads();
-  if (w == 0 && row < nc)
-#pragma unroll
-    for (int f = 0; f < KG; ++f) {
-      float4 s = acc[f];
-#pragma unroll
-      for (int i = 0; i < kW - 1; ++i) {
-        s.x += red[i][lane][4 * f];
-        s.y += red[i][lane][4 * f + 1];
-        s.z += red[i][lane][4 * f + 2];
-        s.w += red[i][lane][4 * f + 3];
+      for (int t = 0; t < 4; ++t) {
+        const int col = c + 4 * k + t;
+        const bool in = r < K && col < nc;
+        b[s][t] = rc[in ? col * K + r : 0];
+        b[s][t] = in ? b[s][t] : 0.0f;
       }
-      reinterpret_cast<float4 *>(ecp)[((size_t)blockIdx.y * nc + row) * KG + f] = s;
     }
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][t], b[s][t], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) tile[w][(4 * k + v) * 16 + r] = acc[v];  // row 4 k + v, field r
+  __syncthreads();
+  const int i = threadIdx.x >> 4, f = threadIdx.x & 15;
+  if (threadIdx.x >= 256 || f >= K || row0 + i >= nc) return;
+  float s = 0.0f;
+#pragma unroll
+  for (int q = 0; q < kGemvWaves; ++q) s += tile[q][threadIdx.x];
+  ec[(size_t)(row0 + i) * K + f] = s;
 }
 
-// E = w1 E + P2 ec at the second level's nodes, ec the sum of its split partials
-template <int K>
-__global__ void __launch_bounds__(256) k_v_coarse_add(Grid g, Grid g1, CGrid cg, int NP1, float w1, int nsplit,
-                                                      const float4 *ecp, float4 *E, const MState *cur) {
+// OUT = w IN + P ec at the nodes of grid gt (S as k_v_coarse_rhs; OUT may be
+// IN); boundary nodes keep IN, zero there
+template <int K, int S>
+__global__ void __launch_bounds__(256) k_v_coarse_add(Grid gt, Hats hats, int NPt, float w, const float4 *ec,
+                                                      const float4 *IN, float4 *OUT, const MState *cur) {
   constexpr int KG = K / 4;
   const int c = blockIdx.y, d = c / KG, grp = c % KG;
-  const int n1 = blockIdx.x * 256 + threadIdx.x;
-  if (n1 >= g1.nn) return;
-  const float4 e0 = E[(size_t)c * NP1 + n1];
+  const int n = blockIdx.x * 256 + threadIdx.x;  // < NPt
+  const float4 e0 = IN[(size_t)c * NPt + n];
   if (group_stopped(cur, grp * 4)) return;
-  const int x = n1 % g1.nx, y = (n1 / g1.nx) % g1.ny, z = n1 / (g1.nx * g1.ny);
-  if (node_on_boundary(g1, x, y, z)) return;  // E is zero there
-  float wx[2], wy[2], wz[2];
-  int qx[2], qy[2], qz[2];
-  hat_pair_at(2 * x, g.nex, cg.mx + 1, wx, qx);
-  hat_pair_at(2 * y, g.ney, cg.my + 1, wy, qy);
-  hat_pair_at(2 * z, g.nez, cg.mz + 1, wz, qz);
-  unsigned o[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-    o[t] = (unsigned)(((qz[t >> 2] * cg.my + qy[(t >> 1) & 1]) * cg.mx + qx[t & 1]) * 3 + d) * KG + grp;
-  float4 acc = make_float4(w1 * e0.x, w1 * e0.y, w1 * e0.z, w1 * e0.w);
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const float4 *es = ecp + (size_t)sp * cg.nc * KG;
+  const int x = n % gt.nx, y = (n / gt.nx) % gt.ny, z = n / (gt.nx * gt.ny);
+  float4 acc = make_float4(w * e0.x, w * e0.y, w * e0.z, w * e0.w);
+  if (n < gt.nn && !node_on_boundary(gt, x, y, z)) {
+    const HatEntry hx = hats.x[S * x], hy = hats.y[S * y], hz = hats.z[S * z];
     float4 e[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) e[t] = es[o[t]];
+    for (int t = 0; t < 8; ++t)
+      e[t] = ec[((t & 1 ? hx.q1 : hx.q0) + (t & 2 ? hy.q1 : hy.q0) + (t & 4 ? hz.q1 : hz.q0) + d) * KG + grp];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) fma4(acc, wx[t & 1] * (wy[(t >> 1) & 1] * wz[t >> 2]), e[t]);
+    for (int t = 0; t < 8; ++t)
+      fma4(acc, (t & 1 ? hx.w1 : hx.w0) * ((t & 2 ? hy.w1 : hy.w0) * (t & 4 ? hz.w1 : hz.w0)), e[t]);
   }
-  E[(size_t)c * NP1 + n1] = acc;
+  OUT[(size_t)c * NPt + n] = acc;
 }
 
 // OUT = w0 Z + P1 E; OUT may be Z.  Along a side a fine node lies on a
@@ -804,25 +801,51 @@ static hipError_t launch_mid(const Grid &g1, int K, const VCycleDev &v, const fl
   return hipGetLastError();
 }
 
+template <int K>
+static void launch_gemv(const VCycleDev &v, const MState *cur, hipStream_t st) {
+  const dim3 grid(nblk(v.cg.nc, kGemvRowsV)), block(64 * kGemvWaves);
+  const int nc = v.cg.nc, steps = (int)nblk(nc, 16 * kGemvWaves);  // of a wave
+  if (steps == 1)
+    hipLaunchKernelGGL((k_v_gemv<K, 1>), grid, block, 0, st, nc, v.ainv, v.rc, v.ec, cur);
+  else if (steps == 2)
+    hipLaunchKernelGGL((k_v_gemv<K, 2>), grid, block, 0, st, nc, v.ainv, v.rc, v.ec, cur);
+  else
+    hipLaunchKernelGGL((k_v_gemv<K, 5>), grid, block, 0, st, nc, v.ainv, v.rc, v.ec, cur);
+}
+
 hipError_t launch_vcycle(const Grid &g, int K, const VCycleDev &v, const StencilOp &op, const float *kinv,
                          const float *R, const float *Z, float *T, float *OUT, double *pr, const void *state,
                          hipStream_t st) {
-  const int NP = mshape(g).NP, NP1 = mshape(v.g1).NP;
+  const int NP = mshape(g).NP;
   const MState *cur = static_cast<const MState *>(state);
-  const dim3 grid1(NP1 / 256, 3 * K / 4), grid0(NP / 256, 3 * K / 4);
+  const dim3 grid0(NP / 256, 3 * K / 4);
   hipError_t e = launch_d_apply<kApplyRes>(g, K, op, Z, R, kinv, v.w0, T, nullptr, state, st);
   if (e != hipSuccess) return e;
+  const Hats hats{v.hat[0], v.hat[1], v.hat[2]};
+  const dim3 nq(nblk(v.cg.nq, 4), 3 * K / 4);
+  float4 *rc4 = reinterpret_cast<float4 *>(v.rc), *ec4 = reinterpret_cast<float4 *>(v.ec);
+  if (!v.mid.nq) {  // two levels
+    MPP_K_DISPATCH(K, {
+      hipLaunchKernelGGL((k_v_coarse_rhs<KK, 1>), nq, dim3(256), 0, st, g, g, v.cg, hats, NP,
+                         reinterpret_cast<const float4 *>(T), rc4, cur);
+      launch_gemv<KK>(v, cur, st);
+      hipLaunchKernelGGL((k_v_coarse_add<KK, 1>), grid0, dim3(256), 0, st, g, hats, NP, v.w0, ec4,
+                         reinterpret_cast<const float4 *>(Z), reinterpret_cast<float4 *>(v.z), cur);
+    });
+    return launch_d_apply<kApplyPost>(g, K, op, v.z, R, kinv, v.w0, OUT, pr, state, st);
+  }
+  const int NP1 = mshape(v.g1).NP;
+  const dim3 grid1(NP1 / 256, 3 * K / 4);
+  float4 *E0 = reinterpret_cast<float4 *>(v.E0);
   MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_v_restrict<KK>, grid1, dim3(256), 0, st, g, v.g1, NP, NP1,
                                        reinterpret_cast<const float4 *>(T), v.kinv1, reinterpret_cast<float4 *>(v.R1),
-                                       reinterpret_cast<float4 *>(v.E0), cur));
+                                       E0, cur));
   if ((e = launch_mid<kApplyRes>(v.g1, K, v, v.E0, v.R1, v.T1, nullptr, state, st)) != hipSuccess) return e;
   MPP_K_DISPATCH(K, {
-    hipLaunchKernelGGL(k_v_coarse_rhs<KK>, dim3(nblk(v.cg.nq, 4), 3 * KK / 4), dim3(256), 0, st, g, v.g1, v.cg, NP1,
-                       reinterpret_cast<const float4 *>(v.T1), reinterpret_cast<float4 *>(v.rc), cur);
-    hipLaunchKernelGGL(k_v_gemv<KK>, dim3(nblk(v.cg.nc, 64), v.nsplit), dim3(64 * kGemvWaves), 0, st, v.cg.nc, v.ainv,
-                       reinterpret_cast<const float4 *>(v.rc), v.ecp, cur);
-    hipLaunchKernelGGL(k_v_coarse_add<KK>, grid1, dim3(256), 0, st, g, v.g1, v.cg, NP1, v.w1, v.nsplit,
-                       reinterpret_cast<const float4 *>(v.ecp), reinterpret_cast<float4 *>(v.E0), cur);
+    hipLaunchKernelGGL((k_v_coarse_rhs<KK, 2>), nq, dim3(256), 0, st, g, v.g1, v.cg, hats, NP1,
+                       reinterpret_cast<const float4 *>(v.T1), rc4, cur);
+    launch_gemv<KK>(v, cur, st);
+    hipLaunchKernelGGL((k_v_coarse_add<KK, 2>), grid1, dim3(256), 0, st, v.g1, hats, NP1, v.w1, ec4, E0, E0, cur);
   });
   if ((e = launch_mid<kApplyPost>(v.g1, K, v, v.E0, v.R1, v.E, nullptr, state, st)) != hipSuccess) return e;
   MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_v_prolong<KK>, grid0, dim3(256), 0, st, g, v.g1, NP, NP1, v.w0,
@@ -849,20 +872,38 @@ namespace {
 // damping * lambda_max < 2
 constexpr int kPowerIts = 12;
 constexpr float kDamp = 1.55f;
+// The two-level form: coarse elements of at most 2 fine ones a side while their
+// inverse has at most kCoarseMaxDofs DOFs (20 elements a side), of at most 3
+// while it has at most 1536 (26).  The second level's five kernels fall away:
+// 60 us an iteration of 8 fields become 40 at 10 to 16 elements a side, 54 at
+// 20 and 47 to 54 at 22 to 26, with as many iterations (22 to 27; 33 at 24).
+// Above, the inverse's set-up (2.1 ms at 2187 DOFs against 1.4) costs more than
+// the iterations gain.
+bool coarse_grid_two_level(const Grid &g, CGrid *out) {
+  for (int width = 2; width <= 3; ++width)
+    if (coarse_grid_wide(g, width, width == 2 ? kCoarseMaxDofs : 1536, out) &&
+        std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= width)
+      return true;
+  return false;
+}
 }  // namespace
 
 int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
                  float *P, float *AP, hipStream_t st, VCycleDev **out) {
   *out = nullptr;
   CGrid cg, mid;
-  if (!coarse_enabled() || !coarse_grid_cycle(g, &cg) || !coarse_grid_by_two(g, &mid)) return MPPD_OK;
+  if (!coarse_enabled()) return MPPD_OK;
+  const bool two = coarse_grid_two_level(g, &cg);
+  if (two)
+    mid = CGrid{};
+  else if (!coarse_grid_cycle(g, &cg) || !coarse_grid_by_two(g, &mid))
+    return MPPD_OK;
   VCycleDev *v = new VCycleDev();
   v->arena = nullptr;
   v->cg = cg;
   v->mid = mid;
-  v->nsplit = (cg.nc + kSplitCols - 1) / kSplitCols;
   Grid &g1 = v->g1;
-  g1 = Grid{};
+  g1 = Grid{};  // (without a second level: 2 nodes a side, unused)
   g1.nx = mid.mx + 2;
   g1.ny = mid.my + 2;
   g1.nz = mid.mz + 2;
@@ -887,17 +928,23 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
       off += (bytes + 255) & ~(size_t)255;
       return o;
     };
-    const size_t n1 = (size_t)s1.NP * 3 * K * sizeof(float);
-    const size_t o_rc = carve((size_t)nc * K * sizeof(float)), o_ecp = carve((size_t)v->nsplit * nc * K * sizeof(float));
+    const size_t n1 = two ? 0 : (size_t)s1.NP * 3 * K * sizeof(float);
+    const size_t o_rc = carve((size_t)nc * K * sizeof(float)), o_ec = carve((size_t)nc * K * sizeof(float));
+    size_t o_hat[3];
+    const int line[3] = {g.nx, g.ny, g.nz}, mq[3] = {cg.mx, cg.my, cg.mz};
+    for (int a = 0; a < 3; ++a) o_hat[a] = carve(line[a] * sizeof(HatEntry));
     const size_t o_z = carve(mixed_vector_len(g, K) * sizeof(float));
     const size_t o_prz = carve(std::max((size_t)K * nb, 2 * 4 * (size_t)std::max(nb, nb1)) * sizeof(double));
     const size_t o_sum = carve(16 * sizeof(double));
     const size_t o_R1 = carve(n1), o_E0 = carve(n1), o_T1 = carve(n1), o_E = carve(n1);
-    const size_t o_k1 = carve((size_t)s1.NP * 3 * sizeof(float));
-    const size_t zeroed = off, o_ainv = carve((size_t)nc * nc * sizeof(float));
-    const size_t o_A1 = carve(mixed_matrix_floats(g1) * sizeof(float));
+    const size_t o_k1 = carve(two ? 0 : (size_t)s1.NP * 3 * sizeof(float));
+    const size_t zeroed = off, o_ainv = carve(((size_t)nc * nc + 16) * sizeof(float));  // (k_v_gemv reads 15 past it)
+    const size_t o_A1 = carve(two ? 0 : mixed_matrix_floats(g1) * sizeof(float));
     hipError_t e = hipMalloc(&v->arena, off);
     if (e == hipSuccess) e = hipMemsetAsync(v->arena, 0, zeroed, st);
+    if (e == hipSuccess)
+      e = hipMemsetAsync(static_cast<char *>(v->arena) + o_ainv + (size_t)nc * nc * sizeof(float), 0,
+                         16 * sizeof(float), st);
     if (e != hipSuccess) {
       rc = hip_fail(e, "preconditioner buffers");
       break;
@@ -905,7 +952,11 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     char *base = static_cast<char *>(v->arena);
     auto at = [base](size_t o) { return reinterpret_cast<float *>(base + o); };
     v->rc = at(o_rc);
-    v->ecp = at(o_ecp);
+    v->ec = at(o_ec);
+    for (int a = 0, stride = 3; a < 3; stride *= mq[a++]) {
+      v->hat[a] = reinterpret_cast<HatEntry *>(base + o_hat[a]);
+      hipLaunchKernelGGL(k_v_hats, dim3(1), dim3(kCoarseMaxLine), 0, st, line[a] - 1, mq[a] + 1, stride, v->hat[a]);
+    }
     v->z = at(o_z);
     v->R1 = at(o_R1);
     v->E0 = at(o_E0);
@@ -929,7 +980,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
       std::swap(a, b);
     }
     hipLaunchKernelGGL(k_v_sums, dim3(1), dim3(kRedThreads), 0, st, p0, p1, nb, sums);
-    if (e == hipSuccess) {
+    if (e == hipSuccess && !two) {
       if ((rc = dalloc(&C, coarse_table_len(mid), false))) break;
       e = launch_cs_table(mid, ke_d, C, st);
       hipLaunchKernelGGL(k_v_asm, dim3(s1.NP / 64), dim3(256), 0, st, g, g1, mid, s1.NP, et_d, C, v->A1, v->kinv1);
@@ -956,7 +1007,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
       return lam > 0.1 && lam < 1e3 ? kDamp / (float)lam : 0.0f;
     };
     v->w0 = damping(sums_h);
-    v->w1 = damping(sums_h + 8);
+    v->w1 = two ? 1.0f : damping(sums_h + 8);
     ok = ok && v->w0 > 0.0f && v->w1 > 0.0f;
   } while (0);
   (void)hipStreamSynchronize(st);  // C may still be in use after a failed step
