@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256) k_elem_ke(Grid g, const double *bmat, con
 
 __global__ void __launch_bounds__(256) k_gather_vals(Grid g, const int *et, const double *ke, int phase_mode,
                                                      double *vals) {
-  gather_vals_row(g, blockIdx.x * blockDim.x + threadIdx.x, et, ke, phase_mode, vals);
+  gather_vals_slice(g, blockIdx.x, et, ke, phase_mode, vals);
 }
 
 __global__ void __launch_bounds__(256) k_elem_be(Grid g, const double *bmat, const material_base *mats, const int *et,
@@ -128,7 +128,7 @@ hipError_t launch_elem_ke(const Grid &g, const double *bmat, const material_base
 
 hipError_t launch_gather_vals(const Grid &g, const int *et, const double *ke, int phase_mode, double *vals,
                               hipStream_t st) {
-  hipLaunchKernelGGL(k_gather_vals, dim3(nblk(g.nrow_pad, 256)), dim3(256), 0, st, g, et, ke, phase_mode, vals);
+  hipLaunchKernelGGL(k_gather_vals, dim3(g.nrow_pad / 64), dim3(256), 0, st, g, et, ke, phase_mode, vals);
   return hipGetLastError();
 }
 

@@ -76,7 +76,8 @@ __global__ void __launch_bounds__(256) kb_elem_ke(const BRve *rv, const int *map
 __global__ void __launch_bounds__(256) kb_gather_vals(const BRve *rv, const int *map, const int *act,
                                                       const int *blk0) {
   MPP_BATCH_PROLOGUE(map)
-  gather_vals_row(R.g, (blockIdx.x - blk0[rid]) * 256 + threadIdx.x, R.et, R.ke, R.phase_mode, R.vals);
+  // four slices per row block
+  gather_vals_slice(R.g, (blockIdx.x - blk0[rid]) * 4 + blockIdx.y, R.et, R.ke, R.phase_mode, R.vals);
 }
 
 __global__ void __launch_bounds__(256) kb_elem_be(const BRve *rv, const int *map, const int *act, const int *blk0) {
@@ -572,7 +573,7 @@ hipError_t launch_b_vars_move(const BLaunch &L, int what, hipStream_t st) {
 }
 hipError_t launch_b_mat(const BLaunch &L, const int *act_ke, const int *act_gather, hipStream_t st) {
   hipLaunchKernelGGL(kb_elem_ke, dim3(L.ke.nb), dim3(64 * kKeWaves), 0, st, L.rv, L.ke.map, act_ke, L.ke.blk0);
-  hipLaunchKernelGGL(kb_gather_vals, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, act_gather, L.row.blk0);
+  hipLaunchKernelGGL(kb_gather_vals, dim3(L.row.nb, 4), dim3(256), 0, st, L.rv, L.row.map, act_gather, L.row.blk0);
   return hipGetLastError();
 }
 hipError_t launch_b_rhs(const BLaunch &L, double *norms, hipStream_t st) {

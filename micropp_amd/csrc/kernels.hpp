@@ -108,23 +108,55 @@ __device__ __forceinline__ void set_bc_node(const Grid &g, int node, const doubl
 }
 
 // ---------------------------------------------------------------------------
-// Element stiffness, get_elem_mat (src/assembly.cpp:140-178).  One wavefront
-// per element (or per material in phase mode); the 8 tangents and C*B*wg are
-// staged in LDS; each lane produces 9 of the 576 entries, summing over
-// (gp, m) in the reference order.  Block lb holds items lb*4 .. lb*4+3.
+// Element stiffness, get_elem_mat (src/assembly.cpp:140-178): Ke = sum_gp B^T
+// (C B wg), one wavefront per element (or per material in phase mode); block
+// lb holds items lb*4 .. lb*4+3.  B of a node holds its three shape gradients
+// (gx, gy, gz) and zeros, so every sum over strain components has three
+// products instead of six; they are added in the reference's order (gp, then
+// component), without contraction, and the zero products left out change no
+// sum (it starts at +0).  The waves share nothing but the gradients, so after
+// those there are no block barriers.
+//
+// What bounds it: FP64 mul and add (about 600 per lane of an element) beside
+// the 4.6 KB written per element.  A lane owns one (gp, node) of C B and one
+// (node, node) 3x3 tile of Ke; sig, C and C B take turns in 9.2 KB of LDS a
+// wave (four blocks a CU).  40^3 J2 elements: 168 us (460 with the zero products,
+// 15 KB a wave and block barriers), 1.8 TB/s of writes.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void wave_lds_sync() {  // LDS written by other lanes of this wave
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// one strain component at a Gauss point with gradients gr[node * 3 + d]
+// (strain_at, the products with B's zeros left out)
+__device__ __forceinline__ double strain_row(const double *gr, const double *ue, int v) {
+#pragma clang fp contract(off)
+  const int d0 = v < 3 ? v : v == 5 ? 1 : 0, d1 = v == 3 ? 1 : 2;
+  double s = 0;
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+    if (v < 3) {
+      s += gr[a * 3 + v] * ue[a * 3 + v];
+    } else {
+      s += gr[a * 3 + d1] * ue[a * 3 + d0];
+      s += gr[a * 3 + d0] * ue[a * 3 + d1];
+    }
+  }
+  return s;
+}
+
+constexpr int kKeWork = 8 * 8 * 18;  // doubles of a wave's turn-taking LDS: C B
 __device__ __forceinline__ void elem_ke_body(const Grid &g, int lb, const double *bmat_g, const material_base *mats,
                                              const int *et, const double *u, const double *vars, int phase_mode,
                                              double *ke) {
 #pragma clang fp contract(off)
-  __shared__ double bm[8 * 144];
+  __shared__ double grad[8 * 24];  // gx, gy, gz of (gp, node)
   __shared__ double ue_s[kKeWaves][24];
-  __shared__ double C_s[kKeWaves][8 * 36];
-  __shared__ double cb_s[kKeWaves][8 * 144];
-  __shared__ double eps_s[kKeWaves][8 * 6];
-  __shared__ double sig_s[kKeWaves][8 * 7 * 6];  // FD tangent: base and 6 perturbed stresses per GP
+  __shared__ double work[kKeWaves][kKeWork];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  stage_bmat(bmat_g, bm);
+  if (tid < 8 * 24) grad[tid] = bmat_g[(tid / 24) * 144 + (tid % 3) * 24 + tid % 24];
   const int item = lb * kKeWaves + w;
   const int nitems = phase_mode ? 3 : g.nelem;
   const bool active = item < nitems;
@@ -143,72 +175,77 @@ __device__ __forceinline__ void elem_ke_body(const Grid &g, int lb, const double
     ue_s[w][lane] = v;
   }
   __syncthreads();
+  if (!active) return;
   // mat_ctan per GP.  Elastic: the closed form, one lane per GP.  Otherwise
   // the forward-difference tangent's 7 stress evaluations per GP (base and
   // 6 perturbed strains) run on 56 lanes at once, then each tangent entry is
   // (s1 - s0) / D_EPS_CTAN as in mat_ctan: the same values bit for bit.
-  const bool fd = active && mats[ph].type != MATERIAL_ELASTIC;
-  if (active && lane < 8) {
-    double eps[6];
-    strain_at(&bm[lane * 144], ue_s[w], eps);
-    if (fd) {
-      for (int i = 0; i < 6; ++i) eps_s[w][lane * 6 + i] = eps[i];
-    } else {
-      mat_ctan(mats[ph], eps, nullptr, &C_s[w][lane * 36]);
+  double *C_s = work[w], *eps_s = C_s + 8 * 36, *sig_s = eps_s + 8 * 6;  // sig: 8 x 7 x 6
+  if (mats[ph].type != MATERIAL_ELASTIC) {
+    if (lane < 48) eps_s[lane] = strain_row(&grad[(lane / 6) * 24], ue_s[w], lane % 6);
+    wave_lds_sync();
+    if (lane < 56) {
+      const int gp = lane / 7, c = lane % 7;  // c = 0: base strain; c > 0: component c - 1 perturbed
+      double e1[6];
+      for (int i = 0; i < 6; ++i) e1[i] = eps_s[gp * 6 + i] + (i == c - 1 ? D_EPS_CTAN : 0.0);
+      const double *h = (vars && !phase_mode) ? vars + ((size_t)item * 8 + gp) * NVAR : nullptr;
+      mat_stress(mats[ph], e1, h, &sig_s[lane * 6]);
     }
-  }
-  __syncthreads();
-  if (fd && lane < 56) {
-    const int gp = lane / 7, c = lane % 7;  // c = 0: base strain; c > 0: component c - 1 perturbed
-    double e1[6];
-    for (int i = 0; i < 6; ++i) e1[i] = eps_s[w][gp * 6 + i];
-    if (c > 0) e1[c - 1] += D_EPS_CTAN;
-    const double *h = (vars && !phase_mode) ? vars + ((size_t)item * 8 + gp) * NVAR : nullptr;
-    mat_stress(mats[ph], e1, h, &sig_s[w][(gp * 7 + c) * 6]);
-  }
-  __syncthreads();
-  if (fd) {
+    wave_lds_sync();
     for (int q = lane; q < 8 * 36; q += 64) {
       const int gp = q / 36, r = (q / 6) % 6, c = q % 6;
-      const double *sg = &sig_s[w][gp * 7 * 6];
-      C_s[w][gp * 36 + r * 6 + c] = (sg[(c + 1) * 6 + r] - sg[r]) / D_EPS_CTAN;
+      const double *sg = &sig_s[gp * 7 * 6];
+      C_s[q] = (sg[(c + 1) * 6 + r] - sg[r]) / D_EPS_CTAN;
+    }
+  } else if (lane < 8) {
+    mat_ctan(mats[ph], nullptr, nullptr, &C_s[lane * 36]);
+  }
+  wave_lds_sync();
+  const int hi = lane >> 3, lo = lane & 7;
+  {  // C B wg of Gauss point hi and node lo: 6 rows x 3 columns
+    const double gx = grad[hi * 24 + lo * 3], gy = grad[hi * 24 + lo * 3 + 1], gz = grad[hi * 24 + lo * 3 + 2];
+    double C[36];
+#pragma unroll
+    for (int q = 0; q < 36; ++q) C[q] = C_s[hi * 36 + q];
+    wave_lds_sync();  // C B takes C's place
+    double *cb = &work[w][lane * 18];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+      const double *c = &C[m * 6];
+      cb[m * 3 + 0] = (c[0] * gx + c[3] * gy + c[4] * gz) * g.wg;
+      cb[m * 3 + 1] = (c[1] * gy + c[3] * gx + c[5] * gz) * g.wg;
+      cb[m * 3 + 2] = (c[2] * gz + c[4] * gx + c[5] * gy) * g.wg;
     }
   }
-  __syncthreads();
-  if (active) {
-    for (int q = lane; q < 8 * 144; q += 64) {
-      const int gp = q / 144, m = (q / 24) % 6, jj = q % 24;
-      const double *C = &C_s[w][gp * 36 + m * 6];
-      const double *b = &bm[gp * 144];
-      double s = 0.0;
-      for (int k = 0; k < 6; ++k) s += C[k] * b[k * 24 + jj];
-      cb_s[w][q] = s * g.wg;
+  wave_lds_sync();
+  // lane (hi, lo) = node pair: rows 3 hi .. 3 hi + 2, columns 3 lo .. 3 lo + 2
+  double acc[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+#pragma unroll 2
+  for (int gp = 0; gp < 8; ++gp) {
+    const double *gr = &grad[gp * 24 + hi * 3], *cb = &work[w][(gp * 8 + lo) * 18];
+    const double gx = gr[0], gy = gr[1], gz = gr[2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      acc[0][c] += gx * cb[0 + c];
+      acc[0][c] += gy * cb[9 + c];
+      acc[0][c] += gz * cb[12 + c];
+      acc[1][c] += gy * cb[3 + c];
+      acc[1][c] += gx * cb[9 + c];
+      acc[1][c] += gz * cb[15 + c];
+      acc[2][c] += gz * cb[6 + c];
+      acc[2][c] += gx * cb[12 + c];
+      acc[2][c] += gy * cb[15 + c];
     }
   }
-  __syncthreads();
-  // Ke = sum_gp B^T (C B wg): lane (bi, bj) owns the 3x3 tile of rows 3 bi ..
-  // 3 bi + 2 and columns 3 bj .. 3 bj + 2 (6 LDS reads per 9 products); each
-  // entry still sums gp, then m, in order
-  if (active) {
-    double *out = ke + (size_t)item * 576;
-    const int bi = lane >> 3, bj = lane & 7;
-    double acc[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-    for (int gp = 0; gp < 8; ++gp)
+  wave_lds_sync();  // Ke takes C B's place on its way out, for whole lines
 #pragma unroll
-      for (int m = 0; m < 6; ++m) {
-        const double *bq = &bm[gp * 144 + m * 24 + 3 * bi];
-        const double *cq = &cb_s[w][gp * 144 + m * 24 + 3 * bj];
-        const double b3[3] = {bq[0], bq[1], bq[2]}, c3[3] = {cq[0], cq[1], cq[2]};
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
+    for (int c = 0; c < 3; ++c) work[w][(3 * hi + a) * 24 + 3 * lo + c] = acc[a][c];
+  wave_lds_sync();
+  double *out = ke + (size_t)item * 576;
 #pragma unroll
-          for (int c = 0; c < 3; ++c) acc[a][c] += b3[a] * c3[c];
-      }
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) out[(3 * bi + a) * 24 + 3 * bj + c] = acc[a][c];
-  }
+  for (int q = 0; q < 9; ++q) out[q * 64 + lane] = work[w][q * 64 + lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -217,58 +254,57 @@ __device__ __forceinline__ void elem_ke_body(const Grid &g, int lb, const double
 // src/ell-common.cpp:166-198) and ell_set_bc_3D (:238-297).  For row
 // (node N, fi) and slot (neighbour M, fj) the contributing elements are those
 // holding both N and M, visited in reference order ex, ey, ez.
+//
+// A block of 256 threads makes one slice (64 rows) in LDS.  A wave takes 8
+// rows at a time: its 8 x 8 lanes load, for each of the 8 elements around the
+// row's node, the row's 3 entries towards local node p: 192 bytes in a line
+// per row and element, all 24 loads of a lane in flight, every entry of ke
+// read once.  Then it adds them element by element (LDS operations of a wave
+// keep their order), and the slice is stored by whole lines.  Bound: memory,
+// the element matrices in and the values out.  40^3 elements: 85 us
+// (a thread per row: 188), 5.0 TB/s.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void gather_vals_row(const Grid &g, int row, const int *et, const double *ke,
-                                                int phase_mode, double *vals) {
+constexpr int kGatherPitch = 66;  // doubles per slot of the slice in LDS
+__device__ __forceinline__ void gather_vals_slice(const Grid &g, int slice, const int *et, const double *ke,
+                                                  int phase_mode, double *vals) {
 #pragma clang fp contract(off)
-  if (row >= g.nrow_pad) return;
-  double *out = vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
-  if (row >= g.nrow) {
-    for (int s = 0; s < kSlots; ++s) out[s * 64] = 0.0;
-    return;
-  }
-  const int node = row / 3, fi = row % 3;
-  const int i = node % g.nx, j = (node / g.nx) % g.ny, k = node / (g.nx * g.ny);
-  if (on_boundary(g, i, j, k)) {
-    for (int s = 0; s < kSlots; ++s) out[s * 64] = (s == 13 * 3 + fi) ? 1.0 : 0.0;
-    return;
-  }
-  // element blocks around the node, reference order (a, b, c) = (x, y, z)
-  const double *blk[8];
-  int la[8];
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b)
-      for (int c = 0; c < 2; ++c) {
-        const int q = (a * 2 + b) * 2 + c;
-        const int ex = i - 1 + a, ey = j - 1 + b, ez = k - 1 + c;  // interior node: always inside
-        const int e = (ez * g.ney + ey) * g.nex + ex;
-        blk[q] = ke + (size_t)(phase_mode ? et[e] : e) * 576;
-        la[q] = local_node(1 - a, 1 - b, 1 - c);
-      }
-  for (int n = 0; n < 27; ++n) {
-    const int dz = n / 9 - 1, dy = (n / 3) % 3 - 1, dx = n % 3 - 1;
-    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-    for (int a = 0; a < 2; ++a) {
-      const int px = 1 - a + dx;
-      if (px < 0 || px > 1) continue;
-      for (int b = 0; b < 2; ++b) {
-        const int py = 1 - b + dy;
-        if (py < 0 || py > 1) continue;
-        for (int c = 0; c < 2; ++c) {
-          const int pz = 1 - c + dz;
-          if (pz < 0 || pz > 1) continue;
-          const int q = (a * 2 + b) * 2 + c;
-          const double *r = blk[q] + (la[q] * 3 + fi) * 24 + local_node(px, py, pz) * 3;
-          acc0 += r[0];
-          acc1 += r[1];
-          acc2 += r[2];
-        }
-      }
+  __shared__ double acc[kSlots * kGatherPitch];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, p = lane & 7;
+  for (int t = threadIdx.x; t < kSlots * kGatherPitch; t += 256) acc[t] = 0.0;
+  __syncthreads();
+  const int px = kHexPos[p][0], py = kHexPos[p][1], pz = kHexPos[p][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = (h * 4 + w) * 8 + (lane >> 3), row = slice * 64 + r;  // (rows of one wave only)
+    if (row >= g.nrow) continue;
+    const int node = row / 3, fi = row % 3;
+    const int i = node % g.nx, j = (node / g.nx) % g.ny, k = node / (g.nx * g.ny);
+    if (on_boundary(g, i, j, k)) {
+      if (p == 0) acc[(13 * 3 + fi) * kGatherPitch + r] = 1.0;
+      continue;
     }
-    out[(n * 3 + 0) * 64] = acc0;
-    out[(n * 3 + 1) * 64] = acc1;
-    out[(n * 3 + 2) * 64] = acc2;
+    double v[8][3];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {  // reference order (a, b, c) = (x, y, z)
+      const int a = q >> 2, b = (q >> 1) & 1, c = q & 1;
+      const int e = ((k - 1 + c) * g.ney + j - 1 + b) * g.nex + i - 1 + a;  // interior node: always inside
+      const double *s = ke + (size_t)(phase_mode ? et[e] : e) * 576 + (local_node(1 - a, 1 - b, 1 - c) * 3 + fi) * 24 + p * 3;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) v[q][d] = s[d];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      // neighbour of the node at local node p of element q
+      const int n = ((pz + (q & 1)) * 3 + py + ((q >> 1) & 1)) * 3 + px + (q >> 2);
+      double *o = &acc[n * 3 * kGatherPitch + r];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) o[d * kGatherPitch] += v[q][d];
+      wave_lds_sync();
+    }
   }
+  __syncthreads();
+  double *out = vals + (size_t)slice * kSlots * 64;
+  for (int t = threadIdx.x; t < kSlots * 64; t += 256) out[t] = acc[(t >> 6) * kGatherPitch + (t & 63)];
 }
 
 // ---------------------------------------------------------------------------
