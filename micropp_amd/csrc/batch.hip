@@ -165,17 +165,23 @@ __global__ void __launch_bounds__(256) kb_cg_init_state(const BRve *rv, const in
 // (b & 7) * per + (b >> 3), so each XCD streams a contiguous run of blocks
 // (blocks are dispatched round-robin over the 8 XCDs).  The arithmetic is
 // the same in every shape.
-template <int CH, bool XCD>
+// DICT: some RVE's matrix is a stencil table (its branch costs the others 40
+// registers, hence kernels of their own).
+template <int CH, bool XCD, bool DICT>
 __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *at, CgState *cg, const int *a0on,
                                                    int nb, int per, int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
   if (b >= nb) return;
   const int rid = at[b].x, k = parity & 1;
   const BRve &R = rv[rid];
-  // vals and a0 are assembled here: the stencil columns follow from the grid
-  const double *A = cg_matrix(R, a0on, rid);
-  cg_step1_body64<CH>(R.g, at[b].y, R.nb_row, A, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap, R.part, cg + 2 * rid + k,
-                      cg + 2 * rid + (k ^ 1));
+  __shared__ double seg[kSegDoubles];
+  CgState *cur = cg + 2 * rid + k, *nxt = cg + 2 * rid + (k ^ 1);
+  if (DICT && R.dict.tab)
+    cg_step1_body64<CH, 1>(R.g, at[b].y, R.nb_row, R.dict.tab, R.dict.code, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap,
+                           R.part, cur, nxt, seg);
+  else  // vals and a0 are assembled here: the stencil columns follow from the grid
+    cg_step1_body64<CH>(R.g, at[b].y, R.nb_row, cg_matrix(R, a0on, rid), nullptr, R.kinv, R.r, R.p[k], R.p[k ^ 1],
+                        R.Ap, R.part, cur, nxt, seg);
 }
 
 __global__ void __launch_bounds__(256) kb_cg_step2(const BRve *rv, const int2 *at, const CgState *cg, int parity) {
@@ -597,16 +603,21 @@ hipError_t launch_b_cg_init(const BLaunch &L, double min_err, double rel_err, in
   hipLaunchKernelGGL(kb_cg_init_state, dim3(L.nrve), dim3(256), 0, st, L.rv, L.act, min_err, rel_err, max_its);
   return hipGetLastError();
 }
-hipError_t launch_b_spmv(const BLaunch &L, int shape, int parity, hipStream_t st) {
+template <int CH, bool XCD>
+static void launch_step1(const BLaunch &L, int parity, hipStream_t st) {
   const int nb = L.row.nb, per = (nb + 7) / 8;
-  const dim3 plain(nb), xcd(8 * per);
+  const auto k = L.dict ? kb_cg_step1<CH, XCD, true> : kb_cg_step1<CH, XCD, false>;
+  hipLaunchKernelGGL(k, dim3(XCD ? 8 * per : nb), dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity);
+}
+
+hipError_t launch_b_spmv(const BLaunch &L, int shape, int parity, hipStream_t st) {
   switch (shape) {
-    case 0: hipLaunchKernelGGL((kb_cg_step1<9, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
-    case 1: hipLaunchKernelGGL((kb_cg_step1<27, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
-    case 2: hipLaunchKernelGGL((kb_cg_step1<81, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
-    case 3: hipLaunchKernelGGL((kb_cg_step1<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
-    case 4: hipLaunchKernelGGL((kb_cg_step1<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
-    case 5: hipLaunchKernelGGL((kb_cg_step1<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity); break;
+    case 0: launch_step1<9, false>(L, parity, st); break;
+    case 1: launch_step1<27, false>(L, parity, st); break;
+    case 2: launch_step1<81, false>(L, parity, st); break;
+    case 3: launch_step1<9, true>(L, parity, st); break;
+    case 4: launch_step1<27, true>(L, parity, st); break;
+    case 5: launch_step1<81, true>(L, parity, st); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

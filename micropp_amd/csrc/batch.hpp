@@ -20,6 +20,7 @@ struct BRve {
   const int *cols;             // SELL-64 columns (shared by RVEs of one size)
   double *vals;                // SELL-64 values
   const double *a0;            // the initial matrix (use_A0; shared by equal RVEs), else nullptr
+  Stencil64 dict;              // phase mode: vals (and a0) as a stencil table (kDictNodes; shared by equal RVEs)
   double *ke;                  // 576 per element, or per phase in phase mode
   double *be;                  // 24 per element
   double *uw, *u_n, *u_k;      // working / converged / current displacements
@@ -90,6 +91,7 @@ struct BLaunch {
   // (kGemvRows a block); coarse = some RVE has a coarse level
   BShape node, upd, gemv;
   int coarse = 0;
+  int dict = 0;  // some RVE's matrix is a stencil table
   int spmv_shape = kSpmvDefault;    // see launch_b_spmv
   int spmv_shape32 = kSpmvDefault;  // the same choice for the inner FP32 SpMV (launch_bm_spmv)
 };

@@ -69,6 +69,7 @@ struct mppd_batch {
   BOuter *outer_d = nullptr, *outer_h = nullptr;
   CgState *cg = nullptr;
   std::map<std::tuple<int, int, int>, int *> cols;
+  std::vector<void *> dicts;  // stencil tables of the all-elastic RVEs
   // per-call device arrays and pinned staging
   int *mask_d[M_NUM] = {};
   int *mask_h[M_NUM] = {};
@@ -116,6 +117,7 @@ struct mppd_batch {
     BShape *const shapes[kShapes] = {&L.row, &L.elem, &L.ke, &L.node, &L.upd, &L.gemv};
     for (int k = 0; k < kShapes; ++k) *shapes[k] = {nb[k], map_d[k], blk0_d[k], at_d[k]};
     L.coarse = coarse_any;
+    L.dict = !dicts.empty();
     L.spmv_shape = spmv_shape;
     L.spmv_shape32 = spmv_shape32;
     return L;
@@ -757,6 +759,7 @@ void destroy(mppd_batch *B) {
                   (void *)B->pend_d})
     dfree(p);
   for (auto &kv : B->cols) dfree(kv.second);
+  for (void *p : B->dicts) dfree(p);
   for (int k = 0; k < M_NUM; ++k) {
     dfree(B->mask_d[k]);
     if (B->mask_h[k]) (void)hipHostFree(B->mask_h[k]);
@@ -790,6 +793,29 @@ bool same_rve(const mppd_batch_rve &a, const mppd_batch_rve &b) {
       return false;
   }
   return true;
+}
+
+// Stencil tables of the all-elastic RVEs of kDictNodes nodes and more, equal
+// RVEs sharing one.
+int setup_dict(mppd_batch *B, const mppd_batch_rve *in) {
+  for (int r = 0; r < B->n; ++r) {
+    BRve &R = B->h[r];
+    if (!R.phase_mode || R.g.nn < kDictNodes) continue;
+    for (int q = 0; q < r && !R.dict.tab; ++q)
+      if (B->h[q].dict.tab && same_rve(in[q], in[r])) R.dict = B->h[q].dict;
+    if (R.dict.tab) continue;
+    uint16_t *code = nullptr;
+    double *tab = nullptr;
+    int rc = dalloc(&code, stencil64_codes(R.g), false);
+    if (rc) return rc;
+    B->dicts.push_back(code);
+    if ((rc = dalloc(&tab, stencil64_table(), false))) return rc;
+    B->dicts.push_back(tab);
+    R.dict.code = code;
+    R.dict.tab = tab;
+    MPP_HIP(launch_stencil64(R.g, R.et, R.ke, R.dict, B->st));
+  }
+  return upload_table(B);
 }
 
 // use_A0: the initial matrix of each distinct RVE (assembly_mat at u = 0
@@ -1056,6 +1082,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
   if ((rc = set_mask(B, M_KE, ph))) return rc;
   if ((rc = set_mask(B, M_GATHER, std::vector<int>(n, 0)))) return rc;
   MPP_HIP(launch_b_mat(B->launch(M_MAIN), B->mask_d[M_KE], B->mask_d[M_GATHER], B->st));
+  if ((rc = setup_dict(B, in))) return rc;
   if (B->prm.use_A0 && (rc = setup_a0(B, in))) return rc;
   // the SpMV shape, then the CG graph (its kernels read the table and masks
   // through fixed pointers)
@@ -1405,6 +1432,8 @@ int mppd_batch_slot_bytes(const mppd_rve *r, size_t *bytes) {
   b += (size_t)(r->all_elastic ? 3 : g.nelem) * 576 * sizeof(double);
   b += (size_t)g.nelem * (24 * sizeof(double) + sizeof(int));
   if (!r->all_elastic) b += (size_t)g.nelem * 8 * NVAR * 3 * sizeof(double);
+  if (r->all_elastic && g.nn >= kDictNodes)
+    b += stencil64_codes(g) * sizeof(uint16_t) + stencil64_table() * sizeof(double);
   b += std::max(3 * nb_row, 6 * nb_elem) * sizeof(double) + 2 * sizeof(CgState) + 8 * 144 * sizeof(double);
   *bytes = b;
   return MPPD_OK;

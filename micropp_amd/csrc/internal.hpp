@@ -254,6 +254,21 @@ hipError_t launch_elem_fields(const Grid &g, const double *bmat, const material_
 // part needs 3 * (nrow_pad / 256) doubles.  Before state[q & 1] is read after
 // q iterations, launch_cg_tail(.., q, ..) takes in the last one's sums.
 hipError_t launch_spmv(const Grid &g, const int *cols, const double *vals, const double *x, double *y, hipStream_t st);
+// The FP64 matrix of an all-elastic RVE as a stencil table: code[node] (of
+// nrow_pad / 3 + 1) and 81 values of each of a code's three rows
+struct Stencil64 {
+  uint16_t *code = nullptr;
+  double *tab = nullptr;
+};
+constexpr int kStencilCodes = 6561 + 2;  // 3^8 phase patterns, a boundary node, a padding node
+// Nodes from which an all-elastic RVE's FP64 CG reads the table: its 12.8 MB
+// (of which a solve touches the RVE's own patterns) against 1944 bytes a node
+// of stored values.  Below, both come from L2: 16^3 nodes 10.3 us an iteration
+// either way, 21^3 10.0 / 10.7, 26^3 11.0 / 12.7, 51^3 34.0 / 58.0.
+constexpr int kDictNodes = 8000;
+inline size_t stencil64_codes(const Grid &g) { return (size_t)g.nrow_pad / 3 + 1; }
+inline size_t stencil64_table() { return (size_t)kStencilCodes * 3 * kSlots; }
+hipError_t launch_stencil64(const Grid &g, const int *et, const double *ke, const Stencil64 &s, hipStream_t st);
 // The working set of one Jacobi-PCG: vectors of nrow_pad doubles, the partial
 // table and the state pair.
 struct CgVecs {
@@ -263,12 +278,12 @@ struct CgVecs {
 hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, const CgVecs &w, double min_err,
                           double rel_err, int max_its, hipStream_t st);
 // step1 of an iteration; cols == nullptr: the matrix was assembled here and
-// the stencil columns are computed.  dir = false leaves out the kernel that
+// the stencil columns are computed; dict: it is dict's, whose table is read.  dir = false leaves out the kernel that
 // forms p where step1 does not (timing of the SpMV alone, after one call with it)
-hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
-                           hipStream_t st, bool dir = true);
-hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
-                          hipStream_t st);
+hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const Stencil64 *dict, const CgVecs &w,
+                           int parity, hipStream_t st, bool dir = true);
+hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const Stencil64 *dict, const CgVecs &w,
+                          int parity, hipStream_t st);
 hipError_t launch_cg_tail(const Grid &g, const CgVecs &w, int queued, hipStream_t st);
 hipError_t launch_axpy(int n, double a, const double *x, double *y, hipStream_t st);
 hipError_t launch_copy(int n, const double *x, double *y, hipStream_t st);

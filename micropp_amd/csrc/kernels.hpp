@@ -543,7 +543,7 @@ __device__ __forceinline__ T row_dot_grid(const Grid &g, const T *vals, const T 
 // gathering them from L1/L2: the same values in the same slot order, so the
 // result is bit-identical to row_dot_grid.  ly and lz are the LDS distances,
 // in nodes, of a line and of a plane.  Every thread of the block must call it.
-constexpr int kSegNodes = 88;
+constexpr int kSegNodes = 88, kSegDoubles = 9 * kSegNodes * 3;
 struct SegPitch {
   int ly, lz;
 };
@@ -567,8 +567,16 @@ __device__ __forceinline__ SegPitch stage_runs(const Grid &g, int row0, T *seg /
 
 // One row's products with the staged runs (own: its node there), in slot
 // order: the first chunk's values are loaded by the caller, each later chunk's
-// before the products of the one in front.
-template <int CH, typename T>
+// before the products of the one in front.  Slot k's value is v[k * VS]: VS =
+// 64 in a stored matrix (streamed once), 1 in a row of a stencil table.
+template <int VS, typename T>
+__device__ __forceinline__ T load_value(const T *v, int k) {
+  if constexpr (VS == 64)
+    return __builtin_nontemporal_load(&v[k * 64]);
+  else
+    return v[k * VS];
+}
+template <int CH, int VS = 64, typename T>
 __device__ __forceinline__ T dot_runs(const T *v, T (&vi)[2][CH], const T *own, SegPitch pt) {
 #pragma clang fp contract(off)
   static_assert(kSlots % CH == 0 && CH % 3 == 0, "chunks tile the row in whole neighbours");
@@ -577,7 +585,7 @@ __device__ __forceinline__ T dot_runs(const T *v, T (&vi)[2][CH], const T *own, 
   for (int ch = 0; ch < kSlots / CH; ++ch) {
     if (ch + 1 < kSlots / CH)
 #pragma unroll
-      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = __builtin_nontemporal_load(&v[((ch + 1) * CH + k) * 64]);
+      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = load_value<VS>(v, (ch + 1) * CH + k);
 #pragma unroll
     for (int k = 0; k < CH; k += 3) {
       const int n = (ch * CH + k) / 3;
@@ -723,26 +731,31 @@ __device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, do
 // chunk of the row's values does not depend on any of the others, so it is
 // loaded before them, and each later chunk before the previous one's products;
 // the barriers in between wait for LDS alone.
-template <int CH>
-__device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, const double *vals, const double *kinv,
-                                                const double *r, const double *p, double *pn, double *Ap,
-                                                double *part1, const CgState *cur, CgState *nxt) {
+// code != nullptr: the matrix of an all-elastic RVE as a stencil table (tab, in
+// place of vals: 81 values of each of the three rows per code, k_s_table), the
+// same values in the same order (kDictNodes).  51^3 nodes: 22.6 us against 47.2
+// with the stored matrix, what is left being LDS and L1 reads; 31^3 8.6 / 12.5.
+template <int CH, int VS = 64>
+__device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, const double *vals,
+                                                const uint16_t *code, const double *kinv, const double *r,
+                                                const double *p, double *pn, double *Ap, double *part1,
+                                                const CgState *cur, CgState *nxt, double *seg /* LDS, kSegDoubles */) {
 #pragma clang fp contract(off)
-  __shared__ double seg[9 * kSegNodes * 3];
   __shared__ double lds[4];
   CgRegs c = cg_load(cur);
   const int row0 = lb * 256, row = row0 + threadIdx.x;
-  const double *v = vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
+  const double *v = VS == 64 ? vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63)
+                             : vals + ((size_t)code[row / 3] * 3 + row % 3) * kSlots;
   double vi[2][CH];
   if (!c.done)
 #pragma unroll
-    for (int k = 0; k < CH; ++k) vi[0][k] = __builtin_nontemporal_load(&v[k * 64]);
+    for (int k = 0; k < CH; ++k) vi[0][k] = load_value<VS>(v, k);
   if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
   const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return cg_dir(c, kinv[q], r[q], p[q]); });
   const double *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
   // rows past the last node lie on its run's clamped end; p is zero there
   const double pv = row < g.nrow ? own[row % 3] : 0.0;
-  const double acc = dot_runs<CH>(v, vi, own, pt);
+  const double acc = dot_runs<CH, VS>(v, vi, own, pt);
   pn[row] = pv;
   Ap[row] = acc;
   double t[1] = {pv * acc};

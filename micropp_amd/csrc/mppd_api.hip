@@ -72,7 +72,14 @@ struct mppd_solver {
   // vals came from this library's assembly (nonzeros only on in-grid stencil
   // slots), so the CG SpMV computes the columns; false after a host upload
   bool vals_stencil = true;
+  // vals hold the all-elastic RVE's matrix, and with nodes enough (kDictNodes)
+  // dict, its stencil table, made with the first assembly
+  bool vals_phase = false;
+  Stencil64 dict;
+  const int *cg_cols() const { return vals_stencil ? nullptr : cols; }
+  const Stencil64 *cg_dict() const { return vals_phase && dict.tab ? &dict : nullptr; }
 };
+
 
 // FP32 inner-solve buffers of mppd_newton_mixed: a 4-field system (field 0
 // carries the Newton correction) in the layout of mixed.hip
@@ -317,6 +324,10 @@ int mppd_solver_create(mppd_solver **out, mppd_rve *r) {
     if ((rc = dalloc(&s->cols, np * kSlots, false))) break;
     if ((rc = dalloc(&s->vals, np * kSlots, st))) break;
     if ((rc = dalloc(&s->ke, (s->phase_mode ? 3 : (size_t)g.nelem) * 576, false))) break;
+    if (s->phase_mode && g.nn >= kDictNodes) {
+      if ((rc = dalloc(&s->dict.code, stencil64_codes(g), false))) break;
+      if ((rc = dalloc(&s->dict.tab, stencil64_table(), false))) break;
+    }
     if ((rc = dalloc(&s->be, (size_t)g.nelem * 24, false))) break;
     double **vecs[] = {&s->x, &s->rr, &s->p, &s->p2, &s->Ap, &s->kinv, &s->b, &s->du};
     for (double **v : vecs)
@@ -344,7 +355,7 @@ int mppd_solver_destroy(mppd_solver *s) {
   if (!s) return MPPD_OK;
   if (s->st) (void)hipStreamSynchronize(s->st);
   for (void *p : {(void *)s->cols, (void *)s->vals, (void *)s->ke, (void *)s->be, (void *)s->x, (void *)s->rr,
-                  (void *)s->p, (void *)s->p2, (void *)s->Ap, (void *)s->kinv, (void *)s->b, (void *)s->du,
+                  (void *)s->p, (void *)s->p2, (void *)s->dict.code, (void *)s->dict.tab, (void *)s->Ap, (void *)s->kinv, (void *)s->b, (void *)s->du,
                   (void *)s->partials, (void *)s->cg, (void *)s->red})
     dfree(p);
   if (s->cg_h) (void)hipHostFree(s->cg_h);
@@ -401,6 +412,7 @@ int mppd_ell_upload_vals(mppd_solver *s, const double *vals_h) {
   if (e == hipSuccess) e = launch_rows_to_sell(g, v, s->vals, s->st);
   if (e == hipSuccess) e = hipStreamSynchronize(s->st);
   dfree(v);
+  s->vals_phase = false;
   s->vals_stencil = false;  // any slot may hold a value: the CG reads the columns
   return e == hipSuccess ? MPPD_OK : hip_fail(e, "ell_upload_vals");
 }
@@ -437,13 +449,17 @@ static hipError_t mat_async(mppd_solver *s, const double *u_d, const double *var
   if (s->phase_mode) {
     if (!s->ke_phase_ready) {
       e = launch_elem_ke(r->g, r->bmat, r->mats_d, r->et, nullptr, nullptr, 1, s->ke, s->st);
+      if (e == hipSuccess && s->dict.tab) e = launch_stencil64(r->g, r->et, s->ke, s->dict, s->st);
       if (e == hipSuccess) s->ke_phase_ready = 1;
     }
   } else {
     e = launch_elem_ke(r->g, r->bmat, r->mats_d, r->et, u_d, vars_d, 0, s->ke, s->st);
   }
   if (e == hipSuccess) e = launch_gather_vals(r->g, r->et, s->ke, s->phase_mode, s->vals, s->st);
-  if (e == hipSuccess) s->vals_stencil = true;  // every slot written, zero off the in-grid stencil
+  if (e == hipSuccess) {
+    s->vals_stencil = true;  // every slot written, zero off the in-grid stencil
+    s->vals_phase = s->phase_mode;
+  }
   return e;
 }
 
@@ -487,7 +503,7 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
     const int n = std::min(chunk, max_its - queued);
     if (n <= 0) break;
     for (int i = 0; i < n; ++i)
-      MPP_HIP(launch_cg_iter(g, A->vals_stencil ? nullptr : A->cols, A->vals, v, queued + i, st));
+      MPP_HIP(launch_cg_iter(g, A->cg_cols(), A->vals, A->cg_dict(), v, queued + i, st));
     queued += n;
     MPP_HIP(launch_cg_tail(g, v, queued, st));
     MPP_HIP(hipMemcpyAsync(w.state_h, v.state + (queued & 1), sizeof(CgState), hipMemcpyDeviceToHost, st));
@@ -674,20 +690,20 @@ int mppd_cg_profile(mppd_solver *s, const double *b_d, int iters, double *spmv_m
   const Grid &g = s->r->g;
   // min_err = rel_err = 0: the stopping test never holds within iters + 1
   const CgVecs v = cg_vecs(s);
-  const int *cols = s->vals_stencil ? nullptr : s->cols;
+  const int *cols = s->cg_cols();
   MPP_HIP(launch_cg_init(g, s->vals, b_d, v, 0.0, 0.0, iters + 1, s->st));
   hipEvent_t ev[3];
   for (auto &x : ev) MPP_HIP(hipEventCreate(&x));
   // (1) step1 back to back: it reads p[0], r and state[0] and writes p[1], Ap,
   // its partials and state[1], so repeating it changes nothing
-  hipError_t e = launch_cg_step1(g, cols, s->vals, v, 0, s->st);
+  hipError_t e = launch_cg_step1(g, cols, s->vals, s->cg_dict(), v, 0, s->st);
   if (e == hipSuccess) e = hipEventRecord(ev[0], s->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_cg_step1(g, cols, s->vals, v, 0, s->st, false);
+    e = launch_cg_step1(g, cols, s->vals, s->cg_dict(), v, 0, s->st, false);
   // (2) whole iterations
   if (e == hipSuccess) e = hipEventRecord(ev[1], s->st);
   for (int i = 0; i < iters && e == hipSuccess; ++i)
-    e = launch_cg_iter(g, cols, s->vals, v, i, s->st);
+    e = launch_cg_iter(g, cols, s->vals, s->cg_dict(), v, i, s->st);
   if (e == hipSuccess) e = hipEventRecord(ev[2], s->st);
   if (e == hipSuccess) e = hipStreamSynchronize(s->st);
   float ms1 = 0.f, ms2 = 0.f;

@@ -19,7 +19,8 @@
 // shuffled block sums: 6^3 nodes 9.3 / 14.1, 11^3 10.0 / 15.6, 21^3 10.7 /
 // 16.2, 31^3 17.7 / 23.0, 41^3 33.0 / 37.8, 51^3 58.0 / 60.4.  Small RVEs wait
 // for launches and block sums (kernels of about 6 and 3 us), 51^3 for 259 MB of
-// values a pass (5.5 TB/s).
+// values a pass (5.5 TB/s); with the stencil table of an all-elastic RVE 51^3
+// takes 34.0, 31^3 13.2.
 #include "kernels.hpp"
 
 namespace mpp {
@@ -49,7 +50,57 @@ __global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const
                                                   double *part, const CgState *cur, CgState *nxt) {
   const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (lb >= nb) return;
-  cg_step1_body64<kChunk>(g, lb, nb, vals, kinv, r, p, pn, Ap, part, cur, nxt);
+  __shared__ double seg[kSegDoubles];
+  cg_step1_body64<kChunk>(g, lb, nb, vals, nullptr, kinv, r, p, pn, Ap, part, cur, nxt, seg);
+}
+
+__global__ void __launch_bounds__(256) k_cg_step1_dict(Grid g, int nb, int per, const double *tab,
+                                                       const uint16_t *code, const double *kinv, const double *r,
+                                                       const double *p, double *pn, double *Ap, double *part,
+                                                       const CgState *cur, CgState *nxt) {
+  const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (lb >= nb) return;
+  __shared__ double seg[kSegDoubles];
+  cg_step1_body64<kChunk, 1>(g, lb, nb, tab, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
+}
+
+// code[n]: sum over the elements q = (a*2+b)*2+c around interior node n of
+// phase * 3^q; the last two for a boundary node and a padding node
+__global__ void __launch_bounds__(256) k_s_code(Grid g, int n, const int *et, uint16_t *code) {
+  const int node = blockIdx.x * 256 + threadIdx.x;
+  if (node >= n) return;
+  const int i = node % g.nx, j = (node / g.nx) % g.ny, k = node / (g.nx * g.ny);
+  int c = kStencilCodes - 1;
+  if (node < g.nn) {
+    c = kStencilCodes - 2;
+    if (!on_boundary(g, i, j, k)) {
+      c = 0;
+      for (int q = 7; q >= 0; --q)
+        c = 3 * c + et[((k - 1 + (q & 1)) * g.ney + j - 1 + ((q >> 1) & 1)) * g.nex + i - 1 + (q >> 2)];
+    }
+  }
+  code[node] = (uint16_t)c;
+}
+
+// one block per code, a thread per value: the sums of gather_vals_slice
+__global__ void __launch_bounds__(256) k_s_table(const double *ke, double *tab) {
+#pragma clang fp contract(off)
+  const int code = blockIdx.x, t = threadIdx.x;
+  if (t >= 3 * kSlots) return;
+  const int fi = t / kSlots, slot = t % kSlots, n = slot / 3, fj = slot % 3;
+  double acc = 0.0;
+  if (code == kStencilCodes - 2) {
+    acc = slot == 13 * 3 + fi ? 1.0 : 0.0;
+  } else if (code < kStencilCodes - 2) {
+    int rest = code;
+    for (int q = 0; q < 8; ++q, rest /= 3) {
+      const int a = q >> 2, b = (q >> 1) & 1, c = q & 1;
+      const int px = n % 3 - a, py = (n / 3) % 3 - b, pz = n / 9 - c;  // neighbour n in element q
+      if (px < 0 || px > 1 || py < 0 || py > 1 || pz < 0 || pz > 1) continue;
+      acc += ke[(rest % 3) * 576 + (local_node(1 - a, 1 - b, 1 - c) * 3 + fi) * 24 + local_node(px, py, pz) * 3 + fj];
+    }
+  }
+  tab[(size_t)code * 3 * kSlots + t] = acc;
 }
 
 __global__ void __launch_bounds__(256) k_cg_dir(const double *kinv, const double *r, const double *p, double *pn,
@@ -101,8 +152,15 @@ hipError_t launch_cg_init(const Grid &g, const double *vals, const double *b, co
   return hipGetLastError();
 }
 
-hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
-                           hipStream_t st, bool dir) {
+hipError_t launch_stencil64(const Grid &g, const int *et, const double *ke, const Stencil64 &s, hipStream_t st) {
+  const int n = g.nrow_pad / 3 + 1;
+  hipLaunchKernelGGL(k_s_code, dim3(nblk(n, 256)), dim3(256), 0, st, g, n, et, s.code);
+  hipLaunchKernelGGL(k_s_table, dim3(kStencilCodes), dim3(256), 0, st, ke, s.tab);
+  return hipGetLastError();
+}
+
+hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, const Stencil64 *dict, const CgVecs &w,
+                           int parity, hipStream_t st, bool dir) {
   const int nb = (int)nblk(g.nrow_pad, 256), per = (nb + 7) / 8, k = parity & 1;
   CgState *cur = w.state + k, *nxt = w.state + (k ^ 1);
   if (cols) {
@@ -110,6 +168,9 @@ hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, c
       hipLaunchKernelGGL(k_cg_dir, dim3(nb), dim3(256), 0, st, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.part + nb, cur, nxt);
     hipLaunchKernelGGL(k_cg_spmv_cols, dim3(8 * per), dim3(256), 0, st, nb, per, cols, vals, w.p[k ^ 1], w.Ap, w.part,
                        nxt);
+  } else if (dict) {
+    hipLaunchKernelGGL(k_cg_step1_dict, dim3(8 * per), dim3(256), 0, st, g, nb, per, dict->tab, dict->code, w.kinv,
+                       w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   } else {
     hipLaunchKernelGGL(k_cg_step1, dim3(8 * per), dim3(256), 0, st, g, nb, per, vals, w.kinv, w.r, w.p[k], w.p[k ^ 1],
                        w.Ap, w.part, cur, nxt);
@@ -117,9 +178,9 @@ hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, c
   return hipGetLastError();
 }
 
-hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const CgVecs &w, int parity,
-                          hipStream_t st) {
-  const hipError_t e = launch_cg_step1(g, cols, vals, w, parity, st);
+hipError_t launch_cg_iter(const Grid &g, const int *cols, const double *vals, const Stencil64 *dict, const CgVecs &w,
+                          int parity, hipStream_t st) {
+  const hipError_t e = launch_cg_step1(g, cols, vals, dict, w, parity, st);
   if (e != hipSuccess) return e;
   const int n = (parity & 1) ^ 1;
   hipLaunchKernelGGL(k_cg_step2, dim3(nblk(g.nrow_pad, 256)), dim3(256), 0, st, w.x, w.r, w.p[n], w.Ap, w.kinv, w.part,
