@@ -166,8 +166,8 @@ __global__ void __launch_bounds__(256) kb_cg_init_state(const BRve *rv, const in
 // (blocks are dispatched round-robin over the 8 XCDs).  The arithmetic is
 // the same in every shape.
 // DICT: some RVE's matrix is a stencil table (its branch costs the others 40
-// registers, hence kernels of their own).
-template <int CH, bool XCD, bool DICT>
+// registers, hence kernels of their own).  SRC: the stored ones (mat_source).
+template <int CH, bool XCD, bool DICT, int SRC>
 __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *at, CgState *cg, const int *a0on,
                                                    int nb, int per, int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
@@ -177,10 +177,10 @@ __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *a
   __shared__ double seg[kSegDoubles];
   CgState *cur = cg + 2 * rid + k, *nxt = cg + 2 * rid + (k ^ 1);
   if (DICT && R.dict.tab)
-    cg_step1_body64<CH, 1>(R.g, at[b].y, R.nb_row, R.dict.tab, R.dict.code, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap,
+    cg_step1_body64<CH, kMatTable>(R.g, at[b].y, R.nb_row, R.dict.tab, R.dict.code, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap,
                            R.part, cur, nxt, seg);
   else  // vals and a0 are assembled here: the stencil columns follow from the grid
-    cg_step1_body64<CH>(R.g, at[b].y, R.nb_row, cg_matrix(R, a0on, rid), nullptr, R.kinv, R.r, R.p[k], R.p[k ^ 1],
+    cg_step1_body64<CH, SRC>(R.g, at[b].y, R.nb_row, cg_matrix(R, a0on, rid), nullptr, R.kinv, R.r, R.p[k], R.p[k ^ 1],
                         R.Ap, R.part, cur, nxt, seg);
 }
 
@@ -383,15 +383,15 @@ __global__ void __launch_bounds__(256) kb_m_outer(const BRve *rv, const int *act
 // r lives in two vectors, read from r[k & 1] and written to r[(k + 1) & 1].
 // States as in the FP64 CG (kernels.hpp).  FP32 residual rows: row = node * 3
 // + d; sums run in fixed orders, those over the rows in FP64.
-// What bounds it: the SpMV streams 324 bytes per row (5.8 TB/s with eight
+// What bounds it: the SpMV streams 324 bytes per row (6.3 TB/s with eight
 // RVEs of 25..31 nodes a side live); the other kernels, and the SpMV once most
 // RVEs have stopped, wait for their launch, the state and the partial sums
 // (4 to 6 us each), hence as few of them as the data allow.
-// Eight J2 RVEs of 25..31 nodes a side, all live, us: SpMV 30, dir 4.4, upd
+// Eight J2 RVEs of 25..31 nodes a side, all live, us: SpMV 28.6, dir 4.4, upd
 // 11.3, gemv 4.8 (eight kernels before, of 4 to 7 beside the SpMV); two live:
 // 10, 3.4, 5.3, 3.5.  With a coarse level on every side (not only those with a
 // suitable divisor) the slowest of them takes 392 iterations a load step
-// instead of 1233, and the step 33 ms instead of 75.
+// instead of 1233, and the step 28 ms instead of 75.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void m_scalars(CgRegs &c, const BRve &R) {
 #pragma clang fp contract(off)
@@ -446,14 +446,14 @@ __global__ void __launch_bounds__(256) kb_m_dir(const BRve *rv, const int2 *at, 
   for (int d = 0; d < 3; ++d) R.p32[node * 3 + d] = c.its == 0 ? z[d] : (float)(z[d] + c.beta * p[d]);
 }
 
-template <int CH, bool XCD>
+template <int CH, bool XCD, int SRC>
 __global__ void __launch_bounds__(256) kb_m_spmv(const BRve *rv, const int2 *at, const CgState *cg, int nb, int per,
                                                  int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
   if (b >= nb) return;
   const int rid = at[b].x;
   const BRve &R = rv[rid];
-  cg_spmv_body32<CH>(R.g, at[b].y, R.vals32, R.p32, R.Ap32, R.part, cg + 2 * rid + ((parity & 1) ^ 1));
+  cg_spmv_body32<CH, SRC>(R.g, at[b].y, R.vals32, R.p32, R.Ap32, R.part, cg + 2 * rid + ((parity & 1) ^ 1));
 }
 
 // START: r_c of the residual kb_m_resid has stored (RVEs in act); the row
@@ -606,7 +606,9 @@ hipError_t launch_b_cg_init(const BLaunch &L, double min_err, double rel_err, in
 template <int CH, bool XCD>
 static void launch_step1(const BLaunch &L, int parity, hipStream_t st) {
   const int nb = L.row.nb, per = (nb + 7) / 8;
-  const auto k = L.dict ? kb_cg_step1<CH, XCD, true> : kb_cg_step1<CH, XCD, false>;
+  const bool stream = mat_source((double)nb * 256 * kSlots * sizeof(double)) == kMatStream;
+  const auto k = L.dict ? (stream ? kb_cg_step1<CH, XCD, true, kMatStream> : kb_cg_step1<CH, XCD, true, kMatCached>)
+                        : (stream ? kb_cg_step1<CH, XCD, false, kMatStream> : kb_cg_step1<CH, XCD, false, kMatCached>);
   hipLaunchKernelGGL(k, dim3(XCD ? 8 * per : nb), dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity);
 }
 
@@ -678,16 +680,21 @@ hipError_t launch_bm_resid(const BLaunch &L, int first, double rel, double abs_t
                      max_inner, tight, tight_factor, out);
   return hipGetLastError();
 }
-hipError_t launch_bm_spmv(const BLaunch &L, int shape, int parity, hipStream_t st) {
+template <int CH, bool XCD>
+static void launch_m_spmv(const BLaunch &L, int parity, hipStream_t st) {
   const int nb = L.row.nb, per = (nb + 7) / 8;
-  const dim3 plain(nb), xcd(8 * per);
+  const bool stream = mat_source((double)nb * 256 * kSlots * sizeof(float)) == kMatStream;
+  const auto k = stream ? kb_m_spmv<CH, XCD, kMatStream> : kb_m_spmv<CH, XCD, kMatCached>;
+  hipLaunchKernelGGL(k, dim3(XCD ? 8 * per : nb), dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity);
+}
+hipError_t launch_bm_spmv(const BLaunch &L, int shape, int parity, hipStream_t st) {
   switch (shape) {
-    case 0: hipLaunchKernelGGL((kb_m_spmv<9, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
-    case 1: hipLaunchKernelGGL((kb_m_spmv<27, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
-    case 2: hipLaunchKernelGGL((kb_m_spmv<81, false>), plain, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
-    case 3: hipLaunchKernelGGL((kb_m_spmv<9, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
-    case 4: hipLaunchKernelGGL((kb_m_spmv<27, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
-    case 5: hipLaunchKernelGGL((kb_m_spmv<81, true>), xcd, dim3(256), 0, st, L.rv, L.row.at, L.cg, nb, per, parity); break;
+    case 0: launch_m_spmv<9, false>(L, parity, st); break;
+    case 1: launch_m_spmv<27, false>(L, parity, st); break;
+    case 2: launch_m_spmv<81, false>(L, parity, st); break;
+    case 3: launch_m_spmv<9, true>(L, parity, st); break;
+    case 4: launch_m_spmv<27, true>(L, parity, st); break;
+    case 5: launch_m_spmv<81, true>(L, parity, st); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

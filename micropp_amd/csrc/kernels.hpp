@@ -567,16 +567,24 @@ __device__ __forceinline__ SegPitch stage_runs(const Grid &g, int row0, T *seg /
 
 // One row's products with the staged runs (own: its node there), in slot
 // order: the first chunk's values are loaded by the caller, each later chunk's
-// before the products of the one in front.  Slot k's value is v[k * VS]: VS =
-// 64 in a stored matrix (streamed once), 1 in a row of a stencil table.
-template <int VS, typename T>
+// before the products of the one in front.
+// Where the values come from: a stored matrix (slot k at v[k * 64]) read past
+// the caches or through them, or a row of a stencil table (v[k]).
+enum MatSource { kMatStream, kMatCached, kMatTable };
+template <int SRC, typename T>
 __device__ __forceinline__ T load_value(const T *v, int k) {
-  if constexpr (VS == 64)
+  if constexpr (SRC == kMatStream)
     return __builtin_nontemporal_load(&v[k * 64]);
   else
-    return v[k * VS];
+    return v[SRC == kMatTable ? k : k * 64];
 }
-template <int CH, int VS = 64, typename T>
+// The stored matrix of a CG is read once an iteration.  While most of it (of
+// every RVE of a launch) fits the 256 MB last-level cache, plain loads find it
+// there, or in L2; beyond, non-temporal ones keep it from evicting the vectors.
+// us per SpMV, plain / non-temporal: 21 MB 6.4 / 8.5, 101 MB 18.4 / 18.8, 171 MB
+// (FP32) 28.7 / 30.0, 270 MB (FP32) 42.1 / 43.0, 381 MB 72.8 / 65.0.
+inline int mat_source(double bytes) { return bytes > 320e6 ? kMatStream : kMatCached; }
+template <int CH, int SRC, typename T>
 __device__ __forceinline__ T dot_runs(const T *v, T (&vi)[2][CH], const T *own, SegPitch pt) {
 #pragma clang fp contract(off)
   static_assert(kSlots % CH == 0 && CH % 3 == 0, "chunks tile the row in whole neighbours");
@@ -585,7 +593,7 @@ __device__ __forceinline__ T dot_runs(const T *v, T (&vi)[2][CH], const T *own, 
   for (int ch = 0; ch < kSlots / CH; ++ch) {
     if (ch + 1 < kSlots / CH)
 #pragma unroll
-      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = load_value<VS>(v, (ch + 1) * CH + k);
+      for (int k = 0; k < CH; ++k) vi[(ch + 1) & 1][k] = load_value<SRC>(v, (ch + 1) * CH + k);
 #pragma unroll
     for (int k = 0; k < CH; k += 3) {
       const int n = (ch * CH + k) / 3;
@@ -726,7 +734,7 @@ __device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, do
 }
 
 // step1 of a matrix assembled here (computed stencil columns).  What bounds
-// it: at 50^3 nodes the 648 bytes of values per row from HBM; on RVEs of a few
+// it: at 50^3 nodes the 648 bytes of values per row; on RVEs of a few
 // thousand rows the chain of waits (state, sums, stage, values).  The first
 // chunk of the row's values does not depend on any of the others, so it is
 // loaded before them, and each later chunk before the previous one's products;
@@ -735,7 +743,7 @@ __device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, do
 // place of vals: 81 values of each of the three rows per code, k_s_table), the
 // same values in the same order (kDictNodes).  51^3 nodes: 22.6 us against 47.2
 // with the stored matrix, what is left being LDS and L1 reads; 31^3 8.6 / 12.5.
-template <int CH, int VS = 64>
+template <int CH, int SRC>
 __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, const double *vals,
                                                 const uint16_t *code, const double *kinv, const double *r,
                                                 const double *p, double *pn, double *Ap, double *part1,
@@ -744,18 +752,18 @@ __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, c
   __shared__ double lds[4];
   CgRegs c = cg_load(cur);
   const int row0 = lb * 256, row = row0 + threadIdx.x;
-  const double *v = VS == 64 ? vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63)
-                             : vals + ((size_t)code[row / 3] * 3 + row % 3) * kSlots;
+  const double *v = SRC == kMatTable ? vals + ((size_t)code[row / 3] * 3 + row % 3) * kSlots
+                                     : vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
   double vi[2][CH];
   if (!c.done)
 #pragma unroll
-    for (int k = 0; k < CH; ++k) vi[0][k] = load_value<VS>(v, k);
+    for (int k = 0; k < CH; ++k) vi[0][k] = load_value<SRC>(v, k);
   if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
   const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return cg_dir(c, kinv[q], r[q], p[q]); });
   const double *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
   // rows past the last node lie on its run's clamped end; p is zero there
   const double pv = row < g.nrow ? own[row % 3] : 0.0;
-  const double acc = dot_runs<CH, VS>(v, vi, own, pt);
+  const double acc = dot_runs<CH, SRC>(v, vi, own, pt);
   pn[row] = pv;
   Ap[row] = acc;
   double t[1] = {pv * acc};
@@ -820,7 +828,7 @@ __device__ __forceinline__ void cg_tail_body(const double *part2, int nb, CgStat
 
 // Ap = A p and the partials of p.Ap of the FP32 inner CG (mixed-precision
 // batch), p in memory; products of p and Ap are formed in FP64
-template <int CH>
+template <int CH, int SRC>
 __device__ __forceinline__ void cg_spmv_body32(const Grid &g, int lb, const float *vals, const float *p, float *Ap,
                                                double *part1, const CgState *cur) {
 #pragma clang fp contract(off)
@@ -831,11 +839,11 @@ __device__ __forceinline__ void cg_spmv_body32(const Grid &g, int lb, const floa
   if (cur->done) return;
   float vi[2][CH];
 #pragma unroll
-  for (int k = 0; k < CH; ++k) vi[0][k] = __builtin_nontemporal_load(&v[k * 64]);
+  for (int k = 0; k < CH; ++k) vi[0][k] = load_value<SRC>(v, k);
   const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return p[q]; });
   const float *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
   const float pv = row < g.nrow ? own[row % 3] : 0.0f;
-  const float y = dot_runs<CH>(v, vi, own, pt);
+  const float y = dot_runs<CH, SRC>(v, vi, own, pt);
   Ap[row] = y;
   double t[1] = {(double)pv * (double)y};
   block_sum<1, 256>(t, lds);

@@ -45,23 +45,14 @@ __global__ void __launch_bounds__(256) k_cg_init_state(const double *part, int n
 // Blocks are dispatched round-robin over the 8 XCDs: the 8 * per launched
 // blocks give XCD x the row blocks [x * per, (x + 1) * per), so each XCD's
 // L2 holds a contiguous slab of the gathered vector (2-5% faster SpMV).
-__global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const double *vals, const double *kinv,
-                                                  const double *r, const double *p, double *pn, double *Ap,
-                                                  double *part, const CgState *cur, CgState *nxt) {
+template <int SRC>
+__global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const double *vals, const uint16_t *code,
+                                                  const double *kinv, const double *r, const double *p, double *pn,
+                                                  double *Ap, double *part, const CgState *cur, CgState *nxt) {
   const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (lb >= nb) return;
   __shared__ double seg[kSegDoubles];
-  cg_step1_body64<kChunk>(g, lb, nb, vals, nullptr, kinv, r, p, pn, Ap, part, cur, nxt, seg);
-}
-
-__global__ void __launch_bounds__(256) k_cg_step1_dict(Grid g, int nb, int per, const double *tab,
-                                                       const uint16_t *code, const double *kinv, const double *r,
-                                                       const double *p, double *pn, double *Ap, double *part,
-                                                       const CgState *cur, CgState *nxt) {
-  const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (lb >= nb) return;
-  __shared__ double seg[kSegDoubles];
-  cg_step1_body64<kChunk, 1>(g, lb, nb, tab, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
+  cg_step1_body64<kChunk, SRC>(g, lb, nb, vals, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
 }
 
 // code[n]: sum over the elements q = (a*2+b)*2+c around interior node n of
@@ -168,12 +159,12 @@ hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, c
       hipLaunchKernelGGL(k_cg_dir, dim3(nb), dim3(256), 0, st, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.part + nb, cur, nxt);
     hipLaunchKernelGGL(k_cg_spmv_cols, dim3(8 * per), dim3(256), 0, st, nb, per, cols, vals, w.p[k ^ 1], w.Ap, w.part,
                        nxt);
-  } else if (dict) {
-    hipLaunchKernelGGL(k_cg_step1_dict, dim3(8 * per), dim3(256), 0, st, g, nb, per, dict->tab, dict->code, w.kinv,
-                       w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   } else {
-    hipLaunchKernelGGL(k_cg_step1, dim3(8 * per), dim3(256), 0, st, g, nb, per, vals, w.kinv, w.r, w.p[k], w.p[k ^ 1],
-                       w.Ap, w.part, cur, nxt);
+    const int src = dict ? kMatTable : mat_source((double)g.nrow_pad * kSlots * sizeof(double));
+    const auto step1 = src == kMatTable ? k_cg_step1<kMatTable> : src == kMatStream ? k_cg_step1<kMatStream>
+                                                                                  : k_cg_step1<kMatCached>;
+    hipLaunchKernelGGL(step1, dim3(8 * per), dim3(256), 0, st, g, nb, per, dict ? dict->tab : vals,
+                       dict ? dict->code : nullptr, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   }
   return hipGetLastError();
 }
