@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(256) k_norm_finish(const double *part, int npa
   if (threadIdx.x == 0) red->v[0] = sqrt(t[0]);
 }
 
-__global__ void __launch_bounds__(256) k_ave_stress(Grid g, const double *bmat, const material_base *mats,
+__global__ void __launch_bounds__(8 * kAveElems) k_ave_stress(Grid g, const double *bmat, const material_base *mats,
                                                     const int *et, const double *u, const double *vars, double *part) {
   ave_stress_body(g, blockIdx.x, bmat, mats, et, u, vars, part);
 }
@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(256) k_ave_stress(Grid g, const double *bmat, 
 // one block: the 6 averages from the per-block partials
 __global__ void __launch_bounds__(256) k_ave_finish(const double *part, int nparts, double vol, RedState *red) {
   double t[6];
-  seg_sum<6>(part, nparts, t);
+  ave_total(part, nparts, t);
   if (threadIdx.x == 0)
     for (int v = 0; v < 6; ++v) red->v[v] = t[v] / vol;
 }
@@ -134,7 +134,7 @@ hipError_t launch_gather_vals(const Grid &g, const int *et, const double *ke, in
 
 hipError_t launch_elem_be(const Grid &g, const double *bmat, const material_base *mats_d, const int *et,
                           const double *u, const double *vars, double *be, hipStream_t st) {
-  hipLaunchKernelGGL(k_elem_be, dim3(nblk(g.nelem, 256)), dim3(256), 0, st, g, bmat, mats_d, et, u, vars, be);
+  hipLaunchKernelGGL(k_elem_be, dim3(nblk(g.nelem, kGpElems)), dim3(8 * kGpElems), 0, st, g, bmat, mats_d, et, u, vars, be);
   return hipGetLastError();
 }
 
@@ -149,7 +149,7 @@ hipError_t launch_gather_rhs(const Grid &g, const double *be, double *b, double 
 hipError_t launch_ave_stress(const Grid &g, const double *bmat, const material_base *mats_d, const int *et,
                              const double *u, const double *vars, double *partials, RedState *red, hipStream_t st) {
   const unsigned nb = nblk(g.nelem, 256);
-  hipLaunchKernelGGL(k_ave_stress, dim3(nb), dim3(256), 0, st, g, bmat, mats_d, et, u, vars, partials);
+  hipLaunchKernelGGL(k_ave_stress, dim3(nb * 256 / kAveElems), dim3(8 * kAveElems), 0, st, g, bmat, mats_d, et, u, vars, partials);
   hipLaunchKernelGGL(k_ave_finish, dim3(1), dim3(256), 0, st, partials, (int)nb, g.vol_tot, red);
   return hipGetLastError();
 }
@@ -163,7 +163,7 @@ hipError_t launch_elem_fields(const Grid &g, const double *bmat, const material_
 
 hipError_t launch_vars_new(const Grid &g, const double *bmat, const material_base *mats_d, const int *et,
                            const double *u, const double *vars_old, double *vars_new, RedState *red, hipStream_t st) {
-  hipLaunchKernelGGL(k_vars_new, dim3(nblk(g.nelem, 256)), dim3(256), 0, st, g, bmat, mats_d, et, u, vars_old,
+  hipLaunchKernelGGL(k_vars_new, dim3(nblk(g.nelem, kGpElems)), dim3(8 * kGpElems), 0, st, g, bmat, mats_d, et, u, vars_old,
                      vars_new, red);
   return hipGetLastError();
 }

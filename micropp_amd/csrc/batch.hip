@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(256) kb_gather_vals(const BRve *rv, const int 
 
 __global__ void __launch_bounds__(256) kb_elem_be(const BRve *rv, const int *map, const int *act, const int *blk0) {
   MPP_BATCH_PROLOGUE(map)
-  elem_be_body(R.g, blockIdx.x - blk0[rid], R.bmat, R.mats, R.et, R.uw, R.use_vars ? R.vars_n : nullptr, R.be);
+  elem_be_body(R.g, (blockIdx.x - blk0[rid]) * (256 / kGpElems) + blockIdx.y, R.bmat, R.mats, R.et, R.uw, R.use_vars ? R.vars_n : nullptr, R.be);
 }
 
 __global__ void __launch_bounds__(256) kb_gather_rhs(const BRve *rv, const int *map, const int *act,
@@ -102,10 +102,10 @@ __global__ void __launch_bounds__(256) kb_norm_finish(const BRve *rv, const int 
 }
 
 // u = uw (which 0) or u_k (which 1); vars as the RVE's use_vars says
-__global__ void __launch_bounds__(256) kb_ave_stress(const BRve *rv, const int *map, const int *act, const int *blk0,
+__global__ void __launch_bounds__(8 * kAveElems) kb_ave_stress(const BRve *rv, const int *map, const int *act, const int *blk0,
                                                      int which) {
   MPP_BATCH_PROLOGUE(map)
-  ave_stress_body(R.g, blockIdx.x - blk0[rid], R.bmat, R.mats, R.et, which ? R.u_k : R.uw,
+  ave_stress_body(R.g, (blockIdx.x - blk0[rid]) * (256 / kAveElems) + blockIdx.y, R.bmat, R.mats, R.et, which ? R.u_k : R.uw,
                   R.use_vars ? R.vars_n : nullptr, R.part);
 }
 
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(256) kb_ave_finish(const BRve *rv, const int *
   if (!act[rid]) return;
   const BRve &R = rv[rid];
   double t[6];
-  seg_sum<6>(R.part, R.nb_elem, t);
+  ave_total(R.part, R.nb_elem, t);
   if (threadIdx.x == 0)
     for (int v = 0; v < 6; ++v) out[(size_t)rid * 6 + v] = t[v] / R.g.vol_tot;
 }
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256) kb_ave_finish(const BRve *rv, const int *
 __global__ void __launch_bounds__(256) kb_vars_new(const BRve *rv, const int *map, const int *act, const int *blk0,
                                                    int *flags) {
   MPP_BATCH_PROLOGUE(map)
-  vars_new_body(R.g, blockIdx.x - blk0[rid], R.bmat, R.mats, R.et, R.u_k, R.use_vars ? R.vars_n : nullptr,
+  vars_new_body(R.g, (blockIdx.x - blk0[rid]) * (256 / kGpElems) + blockIdx.y, R.bmat, R.mats, R.et, R.u_k, R.use_vars ? R.vars_n : nullptr,
                 R.use_vars ? R.vars_k : R.vars_aux, flags + rid);
 }
 
@@ -583,19 +583,19 @@ hipError_t launch_b_mat(const BLaunch &L, const int *act_ke, const int *act_gath
   return hipGetLastError();
 }
 hipError_t launch_b_rhs(const BLaunch &L, double *norms, hipStream_t st) {
-  hipLaunchKernelGGL(kb_elem_be, dim3(L.elem.nb), dim3(256), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0);
+  hipLaunchKernelGGL(kb_elem_be, dim3(L.elem.nb, 256 / kGpElems), dim3(8 * kGpElems), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0);
   hipLaunchKernelGGL(kb_gather_rhs, dim3(L.row.nb), dim3(256), 0, st, L.rv, L.row.map, L.act, L.row.blk0);
   hipLaunchKernelGGL(kb_norm_finish, dim3(L.nrve), dim3(256), 0, st, L.rv, L.act, norms);
   return hipGetLastError();
 }
 hipError_t launch_b_ave(const BLaunch &L, int which, double *sig, hipStream_t st) {
-  hipLaunchKernelGGL(kb_ave_stress, dim3(L.elem.nb), dim3(256), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0, which);
+  hipLaunchKernelGGL(kb_ave_stress, dim3(L.elem.nb, 256 / kAveElems), dim3(8 * kAveElems), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0, which);
   hipLaunchKernelGGL(kb_ave_finish, dim3(L.nrve), dim3(256), 0, st, L.rv, L.act, sig);
   return hipGetLastError();
 }
 hipError_t launch_b_vars_new(const BLaunch &L, int *flags, hipStream_t st) {
   hipLaunchKernelGGL(kb_zero_ints, dim3((L.nrve + 255) / 256), dim3(256), 0, st, L.nrve, flags);
-  hipLaunchKernelGGL(kb_vars_new, dim3(L.elem.nb), dim3(256), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0, flags);
+  hipLaunchKernelGGL(kb_vars_new, dim3(L.elem.nb, 256 / kGpElems), dim3(8 * kGpElems), 0, st, L.rv, L.elem.map, L.act, L.elem.blk0, flags);
   return hipGetLastError();
 }
 hipError_t launch_b_cg_init(const BLaunch &L, double min_err, double rel_err, int max_its, hipStream_t st) {

@@ -26,7 +26,7 @@ struct BRve {
   double *uw, *u_n, *u_k;      // working / converged / current displacements
   double *x, *r, *p[2], *Ap, *kinv, *b;
   double *vars_n, *vars_k, *vars_aux;
-  double *part;                // partials: max(3 nb_row, 6 nb_elem)
+  double *part;                // partials: max(3 nb_row, 24 nb_elem)
   CgState *cg;                 // ping-pong pair
   // mixed precision (nullptr without): the FP32 copy of the matrix being
   // solved (vals' layout), the inner CG's FP32 vectors and Jacobi weights;

@@ -984,7 +984,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     kes += (size_t)(R.phase_mode ? 3 : g.nelem) * 576;
     bes += (size_t)g.nelem * 24;
     if (!v->all_elastic) nvars += (size_t)g.nelem * 8 * NVAR;
-    parts += std::max<size_t>(3 * (size_t)R.nb_row, 6 * (size_t)R.nb_elem);
+    parts += std::max<size_t>(3 * (size_t)R.nb_row, 24 * (size_t)R.nb_elem);
   }
   // the coarse nodes' blocks, which take longest, start first
   std::stable_partition(at[4].begin(), at[4].end(), [&](const int2 &b) { return b.y >= B->h[b.x].nb_row; });
@@ -1041,7 +1041,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     o_slot += (size_t)g.nrow_pad * kSlots;
     o_ke += (size_t)(R.phase_mode ? 3 : g.nelem) * 576;
     o_be += (size_t)g.nelem * 24;
-    o_part += std::max<size_t>(3 * (size_t)R.nb_row, 6 * (size_t)R.nb_elem);
+    o_part += std::max<size_t>(3 * (size_t)R.nb_row, 24 * (size_t)R.nb_elem);
   }
   if (B->prm.mixed_precision) {
     constexpr int kVecs32 = 6;  // x32 r32[2] p32 Ap32 kinv32
@@ -1434,7 +1434,7 @@ int mppd_batch_slot_bytes(const mppd_rve *r, size_t *bytes) {
   if (!r->all_elastic) b += (size_t)g.nelem * 8 * NVAR * 3 * sizeof(double);
   if (r->all_elastic && g.nn >= kDictNodes)
     b += stencil64_codes(g) * sizeof(uint16_t) + stencil64_table() * sizeof(double);
-  b += std::max(3 * nb_row, 6 * nb_elem) * sizeof(double) + 2 * sizeof(CgState) + 8 * 144 * sizeof(double);
+  b += std::max(3 * nb_row, 24 * nb_elem) * sizeof(double) + 2 * sizeof(CgState) + 8 * 144 * sizeof(double);
   *bytes = b;
   return MPPD_OK;
 }

@@ -308,33 +308,72 @@ __device__ __forceinline__ void gather_vals_slice(const Grid &g, int slice, cons
 }
 
 // ---------------------------------------------------------------------------
-// Element internal forces, get_elem_rhs (src/assembly.cpp:123-138): one
-// thread per element; B staged in LDS.
+// The Gauss-point kernels: a thread per Gauss point (8 lanes an element), so
+// that an RVE of a few hundred elements is not a handful of waves that each
+// evaluate eight laws in a row.  gp_stage puts the gradients and the
+// displacements of the block's NE elements (from e0 on) into LDS, gp_strain is
+// get_strain at the thread's point (strain_row, in the reference's order).
+// ---------------------------------------------------------------------------
+template <int NE>
+__device__ __forceinline__ void gp_stage(const Grid &g, int e0, const double *bmat_g, const double *u,
+                                         double *grad /* [8 * 24] */, double *ue /* [NE * 24] */) {
+  for (int t = threadIdx.x; t < 8 * 24; t += 8 * NE) grad[t] = bmat_g[(t / 24) * 144 + (t % 3) * 24 + t % 24];
+  for (int t = threadIdx.x; t < NE * 24; t += 8 * NE) {
+    const int e = e0 + t / 24, i = t % 24;
+    if (e >= g.nelem) break;
+    int ex, ey, ez;
+    elem_coords(g, e, ex, ey, ez);
+    ue[t] = u[(size_t)elem_node(g, ex, ey, ez, i / 3) * 3 + i % 3];
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void gp_strain(const double *grad, const double *ue, double *eps) {
+#pragma unroll
+  for (int v = 0; v < 6; ++v) eps[v] = strain_row(&grad[(threadIdx.x & 7) * 24], &ue[(threadIdx.x >> 3) * 24], v);
+}
+
+constexpr int kGpElems = 32;    // elements per block of 256 threads
+constexpr int kAveElems = 64;   // elements per block of 512 (ave_stress_body)
+
+// ---------------------------------------------------------------------------
+// Element internal forces, get_elem_rhs (src/assembly.cpp:123-138).  The
+// stresses of the block's points go through LDS; then three of the 24 entries
+// of an element per thread, summed over (gp, component) in the reference's
+// order, B's zeros left out (elem_ke_body).  40^3 J2 elements 25
+// us, 125 elements 6 (a thread per element: 37.5 and 24).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void elem_be_body(const Grid &g, int lb, const double *bmat_g, const material_base *mats,
                                              const int *et, const double *u, const double *vars, double *be) {
 #pragma clang fp contract(off)
-  __shared__ double bm[8 * 144];
-  stage_bmat(bmat_g, bm);
-  __syncthreads();
-  const int e = lb * 256 + threadIdx.x;
-  if (e >= g.nelem) return;
-  int ex, ey, ez;
-  elem_coords(g, e, ex, ey, ez);
-  double ue[24];
-  gather_ue(g, ex, ey, ez, u, ue);
-  const material_base &m = mats[et[e]];
-  double acc[24];
-  for (int i = 0; i < 24; ++i) acc[i] = 0;
-  for (int gp = 0; gp < 8; ++gp) {
-    double eps[6], sig[6];
-    strain_at(&bm[gp * 144], ue, eps);
-    mat_stress(m, eps, vars ? vars + ((size_t)e * 8 + gp) * NVAR : nullptr, sig);
-    for (int i = 0; i < 24; ++i)
-      for (int v = 0; v < 6; ++v) acc[i] += bm[gp * 144 + v * 24 + i] * sig[v] * g.wg;
+  __shared__ double grad[8 * 24], ue[kGpElems * 24], sig_s[kGpElems * 48];
+  const int e0 = lb * kGpElems;
+  gp_stage<kGpElems>(g, e0, bmat_g, u, grad, ue);
+  const int e = e0 + (threadIdx.x >> 3);
+  if (e < g.nelem) {
+    double eps[6];
+    gp_strain(grad, ue, eps);
+    mat_stress(mats[et[e]], eps, vars ? vars + ((size_t)e0 * 8 + threadIdx.x) * NVAR : nullptr,
+               &sig_s[threadIdx.x * 6]);
   }
-  double *out = be + (size_t)e * 24;
-  for (int i = 0; i < 24; ++i) out[i] = acc[i];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int t = k * 256 + threadIdx.x, i = t % 24, a = i / 3, d = i % 3;
+    if (e0 + t / 24 >= g.nelem) break;
+    // the three components with row i of B not zero, ascending, and its entries there
+    const int v0 = d, v1 = d == 2 ? 4 : 3, v2 = d == 0 ? 4 : 5;
+    const int g0 = d, g1 = d == 1 ? 0 : d == 0 ? 1 : 0, g2 = d == 0 ? 2 : d == 1 ? 2 : 1;
+    double acc = 0;
+#pragma unroll
+    for (int gp = 0; gp < 8; ++gp) {
+      const double *b = &grad[gp * 24 + a * 3], *sig = &sig_s[(t / 24) * 48 + gp * 6];
+      acc += b[g0] * sig[v0] * g.wg;
+      acc += b[g1] * sig[v1] * g.wg;
+      acc += b[g2] * sig[v2] * g.wg;
+    }
+    be[(size_t)e0 * 24 + t] = acc;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -370,32 +409,53 @@ __device__ __forceinline__ void gather_rhs_body(const Grid &g, int lb, const dou
 
 // ---------------------------------------------------------------------------
 // calc_ave_stress (src/average.cpp:57-82): per-element sums over the Gauss
-// points; the block's partial of the 6 components goes to part[lb * 6 ..].
+// points, and the sum of a block's 64 elements (one wave of them) to
+// part[lb * 6 ..]; ave_total adds those.  40^3 J2 elements
+// 15.5 us, 125 elements 5 (a thread per element: 21 and 13).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void ave_stress_body(const Grid &g, int lb, const double *bmat_g, const material_base *mats,
                                                 const int *et, const double *u, const double *vars, double *part) {
 #pragma clang fp contract(off)
-  __shared__ double bm[8 * 144];
-  __shared__ double lds[4 * 6];
-  stage_bmat(bmat_g, bm);
-  __syncthreads();
-  const int e = lb * 256 + threadIdx.x;
-  double s6[6] = {0, 0, 0, 0, 0, 0};
+  __shared__ double grad[8 * 24], ue[kAveElems * 24], sig_s[kAveElems * 48];
+  const int e0 = lb * kAveElems;
+  gp_stage<kAveElems>(g, e0, bmat_g, u, grad, ue);
+  const int e = e0 + (threadIdx.x >> 3);
   if (e < g.nelem) {
-    int ex, ey, ez;
-    elem_coords(g, e, ex, ey, ez);
-    double ue[24];
-    gather_ue(g, ex, ey, ez, u, ue);
-    const material_base &m = mats[et[e]];
-    for (int gp = 0; gp < 8; ++gp) {
-      double eps[6], sig[6];
-      strain_at(&bm[gp * 144], ue, eps);
-      mat_stress(m, eps, vars ? vars + ((size_t)e * 8 + gp) * NVAR : nullptr, sig);
-      for (int v = 0; v < 6; ++v) s6[v] += sig[v] * g.wg;
-    }
+    double eps[6];
+    gp_strain(grad, ue, eps);
+    mat_stress(mats[et[e]], eps, vars ? vars + ((size_t)e0 * 8 + threadIdx.x) * NVAR : nullptr,
+               &sig_s[threadIdx.x * 6]);
   }
-  block_sum<6, 256>(s6, lds);
-  if (threadIdx.x < 6) part[(size_t)lb * 6 + threadIdx.x] = s6[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  double s6[6] = {0, 0, 0, 0, 0, 0};
+  if (e0 + (int)threadIdx.x < g.nelem)
+    for (int gp = 0; gp < 8; ++gp)
+#pragma unroll
+      for (int v = 0; v < 6; ++v) s6[v] += sig_s[threadIdx.x * 48 + gp * 6 + v] * g.wg;
+#pragma unroll
+  for (int v = 0; v < 6; ++v) {
+    const double s = wave_sum(s6[v]);
+    if (threadIdx.x == 0) part[(size_t)lb * 6 + v] = s;
+  }
+}
+
+// the 6 totals of nb blocks of 256 elements, four partials each, by one block
+// of 256 threads (every thread gets them)
+__device__ __forceinline__ void ave_total(const double *part, int nb, double (&t)[6]) {
+#pragma clang fp contract(off)
+  __shared__ double lds[4 * 6];
+#pragma unroll
+  for (int v = 0; v < 6; ++v) t[v] = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 256)
+#pragma unroll
+    for (int v = 0; v < 6; ++v) {
+      double s = 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) s += part[((size_t)b * 4 + w) * 6 + v];
+      t[v] += s;
+    }
+  block_sum<6, 256>(t, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -436,30 +496,24 @@ __device__ __forceinline__ void elem_fields_body(const Grid &g, int lb, const do
 
 // ---------------------------------------------------------------------------
 // calc_vars_new (src/update.cpp:32-56): evolute per Gauss point; any
-// nonlinear point sets *flag.
+// nonlinear point sets *flag.  40^3 J2 elements 13 us, 125
+// elements 4.4 (a thread per element: 20.5 and 13).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void vars_new_body(const Grid &g, int lb, const double *bmat_g, const material_base *mats,
                                               const int *et, const double *u, const double *vars_old,
                                               double *vars_new, int *flag) {
 #pragma clang fp contract(off)
-  __shared__ double bm[8 * 144];
-  stage_bmat(bmat_g, bm);
-  __syncthreads();
-  const int e = lb * 256 + threadIdx.x;
+  __shared__ double grad[8 * 24], ue[kGpElems * 24];
+  const int e0 = lb * kGpElems;
+  gp_stage<kGpElems>(g, e0, bmat_g, u, grad, ue);
+  const int e = e0 + (threadIdx.x >> 3);
   if (e >= g.nelem) return;
-  int ex, ey, ez;
-  elem_coords(g, e, ex, ey, ez);
-  double ue[24];
-  gather_ue(g, ex, ey, ez, u, ue);
-  const material_base &m = mats[et[e]];
-  int nl = 0;
-  for (int gp = 0; gp < 8; ++gp) {
-    double eps[6];
-    strain_at(&bm[gp * 144], ue, eps);
-    const size_t off = ((size_t)e * 8 + gp) * NVAR;
-    nl |= mat_evolute(m, eps, vars_old ? vars_old + off : nullptr, vars_new + off);
-  }
-  if (nl) atomicOr(flag, 1);
+  double eps[6];
+  gp_strain(grad, ue, eps);
+  const size_t off = ((size_t)e0 * 8 + threadIdx.x) * NVAR;
+  const int nl = mat_evolute(mats[et[e]], eps, vars_old ? vars_old + off : nullptr, vars_new + off);
+  const unsigned long long any = __ballot(nl != 0);  // one atomic per wave
+  if (any && (int)(threadIdx.x & 63) == __ffsll(any) - 1) atomicOr(flag, 1);
 }
 
 // ---------------------------------------------------------------------------

@@ -334,7 +334,7 @@ int mppd_solver_create(mppd_solver **out, mppd_rve *r) {
       if ((rc = dalloc(v, np, st))) break;
     if (rc) break;
     const size_t nb = std::max(round_up(np, 256) / 256, round_up((size_t)g.nelem, 256) / 256) + 1;
-    if ((rc = dalloc(&s->partials, nb * 8, st))) break;
+    if ((rc = dalloc(&s->partials, nb * 24, st))) break;  // 4 x 6 per 256 elements (ave_stress), 3 per 256 rows
     if ((rc = dalloc(&s->cg, 2, st))) break;  // ping-pong pair
     if ((rc = dalloc(&s->red, 1, st))) break;
     e = hipHostMalloc((void **)&s->cg_h, sizeof(CgState), hipHostMallocDefault);
