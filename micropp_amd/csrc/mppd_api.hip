@@ -67,6 +67,7 @@ struct mppd_solver {
   double *b = nullptr, *du = nullptr;
   double *partials = nullptr;
   CgState *cg = nullptr, *cg_h = nullptr;
+  int cg_expect = 0;  // iterations of the last CG
   RedState *red = nullptr, *red_h = nullptr;
   struct MixedLin *ml = nullptr;  // mppd_newton_mixed buffers, made on first use
   // vals came from this library's assembly (nonzeros only on in-grid stencil
@@ -480,28 +481,27 @@ int mppd_ell_mvp(mppd_solver *s, const double *x_d, double *y_d) {
 struct CgWork {
   CgVecs v;
   CgState *state_h;
+  int *expect;  // iterations of the solver's last CG (0: none yet)
 };
 
 static CgVecs cg_vecs(const mppd_solver *s) {
   return CgVecs{s->x, s->rr, {s->p, s->p2}, s->Ap, s->kinv, s->partials, s->cg};
 }
 
-// CG on the device; the host queues iterations in chunks sized from the
-// observed convergence rate and reads the 64-byte state between chunks.
+// CG on the device; the host queues iterations in chunks sized from the last
+// solve and the observed convergence rate and reads the state between chunks.
 // After `queued` iterations the current state is state[queued & 1].
 static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipStream_t st, const double *b_d,
                      double min_err, double rel_err, int max_its, int *its_out, double *err_out) {
   const CgVecs &v = w.v;
   MPP_HIP(launch_cg_init(g, A->vals, b_d, v, min_err, rel_err, max_its, st));
-  int queued = 0;
-  MPP_HIP(hipMemcpyAsync(w.state_h, v.state, sizeof(CgState), hipMemcpyDeviceToHost, st));
-  MPP_HIP(hipStreamSynchronize(st));
-  double pn_prev = w.state_h->pn;
-  int its_prev = 0;
-  int chunk = 32;
-  while (!w.state_h->done) {
-    const int n = std::min(chunk, max_its - queued);
-    if (n <= 0) break;
+  int queued = 0, its_prev = 0;
+  double pn_prev = 0;  // of the first look: pn0
+  // as many as the last solve took before the first look (an iteration queued
+  // past the end costs 3 us, a look about 10)
+  int chunk = *w.expect > 0 ? std::max(4, std::min(256, *w.expect + 1)) : 32;
+  for (;;) {
+    const int n = std::max(0, std::min(chunk, max_its - queued));
     for (int i = 0; i < n; ++i)
       MPP_HIP(launch_cg_iter(g, A->cg_cols(), A->vals, A->cg_dict(), v, queued + i, st));
     queued += n;
@@ -509,7 +509,8 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
     MPP_HIP(hipMemcpyAsync(w.state_h, v.state + (queued & 1), sizeof(CgState), hipMemcpyDeviceToHost, st));
     MPP_HIP(hipStreamSynchronize(st));
     const CgState &c = *w.state_h;
-    if (c.done) break;
+    if (c.done || queued >= max_its) break;
+    if (its_prev == 0) pn_prev = c.pn0;
     // next chunk: iterations still needed at the observed rate, within [4, 256]
     const double target = std::max(c.min_err, c.pn0 * c.rel_err);
     const int dit = c.its - its_prev;
@@ -523,6 +524,7 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
     pn_prev = c.pn;
     its_prev = c.its;
   }
+  *w.expect = w.state_h->its;
   if (its_out) *its_out = w.state_h->its;
   if (err_out) *err_out = w.state_h->rz;
   return MPPD_OK;
@@ -530,7 +532,8 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
 
 static int cg_run(mppd_solver *s, const mppd_solver *A, const double *b_d, double min_err, double rel_err,
                   int max_its, int *its_out, double *err_out) {
-  return cg_run_on(s->r->g, A, CgWork{cg_vecs(s), s->cg_h}, s->st, b_d, min_err, rel_err, max_its, its_out, err_out);
+  const CgWork w{cg_vecs(s), s->cg_h, &s->cg_expect};
+  return cg_run_on(s->r->g, A, w, s->st, b_d, min_err, rel_err, max_its, its_out, err_out);
 }
 
 // A0's matrix is read with s's row layout: it must be a solver of an RVE grid
@@ -607,7 +610,8 @@ int mppd_cg_noalloc(mppd_solver *s, const mppd_solver *A0, const double *b_d, do
   double *v = ptr + kNoAllocHead;
   const auto vec = [v](int i) { return v + i * kNoAllocRows; };
   const CgWork w{
-      CgVecs{vec(0), vec(1), {vec(2), vec(3)}, vec(4), vec(5), vec(6), reinterpret_cast<CgState *>(ptr)}, s->cg_h};
+      CgVecs{vec(0), vec(1), {vec(2), vec(3)}, vec(4), vec(5), vec(6), reinterpret_cast<CgState *>(ptr)}, s->cg_h,
+      &s->cg_expect};
   if (int rc = cg_run_on(g, A0 ? A0 : s, w, s->st, b_d, min_err, rel_err, max_its, its, err)) return rc;
   MPP_HIP(launch_copy(g.nrow, w.v.x, x_d, s->st));
   MPP_HIP(hipStreamSynchronize(s->st));
@@ -663,11 +667,10 @@ int mppd_newton(mppd_solver *s, const mppd_solver *A0, const double eps[6], cons
       break;
     }
     const mppd_solver *A = s;
-    if (!A0 || its > p->its_with_A0 - 1) {
-      MPP_HIP(mat_async(s, u_d, vars_old_d));
-    } else {
+    if (A0 && its <= p->its_with_A0 - 1)
       A = A0;
-    }
+    else if (!s->vals_phase)  // (an all-elastic RVE's matrix is assembled once)
+      MPP_HIP(mat_async(s, u_d, vars_old_d));
     int cg_its = 0;
     double err = 0;
     int rc = cg_run(s, A, s->b, p->cg_abs_tol, p->cg_rel_tol, p->cg_max_its, &cg_its, &err);
