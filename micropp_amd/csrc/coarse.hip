@@ -562,9 +562,9 @@ int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double
   int *info_d = nullptr;
   int rc = MPPD_OK;
   do {
-    // one allocation for the temporaries: Ab | Lb | Wp | C | KE
-    if ((rc = dalloc(&buf, 2 * nband + nw + nC + nKE, false))) break;
-    if ((rc = dalloc(&info_d, 1, false))) break;
+    // one allocation for the temporaries: Ab | Lb | Wp | C | KE | info
+    if ((rc = dalloc(&buf, 2 * nband + nw + nC + nKE + 1, false))) break;
+    info_d = reinterpret_cast<int *>(buf + 2 * nband + nw + nC + nKE);
     double *Ab = buf, *Lb = Ab + nband, *Wp = Lb + nband, *C = Wp + nw, *KE = C + nC;
     hipError_t e = hipMemsetAsync(info_d, 0, sizeof(int), st);
     if (e != hipSuccess) {
@@ -592,7 +592,6 @@ int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double
   } while (0);
   (void)hipStreamSynchronize(st);  // the temporaries below may still be in use after a failed step
   dfree(buf);
-  dfree(info_d);
   return rc;
 }
 

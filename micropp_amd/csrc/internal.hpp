@@ -12,10 +12,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <cstdlib>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "material_base.h"
 #include "mppd.h"
@@ -81,6 +84,31 @@ inline int dalloc(T **p, size_t n, bool zero = true) {
   }
   return MPPD_OK;
 }
+
+// The device buffers of an object as one allocation with 256-byte aligned
+// parts: hipMalloc and hipFree cost 20 to 700 us each, a set of one or two
+// dozen buffers several milliseconds.  add() every part, then alloc().
+class Arena {
+ public:
+  template <typename T>
+  void add(T **p, size_t n) {
+    parts_.push_back({reinterpret_cast<void **>(p), size_});
+    size_ += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+  }
+  size_t size() const { return size_; }
+  // *base owns the parts
+  int alloc(void **base) {
+    *base = nullptr;
+    const hipError_t e = hipMalloc(base, size_);
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc");
+    for (auto &p : parts_) *p.first = static_cast<char *>(*base) + p.second;
+    return MPPD_OK;
+  }
+
+ private:
+  size_t size_ = 0;
+  std::vector<std::pair<void **, size_t>> parts_;
+};
 
 // Device allocation of n elements, zero-filled on stream st: the fill is
 // ordered before st's later work, and the caller synchronizes st before the
@@ -392,6 +420,7 @@ struct mppd_rve {
   double *bmat = nullptr;
   int *et = nullptr;
   double *spheres = nullptr;
+  void *arena = nullptr;  // owns the above
   int nsph = 0;
   double vf[2] = {0, 0};
   int all_elastic = 1;

@@ -84,6 +84,7 @@ struct micropp<tdim>::impl {
   mppd_rve *rve = nullptr;
   mppd_solver *sol = nullptr;
   mppd_solver *A0 = nullptr;
+  double *fields = nullptr;   // owns u, vars_aux and the GPs' u_n and u_k: one allocation (device)
   double *u = nullptr;        // working displacement (device)
   double *vars_aux = nullptr;  // vars_new when the GP has no history yet (device)
   std::vector<int> fe_ids;     // GPs with FE_ONE_WAY / FE_FULL coupling
@@ -112,9 +113,8 @@ struct micropp<tdim>::impl {
       mppd_solver_destroy(wk[k].sol);
     }
     for (auto &q : gp)
-      for (double *p : {q.vars_n, q.vars_k, q.u_n, q.u_k}) mppd_free(p);
-    mppd_free(u);
-    mppd_free(vars_aux);
+      for (double *p : {q.vars_n, q.vars_k}) mppd_free(p);
+    mppd_free(fields);
     mppd_solver_destroy(A0);
     mppd_solver_destroy(sol);
     mppd_rve_destroy(rve);
@@ -573,19 +573,29 @@ micropp<tdim>::micropp(const micropp_params_t &params, const micropp_options_t &
     check(mppd_rve_volume_fractions(s.rve, vf), "volume fractions");
     s.Vm = vf[0];
     s.Vf = vf[1];
-    s.u = dzeros(s.nndim);
-    s.vars_aux = dzeros(s.nvars);
-    s.wk.push_back(worker{s.sol, s.u, s.vars_aux});
     s.gp.resize(s.ngp);
-    int n_fe = 0;
+    int n_fe = 0, n_u = 0;
+    for (int g = 0; g < s.ngp; ++g) {
+      const int c = params.coupling ? params.coupling[g] : FE_ONE_WAY;
+      n_u += !params.coupling || c == FE_ONE_WAY || c == FE_FULL;
+    }
+    // each part on a 256-byte boundary
+    const auto whole = [](size_t n) { return (n + 31) / 32 * 32; };
+    const size_t nu = whole(s.nndim), nv = whole(s.nvars);
+    s.fields = dzeros(nu * (1 + 2 * (size_t)n_u) + nv);
+    s.u = s.fields;
+    s.vars_aux = s.fields + nu;
+    double *next = s.vars_aux + nv;
+    s.wk.push_back(worker{s.sol, s.u, s.vars_aux});
     for (int g = 0; g < s.ngp; ++g) {
       gp_state &q = s.gp[g];
       q.coupling = params.coupling ? params.coupling[g] : FE_ONE_WAY;
       if (q.coupling == FE_LINEAR || q.coupling == FE_ONE_WAY || q.coupling == FE_FULL) n_fe++;
       if (q.coupling == FE_ONE_WAY || q.coupling == FE_FULL) s.fe_ids.push_back(g);
       if (!params.coupling || q.coupling == FE_ONE_WAY || q.coupling == FE_FULL) {
-        q.u_n = dzeros(s.nndim);
-        q.u_k = dzeros(s.nndim);
+        q.u_n = next;
+        q.u_k = next + nu;
+        next += 2 * nu;
       }
     }
     if (s.use_A0) {

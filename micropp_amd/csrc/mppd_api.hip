@@ -57,6 +57,7 @@ using namespace mpp;
 struct mppd_solver {
   mppd_rve *r = nullptr;
   hipStream_t st = nullptr;
+  void *arena = nullptr;  // owns the device buffers below
   int *cols = nullptr;
   double *vals = nullptr;
   double *ke = nullptr;
@@ -208,17 +209,25 @@ int mppd_rve_create(mppd_rve **out, const int size[3], int micro_type, const dou
   int *bad = nullptr;
   unsigned long long *cnt_d = nullptr;
   do {
-    if ((rc = dalloc(&r->bmat, 8 * 144))) break;
-    if ((rc = dalloc(&r->mats_d, 3))) break;
-    if ((rc = dalloc(&r->et, (size_t)g.nelem))) break;
+    Arena a;
+    a.add(&r->bmat, 8 * 144);
+    a.add(&r->mats_d, 3);
+    a.add(&r->spheres, (size_t)kMaxSpheres * 4);
+    a.add(&bad, 1);
+    a.add(&cnt_d, 2);
+    a.add(&r->et, (size_t)g.nelem);
+    if ((rc = a.alloc(&r->arena))) break;
+    hipError_t e = hipMemset(r->arena, 0, a.size());
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // (the null stream, see dalloc)
+    if (e != hipSuccess) {
+      rc = hip_fail(e, "hipMemset");
+      break;
+    }
     if (hipMemcpy(r->mats_d, r->mats, 3 * sizeof(material_base), hipMemcpyHostToDevice) != hipSuccess) {
       rc = fail(MPPD_ERR_HIP, "materials upload");
       break;
     }
-    if ((rc = dalloc(&r->spheres, (size_t)kMaxSpheres * 4))) break;
-    if ((rc = dalloc(&bad, 1))) break;
-    if ((rc = dalloc(&cnt_d, 2))) break;
-    hipError_t e = launch_bmat(g, r->bmat, nullptr);
+    e = launch_bmat(g, r->bmat, nullptr);
     if (e == hipSuccess && micro_type == kMicRandomSpheres) {
       int n = (int)geo[1];
       r->nsph = n < 0 ? 0 : (n > kMaxSpheres ? kMaxSpheres : n);
@@ -247,8 +256,6 @@ int mppd_rve_create(mppd_rve **out, const int size[3], int micro_type, const dou
     r->vf[1] = vfb / g.vol_tot;
     if (bad_h) rc = fail(MPPD_ERR_ARG, "invalid micro_type");
   } while (0);
-  dfree(bad);
-  dfree(cnt_d);
   if (rc) {
     mppd_rve_destroy(r);
     return rc;
@@ -259,10 +266,7 @@ int mppd_rve_create(mppd_rve **out, const int size[3], int micro_type, const dou
 
 int mppd_rve_destroy(mppd_rve *r) {
   if (!r) return MPPD_OK;
-  dfree(r->bmat);
-  dfree(r->mats_d);
-  dfree(r->et);
-  dfree(r->spheres);
+  dfree(r->arena);
   delete r;
   return MPPD_OK;
 }
@@ -320,26 +324,28 @@ int mppd_solver_create(mppd_solver **out, mppd_rve *r) {
       rc = hip_fail(e, "hipStreamCreate");
       break;
     }
-    // zero fills on s->st (synchronized below)
-    hipStream_t st = s->st;
-    if ((rc = dalloc(&s->cols, np * kSlots, false))) break;
-    if ((rc = dalloc(&s->vals, np * kSlots, st))) break;
-    if ((rc = dalloc(&s->ke, (s->phase_mode ? 3 : (size_t)g.nelem) * 576, false))) break;
-    if (s->phase_mode && g.nn >= kDictNodes) {
-      if ((rc = dalloc(&s->dict.code, stencil64_codes(g), false))) break;
-      if ((rc = dalloc(&s->dict.tab, stencil64_table(), false))) break;
-    }
-    if ((rc = dalloc(&s->be, (size_t)g.nelem * 24, false))) break;
+    Arena a;
+    a.add(&s->vals, np * kSlots);
     double **vecs[] = {&s->x, &s->rr, &s->p, &s->p2, &s->Ap, &s->kinv, &s->b, &s->du};
-    for (double **v : vecs)
-      if ((rc = dalloc(v, np, st))) break;
-    if (rc) break;
+    for (double **v : vecs) a.add(v, np);
     const size_t nb = std::max(round_up(np, 256) / 256, round_up((size_t)g.nelem, 256) / 256) + 1;
-    if ((rc = dalloc(&s->partials, nb * 24, st))) break;  // 4 x 6 per 256 elements (ave_stress), 3 per 256 rows
-    if ((rc = dalloc(&s->cg, 2, st))) break;  // ping-pong pair
-    if ((rc = dalloc(&s->red, 1, st))) break;
-    e = hipHostMalloc((void **)&s->cg_h, sizeof(CgState), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&s->red_h, sizeof(RedState), hipHostMallocDefault);
+    a.add(&s->partials, nb * 24);  // 4 x 6 per 256 elements (ave_stress), 3 per 256 rows
+    a.add(&s->cg, 2);              // ping-pong pair
+    a.add(&s->red, 1);
+    const size_t zeroed = a.size();
+    a.add(&s->cols, np * kSlots);
+    a.add(&s->ke, (s->phase_mode ? 3 : (size_t)g.nelem) * 576);
+    if (s->phase_mode && g.nn >= kDictNodes) {
+      a.add(&s->dict.code, stencil64_codes(g));
+      a.add(&s->dict.tab, stencil64_table());
+    }
+    a.add(&s->be, (size_t)g.nelem * 24);
+    if ((rc = a.alloc(&s->arena))) break;
+    e = hipMemsetAsync(s->arena, 0, zeroed, s->st);  // (synchronized below)
+    static_assert(sizeof(CgState) % alignof(RedState) == 0, "one pinned block");
+    if (e == hipSuccess)
+      e = hipHostMalloc((void **)&s->cg_h, sizeof(CgState) + sizeof(RedState), hipHostMallocDefault);
+    if (e == hipSuccess) s->red_h = reinterpret_cast<RedState *>(s->cg_h + 1);
     if (e == hipSuccess) e = launch_ell_cols(g, s->cols, s->st);
     if (e == hipSuccess) e = hipStreamSynchronize(s->st);
     if (e != hipSuccess) rc = hip_fail(e, "solver set-up");
@@ -355,12 +361,8 @@ int mppd_solver_create(mppd_solver **out, mppd_rve *r) {
 int mppd_solver_destroy(mppd_solver *s) {
   if (!s) return MPPD_OK;
   if (s->st) (void)hipStreamSynchronize(s->st);
-  for (void *p : {(void *)s->cols, (void *)s->vals, (void *)s->ke, (void *)s->be, (void *)s->x, (void *)s->rr,
-                  (void *)s->p, (void *)s->p2, (void *)s->dict.code, (void *)s->dict.tab, (void *)s->Ap, (void *)s->kinv, (void *)s->b, (void *)s->du,
-                  (void *)s->partials, (void *)s->cg, (void *)s->red})
-    dfree(p);
-  if (s->cg_h) (void)hipHostFree(s->cg_h);
-  if (s->red_h) (void)hipHostFree(s->red_h);
+  dfree(s->arena);
+  if (s->cg_h) (void)hipHostFree(s->cg_h);  // and red_h
   mixed_lin_free(s->ml);
   if (s->st) (void)hipStreamDestroy(s->st);
   delete s;
