@@ -364,8 +364,9 @@ hipError_t launch_m_resid(const Grid &g, int K, const int *et, const double *ke,
                           double abs_tol, double tau_min, int max_inner, void *state, hipStream_t st,
                           const int *active = nullptr);
 // field f of U from / into a displacement vector in the reference numbering (node * 3 + d)
-hipError_t launch_m_load_u(const Grid &g, int K, int f, const double *u, double *U, hipStream_t st);
-hipError_t launch_m_store_u(const Grid &g, int K, int f, const double *U, double *u, hipStream_t st);
+// U's K fields = the n <= K vectors u[k] (a null one, or null u: zero), zero beyond; and back to those not null
+hipError_t launch_m_load_u(const Grid &g, int K, int n, const double *const *u, double *U, hipStream_t st);
+hipError_t launch_m_store_u(const Grid &g, int K, int n, const double *U, double *const *u, hipStream_t st);
 // adjoint: G (3 x 24 x 6 doubles) and the sources F of fields 0 .. nadj-1
 hipError_t launch_m_adj_src(const Grid &g, int K, int nadj, const double *bmat, const material_base *mats_d,
                             const int *et, double *G, double *F, hipStream_t st);

@@ -94,20 +94,31 @@ __global__ void __launch_bounds__(256) k_m_setbc(Grid g, int NP, const double *e
 }
 
 // ---------------------------------------------------------------------------
-// One field of U from / into a displacement vector in the reference DOF
+// The fields of U from / into displacement vectors in the reference DOF
 // numbering (u[node * 3 + d]); padding nodes of U are zero after a load.
 // ---------------------------------------------------------------------------
+// All fields in one launch (16 fields of 30^3 elements: 5 us each way instead
+// of 16 kernels of 2.8); a field without a vector loads as zero.
+struct FieldIn {
+  const double *u[16];
+};
+struct FieldOut {
+  double *u[16];
+};
+
 template <int K>
-__global__ void __launch_bounds__(256) k_m_load_u(Grid g, int NP, int f, const double *u, double *U) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_m_load_u(Grid g, int NP, FieldIn in, double *U) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x, f = blockIdx.y;
   if (n >= NP) return;
-  for (int d = 0; d < 3; ++d) U[(size_t)(d * K + f) * NP + n] = (n < g.nn) ? u[(size_t)n * 3 + d] : 0.0;
+  const double *u = in.u[f];
+  for (int d = 0; d < 3; ++d) U[(size_t)(d * K + f) * NP + n] = u && n < g.nn ? u[(size_t)n * 3 + d] : 0.0;
 }
 
 template <int K>
-__global__ void __launch_bounds__(256) k_m_store_u(Grid g, int NP, int f, const double *U, double *u) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= g.nn) return;
+__global__ void __launch_bounds__(256) k_m_store_u(Grid g, int NP, const double *U, FieldOut out) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x, f = blockIdx.y;
+  double *u = out.u[f];
+  if (n >= g.nn || !u) return;
   for (int d = 0; d < 3; ++d) u[(size_t)n * 3 + d] = U[(size_t)(d * K + f) * NP + n];
 }
 
@@ -1553,15 +1564,19 @@ hipError_t launch_m_setbc(const Grid &g, int K, const double *eps, double *U, hi
   return hipGetLastError();
 }
 
-hipError_t launch_m_load_u(const Grid &g, int K, int f, const double *u, double *U, hipStream_t st) {
+hipError_t launch_m_load_u(const Grid &g, int K, int n, const double *const *u, double *U, hipStream_t st) {
   const MLaunch s = mshape(g);
-  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_load_u<KK>, dim3(s.NP / 256), dim3(256), 0, st, g, s.NP, f, u, U));
+  FieldIn in{};
+  for (int k = 0; k < n; ++k) in.u[k] = u ? u[k] : nullptr;
+  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_load_u<KK>, dim3(s.NP / 256, KK), dim3(256), 0, st, g, s.NP, in, U));
   return hipGetLastError();
 }
 
-hipError_t launch_m_store_u(const Grid &g, int K, int f, const double *U, double *u, hipStream_t st) {
+hipError_t launch_m_store_u(const Grid &g, int K, int n, const double *U, double *const *u, hipStream_t st) {
   const MLaunch s = mshape(g);
-  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_store_u<KK>, dim3(nblk(g.nn, 256)), dim3(256), 0, st, g, s.NP, f, U, u));
+  FieldOut out{};
+  for (int k = 0; k < n; ++k) out.u[k] = u[k];
+  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_store_u<KK>, dim3(nblk(g.nn, 256), n), dim3(256), 0, st, g, s.NP, U, out));
   return hipGetLastError();
 }
 

@@ -1063,9 +1063,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
   if (max_inner < 1 || max_outer < 1) return fail(MPPD_ERR_ARG, "bad mixed parameters");
   for (int i = 0; i < K * 6; ++i) m->eps_h[i] = (i / 6 < n) ? eps_h[i] : 0.0;
   MPP_HIP(hipMemcpyAsync(m->eps_d, m->eps_h, K * 6 * sizeof(double), hipMemcpyHostToDevice, m->st));
-  MPP_HIP(hipMemsetAsync(m->U, 0, mixed_vector_len(g, K) * sizeof(double), m->st));
-  for (int k = 0; k < n; ++k)
-    if (u_in && u_in[k]) MPP_HIP(launch_m_load_u(g, K, k, u_in[k], m->U, m->st));
+  MPP_HIP(launch_m_load_u(g, K, n, u_in, m->U, m->st));
   MPP_HIP(launch_m_setbc(g, K, m->eps_d, m->U, m->st));
   std::vector<int> its(K, 0), run(K, 0), conv(K, 0), cost(K, 0), cflag(K, 0);
   std::vector<double> rn(K), rn0(K), norm0(K), pn(K), pn0(K);
@@ -1132,8 +1130,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
     if ((rc = msolver_averages(m))) return rc;
     for (int i = 0; i < n * 6; ++i) sig_h[i] = m->sig_h[i];
   }
-  for (int k = 0; k < n; ++k)
-    if (u_out && u_out[k]) MPP_HIP(launch_m_store_u(g, K, k, m->U, u_out[k], m->st));
+  if (u_out) MPP_HIP(launch_m_store_u(g, K, n, m->U, u_out, m->st));
   MPP_HIP(hipStreamSynchronize(m->st));
   for (int k = 0; k < n; ++k) {
     out[3 * k] = its[k];
