@@ -544,8 +544,8 @@ __global__ void __launch_bounds__(256) k_m_spmv(Grid g, int NP, int nsl, int per
 // (r, z) with z = kinv R.  Every block re-sums the (p, Ap) partials of its
 // four fields (part1[field * nsl + slice]) in the same fixed order, so all
 // blocks agree bit for bit; block (0, g) records alpha of group g in the
-// state for k_m_pupd.  Grid (blocks of kVecNodes nodes, 3 K/4 components
-// c = d * K/4 + g), each thread kVecNodes / 256 nodes; partial tables pz / pr
+// state for k_m_pupd.  Grid (blocks of 256 J nodes, 3 K/4 components
+// c = d * K/4 + g), each thread J nodes; partial tables pz / pr
 // [(field * 3 + d) * gridDim.x + block] (the 3 gridDim.x partials of a field
 // contiguous; pr = pz + 3 K gridDim.x).  X is advanced in k_m_pupd, which
 // reads P anyway.
@@ -555,7 +555,7 @@ __global__ void __launch_bounds__(256) k_m_spmv(Grid g, int NP, int nsl, int per
 // Its partials then number ceil(ny nz / lpb) per (field, d) (gridDim.x).
 // kPcCycle (multilevel preconditioner): z = kinv r goes to T1 (R's layout).
 enum { kPcJacobi = 0, kPcCoarse = 1, kPcCycle = 2 };
-template <int K, int PC>
+template <int K, int PC, int J = kVecNodes / 256>
 __global__ void __launch_bounds__(kRedThreads) k_m_upd(int NP, int nsl, const double *part1, const float *kinv,
                                                        const float4 *AP, float4 *R, double *pz, double *pr,
                                                        MState *cur, Grid g, CGrid cg, int lpb, float4 *T1) {
@@ -573,8 +573,7 @@ __global__ void __launch_bounds__(kRedThreads) k_m_upd(int NP, int nsl, const do
   // the barriers below)
   if constexpr (COARSE)
     for (int s2 = threadIdx.x; s2 < 2 * cg.hx - 1; s2 += kRedThreads) wt[s2] = hat(1 + s2, 1, cg.hx);
-  constexpr int J = kVecNodes / 256;
-  int nbeg = blockIdx.x * kVecNodes, nend = min(nbeg + kVecNodes, NP), l0 = 0, l1 = 0;
+  int nbeg = blockIdx.x * (256 * J), nend = min(nbeg + 256 * J, NP), l0 = 0, l1 = 0;
   if constexpr (COARSE) {
     l0 = blockIdx.x * lpb;
     l1 = min(l0 + lpb, g.ny * g.nz);
@@ -984,7 +983,7 @@ __global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int row, const double *
 // (beta, ||z||, stop flags, iteration count).  Grid as k_m_upd.
 // COARSE (two-level and multilevel preconditioners): z is read from Z instead
 // of being formed from kinv and R.  rowz, row: partials per field of pz, pr.
-template <int K, bool COARSE>
+template <int K, bool COARSE, int J = kVecNodes / 256>
 __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kinv, const float4 *R, const float4 *Z,
                                                         float4 *P, float4 *X, const double *pz, int rowz,
                                                         const double *pr, int row, const MState *cur,
@@ -1012,10 +1011,9 @@ __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kin
     rows_load<4>(pr + (size_t)r0 * row, row, row, srz);
   }
   asm volatile("" ::: "memory");
-  constexpr int J = kVecNodes / 256;
   float kvv[J];
   float4 rvv[J], pvv[J], xvv[J];
-  const int n0 = blockIdx.x * kVecNodes + threadIdx.x;
+  const int n0 = blockIdx.x * (256 * J) + threadIdx.x;
 #pragma unroll
   for (int jn = 0; jn < J; ++jn) {
     const int n = min(n0 + jn * 256, NP - 1);
@@ -1656,20 +1654,29 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &
                        reinterpret_cast<const float4 *>(coarse->z), p4, x4, pz, 3 * nbu, pr, 3 * nbx, cur, nxt);
     return hipGetLastError();
   }
+  // two nodes a thread while eight leave the grid short of blocks
+  const bool narrow = (size_t)nbx * (3 * K / 4) < kVecWide;
+  const int nbn = narrow ? (int)nblk(s.NP, 512) : nbx;
+  const dim3 ngrid(nbn, 3 * K / 4);
+  pr = pz + (size_t)3 * K * nbn;
   MPP_K_DISPATCH(K, {
     if (vc) {
       // R -= alpha AP and D^-1 R, then z = M R into AP (with the (r, z)
       // partials), and the p-update from it
-      hipLaunchKernelGGL((k_m_upd<KK, kPcCycle>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
+      const auto upd = narrow ? (k_m_upd<KK, kPcCycle, 2>) : (k_m_upd<KK, kPcCycle>);
+      const auto pupd = narrow ? (k_m_pupd<KK, true, 2>) : (k_m_pupd<KK, true>);
+      hipLaunchKernelGGL(upd, ngrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
                          reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, reinterpret_cast<float4 *>(vc->z));
       if ((e = launch_vcycle(g, K, *vc, op, kinv, R, vc->z, AP, AP, pr, cur, st)) != hipSuccess) return e;
-      hipLaunchKernelGGL((k_m_pupd<KK, true>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, ap4, p4, x4, pz,
-                         3 * nbx, pr, np1, cur, nxt);
+      hipLaunchKernelGGL(pupd, ngrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, ap4, p4, x4, pz, 3 * nbn, pr, np1, cur,
+                         nxt);
     } else {
-      hipLaunchKernelGGL((k_m_upd<KK, kPcJacobi>), vgrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
+      const auto upd = narrow ? (k_m_upd<KK, kPcJacobi, 2>) : (k_m_upd<KK, kPcJacobi>);
+      const auto pupd = narrow ? (k_m_pupd<KK, false, 2>) : (k_m_pupd<KK, false>);
+      hipLaunchKernelGGL(upd, ngrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
                          reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, nullptr);
-      hipLaunchKernelGGL((k_m_pupd<KK, false>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, nullptr, p4, x4, pz,
-                         3 * nbx, pr, 3 * nbx, cur, nxt);
+      hipLaunchKernelGGL(pupd, ngrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, nullptr, p4, x4, pz, 3 * nbn, pr,
+                         3 * nbn, cur, nxt);
     }
   });
   return hipGetLastError();

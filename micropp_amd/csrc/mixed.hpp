@@ -17,6 +17,12 @@ constexpr int kNodeQuads = kRowQuads * kRows;  // 63 float4 per node
 __host__ __device__ constexpr int mslot(int nb, int fi, int fj) { return (nb / 3) * 28 + (nb % 3) * 9 + fi * 3 + fj; }
 constexpr int kRedThreads = 256;  // threads of the one-block reducers
 constexpr int kVecNodes = 2048;   // nodes per block of the vector kernels
+// Blocks of kVecNodes nodes from which the vector kernels of the multi-RHS CG
+// keep them; with fewer, blocks of 512 nodes.  Iteration, us, 512 / 2048 nodes:
+// 11^3 nodes of 8 fields (6 blocks) 37.0 / 38.5, 26^3 of 16 (108) 64.2 / 67.6,
+// 31^3 of 16 (180) 81.4 / 83.9, 41^3 of 8 (204) 86.6 / 85.3, 46^3 of 12 (432)
+// 127 / 121.
+constexpr size_t kVecWide = 200;
 
 // inner CG scalars per field: rz = (r, z), alpha / beta of the iteration, pn
 // the current ||z||, pn0 the start value, tau the relative stop
