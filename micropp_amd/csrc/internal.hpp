@@ -292,7 +292,7 @@ constexpr int kStencilCodes = 6561 + 2;  // 3^8 phase patterns, a boundary node,
 // Nodes from which an all-elastic RVE's FP64 CG reads the table: its 12.8 MB
 // (of which a solve touches the RVE's own patterns) against 1944 bytes a node
 // of stored values.  Below, both come from L2: 16^3 nodes 10.3 us an iteration
-// either way, 21^3 10.0 / 10.7, 26^3 11.0 / 12.7, 51^3 34.0 / 58.0.
+// either way, 21^3 10.0 / 10.7, 26^3 11.0 / 12.7, 51^3 28.3 / 58.0.
 constexpr int kDictNodes = 8000;
 inline size_t stencil64_codes(const Grid &g) { return (size_t)g.nrow_pad / 3 + 1; }
 inline size_t stencil64_table() { return (size_t)kStencilCodes * 3 * kSlots; }

@@ -20,7 +20,7 @@
 // 16.2, 31^3 17.7 / 23.0, 41^3 33.0 / 37.8, 51^3 58.0 / 60.4.  Small RVEs wait
 // for launches and block sums (kernels of about 6 and 3 us), 51^3 for 259 MB of
 // values a pass (5.5 TB/s); with the stencil table of an all-elastic RVE 51^3
-// takes 34.0, 31^3 13.2.
+// takes 28.3, 31^3 13.2.
 #include "kernels.hpp"
 
 namespace mpp {
@@ -53,6 +53,89 @@ __global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const
   if (lb >= nb) return;
   __shared__ double seg[kSegDoubles];
   cg_step1_body64<kChunk, SRC>(g, lb, nb, vals, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
+}
+
+// step1 on the stencil table with a thread per node: the three rows share the
+// staged values, and a wave whose interior nodes have one code (most of them,
+// away from phase interfaces) takes the 243 values as scalars.  Blocks of 256
+// nodes, three row blocks each, whose partials are those of k_cg_step1: the
+// same rows in the same tree.
+constexpr int kNodeBlock = 256;
+// Row blocks from which it runs: fewer than two node blocks a CU leave its nine
+// lines of scalar loads, one after the other, in the open.  Iteration, us, by
+// node / by row: 31^3 nodes (350 row blocks) 15.7 / 13.4, 41^3 (808) 23.1 /
+// 21.3, 46^3 (1141) 24.9 / 28.1, 51^3 (1555) 28.3 / 33.7.  Lines of more than
+// 256 nodes would need more LDS than a launch has by default.
+constexpr int kNodeRowBlocks = 1100, kNodeMaxLine = 256;
+__global__ void __launch_bounds__(kNodeBlock) k_cg_step1_node(Grid g, int nb, int nblocks, int per,
+                                                              const double *__restrict__ tab,
+                                                              const uint16_t *__restrict__ code, const double *kinv,
+                                                              const double *r, const double *p, double *pn, double *Ap,
+                                                              double *part1, const CgState *cur, CgState *nxt) {
+#pragma clang fp contract(off)
+  extern __shared__ double seg[];  // three runs of nodes, one per dz; then the products
+  const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (lb >= nblocks) return;
+  CgRegs c = cg_load(cur);
+  const int n0 = lb * kNodeBlock, n = n0 + threadIdx.x;
+  const int own_code = code[min(n, g.nrow_pad / 3)];
+  if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
+  const int len = kNodeBlock + 2 + 2 * g.nx, nxny = g.nx * g.ny, hi = g.nn - 1;
+  for (int dz = -1; dz <= 1; ++dz)
+#pragma unroll 2
+    for (int e3 = threadIdx.x; e3 < 3 * len; e3 += kNodeBlock) {
+      const int q = 3 * min(max(n0 - 1 - g.nx + dz * nxny + e3 / 3, 0), hi) + e3 % 3;
+      seg[(dz + 1) * 3 * len + e3] = cg_dir(c, kinv[q], r[q], p[q]);
+    }
+  lds_barrier();
+  const double *own = seg + (threadIdx.x + 1 + g.nx + len) * 3;
+  const bool row = own_code < kStencilCodes - 2, node = n < g.nn;
+  double acc[3] = {0.0, 0.0, 0.0};
+  const unsigned long long rows = __ballot(row);
+  const int first = rows ? __ffsll(rows) - 1 : 0;
+  const int wave_code = __builtin_amdgcn_readlane(own_code, first);
+  // line m of the stencil's nine: 3 neighbours x 3 values for each of the rows
+  const auto line = [&](const auto *t, int m) {
+    const double *x = own + ((m / 3 - 1) * len + (m % 3 - 1) * g.nx - 1) * 3;
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+      for (int fi = 0; fi < 3; ++fi) acc[fi] += t[fi * kSlots + m * 9 + k] * x[k];
+  };
+  if (__ballot(row && own_code != wave_code) == 0) {
+    // the constant address space makes these scalar loads
+    typedef const __attribute__((address_space(4))) double *Scalars;
+    const Scalars t = (Scalars)(uintptr_t)(tab + (size_t)wave_code * 3 * kSlots);
+#pragma unroll 1
+    for (int m = 0; m < 9; ++m) line(t, m);
+  } else {
+    const double *t = tab + (size_t)own_code * 3 * kSlots;
+#pragma unroll 1
+    for (int m = 0; m < 9; ++m) line(t, m);
+  }
+  double pv[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    pv[d] = node ? own[d] : 0.0;
+    if (!row) acc[d] = node ? 0.0 + pv[d] : 0.0;  // a Dirichlet row's only value is its 1.0
+  }
+  lds_barrier();
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int q = 3 * n + d;
+    if (q < g.nrow_pad) {
+      pn[q] = pv[d];
+      Ap[q] = acc[d];
+    }
+    seg[threadIdx.x * 3 + d] = pv[d] * acc[d];
+  }
+  lds_barrier();
+  __shared__ double lds[4 * 3];
+  double t[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) t[k] = seg[k * 256 + threadIdx.x];
+  block_sum<3, 256>(t, lds);
+  if (threadIdx.x < 3 && lb * 3 + (int)threadIdx.x < nb) part1[lb * 3 + threadIdx.x] = t[threadIdx.x];
 }
 
 // code[n]: sum over the elements q = (a*2+b)*2+c around interior node n of
@@ -159,6 +242,11 @@ hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, c
       hipLaunchKernelGGL(k_cg_dir, dim3(nb), dim3(256), 0, st, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.part + nb, cur, nxt);
     hipLaunchKernelGGL(k_cg_spmv_cols, dim3(8 * per), dim3(256), 0, st, nb, per, cols, vals, w.p[k ^ 1], w.Ap, w.part,
                        nxt);
+  } else if (dict && nb >= kNodeRowBlocks && g.nx <= kNodeMaxLine) {
+    const int nn = (nb + 2) / 3, pern = (nn + 7) / 8;
+    const size_t lds = (size_t)3 * 3 * (kNodeBlock + 2 + 2 * g.nx) * sizeof(double);
+    hipLaunchKernelGGL(k_cg_step1_node, dim3(8 * pern), dim3(kNodeBlock), lds, st, g, nb, nn, pern, dict->tab,
+                       dict->code, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   } else {
     const int src = dict ? kMatTable : mat_source((double)g.nrow_pad * kSlots * sizeof(double));
     const auto step1 = src == kMatTable ? k_cg_step1<kMatTable> : src == kMatStream ? k_cg_step1<kMatStream>

@@ -48,10 +48,11 @@ def test_solve_by_computed_and_by_uploaded_columns(mp, oracle, size):
         assert abs(it6 - io) <= 1 and np.abs(x.numpy() - xo).max() <= 1e-5 * np.abs(xo).max()
 
 
-@pytest.mark.parametrize("size", [(20, 20, 20), (21, 20, 19), (90, 10, 9)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("size", [(20, 20, 20), (21, 20, 19), (90, 10, 9), (47, 46, 45), (256, 25, 15), (257, 25, 15)],
+                         ids=lambda s: "x".join(map(str, s)))
 def test_stencil_table_of_elastic_rves(mp, size):
     """From 8000 nodes on (20^3; 7980 stay below) an all-elastic RVE's CG reads a stencil table instead of the
-    matrix; three phases.  Solved bit for bit as the uploaded matrix, alone and beside a J2 RVE in a batch, whose
+    matrix, from 1100 row blocks on (47x46x45) with a thread per node unless a line has more than 256; three phases.  Solved bit for bit as the uploaded matrix, alone and beside a J2 RVE in a batch, whose
     Newton then needs what a batch of the elastic RVE alone needs."""
     mats = [mp.material(0, 1e6, 0.3), mp.material(0, 1e7, 0.25), mp.material(0, 3e6, 0.2)]
     geo = (0.3, 0.15, 0.0, 0.0)
