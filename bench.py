@@ -12,13 +12,16 @@ of its initial value.  A step yields 6 RVE solves (sigma + ctan).
 
 Paths
   mixed (value): the 12 solves of a step run together -- FP32 multi-RHS
-        Jacobi-PCG inner solves, FP64 residual / update / averages.
+        PCG inner solves with a V-cycle preconditioner, FP64 residual /
+        update / averages.
   plain: the reference algorithm on the GPU, one FP64 Newton/CG solve after
-        another (the reference ELL values; the SpMV computes the stencil
-        columns instead of loading them, with bit-identical results).
-roofline: the dominant kernel of the mixed path (the FP32 multi-RHS SpMV),
-  timed with HIP events on its own stream; algorithmic bytes per node =
-  252 x 4 (coefficients incl. the 9 row pads) + 2 x 3K x 4 (p in, Ap out).
+        another (the reference ELL values, out of a table of phase patterns
+        by a 16-bit code per node, with bit-identical results).
+roofline: the dominant kernel of the mixed path (the FP32 multi-RHS operator,
+  three applications an inner iteration), timed with HIP events on its own
+  stream; algorithmic bytes per node = 2 (stencil code) + 2 x 3K x 4 (p in,
+  Ap out).  Of the plain path, the kernel that forms p and Ap: 2 + 5 x 24 (D^-1,
+  r and p in, p and Ap out).
 Secondary lines (not value; --no-batch skips them):
   drop_in: the same workload through the micropp3_* interface (one mixed-
         precision micropp<3> instance with 6 Gauss points; its constructor
@@ -52,7 +55,9 @@ CG_TOL, CG_MAX = 1e-8, 2000
 D_EPS = 1e-8
 HBM_PEAK_GBS = 8000.0
 BYTES_PER_ROW_SPMV64 = 81 * 8 + 16  # values + p in + Ap out (columns are computed)
-BYTES_PER_NODE_SPMV32 = 252 * 4 + 2 * 3 * K * 4
+BYTES_PER_NODE_SPMV32 = 252 * 4 + 2 * 3 * K * 4  # a stored node-block matrix (single mixed Newton)
+BYTES_PER_NODE_APPLY32 = 2 + 2 * 3 * K * 4
+BYTES_PER_NODE_TABLE64 = 2 + 5 * 24
 
 
 def workload(seed=SEED):
@@ -592,9 +597,9 @@ def main():
     value = N_STRAINS / dt_mixed
     spmv_ms, iter_ms = ms.profile(args.profile_iters)
     nodes = SIZE ** 3
-    spmv_bytes = BYTES_PER_NODE_SPMV32 * nodes
+    spmv_bytes = BYTES_PER_NODE_APPLY32 * nodes
     achieved = spmv_bytes / (spmv_ms * 1e-3) / 1e9
-    traffic, traffic_src = pmc_traffic(f"k_m_spmv{K}_50cube_traffic.md")
+    traffic, traffic_src = pmc_traffic(f"k_d_apply{K}_50cube_traffic.md")
 
     line = {
         "metric": "RVE solves/s (sigma+ctan) at 50^3, 1 GPU",
@@ -616,7 +621,8 @@ def main():
                    "outer_steps": stats[0], "inner_iterations": stats[1]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": f"k_m_spmv<{K}> (FP32 node-block SpMV, {K} RHS in 4-field groups, + p.Ap)",
+                     "kernel": f"k_d_apply<{K}> (FP32 operator from a stencil dictionary, {K} RHS in 4-field groups, "
+                               "+ p.Ap)",
                      "bytes_per_launch": spmv_bytes, "avg_ms": spmv_ms, "inner_iteration_ms": iter_ms},
     }
 
@@ -632,14 +638,14 @@ def main():
         solver.assembly_mat(u)
         solver.assembly_rhs(u, None, b)
         p_spmv_ms, p_iter_ms = mp.cg_profile(solver, b, args.profile_iters)
-        p_bytes = BYTES_PER_ROW_SPMV64 * 3 * nodes
+        p_bytes = BYTES_PER_NODE_TABLE64 * nodes
         p_ach = p_bytes / (p_spmv_ms * 1e-3) / 1e9
-        p_traffic, p_src = pmc_traffic("k_cg_step1_50cube_traffic.md")
+        p_traffic, p_src = pmc_traffic("k_cg_step1_node_50cube_traffic.md")
         line["plain_fp64"] = {"value": N_STRAINS / dt_plain, "ms_per_step": 1e3 * dt_plain,
                               "cg_iterations_per_step": cg_its,
                               "roofline": {"bound": "hbm", "achieved": p_ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                            "frac": p_ach / HBM_PEAK_GBS, "traffic": p_traffic,
-                                           "traffic_source": p_src, "kernel": "k_cg_step1 (FP64 ELL SpMV, stencil columns computed, + p.Ap)",
+                                           "traffic_source": p_src, "kernel": "k_cg_step1_node (FP64 p = z + beta p and SpMV from a stencil table, + p.Ap)",
                                            "bytes_per_launch": p_bytes, "avg_ms": p_spmv_ms,
                                            "cg_iteration_ms": p_iter_ms}}
         line["speedup_vs_plain_fp64"] = value / (N_STRAINS / dt_plain)

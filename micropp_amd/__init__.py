@@ -628,7 +628,7 @@ class MSolver:
         return a.value, t.value
 
     def coarse(self, inverse=True):
-        """The coarse level of the two-level inner preconditioner: (dims {nc, hx, hy, hz, mx, my, mz}, the FP32
+        """The coarsest level of the inner preconditioner: (dims {nc, hx, hy, hz, mx, my, mz}, the FP32
         inverse of the Galerkin coarse matrix, nc x nc, or None).  nc = 0 without a coarse level."""
         dims = np.zeros(7, dtype=np.int32)
         _chk(load().mppd_msolver_coarse(self.h, _ip(dims), None), "mppd_msolver_coarse")

@@ -6,15 +6,18 @@
 // FP64 defect correction (a Newton iteration of the linear problem): the
 // residual b - A u is computed matrix-free in FP64 from the element
 // stiffness of each phase, and u += d is applied in FP64.  The correction d
-// comes from an FP32 Jacobi-preconditioned CG on all K systems at once: one
-// pass over the FP32 matrix serves K vectors.  The volume averages are FP64.
+// comes from an FP32 preconditioned CG on all K systems at once, on the
+// operator and with the multilevel preconditioner of vcycle.hip.  The volume
+// averages are FP64.  With K = 4 the same kernels serve the mixed-precision
+// Newton of any law: an FP32 copy of its tangent as a stored matrix (below)
+// and an additive coarse level (coarse.hip).
 //
 // The inner CG keeps the reference's recurrence (alpha from (p, Ap) computed
 // directly: the single-reduction Chronopoulos-Gear form, tried here, loses
 // that denominator to cancellation in FP32 after ~150 iterations and
 // diverges), with the stopping test on ||z||, the reference CG's metric.
 //
-// FP32 matrix layout (node-blocked SELL-64): the 27 neighbour blocks of 3x3
+// Layout of the stored FP32 matrix (node-blocked SELL-64): the 27 neighbour blocks of 3x3
 // coefficients of a node (nb as in the reference ELL) in 9 stencil rows
 // (dz, dy) of 3 neighbours (dx = -1, 0, 1); a row's 27 floats plus 1 pad are 7
 // float4, so slot (nb, fi, fj) is float (nb / 3) * 28 + (nb % 3) * 9 + fi * 3
@@ -26,7 +29,7 @@
 //
 // FP32 vectors group 4 fields: float4 (d * K/4 + g) * NP + n holds fields
 // 4g .. 4g+3 of DOF direction d at node n (NP = nodes rounded up to 256).  A
-// wave of the SpMV owns 64 consecutive nodes and one field group, so every
+// wave of k_m_spmv owns 64 consecutive nodes and one field group, so every
 // matrix load and every neighbour gather is one contiguous 1 KB line.  The
 // FP64 displacements U are per field: component c = d * K + k of node n at
 // c * NP + n.
