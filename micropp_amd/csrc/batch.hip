@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(256) kb_cg_init_state(const BRve *rv, const in
 // the same in every shape.
 // DICT: some RVE's matrix is a stencil table (its branch costs the others 40
 // registers, hence kernels of their own).  SRC: the stored ones (mat_source).
-template <int CH, bool XCD, bool DICT, int SRC>
+template <int CH, bool XCD, bool DICT, int SRC, bool AHEAD>
 __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *at, CgState *cg, const int *a0on,
                                                    int nb, int per, int parity) {
   const int b = XCD ? (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3)) : (int)blockIdx.x;
@@ -177,10 +177,10 @@ __global__ void __launch_bounds__(256) kb_cg_step1(const BRve *rv, const int2 *a
   __shared__ double seg[kSegDoubles];
   CgState *cur = cg + 2 * rid + k, *nxt = cg + 2 * rid + (k ^ 1);
   if (DICT && R.dict.tab)
-    cg_step1_body64<CH, kMatTable>(R.g, at[b].y, R.nb_row, R.dict.tab, R.dict.code, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap,
+    cg_step1_body64<CH, kMatTable, AHEAD>(R.g, at[b].y, R.nb_row, R.dict.tab, R.dict.code, R.kinv, R.r, R.p[k], R.p[k ^ 1], R.Ap,
                            R.part, cur, nxt, seg);
   else  // vals and a0 are assembled here: the stencil columns follow from the grid
-    cg_step1_body64<CH, SRC>(R.g, at[b].y, R.nb_row, cg_matrix(R, a0on, rid), nullptr, R.kinv, R.r, R.p[k], R.p[k ^ 1],
+    cg_step1_body64<CH, SRC, AHEAD>(R.g, at[b].y, R.nb_row, cg_matrix(R, a0on, rid), nullptr, R.kinv, R.r, R.p[k], R.p[k ^ 1],
                         R.Ap, R.part, cur, nxt, seg);
 }
 
@@ -607,8 +607,13 @@ template <int CH, bool XCD>
 static void launch_step1(const BLaunch &L, int parity, hipStream_t st) {
   const int nb = L.row.nb, per = (nb + 7) / 8;
   const bool stream = mat_source((double)nb * 256 * kSlots * sizeof(double)) == kMatStream;
-  const auto k = L.dict ? (stream ? kb_cg_step1<CH, XCD, true, kMatStream> : kb_cg_step1<CH, XCD, true, kMatCached>)
-                        : (stream ? kb_cg_step1<CH, XCD, false, kMatStream> : kb_cg_step1<CH, XCD, false, kMatCached>);
+  const bool ahead = cg_ahead(nb, L.nx_max);
+  const auto k = stream ? (L.dict ? kb_cg_step1<CH, XCD, true, kMatStream, false>
+                                  : kb_cg_step1<CH, XCD, false, kMatStream, false>)
+                 : L.dict ? (ahead ? kb_cg_step1<CH, XCD, true, kMatCached, true>
+                                   : kb_cg_step1<CH, XCD, true, kMatCached, false>)
+                          : (ahead ? kb_cg_step1<CH, XCD, false, kMatCached, true>
+                                   : kb_cg_step1<CH, XCD, false, kMatCached, false>);
   hipLaunchKernelGGL(k, dim3(XCD ? 8 * per : nb), dim3(256), 0, st, L.rv, L.row.at, L.cg, L.a0on, nb, per, parity);
 }
 

@@ -92,6 +92,7 @@ struct BLaunch {
   BShape node, upd, gemv;
   int coarse = 0;
   int dict = 0;  // some RVE's matrix is a stencil table
+  int nx_max = 0;
   int spmv_shape = kSpmvDefault;    // see launch_b_spmv
   int spmv_shape32 = kSpmvDefault;  // the same choice for the inner FP32 SpMV (launch_bm_spmv)
 };

@@ -118,6 +118,7 @@ struct mppd_batch {
     for (int k = 0; k < kShapes; ++k) *shapes[k] = {nb[k], map_d[k], blk0_d[k], at_d[k]};
     L.coarse = coarse_any;
     L.dict = !dicts.empty();
+    for (const BRve &R : h) L.nx_max = std::max(L.nx_max, R.g.nx);
     L.spmv_shape = spmv_shape;
     L.spmv_shape32 = spmv_shape32;
     return L;

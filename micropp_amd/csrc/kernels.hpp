@@ -787,6 +787,13 @@ __device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, do
   return c.its == 0 ? z : z + c.beta * p;
 }
 
+// AHEAD of cg_step1_body64: lines of at most 41 nodes (two entries of a run per
+// thread, and one run per plane), and so few row blocks that the 36 registers
+// more do not keep any of them waiting.  Iteration, us, ahead / not: 6^3 nodes
+// 8.7 / 9.5, 11^3 9.0 / 10.4, 21^3 9.5 / 10.4, 31^3 12.7 / 13.2, eight J2 RVEs of
+// 11^3 9.3 / 10.1.
+inline bool cg_ahead(int row_blocks, int nx) { return row_blocks <= 768 && 3 * (kSegNodes + 2 * nx) <= 512; }
+
 // step1 of a matrix assembled here (computed stencil columns).  What bounds
 // it: at 50^3 nodes the 648 bytes of values per row; on RVEs of a few
 // thousand rows the chain of waits (state, sums, stage, values).  The first
@@ -797,7 +804,7 @@ __device__ __forceinline__ double cg_dir(const CgRegs &c, double k, double r, do
 // place of vals: 81 values of each of the three rows per code, k_s_table), the
 // same values in the same order (kDictNodes).  51^3 nodes: 22.6 us against 47.2
 // with the stored matrix, what is left being LDS and L1 reads; 31^3 8.6 / 12.5.
-template <int CH, int SRC>
+template <int CH, int SRC, bool AHEAD>
 __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, const double *vals,
                                                 const uint16_t *code, const double *kinv, const double *r,
                                                 const double *p, double *pn, double *Ap, double *part1,
@@ -812,8 +819,33 @@ __device__ __forceinline__ void cg_step1_body64(const Grid &g, int lb, int nb, c
   if (!c.done)
 #pragma unroll
     for (int k = 0; k < CH; ++k) vi[0][k] = load_value<SRC>(v, k);
+  // AHEAD: the (at most two) entries of each plane's run that the thread
+  // stages, loaded before the sums that beta waits for
+  const int len = kSegNodes + 2 * g.nx, n_lo = row0 / 3, hi = g.nn - 1;
+  double pre[AHEAD ? 18 : 1];
+  if constexpr (AHEAD) {
+    if (!c.done)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const int e3 = min((int)threadIdx.x + (k & 1) * 256, 3 * len - 1);
+        const int q = 3 * min(max(n_lo - 1 - g.nx + (k / 2 - 1) * g.nx * g.ny + e3 / 3, 0), hi) + e3 % 3;
+        pre[k * 3] = kinv[q];
+        pre[k * 3 + 1] = r[q];
+        pre[k * 3 + 2] = p[q];
+      }
+  }
   if (!cg_enter(c, lb, nb, part1 + nb, nxt)) return;
-  const SegPitch pt = stage_runs(g, row0, seg, [&](int q) { return cg_dir(c, kinv[q], r[q], p[q]); });
+  SegPitch pt{g.nx, len};
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const int e3 = threadIdx.x + (k & 1) * 256;
+      if (e3 < 3 * len) seg[(k / 2) * 3 * len + e3] = cg_dir(c, pre[k * 3], pre[k * 3 + 1], pre[k * 3 + 2]);
+    }
+    lds_barrier();
+  } else {
+    pt = stage_runs(g, row0, seg, [&](int q) { return cg_dir(c, kinv[q], r[q], p[q]); });
+  }
   const double *own = seg + (row / 3 - row0 / 3 + 1 + pt.ly + pt.lz) * 3;
   // rows past the last node lie on its run's clamped end; p is zero there
   const double pv = row < g.nrow ? own[row % 3] : 0.0;

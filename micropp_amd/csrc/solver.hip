@@ -16,11 +16,11 @@
 // holds identical scalars.  The parity is a kernel argument, so a run of
 // iterations can be queued or captured in a graph ahead of time.
 // Time per iteration (us) in two kernels, and as three (SpMV, x and r, p) with
-// shuffled block sums: 6^3 nodes 9.3 / 14.1, 11^3 10.0 / 15.6, 21^3 10.7 /
-// 16.2, 31^3 17.7 / 23.0, 41^3 33.0 / 37.8, 51^3 58.0 / 60.4.  Small RVEs wait
-// for launches and block sums (kernels of about 6 and 3 us), 51^3 for 259 MB of
+// shuffled block sums: 6^3 nodes 8.7 / 14.1, 11^3 9.0 / 15.6, 21^3 9.9 /
+// 16.2, 31^3 17.2 / 23.0, 41^3 33.0 / 37.8, 51^3 58.0 / 60.4.  Small RVEs wait
+// for launches and block sums (kernels of about 5 and 3 us), 51^3 for 259 MB of
 // values a pass (5.5 TB/s); with the stencil table of an all-elastic RVE 51^3
-// takes 28.3, 31^3 13.2.
+// takes 28.3, 31^3 12.7.
 #include "kernels.hpp"
 
 namespace mpp {
@@ -45,14 +45,14 @@ __global__ void __launch_bounds__(256) k_cg_init_state(const double *part, int n
 // Blocks are dispatched round-robin over the 8 XCDs: the 8 * per launched
 // blocks give XCD x the row blocks [x * per, (x + 1) * per), so each XCD's
 // L2 holds a contiguous slab of the gathered vector (2-5% faster SpMV).
-template <int SRC>
+template <int SRC, bool AHEAD>
 __global__ void __launch_bounds__(256) k_cg_step1(Grid g, int nb, int per, const double *vals, const uint16_t *code,
                                                   const double *kinv, const double *r, const double *p, double *pn,
                                                   double *Ap, double *part, const CgState *cur, CgState *nxt) {
   const int lb = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (lb >= nb) return;
   __shared__ double seg[kSegDoubles];
-  cg_step1_body64<kChunk, SRC>(g, lb, nb, vals, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
+  cg_step1_body64<kChunk, SRC, AHEAD>(g, lb, nb, vals, code, kinv, r, p, pn, Ap, part, cur, nxt, seg);
 }
 
 // step1 on the stencil table with a thread per node: the three rows share the
@@ -249,8 +249,10 @@ hipError_t launch_cg_step1(const Grid &g, const int *cols, const double *vals, c
                        dict->code, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   } else {
     const int src = dict ? kMatTable : mat_source((double)g.nrow_pad * kSlots * sizeof(double));
-    const auto step1 = src == kMatTable ? k_cg_step1<kMatTable> : src == kMatStream ? k_cg_step1<kMatStream>
-                                                                                  : k_cg_step1<kMatCached>;
+    const bool ahead = cg_ahead(nb, g.nx);
+    const auto step1 = src == kMatTable    ? (ahead ? k_cg_step1<kMatTable, true> : k_cg_step1<kMatTable, false>)
+                       : src == kMatCached ? (ahead ? k_cg_step1<kMatCached, true> : k_cg_step1<kMatCached, false>)
+                                           : k_cg_step1<kMatStream, false>;
     hipLaunchKernelGGL(step1, dim3(8 * per), dim3(256), 0, st, g, nb, per, dict ? dict->tab : vals,
                        dict ? dict->code : nullptr, w.kinv, w.r, w.p[k], w.p[k ^ 1], w.Ap, w.part, cur, nxt);
   }

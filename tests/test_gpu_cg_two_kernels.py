@@ -20,8 +20,8 @@ def mp():
     return micropp_amd
 
 
-# lines of 87, 88 and 89 nodes, fewer rows than a block, whole blocks and a remainder
-SIZES = [(2, 2, 2), (3, 3, 2), (5, 4, 6), (87, 3, 4), (88, 4, 3), (89, 3, 4), (17, 30, 9), (32, 16, 8), (23, 31, 50)]
+# lines of 41 nodes (staged ahead) and 42, of 87, 88 and 89, fewer rows than a block, whole blocks and a remainder
+SIZES = [(2, 2, 2), (3, 3, 2), (5, 4, 6), (41, 5, 6), (42, 5, 6), (87, 3, 4), (88, 4, 3), (89, 3, 4), (17, 30, 9), (32, 16, 8), (23, 31, 50)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
