@@ -511,10 +511,17 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out) {
 
 // At h = 4 to 5 the second level's smoother covers what lies between the grids
 // (50^3, contrast 10: 21 iterations at h = 5, 26 at h = 7; 30^3: 17 at h = 3, 19
-// at h = 5), while the dense inverse stays small: 375 coarse DOFs at 30^3
-// against 2187 at h = 3, whose inverse (19 MB read an iteration) and
-// factorisation (1.2 ms) cost more than the two iterations.
-bool coarse_grid_cycle(const Grid &g, CGrid *out) { return coarse_grid_wide(g, 5, kCoarseMaxDofs, out); }
+// at h = 5), while the dense inverse stays small.  Elements at most 4 wide while
+// their inverse has at most 1100 DOFs (4.8 MB, 4 us an iteration; its set-up
+// costs 0.1 ms more): 30^3 elements 29 iterations to 1e-10 become 25, 29 x 37 x
+// 23 38 become 33, sigma and ctan 9% sooner.  2187 DOFs (30^3 at h = 3, 40^3 at h
+// = 4: 19 MB read an iteration and 0.7 ms more set-up) cost more than they save.
+bool coarse_grid_cycle(const Grid &g, CGrid *out) {
+  if (coarse_grid_wide(g, 4, 1100, out) &&
+      std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= 4)
+    return true;
+  return coarse_grid_wide(g, 5, kCoarseMaxDofs, out);
+}
 
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
   if (g.nex < 4 || g.ney < 4 || g.nez < 4) return false;

@@ -198,7 +198,7 @@ bool coarse_enabled();
 bool coarse_grid(const Grid &g, int max_dofs, CGrid *out);
 // the grid of twice the spacing (an odd side's last element 1 wide; false: a side of fewer than 4 elements)
 bool coarse_grid_by_two(const Grid &g, CGrid *out);
-// the coarse grid of the multilevel preconditioner: about 5 fine elements per coarse element and side, coarse node q
+// the coarse grid of the multilevel preconditioner: 4 or 5 fine elements per coarse element and side, coarse node q
 // of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
 // divide the side, l = h + 1); false: none
 bool coarse_grid_cycle(const Grid &g, CGrid *out);

@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 // application an iteration instead of three), 160 us an iteration against 85:
 // sigma and ctan of six strains to 1e-10 in 4.8 ms against 7.5 ms.  Sides
 // without a common divisor (29 x 37 x 23 elements) had no coarse level before:
-// 38 iterations against 250, 2.4 ms against 5.9 ms.
+// 33 iterations against 250, 2.3 ms against 5.9 ms.
 // ---------------------------------------------------------------------------
 
 // the coarse hats along a side of ne fine elements and d coarse ones, node q at
