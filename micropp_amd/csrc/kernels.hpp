@@ -288,7 +288,8 @@ __device__ __forceinline__ void gather_vals_slice(const Grid &g, int slice, cons
     for (int q = 0; q < 8; ++q) {  // reference order (a, b, c) = (x, y, z)
       const int a = q >> 2, b = (q >> 1) & 1, c = q & 1;
       const int e = ((k - 1 + c) * g.ney + j - 1 + b) * g.nex + i - 1 + a;  // interior node: always inside
-      const double *s = ke + (size_t)(phase_mode ? et[e] : e) * 576 + (local_node(1 - a, 1 - b, 1 - c) * 3 + fi) * 24 + p * 3;
+      const int la = local_node(1 - a, 1 - b, 1 - c);
+      const double *s = ke + (size_t)(phase_mode ? et[e] : e) * 576 + (la * 3 + fi) * 24 + p * 3;
 #pragma unroll
       for (int d = 0; d < 3; ++d) v[q][d] = s[d];
     }
