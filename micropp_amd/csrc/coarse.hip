@@ -46,14 +46,14 @@ __device__ __forceinline__ int hex_corner(int ox, int oy, int oz) { return oz * 
 
 // C[(pos * 3 + phase) * 576 + r * 24 + c] = (P_e^T Ke_phase P_e)[r][c] for the
 // fine element at position pos = (pz ny + py) nx + px, nx = npos(hx, lx) ...
-// (p < h: the position in an element h wide; h + p: in one l wide):
-// block (pos, phase), one thread per entry
-__global__ void __launch_bounds__(576) k_cs_table(CGrid cg, const double *ke, double *C) {
+// (p < h: the position in an element h wide; h + p: in one l wide), from
+// plane z0 of positions on: block (pos, phase), one thread per entry
+__global__ void __launch_bounds__(576) k_cs_table(CGrid cg, int z0, const double *ke, double *C) {
   __shared__ double N[8][8];  // N[a][A]: coarse corner A's hat at the fine element's node a
   __shared__ double K[576];
   const int pos = blockIdx.x, ph = blockIdx.y, t = threadIdx.x;
   const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
-  const int px = pos % nx, py = (pos / nx) % ny, pz = pos / (nx * ny);
+  const int px = pos % nx, py = (pos / nx) % ny, pz = z0 + pos / (nx * ny);
   K[t] = ke[(size_t)ph * 576 + t];
   if (t < 64) {
     const int a = t >> 3, A = t & 7;
@@ -74,9 +74,11 @@ __global__ void __launch_bounds__(576) k_cs_table(CGrid cg, const double *ke, do
 }
 
 // KE[E * 576 + t]: the stiffness of coarse element E, the sum of its fine
-// elements' C entries in position order; block E, one thread per entry
-__global__ void __launch_bounds__(576) k_cs_elem(Grid g, CGrid cg, int dx, int dy, const int *et, const double *C,
-                                                 double *KE) {
+// elements' C entries in position order; block E, one thread per entry.  C
+// holds nz planes of positions from zp on: slabs in ascending order continue
+// the sum, from zero at the first (zp = 0)
+__global__ void __launch_bounds__(576) k_cs_elem(Grid g, CGrid cg, int dx, int dy, int zp, int nz, const int *et,
+                                                 const double *C, double *KE) {
   const int E = blockIdx.x, t = threadIdx.x;
   const int Ex = E % dx, Ey = (E / dx) % dy, Ez = E / (dx * dy);
   const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
@@ -84,12 +86,12 @@ __global__ void __launch_bounds__(576) k_cs_elem(Grid g, CGrid cg, int dx, int d
   const int wx = cnode(Ex + 1, g.nex, cg.mx + 1) - x0, wy = cnode(Ey + 1, g.ney, cg.my + 1) - y0,
             wz = cnode(Ez + 1, g.nez, cg.mz + 1) - z0;
   const int ox = wx != cg.hx ? cg.hx : 0, oy = wy != cg.hy ? cg.hy : 0, oz = wz != cg.hz ? cg.hz : 0;
-  double s = 0.0;
-  for (int pz = 0; pz < wz; ++pz)
+  double s = zp ? KE[(size_t)E * 576 + t] : 0.0;
+  for (int pz = max(0, zp - oz); pz < min(wz, zp + nz - oz); ++pz)
     for (int py = 0; py < wy; ++py)
       for (int px = 0; px < wx; ++px) {
         const int e = ((z0 + pz) * g.ney + y0 + py) * g.nex + x0 + px;
-        const int pos = ((oz + pz) * ny + oy + py) * nx + ox + px;
+        const int pos = ((oz + pz - zp) * ny + oy + py) * nx + ox + px;
         s += C[((size_t)pos * 3 + et[e]) * 576 + t];
       }
   KE[(size_t)E * 576 + t] = s;
@@ -536,21 +538,21 @@ bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
       m[d] = n - 1;
     }
     if (3 * m[0] * m[1] * m[2] > max_dofs) continue;
-    const CGrid cg = make_grid(h[0], h[1], h[2], l[0], l[1], l[2], m[0], m[1], m[2]);
-    // the set-up's table holds every position along a side (h, and l of the wider elements)
-    if (coarse_table_len(cg) / (3 * 576) > (size_t)kCoarseMaxPos * 4) return false;
-    *out = cg;
+    *out = make_grid(h[0], h[1], h[2], l[0], l[1], l[2], m[0], m[1], m[2]);
     return true;
   }
   return false;
 }
 
-size_t coarse_table_len(const CGrid &cg) {
-  return (size_t)npos(cg.hx, cg.lx) * npos(cg.hy, cg.ly) * npos(cg.hz, cg.lz) * 3 * 576;
+int coarse_table_planes(const CGrid &cg) { return npos(cg.hz, cg.lz); }
+
+size_t coarse_table_len(const CGrid &cg, int nz) {
+  return (size_t)npos(cg.hx, cg.lx) * npos(cg.hy, cg.ly) * nz * 3 * 576;
 }
 
-hipError_t launch_cs_table(const CGrid &cg, const double *ke, double *C, hipStream_t st) {
-  hipLaunchKernelGGL(k_cs_table, dim3((unsigned)(coarse_table_len(cg) / (3 * 576)), 3), dim3(576), 0, st, cg, ke, C);
+hipError_t launch_cs_table(const CGrid &cg, int z0, int nz, const double *ke, double *C, hipStream_t st) {
+  hipLaunchKernelGGL(k_cs_table, dim3((unsigned)(coarse_table_len(cg, nz) / (3 * 576)), 3), dim3(576), 0, st, cg, z0,
+                     ke, C);
   return hipGetLastError();
 }
 
@@ -564,7 +566,12 @@ int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double
   b.nt = (nc + kChT - 1) / kChT;
   b.bt = (3 * (cg.mx * cg.my + cg.mx + 1) + 2 + kChT - 1) / kChT;
   const size_t nband = (size_t)b.nt * (b.bt + 1) * kChTT, nw = tri_slot(b.nt, 0) * kChTT;
-  const size_t nC = coarse_table_len(cg), nKE = (size_t)ncel * 576;
+  // the table in slabs of whole planes of positions: coarse elements of two
+  // widths h and h + 1 have (2 h + 1)^3 positions, 13.8 KB each (51^3 on the
+  // largest cube)
+  const int planes = coarse_table_planes(cg);
+  const int slab = std::clamp((int)((size_t)kCoarseMaxPos * 3 * 576 / coarse_table_len(cg, 1)), 1, planes);
+  const size_t nC = coarse_table_len(cg, slab), nKE = (size_t)ncel * 576;
   double *buf = nullptr;
   int *info_d = nullptr;
   int rc = MPPD_OK;
@@ -578,8 +585,11 @@ int coarse_inverse(const Grid &g, const CGrid &cg, const int *et_d, const double
       rc = hip_fail(e, "coarse factor status");
       break;
     }
-    (void)launch_cs_table(cg, ke_d, C, st);
-    hipLaunchKernelGGL(k_cs_elem, dim3(ncel), dim3(576), 0, st, g, cg, dx, dy, et_d, C, KE);
+    for (int z = 0; z < planes; z += slab) {
+      const int nz = std::min(slab, planes - z);
+      (void)launch_cs_table(cg, z, nz, ke_d, C, st);
+      hipLaunchKernelGGL(k_cs_elem, dim3(ncel), dim3(576), 0, st, g, cg, dx, dy, z, nz, et_d, C, KE);
+    }
     hipLaunchKernelGGL(k_cs_band, dim3((unsigned)((nband + 255) / 256)), dim3(256), 0, st, cg, dx, dy, b, KE, Ab);
     for (int k = -1; k < b.nt; ++k) {
       const int m = k < 0 ? 0 : std::min(b.bt, b.nt - 1 - k);

@@ -164,7 +164,7 @@ struct CoarseDev {
 constexpr int kCoarseSplit = 16;    // column splits of the coarse solve (one partial each)
 constexpr int kCoarseMaxLine = 256;  // nodes per side a coarse level allows
 constexpr int kCoarseMaxDofs = 2200;  // coarse DOFs of a multi-RHS solver (3 x 9^3 = 2187: 10^3 coarse elements)
-constexpr int kCoarseMaxPos = 4096;   // fine elements per coarse element (the set-up's table size)
+constexpr int kCoarseMaxPos = 4096;   // positions of a fine element that the set-up's table holds at once (57 MB)
 // Trilinear hats along one side at one fine index: the interior coarse nodes
 // below and above it, as offsets into the coarse vectors, and their weights
 // (0 for a node on the boundary, with a valid offset).
@@ -204,10 +204,12 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out);
 bool coarse_grid_cycle(const Grid &g, CGrid *out);
 // the same with the narrowest coarse elements of at least `least` fine ones a side and at most max_dofs coarse DOFs
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out);
-// C (device, coarse_table_len(cg) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position
-// (position px of a side: px < h in a regular element, h + px in a last element of another width)
-size_t coarse_table_len(const CGrid &cg);
-hipError_t launch_cs_table(const CGrid &cg, const double *ke, double *C, hipStream_t st);
+// C (device, coarse_table_len(cg, nz) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position,
+// for nz of the coarse_table_planes(cg) planes of positions from z0 on
+// (position px of a side: px < h in an element h wide, h + px in one l wide)
+int coarse_table_planes(const CGrid &cg);
+size_t coarse_table_len(const CGrid &cg, int nz);
+hipError_t launch_cs_table(const CGrid &cg, int z0, int nz, const double *ke, double *C, hipStream_t st);
 // ainv (nc x nc floats, device) = the FP32 inverse of the Galerkin coarse
 // matrix of the RVE (phase map et_d, per-phase element stiffness ke_d) on cg;
 // *ok = false when that matrix is not positive definite

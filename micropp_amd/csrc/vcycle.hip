@@ -981,8 +981,9 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     }
     hipLaunchKernelGGL(k_v_sums, dim3(1), dim3(kRedThreads), 0, st, p0, p1, nb, sums);
     if (e == hipSuccess && !two) {
-      if ((rc = dalloc(&C, coarse_table_len(mid), false))) break;
-      e = launch_cs_table(mid, ke_d, C, st);
+      const int planes = coarse_table_planes(mid);
+      if ((rc = dalloc(&C, coarse_table_len(mid, planes), false))) break;
+      e = launch_cs_table(mid, 0, planes, ke_d, C, st);
       hipLaunchKernelGGL(k_v_asm, dim3(s1.NP / 64), dim3(256), 0, st, g, g1, mid, s1.NP, et_d, C, v->A1, v->kinv1);
       float *a1 = v->E0, *b1 = v->T1;  // four fields fit: K >= 4
       double *q0 = v->prz, *q1 = v->prz + 4 * (size_t)nb1;
