@@ -234,6 +234,10 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
  * and 0 at the neighbouring coarse nodes' (h wide everywhere: max(0, 1 -
  * |i - cx hx| / hx)). */
 int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h);
+/* The damping of its Jacobi smoothers on the fine grid and on the second level
+ * (1 without one; both 0 without a preconditioner).  The preconditioner is
+ * positive definite while each is below 2 / lambda_max(D^-1 A) of its level. */
+int mppd_msolver_damping(const mppd_msolver *m, double w[2]);
 /* newton_raphson (src/solve.cpp:28-82) with mixed-precision linear solves,
  * for an RVE of any material law (a plastic or damaged RVE's Newton tangent
  * included).  The Newton control flow, the residual (assembly_rhs with the

@@ -149,6 +149,7 @@ SIGNATURES = {
     "mppd_msolver_adjoint_many": (_I, [_I, C.c_void_p, _I, _PD, C.c_void_p, _I, _PD, _PD, _PD, _PI, _PD]),
     "mppd_msolver_profile": (_I, [_VP, _I, _PD, _PD]),
     "mppd_msolver_coarse": (_I, [_VP, _PI, C.POINTER(C.c_float)]),
+    "mppd_msolver_damping": (_I, [_VP, _PD]),
     "mppd_msolver_newton": (_I, [_VP, _I, _PD, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, _PD, _PI, _PI]),
     "mppd_newton_mixed": (_I, [_VP, _VP, _PD, _VP, _VP, C.POINTER(NewtonParams), _VP, _PI, _PI]),
     "mppd_batch_params_default": (None, [_VP]),
@@ -639,6 +640,12 @@ class MSolver:
         _chk(load().mppd_msolver_coarse(self.h, _ip(dims), ainv.ctypes.data_as(C.POINTER(C.c_float))),
              "mppd_msolver_coarse")
         return dims, ainv
+
+    def damping(self):
+        """The damping of the preconditioner's Jacobi smoothers: (fine grid, second level)."""
+        w = np.zeros(2)
+        _chk(load().mppd_msolver_damping(self.h, _dp(w)), "mppd_msolver_damping")
+        return float(w[0]), float(w[1])
 
 
 def adjoint_many(msolvers, strains=None, workers=0, rel_tol=1e-8, abs_tol=1e-50, inner_tol=1e-5, max_inner_its=2000,

@@ -1409,4 +1409,11 @@ int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h) {
   return MPPD_OK;
 }
 
+int mppd_msolver_damping(const mppd_msolver *m, double w[2]) {
+  if (!m || !w) return fail(MPPD_ERR_ARG, "bad msolver_damping arguments");
+  w[0] = m->vc ? m->vc->w0 : 0.0;
+  w[1] = m->vc ? m->vc->w1 : 0.0;
+  return MPPD_OK;
+}
+
 }  // extern "C"

@@ -398,7 +398,7 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 // hats at the second level's nodes).  M is symmetric positive definite while w0 and w1 stay
 // below 2 / lambda_max(D^-1 A) of their levels (estimated at set-up by a power
 // iteration on the operators themselves, since isolated stiff elements raise
-// it: 2.7-2.9 for cubes, up to 4.5 in thin cells).
+// it: 2.7-2.9 for cubes, up to 4.5 in thin cells and beside one stiff element).
 //
 // 50^3, contrast 10, 12 fields: 22 iterations to 1e-8 against 73 with the
 // additive two-level form (Jacobi plus the same coarse inverse; one operator
@@ -721,12 +721,29 @@ __global__ void __launch_bounds__(256) k_v_rand(int NP, int stride, const float 
   P[(size_t)d * stride + n] = make_float4(s(3), s(9), s(17), s(25));
 }
 
-// out[q] = the sums of rows q < 4 of two partial tables: out[q], out[4 + q]
-__global__ void __launch_bounds__(kRedThreads) k_v_sums(const double *p0, const double *p1, int n, double *out) {
-  const double a = rows_sum<4>(p0, n, n), b = rows_sum<4>(p1, n, n);
-  if (threadIdx.x < 4) {
-    out[threadIdx.x] = a;
-    out[4 + threadIdx.x] = b;
+// *out = the largest growth of (v, D v) between two iterates of the power
+// iteration, over four fields and the blocks of the kernel that formed it
+// (partials p0, then p1, n a field).  A mode on a few nodes, of one stiff element
+// say, has outgrown what else its block holds after a dozen steps, while the sum
+// over a large grid does not show it yet.  Blocks below kGrowthShare of the mean
+// are left out: a node or two whose value passes through zero grow by anything.
+constexpr double kGrowthShare = 0.1;
+__global__ void __launch_bounds__(kRedThreads) k_v_growth(const double *p0, const double *p1, int n, double *out) {
+  __shared__ double least[4], most[kRedThreads];
+  const double sum = rows_sum<4>(p0, n, n);
+  if (threadIdx.x < 4) least[threadIdx.x] = kGrowthShare * sum / n;
+  __syncthreads();
+  double m = 0.0;
+  for (int f = 0; f < 4; ++f)
+    for (int i = threadIdx.x; i < n; i += kRedThreads) {
+      const double a = p0[(size_t)f * n + i], g = p1[(size_t)f * n + i] / a;
+      if (a > least[f]) m = g < 1e6 ? fmax(m, g) : 1e6;  // (1e6, as for NaN: not usable)
+    }
+  most[threadIdx.x] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kRedThreads; ++i) m = fmax(m, most[i]);
+    *out = m;
   }
 }
 
@@ -868,10 +885,16 @@ void vcycle_free(VCycleDev *v) {
 
 namespace {
 // Smoother damping: kDamp / lambda with lambda the power iteration's estimate
-// after kPowerIts steps, a few percent below lambda_max; the smoothers need
-// damping * lambda_max < 2
+// after kPowerIts steps (k_v_growth); the smoothers need damping * lambda_max <
+// 2.  The estimate is 0.94 to 1.05 lambda_max (damping * lambda_max 1.57 to 1.75)
+// in homogeneous, spherical and random media of contrasts to 1000, with one
+// stiff element on 24^3 to 160^3, in thin cells, with Poisson's ratios to 0.49,
+// and on the second level.  The ratio of the sums over the whole grid instead
+// reads 2.71 where one stiff element makes it 3.52 (80^3, contrast 15), and has
+// to be met with a smaller kDamp: 45 RVEs of 11 to 80 elements a side take 1501
+// iterations against 1511 with 1.55 over that ratio (1531 at kDamp = 1.6).
 constexpr int kPowerIts = 12;
-constexpr float kDamp = 1.55f;
+constexpr float kDamp = 1.65f;
 // The two-level form: coarse elements of at most 2 fine ones a side while their
 // inverse has at most kCoarseMaxDofs DOFs (20 elements a side), of at most 3
 // while it has at most 1536 (26).  The second level's five kernels fall away:
@@ -916,7 +939,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
   g1.nelem = g1.nex * g1.ney * g1.nez;
   const MLaunch s1 = mshape(g1);
   const int nc = cg.nc, nb = stencil_blocks(g, op), nb1 = (int)nblk(s1.NP, kApNodes);
-  double *C = nullptr, sums_h[16] = {};
+  double *C = nullptr, growth_h[2] = {};
   int rc = MPPD_OK;
   bool ok = false;
   do {
@@ -935,7 +958,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     for (int a = 0; a < 3; ++a) o_hat[a] = carve(line[a] * sizeof(HatEntry));
     const size_t o_z = carve(mixed_vector_len(g, K) * sizeof(float));
     const size_t o_prz = carve(std::max((size_t)K * nb, 2 * 4 * (size_t)std::max(nb, nb1)) * sizeof(double));
-    const size_t o_sum = carve(16 * sizeof(double));
+    const size_t o_grow = carve(2 * sizeof(double));
     const size_t o_R1 = carve(n1), o_E0 = carve(n1), o_T1 = carve(n1), o_E = carve(n1);
     const size_t o_k1 = carve(two ? 0 : (size_t)s1.NP * 3 * sizeof(float));
     const size_t zeroed = off, o_ainv = carve(((size_t)nc * nc + 16) * sizeof(float));  // (k_v_gemv reads 15 past it)
@@ -965,10 +988,10 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     v->kinv1 = at(o_k1);
     v->A1 = at(o_A1);
     v->prz = reinterpret_cast<double *>(base + o_prz);
-    double *sums = reinterpret_cast<double *>(base + o_sum);
+    double *growth = reinterpret_cast<double *>(base + o_grow);
     float *ainv = at(o_ainv);
     v->ainv = ainv;
-    // lambda_max(D^-1 A) of the fine operator, on four fields: sums of
+    // lambda_max(D^-1 A) of the fine operator, on four fields: the growth of
     // (v, D v) over the last two iterates
     const int NP = mshape(g).NP;
     double *p0 = v->prz, *p1 = v->prz + 4 * (size_t)nb;
@@ -979,7 +1002,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
       e = launch_d_apply<kApplyPow>(g, K, op, a, nullptr, kinv, 0.0f, b, i & 1 ? p1 : p0, nullptr, st);
       std::swap(a, b);
     }
-    hipLaunchKernelGGL(k_v_sums, dim3(1), dim3(kRedThreads), 0, st, p0, p1, nb, sums);
+    hipLaunchKernelGGL(k_v_growth, dim3(1), dim3(kRedThreads), 0, st, p0, p1, nb, growth);
     if (e == hipSuccess && !two) {
       const int planes = coarse_table_planes(mid);
       if ((rc = dalloc(&C, coarse_table_len(mid, planes), false))) break;
@@ -993,22 +1016,21 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
         e = launch_mid<kApplyPow>(g1, 4, *v, a1, nullptr, b1, i & 1 ? q1 : q0, nullptr, st);
         std::swap(a1, b1);
       }
-      hipLaunchKernelGGL(k_v_sums, dim3(1), dim3(kRedThreads), 0, st, q0, q1, nb1, sums + 8);
+      hipLaunchKernelGGL(k_v_growth, dim3(1), dim3(kRedThreads), 0, st, q0, q1, nb1, growth + 1);
     }
     if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(sums_h, sums, sizeof(sums_h), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(growth_h, growth, sizeof(growth_h), hipMemcpyDeviceToHost, st);
     if (e != hipSuccess) {
       rc = hip_fail(e, "preconditioner set-up");
       break;
     }
     if ((rc = coarse_inverse(g, cg, et_d, ke_d, ainv, st, &ok))) break;  // synchronizes st
-    auto damping = [&](const double *s) {  // NaN or no growth: not usable
-      double lam = 0.0;
-      for (int f = 0; f < 4; ++f) lam = std::max(lam, std::sqrt(s[4 + f] / s[f]));
+    auto damping = [](double growth) {  // NaN or no growth: not usable
+      const double lam = std::sqrt(growth);
       return lam > 0.1 && lam < 1e3 ? kDamp / (float)lam : 0.0f;
     };
-    v->w0 = damping(sums_h);
-    v->w1 = two ? 1.0f : damping(sums_h + 8);
+    v->w0 = damping(growth_h[0]);
+    v->w1 = two ? 1.0f : damping(growth_h[1]);
     ok = ok && v->w0 > 0.0f && v->w1 > 0.0f;
   } while (0);
   (void)hipStreamSynchronize(st);  // C may still be in use after a failed step

@@ -1,0 +1,80 @@
+"""GPU: the multilevel preconditioner stays positive definite: damping * lambda_max(D^-1 A) < 2 on both levels.
+
+lambda_max is the largest eigenvalue of the level's own operator, by Lanczos on the FP64 matrix of the same RVE; a mode
+bound to a few stiff elements does not feel the size of the grid around them, so that of a large RVE is taken from a
+smaller one.  The damping is 1.65 over an estimate of lambda_max, so the product must not pass 1.85 (the estimate 11%
+short)."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+from scipy.sparse.linalg import eigsh
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mp():
+    import micropp_amd
+
+    micropp_amd.load()
+    if not micropp_amd.gpu_available():
+        pytest.skip("no HIP device")
+    return micropp_amd
+
+
+def hats2(ne):
+    """Interior fine nodes x interior nodes of every second one."""
+    i, q = np.arange(1, ne)[:, None], np.arange(1, (ne - 1) // 2 + 1)[None]
+    return sp.csr_matrix(np.maximum(0.0, 1.0 - np.abs(i - 2 * q) / 2))
+
+
+def lambda_max(mp, r, second=False):
+    s = mp.Solver(r)
+    s.assembly_mat(None)
+    cols, vals = s.ell()
+    a = sp.csr_matrix((vals.ravel(), (np.repeat(np.arange(r.nrow), cols.shape[1]), cols.ravel())), shape=(r.nrow,) * 2)
+    nx, ny, nz = r.size
+    inner = np.zeros((nz, ny, nx, 3), dtype=bool)
+    inner[1:-1, 1:-1, 1:-1] = True
+    a = a[inner.ravel()][:, inner.ravel()]
+    if second:
+        p = sp.kron(sp.kron(sp.kron(hats2(nz - 1), hats2(ny - 1)), hats2(nx - 1)), sp.identity(3)).tocsr()
+        a = (p.T @ a @ p).tocsr()
+    d = sp.diags(1.0 / np.sqrt(a.diagonal()))
+    return float(eigsh(d @ a @ d, k=1, which="LA", tol=1e-3, return_eigenvectors=False)[0])
+
+
+def sphere_rve(mp, ne, contrast, elems, nu=0.25):
+    """`elems` stiff elements (1: ne odd, 8: ne even) in the middle of ne^3."""
+    mats = [mp.material(0, 1e6, 0.3), mp.material(0, 1e6 * contrast, nu), mp.material(0, 1e6, 0.3)]
+    return mp.Rve((ne + 1,) * 3, mp.MIC_SPHERE, ((0.1 if elems == 1 else 0.9) / ne, 0.0, 0.0, 0.0), mats)
+
+
+@pytest.mark.parametrize("ne, contrast, nu", [(49, 10.0, 0.25), (81, 15.0, 0.25), (81, 20.0, 0.25), (161, 15.0, 0.25),
+                                              (101, 2.0, 0.45)])
+def test_one_stiff_element(mp, ne, contrast, nu):
+    lam = lambda_max(mp, sphere_rve(mp, 13, contrast, 1, nu))
+    w = mp.MSolver(sphere_rve(mp, ne, contrast, 1, nu), 4).damping()
+    print(f"{ne}: damping {w}, times lambda {w[0] * lam:.3f}", flush=True)
+    assert 1.4 < w[0] * lam < 1.85
+
+
+@pytest.mark.parametrize("ne, contrast", [(42, 15.0), (122, 15.0), (202, 15.0), (202, 1000.0)])
+def test_one_stiff_element_of_the_second_level(mp, ne, contrast):
+    lam = lambda_max(mp, sphere_rve(mp, 22, contrast, 8), second=True)
+    w = mp.MSolver(sphere_rve(mp, ne, contrast, 8), 4).damping()
+    print(f"{ne}: damping {w}, times lambda {w[1] * lam:.3f}", flush=True)
+    assert 1.4 < w[1] * lam < 1.85
+
+
+# two levels (the first), three, thin cells; even sides
+@pytest.mark.parametrize("size, geo, contrast", [
+    ((5, 7, 5), (7.0, 4.0, 0.1, 0.2), 10.0), ((31, 29, 33), (10.0, 8.0, 0.05, 0.15), 10.0),
+    ((31, 31, 31), (12.0, 60.0, 0.01, 0.04), 300.0), ((61, 63, 9), (13.0, 8.0, 0.05, 0.2), 100.0)])
+def test_spheres(mp, size, geo, contrast):
+    mats = [mp.material(0, 1e6, 0.3), mp.material(0, 1e6 * contrast, 0.25), mp.material(0, 1e6, 0.3)]
+    r = mp.Rve(size, mp.MIC3D_RANDOM_SPHERES, geo, mats)
+    w = mp.MSolver(r, 4).damping()
+    product = [w[k] * lambda_max(mp, r, second=k == 1) for k in range(1 if size[0] < 30 else 2)]
+    print(f"{size}: damping {w}, times lambda {product}", flush=True)
+    assert all(1.4 < q < 1.85 for q in product)
