@@ -394,8 +394,8 @@ hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float 
 hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                          float *AP, double *part, void *state, int parity, hipStream_t st,
                          const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr);
-// s0's (r, z) from partials prz[field * row + i]
-hipError_t launch_c_rzfix(int K, int row, const double *prz, void *state, hipStream_t st);
+// s0's (r, z) from partials prz[field * row + i]; guard: with the test of a positive definite preconditioner
+hipError_t launch_c_rzfix(int K, int row, const double *prz, bool guard, void *state, hipStream_t st);
 // blocks per component of the vector kernels (the partial tables' stride)
 size_t coarse_vec_blocks(const Grid &g);
 hipError_t launch_m_accum(const Grid &g, int K, const float *X, double *U, hipStream_t st);
@@ -432,6 +432,7 @@ struct mppd_rve {
 namespace mpp {
 
 void mixed_state_view(const void *state_h, int parity, int *its, int *all_done);
+bool mixed_state_broken(const void *state_h, int parity);
 // field k of the inner state: returns its done flag; *pn its preconditioned
 // residual norm, *target the norm at which it stops
 int mixed_state_field(const void *state_h, int parity, int k, double *pn, double *target);

@@ -348,6 +348,7 @@ __global__ void __launch_bounds__(kRedThreads) k_m_outer(int nparts, const doubl
     s0->its = 0;
     s0->max_its = max_inner;
     s0->all_done = all;
+    s0->broken = 0;
   }
 }
 
@@ -972,11 +973,15 @@ __global__ void __launch_bounds__(kZdotThreads) k_c_zdot(Grid g, CGrid cg, int N
 }
 
 // start: the state's (r, z) of every field from the partials (row per field)
-// of the kernel that formed z
+// of the kernel that formed z.  guard: a preconditioner that is not positive
+// definite stops the CG before its first iteration
 template <int K>
-__global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int row, const double *prz, MState *s0) {
+__global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int row, const double *prz, int guard, MState *s0) {
   const double rz = rows_sum<K>(prz, row, row);
-  if (threadIdx.x < K) s0->rz[threadIdx.x] = rz;
+  const int r = threadIdx.x;
+  if (r >= K) return;
+  s0->rz[r] = rz;
+  if (guard && !s0->done[r] && spd_broken(rz, s0->pn[r], s0->pn0[r], s0->tau[r])) s0->broken = s0->all_done = 1;
 }
 
 // k_m_pupd: X += alpha P; P = kinv R + beta P for the fields still running;
@@ -986,14 +991,15 @@ __global__ void __launch_bounds__(kRedThreads) k_c_rzfix(int row, const double *
 // (beta, ||z||, stop flags, iteration count).  Grid as k_m_upd.
 // COARSE (two-level and multilevel preconditioners): z is read from Z instead
 // of being formed from kinv and R.  rowz, row: partials per field of pz, pr.
+// guard: the CG stops where the preconditioner is not positive definite.
 template <int K, bool COARSE, int J = kVecNodes / 256>
 __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kinv, const float4 *R, const float4 *Z,
                                                         float4 *P, float4 *X, const double *pz, int rowz,
-                                                        const double *pr, int row, const MState *cur,
+                                                        const double *pr, int row, int guard, const MState *cur,
                                                         MState *nxt) {
   constexpr int KG = K / 4;
   __shared__ double beta_s[kMaxRhs];
-  __shared__ int live_s[kMaxRhs], dn_s[kMaxRhs];
+  __shared__ int live_s[kMaxRhs], dn_s[kMaxRhs], bad_s[kMaxRhs];
   const int c = blockIdx.y, grp = c % KG, d = c / KG, r0 = grp * 4;
   const bool head = blockIdx.x == 0 && blockIdx.y == 0;
   if (cur->all_done) {
@@ -1046,6 +1052,7 @@ __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kin
       nxt->tau[r] = cur->tau[r];
       nxt->done[r] = o.done;
       dn_s[r] = o.done;
+      bad_s[r] = guard && !cur->done[r] && spd_broken(rz, o.pn, cur->pn0[r], cur->tau[r]);
       if (r >= r0 && r < r0 + 4) {
         beta_s[r - r0] = o.beta;
         live_s[r - r0] = !o.done && its < cur->max_its;
@@ -1053,11 +1060,12 @@ __global__ void __launch_bounds__(kRedThreads) k_m_pupd(int NP, const float *kin
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      int all = 1;
-      for (int q = 0; q < K; ++q) all &= dn_s[q];
+      int all = 1, bad = 0;
+      for (int q = 0; q < K; ++q) all &= dn_s[q], bad |= bad_s[q];
       nxt->its = its;
       nxt->max_its = cur->max_its;
-      nxt->all_done = all || its >= cur->max_its;
+      nxt->all_done = all || bad || its >= cur->max_its;
+      nxt->broken = bad;
     }
   } else {
     const double zz = rows_finish<4>(szz);
@@ -1654,7 +1662,8 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &
     hipLaunchKernelGGL((k_c_zdot<4, false>), vgrid, dim3(kZdotThreads), 0, st, g, cg, s.NP, kinv, r4,
                        reinterpret_cast<const float4 *>(coarse->ec), reinterpret_cast<float4 *>(coarse->z), pr, cur);
     hipLaunchKernelGGL((k_m_pupd<4, true>), vgrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4,
-                       reinterpret_cast<const float4 *>(coarse->z), p4, x4, pz, 3 * nbu, pr, 3 * nbx, cur, nxt);
+                       reinterpret_cast<const float4 *>(coarse->z), p4, x4, pz, 3 * nbu, pr, 3 * nbx, 0,
+                       cur, nxt);
     return hipGetLastError();
   }
   // two nodes a thread while eight leave the grid short of blocks
@@ -1671,15 +1680,15 @@ hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &
       hipLaunchKernelGGL(upd, ngrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
                          reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, reinterpret_cast<float4 *>(vc->z));
       if ((e = launch_vcycle(g, K, *vc, op, kinv, R, vc->z, AP, AP, pr, cur, st)) != hipSuccess) return e;
-      hipLaunchKernelGGL(pupd, ngrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, ap4, p4, x4, pz, 3 * nbn, pr, np1, cur,
-                         nxt);
+      hipLaunchKernelGGL(pupd, ngrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, ap4, p4, x4, pz, 3 * nbn, pr, np1, 1,
+                         cur, nxt);
     } else {
       const auto upd = narrow ? (k_m_upd<KK, kPcJacobi, 2>) : (k_m_upd<KK, kPcJacobi>);
       const auto pupd = narrow ? (k_m_pupd<KK, false, 2>) : (k_m_pupd<KK, false>);
       hipLaunchKernelGGL(upd, ngrid, dim3(kRedThreads), 0, st, s.NP, np1, part1, kinv, ap4,
                          reinterpret_cast<float4 *>(R), pz, pr, cur, g, CGrid{}, 0, nullptr);
       hipLaunchKernelGGL(pupd, ngrid, dim3(kRedThreads), 0, st, s.NP, kinv, r4, nullptr, p4, x4, pz, 3 * nbn, pr,
-                         3 * nbn, cur, nxt);
+                         3 * nbn, 0, cur, nxt);
     }
   });
   return hipGetLastError();
@@ -1695,11 +1704,11 @@ hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float 
   hipLaunchKernelGGL((k_c_zdot<4, true>), dim3(nbx, 3), dim3(kZdotThreads), 0, st, g, c.cg, s.NP, kinv,
                      reinterpret_cast<const float4 *>(R), reinterpret_cast<const float4 *>(c.ec),
                      reinterpret_cast<float4 *>(P), c.prz, s0);
-  return launch_c_rzfix(K, 3 * nbx, c.prz, state, st);
+  return launch_c_rzfix(K, 3 * nbx, c.prz, false, state, st);
 }
 
-hipError_t launch_c_rzfix(int K, int row, const double *prz, void *state, hipStream_t st) {
-  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_c_rzfix<KK>, dim3(1), dim3(kRedThreads), 0, st, row, prz,
+hipError_t launch_c_rzfix(int K, int row, const double *prz, bool guard, void *state, hipStream_t st) {
+  MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_c_rzfix<KK>, dim3(1), dim3(kRedThreads), 0, st, row, prz, guard ? 1 : 0,
                                        static_cast<MState *>(state)));
   return hipGetLastError();
 }
@@ -1788,6 +1797,9 @@ void mixed_state_view(const void *state_h, int parity, int *its, int *all_done) 
   const MState *ms = static_cast<const MState *>(state_h) + (parity & 1);
   *its = ms->its;
   *all_done = ms->all_done;
+}
+bool mixed_state_broken(const void *state_h, int parity) {
+  return (static_cast<const MState *>(state_h) + (parity & 1))->broken != 0;
 }
 int mixed_state_field(const void *state_h, int parity, int k, double *pn, double *target) {
   const MState *ms = static_cast<const MState *>(state_h) + (parity & 1);

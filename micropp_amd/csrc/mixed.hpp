@@ -25,12 +25,20 @@ constexpr int kVecNodes = 2048;   // nodes per block of the vector kernels
 constexpr size_t kVecWide = 200;
 
 // inner CG scalars per field: rz = (r, z), alpha / beta of the iteration, pn
-// the current ||z||, pn0 the start value, tau the relative stop
+// the current ||z||, pn0 the start value, tau the relative stop; broken: the
+// preconditioner has shown itself not positive definite (spd_broken)
 struct MState {
   double rz[kMaxRhs], alpha[kMaxRhs], beta[kMaxRhs], pn[kMaxRhs], pn0[kMaxRhs], tau[kMaxRhs];
   int done[kMaxRhs];
-  int its, max_its, all_done, pad;
+  int its, max_its, all_done, broken;
 };
+
+// (r, z) not positive on a field that has not reached its stop: z = M r with a
+// preconditioner that is not positive definite (a start value that is not a
+// number is not its doing)
+__device__ __forceinline__ bool spd_broken(double rz, double pn, double pn0, double tau) {
+  return !(rz > 0.0) && !(pn < tau * pn0) && pn0 - pn0 == 0.0;
+}
 
 // all fields, or the four fields r0 .. r0 + 3 of a group, have stopped (one
 // round of loads: no test waits for another's)

@@ -850,21 +850,20 @@ int mppd_msolver_destroy(mppd_msolver *m) {
   return MPPD_OK;
 }
 
-// The K fields: 0 .. nadj-1 adjoint fields (zero boundary values, source
-// a_v / V of field v), then n forward fields with the macro strains eps_h,
-// then idle fields.  FP64 defect correction with FP32 inner CG until every
-// field converges; the solution is left in m->U.
 // Inner FP32 CG of a K-field system, from the start state the outer test has
 // written (state_h holds it), queued in chunks; after q iterations the state
 // is state[q & 1].  The next chunk is sized from each live field's observed
 // convergence rate (iterations still needed, + 2), so few iterations are
 // queued past the end.  *its = iterations run; *finite (may be NULL) = every
-// field's ||z|| is finite at the end (no breakdown).
+// field's ||z|| is finite at the end (no breakdown).  *broken: the multilevel
+// preconditioner vc has shown itself not positive definite ((r, z) <= 0); the
+// CG has stopped there and X is of no use.
 static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                        float *AP, double *part, void *state, void *state_h, int max_inner, hipStream_t st,
                        int *its_out, bool *finite = nullptr, bool stop_on_stall = false,
-                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr) {
+                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr, bool *broken = nullptr) {
   int queued = 0, its = 0, done = 0, its_prev = 0;
+  if (vc) mixed_state_view(state_h, 0, &its, &done);  // (it may be broken at the start)
   // (with the multilevel preconditioner a solve takes about 10 iterations of
   // up to 13 launches each, so few are queued past the end)
   int chunk = vc ? 8 : 32;
@@ -908,6 +907,7 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
     if (stalled && stop_on_stall) break;
   }
   *its_out = its;
+  if (broken) *broken = mixed_state_broken(state_h, queued);
   if (finite) {
     *finite = true;
     for (int k = 0; k < K; ++k) {
@@ -919,6 +919,12 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
   return MPPD_OK;
 }
 
+// The K fields: 0 .. nadj-1 adjoint fields (zero boundary values, source
+// a_v / V of field v), then n forward fields with the macro strains eps_h,
+// then idle fields.  FP64 defect correction with FP32 inner CG until every
+// field converges; the solution is left in m->U.  A correction whose
+// preconditioner was not positive definite is dropped and solved again, and the
+// rest of the call with Jacobi.
 static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, const mppd_mixed_params *p,
                        int stats[2], std::vector<double> &pn, std::vector<double> &pn0, int *all_conv_out) {
   const Grid &g = m->r->g;
@@ -936,20 +942,26 @@ static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, co
     F = m->F;
   }
   int outer = 0, inner_total = 0, all_conv = 0;
+  const VCycleDev *vc = m->vc;
   pn.assign(K, 0.0);
   pn0.assign(K, 0.0);
   for (;;) {
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, F, m->kinv, m->R, m->X, m->P, m->part, outer == 0,
                            p->rel_tol, p->abs_tol, p->inner_tol, p->max_inner_its, m->state, m->st));
-    if (m->vc) MPP_HIP(launch_v_start(g, K, *m->vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
+    if (vc) MPP_HIP(launch_v_start(g, K, *vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
     if (all_conv || outer >= p->max_outer) break;
+    bool broken = false;
     int its = 0, rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
-                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, m->vc);
+                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, vc, &broken);
     if (rc) return rc;
     inner_total += its;
+    if (broken) {
+      vc = nullptr;
+      continue;
+    }
     MPP_HIP(launch_m_accum(g, K, m->X, m->U, m->st));
     ++outer;
   }
@@ -1069,6 +1081,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
   std::vector<double> rn(K), rn0(K), norm0(K), pn(K), pn0(K);
   for (int k = 0; k < n; ++k) run[k] = 1;
   int outer_total = 0, inner_total = 0;
+  const VCycleDev *vc = m->vc;  // (null once it has failed: msolver_run)
   // the residual of the current U for the fields in run, with the outer test
   // and the inner start state (first: targets from this residual)
   auto resid = [&](int first) -> int {
@@ -1077,7 +1090,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
     MPP_HIP(hipMemcpyAsync(m->act_d, m->act_h, K * sizeof(int), hipMemcpyHostToDevice, m->st));
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, nullptr, m->kinv, m->R, m->X, m->P, m->part, first,
                            p->cg_rel_tol, p->cg_abs_tol, inner_tol, max_inner, m->state, m->st, m->act_d));
-    if (m->vc) MPP_HIP(launch_v_start(g, K, *m->vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
+    if (vc) MPP_HIP(launch_v_start(g, K, *vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_norms(m->state_h, K, cflag.data(), rn.data(), rn0.data());
@@ -1114,12 +1127,19 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
       mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
       if (all_conv || outer >= max_outer) break;
       int inner = 0;
+      bool broken = false;
       if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
-                            m->st, &inner, nullptr, false, nullptr, m->vc)))
+                            m->st, &inner, nullptr, false, nullptr, vc, &broken)))
         return rc;
       inner_total += inner;
-      ++outer_total;
       for (int k = 0; k < n; ++k) cost[k] += run[k] ? inner : 0;
+      if (broken) {  // this outer step again, from its residual
+        vc = nullptr;
+        if (outer == 0 && (rc = resid(1))) return rc;
+        --outer;
+        continue;
+      }
+      ++outer_total;
       MPP_HIP(launch_m_accum(g, K, m->X, m->U, m->st));
     }
     // every exit of the loop above follows a residual of the current U, whose

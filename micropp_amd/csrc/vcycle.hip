@@ -12,6 +12,7 @@
 // sums of the element blocks in the reference element order, rounded once.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 
 #include "mixed.hpp"
 
@@ -874,7 +875,7 @@ hipError_t launch_vcycle(const Grid &g, int K, const VCycleDev &v, const Stencil
 hipError_t launch_v_start(const Grid &g, int K, const VCycleDev &v, const StencilOp &op, const float *kinv,
                           const float *R, float *P, float *AP, void *state, hipStream_t st) {
   const hipError_t e = launch_vcycle(g, K, v, op, kinv, R, P, AP, P, v.prz, state, st);
-  return e == hipSuccess ? launch_c_rzfix(K, stencil_blocks(g, op), v.prz, state, st) : e;
+  return e == hipSuccess ? launch_c_rzfix(K, stencil_blocks(g, op), v.prz, true, state, st) : e;
 }
 
 void vcycle_free(VCycleDev *v) {
@@ -1025,9 +1026,13 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
       break;
     }
     if ((rc = coarse_inverse(g, cg, et_d, ke_d, ainv, st, &ok))) break;  // synchronizes st
-    auto damping = [](double growth) {  // NaN or no growth: not usable
+    // test hook: MPPD_VCYCLE_DAMPING in kDamp's place (above 2: a preconditioner
+    // that is not positive definite, and the solver's return to Jacobi)
+    const char *env = std::getenv("MPPD_VCYCLE_DAMPING");
+    const float damp = env ? (float)std::atof(env) : kDamp;
+    auto damping = [damp](double growth) {  // NaN or no growth: not usable
       const double lam = std::sqrt(growth);
-      return lam > 0.1 && lam < 1e3 ? kDamp / (float)lam : 0.0f;
+      return lam > 0.1 && lam < 1e3 ? damp / (float)lam : 0.0f;
     };
     v->w0 = damping(growth_h[0]);
     v->w1 = two ? 1.0f : damping(growth_h[1]);
