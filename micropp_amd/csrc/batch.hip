@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(256) kb_m_outer(const BRve *rv, const int *act
 // upd form r - alpha Ap from the old r, beside the row blocks that store it:
 // r lives in two vectors, read from r[k & 1] and written to r[(k + 1) & 1].
 // States as in the FP64 CG (kernels.hpp).  FP32 residual rows: row = node * 3
-// + d; sums run in fixed orders, those over the rows in FP64.
+// + d; sums over the rows, r_c among them, are FP64 in fixed orders.
 // What bounds it: the SpMV streams 324 bytes per row (6.3 TB/s with eight
 // RVEs of 25..31 nodes a side live); the other kernels, and the SpMV once most
 // RVEs have stopped, wait for their launch, the state and the partial sums
@@ -503,18 +503,21 @@ __global__ void __launch_bounds__(256) kb_m_upd(const BRve *rv, const int2 *at, 
   const int n = wx * wy * ((cz + 2) * R.g.nez / dz - l0);
   const int ox = 3 * cx, oy = 3 * cgd.mx * cy, oz = 3 * cgd.mx * cgd.my * cz;
   const auto weight = [](const HatEntry &h, int o) { return (h.q0 == o ? h.w0 : 0.0f) + (h.q1 == o ? h.w1 : 0.0f); };
-  float acc[3] = {};
+  double acc[3] = {};
 #pragma unroll 2
   for (int s = threadIdx.x; s < n; s += 256) {
     const int i = i0 + s % wx, j = j0 + (s / wx) % wy, l = l0 + s / (wx * wy);
     const float w = weight(R.hat[0][i], ox) * (weight(R.hat[1][j], oy) * weight(R.hat[2][l], oz));
     const int e = ((l * R.g.ny + j) * R.g.nx + i) * 3;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) acc[d] += w * (START ? r[e + d] : (float)(r[e + d] - alpha * Ap[e + d]));
+    for (int d = 0; d < 3; ++d) acc[d] += (double)w * (START ? r[e + d] : (float)(r[e + d] - alpha * Ap[e + d]));
   }
-  __shared__ float ldf[4 * 3];
-  block_sum<3, 256>(acc, ldf);
-  if (threadIdx.x < 3) R.crc[q * 3 + threadIdx.x] = acc[threadIdx.x];
+  __shared__ double ldc[4 * 3];
+  block_sum<3, 256>(acc, ldc);
+  if (threadIdx.x < 3) {
+    R.crc[q * 3 + threadIdx.x] = acc[threadIdx.x];
+    R.crc32[q * 3 + threadIdx.x] = (float)acc[threadIdx.x];
+  }
 }
 
 // e = A_c^-1 r_c: a wave per two coarse rows (the inverse's rows read along
@@ -526,8 +529,9 @@ __global__ void __launch_bounds__(256) kb_c_gemv(const BRve *rv, const int2 *at,
   const BRve &R = rv[rid];
   if (lb * kGemvRows >= nc || (act ? !act[rid] : cg[2 * rid + ((parity & 1) ^ 1)].done != 0)) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, row = lb * kGemvRows + 2 * w;
-  const float *rc = R.crc;
+  const float *rc = R.crc32;
   const float *a0 = R.cainv + (size_t)min(row, nc - 1) * nc, *a1 = R.cainv + (size_t)min(row + 1, nc - 1) * nc;
+  const double r0 = R.crc[min(row, nc - 1)], r1 = R.crc[min(row + 1, nc - 1)];
   float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll 8
   for (int c = lane; c < nc; c += 64) {
@@ -539,8 +543,8 @@ __global__ void __launch_bounds__(256) kb_c_gemv(const BRve *rv, const int2 *at,
   s1 = wave_sum_dpp(s1);
   if (lane == 0) {
     double z = 0.0;
-    if (row < nc) R.cec[row] = s0, z += (double)rc[row] * s0;
-    if (row + 1 < nc) R.cec[row + 1] = s1, z += (double)rc[row + 1] * s1;
+    if (row < nc) R.cec[row] = s0, z += r0 * s0;
+    if (row + 1 < nc) R.cec[row + 1] = s1, z += r1 * s1;
     lds[w] = z;
   }
   lds_barrier();

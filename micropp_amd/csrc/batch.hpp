@@ -35,13 +35,13 @@ struct BRve {
   // mixed precision, two-level preconditioner of the inner CG (cgrid.nc = 0:
   // Jacobi alone): the inverse of the Galerkin coarse matrix of the RVE's
   // initial (elastic) tangent, the restricted residual and the coarse
-  // correction (nc each), the coarse solve's partials of their product, and
-  // the hats along x, y and z
+  // correction (nc each; the residual's FP64 sums and their FP32 values), the
+  // coarse solve's partials of their product, and the hats along x, y and z
   CGrid cgrid;
   const HatEntry *hat[3];
   const float *cainv;
-  float *crc, *cec;
-  double *cpart;
+  float *crc32, *cec;
+  double *crc, *cpart;
   int phase_mode;              // all phases elastic: one Ke per phase
   int use_vars;                // the RVE has history (vars_n / vars_k in use)
   int nb_row, nb_elem;

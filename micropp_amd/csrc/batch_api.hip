@@ -60,7 +60,7 @@ struct mppd_batch {
   int nb[kShapes] = {};
   int coarse_any = 0;    // mixed precision: some RVE has a coarse level
   float *c32 = nullptr;  // coarse arena: inverses, restriction and correction vectors
-  double *cpart = nullptr;  // partials of the coarse solves
+  double *cpart = nullptr;  // restricted residuals and partials of the coarse solves
   HatEntry *hat_d = nullptr;  // hats of the coarse grids
   // arenas
   double *vec = nullptr, *vals = nullptr, *ke = nullptr, *be = nullptr, *vars = nullptr, *part = nullptr;
@@ -877,11 +877,14 @@ int setup_coarse(mppd_batch *B, const mppd_batch_rve *in, size_t c32) {
   const int n = B->n;
   int rc = dalloc(&B->c32, c32, false);
   if (rc) return rc;
-  size_t nparts = 0, nhat = 0;
-  for (const BRve &R : B->h) nhat += R.cgrid.nc ? R.g.nx + R.g.ny + R.g.nz : 0;
+  size_t nparts = 0, nhat = 0, nrc = 0;
+  for (const BRve &R : B->h) {
+    nhat += R.cgrid.nc ? R.g.nx + R.g.ny + R.g.nz : 0;
+    nrc += R.cgrid.nc;
+  }
   std::vector<HatEntry> hats;
   if ((rc = dalloc(&B->hat_d, nhat, false))) return rc;
-  if ((rc = dalloc(&B->cpart, (size_t)B->nb[5], false))) return rc;
+  if ((rc = dalloc(&B->cpart, nrc + (size_t)B->nb[5], false))) return rc;
   double *ke = nullptr;
   if ((rc = dalloc(&ke, 3 * 576, false))) return rc;
   std::vector<int> owner(n, -1);
@@ -913,7 +916,7 @@ int setup_coarse(mppd_batch *B, const mppd_batch_rve *in, size_t c32) {
       owner[r] = r;
       R.cainv = ainv;
     }
-    R.crc = B->c32 + off;
+    R.crc32 = B->c32 + off;
     R.cec = B->c32 + off + cg.nc;
     off += 2 * (size_t)cg.nc;
     const int ne[3] = {g.nex, g.ney, g.nez}, m[3] = {cg.mx, cg.my, cg.mz};
@@ -921,8 +924,9 @@ int setup_coarse(mppd_batch *B, const mppd_batch_rve *in, size_t c32) {
       R.hat[a] = B->hat_d + hats.size();
       add_hats(hats, ne[a], m[a] + 1, stride);
     }
-    R.cpart = B->cpart + nparts;
-    nparts += (size_t)(cg.nc + kGemvRows - 1) / kGemvRows;
+    R.crc = B->cpart + nparts;
+    R.cpart = R.crc + cg.nc;
+    nparts += cg.nc + (size_t)(cg.nc + kGemvRows - 1) / kGemvRows;
   }
   (void)hipStreamSynchronize(B->st);
   dfree(ke);
