@@ -270,6 +270,9 @@ int mppd_newton_mixed(mppd_solver *s, const mppd_solver *A0, const double eps[6]
  * of the iteration (SpMV fused with p.Ap) and every whole iteration with HIP
  * events on the solver's stream.  Averages in milliseconds. */
 int mppd_cg_profile(mppd_solver *s, const double *b_d, int iters, double *spmv_ms, double *iter_ms);
+/* CG iterations the solver's calls have queued since its creation: those run and
+ * those queued past the end of a solve, before the host's next look */
+int mppd_cg_queued(const mppd_solver *s, long *queued);
 
 /* ---- batches of RVEs (replaces the per-GP loop of homogenize,
  * src/homogenize.cpp:68-99 with homogenize_fe_one_way / homogenize_fe_full,

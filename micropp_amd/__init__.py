@@ -141,6 +141,7 @@ SIGNATURES = {
     "mppd_elem_fields": (_I, [_VP, _VP, _VP, _PD, _PD]),
     "mppd_newton": (_I, [_VP, _VP, _PD, _VP, _VP, C.POINTER(NewtonParams), _PI]),
     "mppd_cg_profile": (_I, [_VP, _VP, _I, _PD, _PD]),
+    "mppd_cg_queued": (_I, [_VP, C.POINTER(C.c_long)]),
     "mppd_msolver_create": (_I, [C.POINTER(C.c_void_p), _VP, _I]),
     "mppd_msolver_destroy": (_I, [_VP]),
     "mppd_msolver_solve": (_I, [_VP, _I, _PD, C.c_void_p, _PD, _PI, _PD]),
@@ -502,6 +503,12 @@ class Solver:
         _chk(load().mppd_cg(self.h, None if A0 is None else A0.h, b.ptr, x.ptr, min_err, rel_err, max_its,
                             C.byref(its), C.byref(err)), "mppd_cg")
         return its.value, err.value
+
+    def cg_queued(self):
+        """CG iterations queued since the solver's creation, those past the end of a solve included."""
+        n = C.c_long()
+        _chk(load().mppd_cg_queued(self.h, C.byref(n)), "mppd_cg_queued")
+        return n.value
 
     def ave_stress(self, u: DeviceArray, vars_: DeviceArray | None = None):
         s = np.zeros(6)

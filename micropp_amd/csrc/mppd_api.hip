@@ -54,6 +54,13 @@ int make_material(const material_base &in, material_base &m) {
 
 using namespace mpp;
 
+// What a solver's CG calls tell the next one: iterations of the last, how many in
+// a row took no fewer than the one before (less 8), iterations queued in all
+struct CgPast {
+  int its = 0, regular = 0;
+  long queued = 0;
+};
+
 struct mppd_solver {
   mppd_rve *r = nullptr;
   hipStream_t st = nullptr;
@@ -68,7 +75,7 @@ struct mppd_solver {
   double *b = nullptr, *du = nullptr;
   double *partials = nullptr;
   CgState *cg = nullptr, *cg_h = nullptr;
-  int cg_expect = 0;  // iterations of the last CG
+  CgPast cg_past;
   RedState *red = nullptr, *red_h = nullptr;
   struct MixedLin *ml = nullptr;  // mppd_newton_mixed buffers, made on first use
   // vals came from this library's assembly (nonzeros only on in-grid stencil
@@ -483,11 +490,21 @@ int mppd_ell_mvp(mppd_solver *s, const double *x_d, double *y_d) {
 struct CgWork {
   CgVecs v;
   CgState *state_h;
-  int *expect;  // iterations of the solver's last CG (0: none yet)
+  CgPast *past;
 };
 
 static CgVecs cg_vecs(const mppd_solver *s) {
   return CgVecs{s->x, s->rr, {s->p, s->p2}, s->Ap, s->kinv, s->partials, s->cg};
+}
+
+// Iterations queued before the first look: as many as the last solve took (a look
+// costs about 10 us), but no more than 32 and one for each solve in a row that
+// took no fewer than the one before it: an iteration queued past the end costs 6
+// to 9 us, so a short solve behind a run of long ones pays about what their looks
+// would have cost.  A solve of 4 iterations to 0.3 behind each of 301 to 1e-12
+// (41^3 nodes): 254 us, 1905 with the last solve's count alone.
+static int cg_first_chunk(const CgPast &p) {
+  return p.its > 0 ? std::max(4, std::min({256, p.its + 1, 32 + p.regular})) : 32;
 }
 
 // CG on the device; the host queues iterations in chunks sized from the last
@@ -499,9 +516,7 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
   MPP_HIP(launch_cg_init(g, A->vals, b_d, v, min_err, rel_err, max_its, st));
   int queued = 0, its_prev = 0;
   double pn_prev = 0;  // of the first look: pn0
-  // as many as the last solve took before the first look (an iteration queued
-  // past the end costs 3 us, a look about 10)
-  int chunk = *w.expect > 0 ? std::max(4, std::min(256, *w.expect + 1)) : 32;
+  int chunk = cg_first_chunk(*w.past);
   for (;;) {
     const int n = std::max(0, std::min(chunk, max_its - queued));
     for (int i = 0; i < n; ++i)
@@ -526,7 +541,10 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
     pn_prev = c.pn;
     its_prev = c.its;
   }
-  *w.expect = w.state_h->its;
+  CgPast &past = *w.past;
+  past.regular = w.state_h->its + 8 >= past.its ? std::min(past.regular + 1, 256) : 0;
+  past.its = w.state_h->its;
+  past.queued += queued;
   if (its_out) *its_out = w.state_h->its;
   if (err_out) *err_out = w.state_h->rz;
   return MPPD_OK;
@@ -534,7 +552,7 @@ static int cg_run_on(const Grid &g, const mppd_solver *A, const CgWork &w, hipSt
 
 static int cg_run(mppd_solver *s, const mppd_solver *A, const double *b_d, double min_err, double rel_err,
                   int max_its, int *its_out, double *err_out) {
-  const CgWork w{cg_vecs(s), s->cg_h, &s->cg_expect};
+  const CgWork w{cg_vecs(s), s->cg_h, &s->cg_past};
   return cg_run_on(s->r->g, A, w, s->st, b_d, min_err, rel_err, max_its, its_out, err_out);
 }
 
@@ -613,7 +631,7 @@ int mppd_cg_noalloc(mppd_solver *s, const mppd_solver *A0, const double *b_d, do
   const auto vec = [v](int i) { return v + i * kNoAllocRows; };
   const CgWork w{
       CgVecs{vec(0), vec(1), {vec(2), vec(3)}, vec(4), vec(5), vec(6), reinterpret_cast<CgState *>(ptr)}, s->cg_h,
-      &s->cg_expect};
+      &s->cg_past};
   if (int rc = cg_run_on(g, A0 ? A0 : s, w, s->st, b_d, min_err, rel_err, max_its, its, err)) return rc;
   MPP_HIP(launch_copy(g.nrow, w.v.x, x_d, s->st));
   MPP_HIP(hipStreamSynchronize(s->st));
@@ -687,6 +705,12 @@ int mppd_newton(mppd_solver *s, const mppd_solver *A0, const double eps[6], cons
   out[0] = its;
   out[1] = solver_its;
   out[2] = conv;
+  return MPPD_OK;
+}
+
+int mppd_cg_queued(const mppd_solver *s, long *queued) {
+  if (!s || !queued) return fail(MPPD_ERR_ARG, "bad cg_queued arguments");
+  *queued = s->cg_past.queued;
   return MPPD_OK;
 }
 
