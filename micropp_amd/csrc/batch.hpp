@@ -49,7 +49,7 @@ struct BRve {
 
 // One launch shape: nb blocks in all; map[block] = RVE; blk0[rve] = the
 // RVE's first block; at[block] = {RVE, block within it}, one load instead of
-// two in a row.
+// two in a row.  A shape holds those that its kernels read, null for the others.
 struct BShape {
   int nb;
   const int *map;

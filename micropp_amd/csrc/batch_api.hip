@@ -51,10 +51,11 @@ struct mppd_batch {
   std::vector<BRve> h;
   std::vector<BState> s;
   BRve *rv = nullptr;
-  // launch shapes
   // launch shapes: rows, elements, element stiffness, then the inner CG's
-  // nodes, rows and coarse nodes, coarse rows
-  static constexpr int kShapes = 6;
+  // nodes, rows and coarse nodes, coarse rows.  The first three have map and
+  // blk0, the rows and the inner CG's have at (BShape)
+  static constexpr int kShapes = 6, kMapped = 3;
+  static constexpr bool has_at(int k) { return k == 0 || k >= kMapped; }
   int *map_d[kShapes] = {}, *blk0_d[kShapes] = {};
   int2 *at_d[kShapes] = {};
   int nb[kShapes] = {};
@@ -952,10 +953,11 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
   // sizes, block tables and arena offsets; with mixed precision, each RVE's
   // coarse grid (a small one: its inverse is read by every inner iteration)
   constexpr int kS = mppd_batch::kShapes;
-  std::vector<int> map[kS], blk0[kS];
+  constexpr int kM = mppd_batch::kMapped;
+  std::vector<int> map[kM], blk0[kM];
   std::vector<int2> at[kS];
   size_t rows = 0, slots = 0, kes = 0, bes = 0, nvars = 0, parts = 0, c32 = 0;
-  for (int k = 0; k < kS; ++k) blk0[k].assign(n, 0);
+  for (auto &b : blk0) b.assign(n, 0);
   const bool coarse = B->prm.mixed_precision && coarse_enabled();
   for (int r = 0; r < n; ++r) {
     const mppd_rve *v = B->rves[r];
@@ -980,9 +982,12 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
       c32 += (size_t)cg.nc * cg.nc + 2 * (size_t)cg.nc;
     }
     for (int k = 0; k < kS; ++k) {
-      blk0[k][r] = (int)map[k].size();
-      map[k].insert(map[k].end(), counts[k], r);
-      for (int b = 0; b < counts[k]; ++b) at[k].push_back(make_int2(r, b));
+      B->nb[k] += counts[k];
+      if (k < kM) {
+        blk0[k][r] = (int)map[k].size();
+        map[k].insert(map[k].end(), counts[k], r);
+      }
+      for (int b = 0; b < counts[k] && mppd_batch::has_at(k); ++b) at[k].push_back(make_int2(r, b));
     }
     rows += g.nrow_pad;
     slots += (size_t)g.nrow_pad * kSlots;
@@ -994,11 +999,13 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
   // the coarse nodes' blocks, which take longest, start first
   std::stable_partition(at[4].begin(), at[4].end(), [&](const int2 &b) { return b.y >= B->h[b.x].nb_row; });
   for (int k = 0; k < kS; ++k) {
-    B->nb[k] = (int)map[k].size();
+    if (mppd_batch::has_at(k)) {
+      if ((rc = dalloc(&B->at_d[k], at[k].size(), false))) return rc;
+      MPP_HIP(hipMemcpy(B->at_d[k], at[k].data(), sizeof(int2) * at[k].size(), hipMemcpyHostToDevice));
+    }
+    if (k >= kM) continue;
     if ((rc = dalloc(&B->map_d[k], map[k].size(), false))) return rc;
     if ((rc = dalloc(&B->blk0_d[k], n, false))) return rc;
-    if ((rc = dalloc(&B->at_d[k], at[k].size(), false))) return rc;
-    MPP_HIP(hipMemcpy(B->at_d[k], at[k].data(), sizeof(int2) * at[k].size(), hipMemcpyHostToDevice));
     MPP_HIP(hipMemcpy(B->map_d[k], map[k].data(), sizeof(int) * map[k].size(), hipMemcpyHostToDevice));
     MPP_HIP(hipMemcpy(B->blk0_d[k], blk0[k].data(), sizeof(int) * n, hipMemcpyHostToDevice));
   }
