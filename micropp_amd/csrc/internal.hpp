@@ -42,19 +42,15 @@ struct Grid {
 
 // Jacobi-PCG scalars of one system (device resident).
 struct CgState {
-  double rz, pn0, pn, alpha, beta, min_err, rel_err, pAp;
+  double rz, pn0, pn, beta, min_err, rel_err;
   int its, max_its, done;
-  int fresh;  // FP64 CG: the scalars hold the last step2's sums (kernels.hpp)
-  unsigned cnt;
-  unsigned pad2[3];
+  int fresh;  // the scalars hold the sums of the last iteration queued (kernels.hpp)
 };
 
 // Status of an averaging / norm reduction.
 struct RedState {
   double v[8];
-  unsigned cnt;
   int flag;
-  unsigned pad[2];
 };
 
 size_t round_up(size_t v, size_t m);
@@ -365,8 +361,8 @@ hipError_t launch_m_resid(const Grid &g, int K, const int *et, const double *ke,
                           const float *kinv, float *R, float *X, float *P, double *part, int first, double rel,
                           double abs_tol, double tau_min, int max_inner, void *state, hipStream_t st,
                           const int *active = nullptr);
-// field f of U from / into a displacement vector in the reference numbering (node * 3 + d)
-// U's K fields = the n <= K vectors u[k] (a null one, or null u: zero), zero beyond; and back to those not null
+// U's K fields = the n <= K displacement vectors u[k] (reference numbering, node * 3 + d; a null one, or null u: zero),
+// zero beyond; and back to those not null
 hipError_t launch_m_load_u(const Grid &g, int K, int n, const double *const *u, double *U, hipStream_t st);
 hipError_t launch_m_store_u(const Grid &g, int K, int n, const double *U, double *const *u, hipStream_t st);
 // adjoint: G (3 x 24 x 6 doubles) and the sources F of fields 0 .. nadj-1
@@ -387,10 +383,8 @@ hipError_t launch_m_adj(const Grid &g, int K, const double *bmat, const material
 // it in every iteration.
 hipError_t launch_c_start(const Grid &g, int K, const CoarseDev &c, const float *kinv, const float *R, float *P,
                           void *state, hipStream_t st);
-// the full symmetric FP32 copy of the lower triangle (column-major) of the
-// FP64 inverse a64 (n x n): ainv[i * n + j]
-// (the operator: the stored FP32 matrix A, K = 4 only, or, when A is null, the
-// stencil dictionary op)
+// one iteration of the inner CG (operator: the stored FP32 matrix A, K = 4 only,
+// or, when A is null, the stencil dictionary op)
 hipError_t launch_m_iter(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                          float *AP, double *part, void *state, int parity, hipStream_t st,
                          const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr);
