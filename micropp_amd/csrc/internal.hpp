@@ -362,7 +362,7 @@ hipError_t launch_m_resid(const Grid &g, int K, const int *et, const double *ke,
                           double abs_tol, double tau_min, int max_inner, void *state, hipStream_t st,
                           const int *active = nullptr);
 // U's K fields = the n <= K displacement vectors u[k] (reference numbering, node * 3 + d; a null one, or null u: zero),
-// zero beyond; and back to those not null
+// zero beyond; and back to those not null (the last of those that are the same)
 hipError_t launch_m_load_u(const Grid &g, int K, int n, const double *const *u, double *U, hipStream_t st);
 hipError_t launch_m_store_u(const Grid &g, int K, int n, const double *U, double *const *u, hipStream_t st);
 // adjoint: G (3 x 24 x 6 doubles) and the sources F of fields 0 .. nadj-1

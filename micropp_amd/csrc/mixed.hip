@@ -1584,7 +1584,11 @@ hipError_t launch_m_load_u(const Grid &g, int K, int n, const double *const *u, 
 hipError_t launch_m_store_u(const Grid &g, int K, int n, const double *U, double *const *u, hipStream_t st) {
   const MLaunch s = mshape(g);
   FieldOut out{};
-  for (int k = 0; k < n; ++k) out.u[k] = u[k];
+  for (int k = 0; k < n; ++k) {
+    for (int q = 0; q < k; ++q)
+      if (out.u[q] == u[k]) out.u[q] = nullptr;  // of fields with one vector the last is stored
+    out.u[k] = u[k];
+  }
   MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_m_store_u<KK>, dim3(nblk(g.nn, 256), n), dim3(256), 0, st, g, s.NP, U, out));
   return hipGetLastError();
 }
