@@ -57,7 +57,7 @@ using namespace mpp;
 // What a solver's CG calls tell the next one: iterations of the last, how many in
 // a row took no fewer than the one before (less 8), iterations queued in all
 struct CgPast {
-  int its = 0, regular = 0;
+  int its = -1, regular = 0;  // (-1: none yet)
   long queued = 0;
 };
 
@@ -504,7 +504,7 @@ static CgVecs cg_vecs(const mppd_solver *s) {
 // would have cost.  A solve of 4 iterations to 0.3 behind each of 301 to 1e-12
 // (41^3 nodes): 254 us, 1905 with the last solve's count alone.
 static int cg_first_chunk(const CgPast &p) {
-  return p.its > 0 ? std::max(4, std::min({256, p.its + 1, 32 + p.regular})) : 32;
+  return p.its >= 0 ? std::max(4, std::min({256, p.its + 1, 32 + p.regular})) : 32;
 }
 
 // CG on the device; the host queues iterations in chunks sized from the last

@@ -49,3 +49,16 @@ def test_like_solves_are_queued_at_once(mp):
     out = calls(mp, [1e-6] * 72)
     assert len({its for its, _ in out}) == 1 and 32 < out[0][0] < 96
     assert all(idle == 1 for _, idle in out[-5:])
+
+
+def test_solves_that_need_no_iteration(mp):
+    """A right-hand side of zero is converged at the start: the next such call queues four iterations."""
+    mats = [mp.material(0, 1e6, 0.3), mp.material(0, 1e7, 0.25), mp.material(0, 1e7, 0.25)]
+    r = mp.Rve((12, 12, 12), mp.MIC3D_RANDOM_SPHERES, (7.0, 8.0, 0.05, 0.15), mats)
+    s, b, x = mp.Solver(r), mp.DeviceArray(r.nrow), mp.DeviceArray(r.nrow)
+    s.assembly_mat(None)
+    queued = [0]
+    for _ in range(4):
+        assert s.cg(b, x)[0] == 0 and not x.numpy().any()
+        queued.append(s.cg_queued())
+    assert np.diff(queued).tolist() == [32, 4, 4, 4]
