@@ -238,6 +238,9 @@ int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h);
  * (1 without one; both 0 without a preconditioner).  The preconditioner is
  * positive definite while each is below 2 / lambda_max(D^-1 A) of its level. */
 int mppd_msolver_damping(const mppd_msolver *m, double w[2]);
+/* inner iterations the solver's calls have queued since its creation: those run
+ * (stats[1]) and those past the end of a solve */
+int mppd_msolver_queued(const mppd_msolver *m, long *queued);
 /* newton_raphson (src/solve.cpp:28-82) with mixed-precision linear solves,
  * for an RVE of any material law (a plastic or damaged RVE's Newton tangent
  * included).  The Newton control flow, the residual (assembly_rhs with the

@@ -151,6 +151,7 @@ SIGNATURES = {
     "mppd_msolver_profile": (_I, [_VP, _I, _PD, _PD]),
     "mppd_msolver_coarse": (_I, [_VP, _PI, C.POINTER(C.c_float)]),
     "mppd_msolver_damping": (_I, [_VP, _PD]),
+    "mppd_msolver_queued": (_I, [_VP, C.POINTER(C.c_long)]),
     "mppd_msolver_newton": (_I, [_VP, _I, _PD, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, _PD, _PI, _PI]),
     "mppd_newton_mixed": (_I, [_VP, _VP, _PD, _VP, _VP, C.POINTER(NewtonParams), _VP, _PI, _PI]),
     "mppd_batch_params_default": (None, [_VP]),
@@ -647,6 +648,12 @@ class MSolver:
         _chk(load().mppd_msolver_coarse(self.h, _ip(dims), ainv.ctypes.data_as(C.POINTER(C.c_float))),
              "mppd_msolver_coarse")
         return dims, ainv
+
+    def queued(self):
+        """Inner iterations queued since the solver's creation, those past the end of a solve included."""
+        n = C.c_long()
+        _chk(load().mppd_msolver_queued(self.h, C.byref(n)), "mppd_msolver_queued")
+        return n.value
 
     def damping(self):
         """The damping of the preconditioner's Jacobi smoothers: (fine grid, second level)."""

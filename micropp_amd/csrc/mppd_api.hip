@@ -755,6 +755,7 @@ constexpr int kMaxRhsFields = 16;  // largest K of an msolver
 struct mppd_msolver {
   mppd_rve *r = nullptr;
   int K = 0;
+  long queued = 0;          // inner iterations queued by its calls
   VCycleDev *vc = nullptr;  // multilevel preconditioner of the inner CG (null: Jacobi alone)
   hipStream_t st = nullptr;
   double *ke = nullptr;         // phase table 3 x 576 (FP64)
@@ -885,13 +886,17 @@ int mppd_msolver_destroy(mppd_msolver *m) {
 static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                        float *AP, double *part, void *state, void *state_h, int max_inner, hipStream_t st,
                        int *its_out, bool *finite = nullptr, bool stop_on_stall = false,
-                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr, bool *broken = nullptr) {
+                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr, bool *broken = nullptr,
+                       long *queued_out = nullptr) {
   int queued = 0, its = 0, done = 0, its_prev = 0;
   if (vc) mixed_state_view(state_h, 0, &its, &done);  // (it may be broken at the start)
-  // (with the multilevel preconditioner a solve takes about 10 iterations of
-  // up to 13 launches each, so few are queued past the end)
+  // With the multilevel preconditioner a solve takes about 10 iterations of up
+  // to 13 launches each, so few are queued past the end: an iteration after it
+  // costs about 50 us, a look 10.  (Rates of plateaus overshoot by far: 96
+  // iterations at contrast 1000, 30^3 elements, 18.8 ms with chunks of up to 256,
+  // 7.6 with 16.)
   int chunk = vc ? 8 : 32;
-  const int slack = vc ? 0 : 2, least = vc ? 1 : 4;
+  const int slack = vc ? 0 : 2, least = vc ? 1 : 4, most = vc ? 16 : 256;
   std::vector<double> pn_prev(K, 0.0);
   for (int k = 0; k < K; ++k) {
     double target;
@@ -924,13 +929,14 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
       pn_prev[k] = pnk;
     }
     its_prev = its;
-    chunk = std::max(least, std::min(256, next));
+    chunk = std::max(least, std::min(most, next));
     // FP32 CG that no longer reduces ||z|| by 10% over a chunk of >= 32
     // iterations (rounding, or a nonsymmetric Newton tangent) is stopped: the
     // caller's FP64 defect correction restarts it from the true residual
     if (stalled && stop_on_stall) break;
   }
   *its_out = its;
+  if (queued_out) *queued_out += queued;
   if (broken) *broken = mixed_state_broken(state_h, queued);
   if (finite) {
     *finite = true;
@@ -979,7 +985,7 @@ static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, co
     if (all_conv || outer >= p->max_outer) break;
     bool broken = false;
     int its = 0, rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
-                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, vc, &broken);
+                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, vc, &broken, &m->queued);
     if (rc) return rc;
     inner_total += its;
     if (broken) {
@@ -1153,7 +1159,7 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
       int inner = 0;
       bool broken = false;
       if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
-                            m->st, &inner, nullptr, false, nullptr, vc, &broken)))
+                            m->st, &inner, nullptr, false, nullptr, vc, &broken, &m->queued)))
         return rc;
       inner_total += inner;
       for (int k = 0; k < n; ++k) cost[k] += run[k] ? inner : 0;
@@ -1450,6 +1456,12 @@ int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h) {
     MPP_HIP(hipMemcpyAsync(ainv_h, c->ainv, (size_t)cg.nc * cg.nc * sizeof(float), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
   }
+  return MPPD_OK;
+}
+
+int mppd_msolver_queued(const mppd_msolver *m, long *queued) {
+  if (!m || !queued) return fail(MPPD_ERR_ARG, "bad msolver_queued arguments");
+  *queued = m->queued;
   return MPPD_OK;
 }
 
