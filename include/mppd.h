@@ -226,13 +226,15 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
  * elements per coarse element along x, y, z, interior coarse nodes along x,
  * y, z (all 0 without a coarse level).  Where a side of ne elements is no
  * multiple of its d = m + 1 coarse ones, h is the smaller of two widths, h
- * and h + 1.  ainv_h (may be NULL): nc x nc floats,
+ * and h + 1.  With three levels and a contrast of the moduli above 30 the
+ * widths are even instead, h and h + 2, and an odd side's last one is narrower
+ * by 1.  ainv_h (may be NULL): nc x nc floats,
  * the inverse of the Galerkin matrix P^T A P, P the trilinear hats of the
  * interior coarse nodes; coarse DOF q * 3 + d of node q = ((cz - 1) my +
  * (cy - 1)) mx + (cx - 1), hat of (cx, cy, cz) at fine node (i, j, k) = the
  * product over the sides of the hat that is 1 at fine index floor(cx ne / d)
- * and 0 at the neighbouring coarse nodes' (h wide everywhere: max(0, 1 -
- * |i - cx hx| / hx)). */
+ * (even widths: 2 floor(cx ceil(ne / 2) / d)) and 0 at the neighbouring coarse
+ * nodes' (h wide everywhere: max(0, 1 - |i - cx hx| / hx)). */
 int mppd_msolver_coarse(const mppd_msolver *m, int dims[7], float *ainv_h);
 /* The damping of its Jacobi smoothers on the fine grid and on the second level
  * (1 without one; both 0 without a preconditioner).  The preconditioner is

@@ -32,10 +32,28 @@ int pick_side(int ne, int dmax) {
   return 0;
 }
 
-// positions of a fine element along a side (see k_cs_table)
-__host__ __device__ inline int npos(int h, int l) { return l == h ? h : h + l; }
-// first fine element of coarse element E of d along a side of ne
-__device__ __forceinline__ int cnode(int E, int ne, int d) { return E * ne / d; }
+// Contrast above which the multilevel preconditioner's coarse nodes have even
+// fine indices, i.e. are nodes of its second level.  A coarse hat with its peak
+// between two of them is no sum of its hats, and its Galerkin matrix says
+// nothing about the energy of what the second level makes of it: beside a stiff
+// element too little by up to the contrast.  Solves of 8 fields to 1e-8, ms, at
+// even indices / at floor(q ne / d): 30^3 elements, 40 small spheres, contrast
+// 10 1.85 / 1.84, 300 7.4 / 8.4, 1e4 39 / 86, 1e5 153 / 796; 50^3, a layer, 300
+// 3.4 / 4.0, 1e4 3.7 / 14.9, 1e-5 3.5 / 36.  Over 45 RVEs, to 1e-10, even
+// indices take 1.01 of the time at contrast 3, 1.00 at 10, 0.99 at 30, 0.97 at
+// 100 and 0.93 at 300.
+constexpr double kEvenContrast = 30.0;
+
+// Positions of a fine element along a side: 0 .. h - 1 in a coarse element h
+// wide, then those in one l wide and in the last one (t wide), as far as these
+// widths differ.  The first position in an element w wide, and all of them:
+__host__ __device__ inline int pos0(int w, int h, int l) { return w == h ? 0 : w == l ? h : h + (l == h ? 0 : l); }
+__host__ __device__ inline int npos(int h, int l, int t) { return t == h || t == l ? pos0(0, h, l) : pos0(t, h, l) + t; }
+// the hat of an element's far end at node px + o of position px
+__device__ __forceinline__ double pos_hat(int px, int o, int h, int l, int t) {
+  const int w = px < h ? h : l != h && px < h + l ? l : t;
+  return (double)(px - pos0(w, h, l) + o) / w;
+}
 
 // corner A of a hexahedron (the element's local node order: (0,0,0), (1,0,0),
 // (1,1,0), (0,1,0), then the same at z + 1) and its inverse
@@ -45,21 +63,19 @@ __device__ __forceinline__ int hex_oz(int A) { return A >> 2; }
 __device__ __forceinline__ int hex_corner(int ox, int oy, int oz) { return oz * 4 + (oy ? 3 - ox : ox); }
 
 // C[(pos * 3 + phase) * 576 + r * 24 + c] = (P_e^T Ke_phase P_e)[r][c] for the
-// fine element at position pos = (pz ny + py) nx + px, nx = npos(hx, lx) ...
-// (p < h: the position in an element h wide; h + p: in one l wide), from
-// plane z0 of positions on: block (pos, phase), one thread per entry
+// fine element at position pos = (pz ny + py) nx + px, nx = npos(hx, lx, tx) ...,
+// from plane z0 of positions on: block (pos, phase), one thread per entry
 __global__ void __launch_bounds__(576) k_cs_table(CGrid cg, int z0, const double *ke, double *C) {
   __shared__ double N[8][8];  // N[a][A]: coarse corner A's hat at the fine element's node a
   __shared__ double K[576];
   const int pos = blockIdx.x, ph = blockIdx.y, t = threadIdx.x;
-  const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
+  const int nx = npos(cg.hx, cg.lx, cg.tx), ny = npos(cg.hy, cg.ly, cg.ty);
   const int px = pos % nx, py = (pos / nx) % ny, pz = z0 + pos / (nx * ny);
   K[t] = ke[(size_t)ph * 576 + t];
   if (t < 64) {
     const int a = t >> 3, A = t & 7;
-    const double xi = px < cg.hx ? (double)(px + hex_ox(a)) / cg.hx : (double)(px - cg.hx + hex_ox(a)) / cg.lx,
-                 yi = py < cg.hy ? (double)(py + hex_oy(a)) / cg.hy : (double)(py - cg.hy + hex_oy(a)) / cg.ly,
-                 zi = pz < cg.hz ? (double)(pz + hex_oz(a)) / cg.hz : (double)(pz - cg.hz + hex_oz(a)) / cg.lz;
+    const double xi = pos_hat(px, hex_ox(a), cg.hx, cg.lx, cg.tx), yi = pos_hat(py, hex_oy(a), cg.hy, cg.ly, cg.ty),
+                 zi = pos_hat(pz, hex_oz(a), cg.hz, cg.lz, cg.tz);
     N[a][A] = (hex_ox(A) ? xi : 1.0 - xi) * (hex_oy(A) ? yi : 1.0 - yi) * (hex_oz(A) ? zi : 1.0 - zi);
   }
   __syncthreads();
@@ -81,11 +97,13 @@ __global__ void __launch_bounds__(576) k_cs_elem(Grid g, CGrid cg, int dx, int d
                                                  const double *C, double *KE) {
   const int E = blockIdx.x, t = threadIdx.x;
   const int Ex = E % dx, Ey = (E / dx) % dy, Ez = E / (dx * dy);
-  const int nx = npos(cg.hx, cg.lx), ny = npos(cg.hy, cg.ly);
-  const int x0 = cnode(Ex, g.nex, cg.mx + 1), y0 = cnode(Ey, g.ney, cg.my + 1), z0 = cnode(Ez, g.nez, cg.mz + 1);
-  const int wx = cnode(Ex + 1, g.nex, cg.mx + 1) - x0, wy = cnode(Ey + 1, g.ney, cg.my + 1) - y0,
-            wz = cnode(Ez + 1, g.nez, cg.mz + 1) - z0;
-  const int ox = wx != cg.hx ? cg.hx : 0, oy = wy != cg.hy ? cg.hy : 0, oz = wz != cg.hz ? cg.hz : 0;
+  const int nx = npos(cg.hx, cg.lx, cg.tx), ny = npos(cg.hy, cg.ly, cg.ty);
+  const auto nodex = [&](int q) { return coarse_node(q, g.nex, cg.mx + 1, cg.even & 1); };
+  const auto nodey = [&](int q) { return coarse_node(q, g.ney, cg.my + 1, cg.even & 2); };
+  const auto nodez = [&](int q) { return coarse_node(q, g.nez, cg.mz + 1, cg.even & 4); };
+  const int x0 = nodex(Ex), y0 = nodey(Ey), z0 = nodez(Ez);
+  const int wx = nodex(Ex + 1) - x0, wy = nodey(Ey + 1) - y0, wz = nodez(Ez + 1) - z0;
+  const int ox = pos0(wx, cg.hx, cg.lx), oy = pos0(wy, cg.hy, cg.ly), oz = pos0(wz, cg.hz, cg.lz);
   double s = zp ? KE[(size_t)E * 576 + t] : 0.0;
   for (int pz = max(0, zp - oz); pz < min(wz, zp + nz - oz); ++pz)
     for (int py = 0; py < wy; ++py)
@@ -465,7 +483,7 @@ bool coarse_enabled() {
 }
 
 // the coarse grid of hx, hy, hz (lx, ly, lz) fine elements per coarse element
-// and mx, my, mz interior nodes
+// and mx, my, mz interior nodes, coarse_node's with even = 0
 static CGrid make_grid(int hx, int hy, int hz, int lx, int ly, int lz, int mx, int my, int mz) {
   CGrid cg;
   cg.hx = hx;
@@ -474,6 +492,10 @@ static CGrid make_grid(int hx, int hy, int hz, int lx, int ly, int lz, int mx, i
   cg.lx = lx;
   cg.ly = ly;
   cg.lz = lz;
+  cg.tx = hx;
+  cg.ty = hy;
+  cg.tz = hz;
+  cg.even = 0;
   cg.mx = mx;
   cg.my = my;
   cg.mz = mz;
@@ -518,11 +540,26 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out) {
 // costs 0.1 ms more): 30^3 elements 29 iterations to 1e-10 become 25, 29 x 37 x
 // 23 38 become 33, sigma and ctan 9% sooner.  2187 DOFs (30^3 at h = 3, 40^3 at h
 // = 4: 19 MB read an iteration and 0.7 ms more set-up) cost more than they save.
-bool coarse_grid_cycle(const Grid &g, CGrid *out) {
-  if (coarse_grid_wide(g, 4, 1100, out) &&
-      std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= 4)
-    return true;
-  return coarse_grid_wide(g, 5, kCoarseMaxDofs, out);
+bool coarse_grid_cycle(const Grid &g, double contrast, CGrid *out) {
+  const bool narrow = coarse_grid_wide(g, 4, 1100, out) &&
+                      std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= 4;
+  if (!narrow && !coarse_grid_wide(g, 5, kCoarseMaxDofs, out)) return false;
+  if (contrast <= kEvenContrast) return true;
+  const int ne[3] = {g.nex, g.ney, g.nez}, m[3] = {out->mx, out->my, out->mz};
+  int h[3] = {out->hx, out->hy, out->hz}, l[3] = {out->lx, out->ly, out->lz}, even = 0;
+  for (int a = 0; a < 3; ++a) {
+    if (l[a] == h[a] && h[a] % 2 == 0) continue;  // even already
+    const int n = (ne[a] + 1) / 2, d = m[a] + 1;
+    even |= 1 << a;
+    h[a] = 2 * (n / d);
+    l[a] = h[a] + (n % d ? 2 : 0);
+  }
+  *out = make_grid(h[0], h[1], h[2], l[0], l[1], l[2], m[0], m[1], m[2]);
+  out->even = even;
+  out->tx = ne[0] - coarse_node(m[0], ne[0], m[0] + 1, even & 1);
+  out->ty = ne[1] - coarse_node(m[1], ne[1], m[1] + 1, even & 2);
+  out->tz = ne[2] - coarse_node(m[2], ne[2], m[2] + 1, even & 4);
+  return true;
 }
 
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
@@ -544,10 +581,10 @@ bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
   return false;
 }
 
-int coarse_table_planes(const CGrid &cg) { return npos(cg.hz, cg.lz); }
+int coarse_table_planes(const CGrid &cg) { return npos(cg.hz, cg.lz, cg.tz); }
 
 size_t coarse_table_len(const CGrid &cg, int nz) {
-  return (size_t)npos(cg.hx, cg.lx) * npos(cg.hy, cg.ly) * nz * 3 * 576;
+  return (size_t)npos(cg.hx, cg.lx, cg.tx) * npos(cg.hy, cg.ly, cg.ty) * nz * 3 * 576;
 }
 
 hipError_t launch_cs_table(const CGrid &cg, int z0, int nz, const double *ke, double *C, hipStream_t st) {

@@ -142,9 +142,17 @@ inline bool alloc_fault_injected() {
 struct CGrid {
   int hx, hy, hz;  // fine elements per coarse element
   int lx, ly, lz;  // = h where all are h wide; else some are l wide
+  int tx, ty, tz;  // width of the last, where neither (= h otherwise)
   int mx, my, mz;  // interior coarse nodes per side
   int nq, nc;      // interior coarse nodes, coarse DOFs (3 nq)
+  int even;        // sides (bit 0 x, 1 y, 2 z) whose coarse nodes have even fine indices
 };
+
+// fine index of coarse node q (0 .. d) along a side of ne elements
+__host__ __device__ inline int coarse_node(int q, int ne, int d, int even) {
+  if (!even) return q * ne / d;
+  return q < d ? 2 * (q * ((ne + 1) / 2) / d) : ne;
+}
 // device buffers of the coarse level of one K-field system
 struct CoarseDev {
   CGrid cg;
@@ -175,8 +183,11 @@ struct HatEntry {
 // dense inverse of a coarse Galerkin matrix.  Small RVEs have no second level
 // (mid.nq = 0): their coarse grid is that fine itself.
 struct VCycleDev {
-  CGrid mid, cg;     // second level (h = 2), coarse grid (hats on the fine grid's indices)
-  HatEntry *hat[3];  // the coarse hats along x, y, z
+  CGrid mid, cg;  // second level (h = 2), coarse grid
+  // along x, y, z: the coarse hats at the nodes of the level above, and the
+  // first node there beyond coarse node q (0 .. d - 1), and at or beyond it (1 .. d)
+  const HatEntry *hat[3];
+  const int *past[3], *upto[3];
   Grid g1;           // the second level as a grid: m + 2 nodes a side, the boundary among them
   const float *ainv;          // nc x nc
   float *rc, *ec;             // restricted residual and coarse correction (nc x K)
@@ -194,15 +205,16 @@ bool coarse_enabled();
 bool coarse_grid(const Grid &g, int max_dofs, CGrid *out);
 // the grid of twice the spacing (an odd side's last element 1 wide; false: a side of fewer than 4 elements)
 bool coarse_grid_by_two(const Grid &g, CGrid *out);
-// the coarse grid of the multilevel preconditioner: 4 or 5 fine elements per coarse element and side, coarse node q
-// of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
+// the coarse grid of the multilevel preconditioner of an RVE with this contrast: about 4 or 5 fine elements per coarse
+// element and side; false: none
+bool coarse_grid_cycle(const Grid &g, double contrast, CGrid *out);
+// a coarse grid of elements of at least `least` fine ones a side, as narrow as max_dofs coarse DOFs allow: coarse node
+// q of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
 // divide the side, l = h + 1); false: none
-bool coarse_grid_cycle(const Grid &g, CGrid *out);
-// the same with the narrowest coarse elements of at least `least` fine ones a side and at most max_dofs coarse DOFs
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out);
 // C (device, coarse_table_len(cg, nz) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position,
 // for nz of the coarse_table_planes(cg) planes of positions from z0 on
-// (position px of a side: px < h in an element h wide, h + px in one l wide)
+// (positions of a side: those in an element h wide, in one l wide, in the last one)
 int coarse_table_planes(const CGrid &cg);
 size_t coarse_table_len(const CGrid &cg, int nz);
 hipError_t launch_cs_table(const CGrid &cg, int z0, int nz, const double *ke, double *C, hipStream_t st);
@@ -336,7 +348,8 @@ hipError_t launch_d_spmv(const Grid &g, int K, const StencilOp &op, const float 
                          const void *state, hipStream_t st);
 // the multilevel preconditioner of a K-field system (*out = nullptr: no
 // coarse grid, or MPPD_COARSE=0); P and AP are its scratch during the set-up
-int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
+// (contrast: of the RVE's materials, at least 1)
+int vcycle_setup(const Grid &g, int K, double contrast, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
                  float *P, float *AP, hipStream_t st, VCycleDev **out);
 void vcycle_free(VCycleDev *v);
 // OUT = M R with Z = D^-1 R given (Z may be v.z), T a work vector, and the (r, OUT) partials

@@ -775,6 +775,19 @@ struct mppd_msolver {
 
 extern "C" {
 
+// the largest ratio between the materials' moduli (uniaxial strain, shear)
+static double contrast(const material_base (&mats)[3]) {
+  double lo[2] = {INFINITY, INFINITY}, hi[2] = {0.0, 0.0};
+  for (const material_base &m : mats) {
+    const double c[2] = {m.lambda + 2 * m.mu, m.mu};
+    for (int i = 0; i < 2; ++i) {
+      lo[i] = std::min(lo[i], c[i]);
+      hi[i] = std::max(hi[i], c[i]);
+    }
+  }
+  return std::max(hi[0] / lo[0], hi[1] / lo[1]);
+}
+
 int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
   *out = nullptr;
   if (!r) return fail(MPPD_ERR_ARG, "null rve");
@@ -853,7 +866,7 @@ int mppd_msolver_create(mppd_msolver **out, mppd_rve *r, int nrhs) {
       rc = hip_fail(e, "msolver set-up");
       break;
     }
-    rc = vcycle_setup(g, nrhs, r->et, m->ke, m->op, m->kinv, m->P, m->AP, m->st, &m->vc);
+    rc = vcycle_setup(g, nrhs, contrast(r->mats), r->et, m->ke, m->op, m->kinv, m->P, m->AP, m->st, &m->vc);
   } while (0);
   if (rc) {
     mppd_msolver_destroy(m);

@@ -13,6 +13,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
+#include <vector>
 
 #include "mixed.hpp"
 
@@ -396,7 +398,8 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 // same cycle on that grid (small RVEs, vcycle_setup: P1 the coarse hats and M1
 // the dense inverse, nothing in between) with its Galerkin operator A1 = P1^T A P1 and the
 // dense inverse of the coarse Galerkin matrix as its correction (P2: the coarse
-// hats at the second level's nodes).  M is symmetric positive definite while w0 and w1 stay
+// hats at the second level's nodes; at high contrasts these include the coarse
+// ones, coarse_grid_cycle).  M is symmetric positive definite while w0 and w1 stay
 // below 2 / lambda_max(D^-1 A) of their levels (estimated at set-up by a power
 // iteration on the operators themselves, since isolated stiff elements raise
 // it: 2.7-2.9 for cubes, up to 4.5 in thin cells and beside one stiff element).
@@ -408,23 +411,13 @@ __global__ void __launch_bounds__(256, 3) k_d_apply(Grid g, int NP, int nbi, int
 // without a common divisor (29 x 37 x 23 elements) had no coarse level before:
 // 33 iterations against 250, 2.3 ms against 5.9 ms.
 // ---------------------------------------------------------------------------
-
-// the coarse hats along a side of ne fine elements and d coarse ones, node q at
-// fine index floor(q ne / d) (HatEntry, at every fine index), offsets of stride
-// per interior coarse node
-__global__ void __launch_bounds__(256) k_v_hats(int ne, int d, int stride, HatEntry *out) {
-  const int i = threadIdx.x;  // sides have at most kCoarseMaxLine = 256 nodes
-  if (i > ne) return;
-  const int e = min(((i + 1) * d - 1) / ne, d - 1), a = e * ne / d, b = (e + 1) * ne / d;  // the coarse element
-  const float f = (float)(i - a) / (float)(b - a);
-  out[i] = {e >= 1 ? 1.0f - f : 0.0f, e + 1 < d ? f : 0.0f, (max(e, 1) - 1) * stride, (min(e + 1, d - 1) - 1) * stride};
-}
 // a hat's weight at an index with entry h, the hat's node at offset o
 __device__ __forceinline__ float hat_weight(const HatEntry &h, int o) {
   return (h.q0 == o ? h.w0 : 0.0f) + (h.q1 == o ? h.w1 : 0.0f);
 }
-struct Hats {
+struct Hats {  // along x, y and z (VCycleDev)
   const HatEntry *x, *y, *z;
+  const int *past[3], *upto[3];
 };
 
 // R1 = P1^T T and E0 = D1^-1 R1.  One thread per second-level node (boundary
@@ -527,29 +520,28 @@ __global__ void __launch_bounds__(MODE == kApplyPow ? 192 : 48 * K)
   }
 }
 
-// rc = P^T T for the coarse hats at the nodes of grid gt, node i at fine index
-// S i (the second level, S = 2, or the fine grid itself): a wave per coarse node
-// and component, its lanes over the nodes under the node's hat
-template <int K, int S>
-__global__ void __launch_bounds__(256) k_v_coarse_rhs(Grid g, Grid gt, CGrid cg, Hats hats, int NPt, const float4 *T,
+// rc = P^T T for the coarse hats at the nodes of grid gt (the second level or
+// the fine grid itself): a wave per coarse node and component, its lanes over
+// the nodes under the node's hat
+template <int K>
+__global__ void __launch_bounds__(256) k_v_coarse_rhs(Grid gt, CGrid cg, Hats hats, int NPt, const float4 *T,
                                                       float4 *rc4, const MState *cur) {
   constexpr int KG = K / 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int id = blockIdx.x * 4 + wv, c = blockIdx.y, d = c / KG, grp = c % KG;
   if (id >= cg.nq || group_stopped(cur, grp * 4)) return;
   const int cx = id % cg.mx, cy = (id / cg.mx) % cg.my, cz = id / (cg.mx * cg.my);  // interior index, 0-based
-  const int dx = cg.mx + 1, dy = cg.my + 1, dz = cg.mz + 1;
-  // nodes with a non-zero hat: fine indices S i strictly between the neighbouring coarse nodes
-  const int x0 = cx * g.nex / dx / S + 1, y0 = cy * g.ney / dy / S + 1, z0 = cz * g.nez / dz / S + 1;
-  const int wx = ((cx + 2) * g.nex / dx - 1) / S + 1 - x0, wy = ((cy + 2) * g.ney / dy - 1) / S + 1 - y0;
-  const int n = wx * wy * (((cz + 2) * g.nez / dz - 1) / S + 1 - z0);
+  // nodes with a non-zero hat: strictly between the neighbouring coarse nodes
+  const int x0 = hats.past[0][cx], y0 = hats.past[1][cy], z0 = hats.past[2][cz];
+  const int wx = hats.upto[0][cx + 2] - x0, wy = hats.upto[1][cy + 2] - y0;
+  const int n = wx * wy * (hats.upto[2][cz + 2] - z0);
   const int ox = 3 * cx, oy = 3 * cg.mx * cy, oz = 3 * cg.mx * cg.my * cz;
   const float4 *t = T + (size_t)c * NPt;
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 2
   for (int s = lane; s < n; s += 64) {
     const int r = s / wx, x = x0 + s % wx, y = y0 + r % wy, z = z0 + r / wy;
-    const float w = hat_weight(hats.x[S * x], ox) * (hat_weight(hats.y[S * y], oy) * hat_weight(hats.z[S * z], oz));
+    const float w = hat_weight(hats.x[x], ox) * (hat_weight(hats.y[y], oy) * hat_weight(hats.z[z], oz));
     fma4(acc, w, t[((size_t)z * gt.ny + y) * gt.nx + x]);
   }
   acc = make_float4(wave_sum_dpp(acc.x), wave_sum_dpp(acc.y), wave_sum_dpp(acc.z), wave_sum_dpp(acc.w));
@@ -614,9 +606,9 @@ __global__ void __launch_bounds__(64 * kGemvWaves) k_v_gemv(int nc, const float 
   ec[(size_t)(row0 + i) * K + f] = s;
 }
 
-// OUT = w IN + P ec at the nodes of grid gt (S as k_v_coarse_rhs; OUT may be
-// IN); boundary nodes keep IN, zero there
-template <int K, int S>
+// OUT = w IN + P ec at the nodes of grid gt (as k_v_coarse_rhs; OUT may be IN);
+// boundary nodes keep IN, zero there
+template <int K>
 __global__ void __launch_bounds__(256) k_v_coarse_add(Grid gt, Hats hats, int NPt, float w, const float4 *ec,
                                                       const float4 *IN, float4 *OUT, const MState *cur) {
   constexpr int KG = K / 4;
@@ -627,7 +619,7 @@ __global__ void __launch_bounds__(256) k_v_coarse_add(Grid gt, Hats hats, int NP
   const int x = n % gt.nx, y = (n / gt.nx) % gt.ny, z = n / (gt.nx * gt.ny);
   float4 acc = make_float4(w * e0.x, w * e0.y, w * e0.z, w * e0.w);
   if (n < gt.nn && !node_on_boundary(gt, x, y, z)) {
-    const HatEntry hx = hats.x[S * x], hy = hats.y[S * y], hz = hats.z[S * z];
+    const HatEntry hx = hats.x[x], hy = hats.y[y], hz = hats.z[z];
     float4 e[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t)
@@ -839,15 +831,15 @@ hipError_t launch_vcycle(const Grid &g, int K, const VCycleDev &v, const Stencil
   const dim3 grid0(NP / 256, 3 * K / 4);
   hipError_t e = launch_d_apply<kApplyRes>(g, K, op, Z, R, kinv, v.w0, T, nullptr, state, st);
   if (e != hipSuccess) return e;
-  const Hats hats{v.hat[0], v.hat[1], v.hat[2]};
+  const Hats hats{v.hat[0], v.hat[1], v.hat[2], {v.past[0], v.past[1], v.past[2]}, {v.upto[0], v.upto[1], v.upto[2]}};
   const dim3 nq(nblk(v.cg.nq, 4), 3 * K / 4);
   float4 *rc4 = reinterpret_cast<float4 *>(v.rc), *ec4 = reinterpret_cast<float4 *>(v.ec);
   if (!v.mid.nq) {  // two levels
     MPP_K_DISPATCH(K, {
-      hipLaunchKernelGGL((k_v_coarse_rhs<KK, 1>), nq, dim3(256), 0, st, g, g, v.cg, hats, NP,
+      hipLaunchKernelGGL(k_v_coarse_rhs<KK>, nq, dim3(256), 0, st, g, v.cg, hats, NP,
                          reinterpret_cast<const float4 *>(T), rc4, cur);
       launch_gemv<KK>(v, cur, st);
-      hipLaunchKernelGGL((k_v_coarse_add<KK, 1>), grid0, dim3(256), 0, st, g, hats, NP, v.w0, ec4,
+      hipLaunchKernelGGL(k_v_coarse_add<KK>, grid0, dim3(256), 0, st, g, hats, NP, v.w0, ec4,
                          reinterpret_cast<const float4 *>(Z), reinterpret_cast<float4 *>(v.z), cur);
     });
     return launch_d_apply<kApplyPost>(g, K, op, v.z, R, kinv, v.w0, OUT, pr, state, st);
@@ -860,10 +852,10 @@ hipError_t launch_vcycle(const Grid &g, int K, const VCycleDev &v, const Stencil
                                        E0, cur));
   if ((e = launch_mid<kApplyRes>(v.g1, K, v, v.E0, v.R1, v.T1, nullptr, state, st)) != hipSuccess) return e;
   MPP_K_DISPATCH(K, {
-    hipLaunchKernelGGL((k_v_coarse_rhs<KK, 2>), nq, dim3(256), 0, st, g, v.g1, v.cg, hats, NP1,
+    hipLaunchKernelGGL(k_v_coarse_rhs<KK>, nq, dim3(256), 0, st, v.g1, v.cg, hats, NP1,
                        reinterpret_cast<const float4 *>(v.T1), rc4, cur);
     launch_gemv<KK>(v, cur, st);
-    hipLaunchKernelGGL((k_v_coarse_add<KK, 2>), grid1, dim3(256), 0, st, v.g1, hats, NP1, v.w1, ec4, E0, E0, cur);
+    hipLaunchKernelGGL(k_v_coarse_add<KK>, grid1, dim3(256), 0, st, v.g1, hats, NP1, v.w1, ec4, E0, E0, cur);
   });
   if ((e = launch_mid<kApplyPost>(v.g1, K, v, v.E0, v.R1, v.E, nullptr, state, st)) != hipSuccess) return e;
   MPP_K_DISPATCH(K, hipLaunchKernelGGL(k_v_prolong<KK>, grid0, dim3(256), 0, st, g, v.g1, NP, NP1, v.w0,
@@ -910,9 +902,33 @@ bool coarse_grid_two_level(const Grid &g, CGrid *out) {
       return true;
   return false;
 }
+
+// The tables of a side of ne fine and d coarse elements at the nodes of the
+// level above the coarse one, node i at fine index min(step i, ne): the hats
+// (offsets of stride per interior coarse node), then, each for q = 0 .. d, the
+// first node beyond coarse node q and the first one at or beyond it
+void side_tables(int ne, int d, int even, int step, int stride, std::vector<HatEntry> &hats, std::vector<int> &ends) {
+  const int n = (ne + step - 1) / step + 1;
+  ends.assign(2 * (d + 1), n);
+  int e = 0;
+  for (int i = n - 1; i >= 0; --i)
+    for (int q = 0; q <= d; ++q) {
+      const int x = std::min(step * i, ne), at = coarse_node(q, ne, d, even);
+      if (x > at) ends[q] = i;
+      if (x >= at) ends[d + 1 + q] = i;
+    }
+  for (int i = 0; i < n; ++i) {
+    const int x = std::min(step * i, ne);
+    while (e + 1 < d && x >= coarse_node(e + 1, ne, d, even)) ++e;
+    const int a = coarse_node(e, ne, d, even), b = coarse_node(e + 1, ne, d, even);
+    const float f = (float)(x - a) / (float)(b - a);
+    hats.push_back({e >= 1 ? 1.0f - f : 0.0f, e + 1 < d ? f : 0.0f, (std::max(e, 1) - 1) * stride,
+                    (std::min(e + 1, d - 1) - 1) * stride});
+  }
+}
 }  // namespace
 
-int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
+int vcycle_setup(const Grid &g, int K, double contrast, const int *et_d, const double *ke_d, const StencilOp &op, const float *kinv,
                  float *P, float *AP, hipStream_t st, VCycleDev **out) {
   *out = nullptr;
   CGrid cg, mid;
@@ -920,7 +936,7 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
   const bool two = coarse_grid_two_level(g, &cg);
   if (two)
     mid = CGrid{};
-  else if (!coarse_grid_cycle(g, &cg) || !coarse_grid_by_two(g, &mid))
+  else if (!coarse_grid_cycle(g, contrast, &cg) || !coarse_grid_by_two(g, &mid))
     return MPPD_OK;
   VCycleDev *v = new VCycleDev();
   v->arena = nullptr;
@@ -954,9 +970,16 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     };
     const size_t n1 = two ? 0 : (size_t)s1.NP * 3 * K * sizeof(float);
     const size_t o_rc = carve((size_t)nc * K * sizeof(float)), o_ec = carve((size_t)nc * K * sizeof(float));
-    size_t o_hat[3];
-    const int line[3] = {g.nx, g.ny, g.nz}, mq[3] = {cg.mx, cg.my, cg.mz};
-    for (int a = 0; a < 3; ++a) o_hat[a] = carve(line[a] * sizeof(HatEntry));
+    // the sides' tables (VCycleDev), one copy
+    std::vector<HatEntry> hats[3];
+    std::vector<int> ends[3];
+    size_t o_hat[3], o_end[3];
+    const int ne[3] = {g.nex, g.ney, g.nez}, mq[3] = {cg.mx, cg.my, cg.mz};
+    for (int a = 0, stride = 3; a < 3; stride *= mq[a++]) {
+      side_tables(ne[a], mq[a] + 1, cg.even & (1 << a), two ? 1 : 2, stride, hats[a], ends[a]);
+      o_hat[a] = carve(hats[a].size() * sizeof(HatEntry));
+      o_end[a] = carve(ends[a].size() * sizeof(int));
+    }
     const size_t o_z = carve(mixed_vector_len(g, K) * sizeof(float));
     const size_t o_prz = carve(std::max((size_t)K * nb, 2 * 4 * (size_t)std::max(nb, nb1)) * sizeof(double));
     const size_t o_grow = carve(2 * sizeof(double));
@@ -977,9 +1000,19 @@ int vcycle_setup(const Grid &g, int K, const int *et_d, const double *ke_d, cons
     auto at = [base](size_t o) { return reinterpret_cast<float *>(base + o); };
     v->rc = at(o_rc);
     v->ec = at(o_ec);
-    for (int a = 0, stride = 3; a < 3; stride *= mq[a++]) {
+    std::vector<char> tables(o_z - o_hat[0]);
+    for (int a = 0; a < 3; ++a) {
+      std::memcpy(tables.data() + (o_hat[a] - o_hat[0]), hats[a].data(), hats[a].size() * sizeof(HatEntry));
+      std::memcpy(tables.data() + (o_end[a] - o_hat[0]), ends[a].data(), ends[a].size() * sizeof(int));
       v->hat[a] = reinterpret_cast<HatEntry *>(base + o_hat[a]);
-      hipLaunchKernelGGL(k_v_hats, dim3(1), dim3(kCoarseMaxLine), 0, st, line[a] - 1, mq[a] + 1, stride, v->hat[a]);
+      v->past[a] = reinterpret_cast<int *>(base + o_end[a]);
+      v->upto[a] = v->past[a] + mq[a] + 2;
+    }
+    e = hipMemcpyAsync(base + o_hat[0], tables.data(), tables.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+      rc = hip_fail(e, "preconditioner tables");
+      break;
     }
     v->z = at(o_z);
     v->R1 = at(o_R1);

@@ -1,7 +1,8 @@
-"""GPU: the coarse level of multi-RHS solvers on large RVEs.
+"""GPU: the coarse level of multi-RHS solvers on large RVEs and at high contrast.
 
 Above 80 elements a side a coarse element is 8 or more fine ones wide; with elements of two widths h and h + 1 a fine
-element has (2 h + 1)^3 positions in its coarse element, and the set-up holds them in slabs.  Every side up to 255
+element has (2 h + 1)^3 positions in its coarse element, and the set-up holds them in slabs.  Above a contrast of 30 the
+coarse nodes have even fine indices: up to three widths a side.  Every side up to 255
 elements has a coarse level, whatever divides it."""
 import numpy as np
 import pytest
@@ -22,8 +23,8 @@ def mp():
     return micropp_amd
 
 
-def materials(mp):
-    return [mp.material(0, 1e6, 0.3), mp.material(0, 1e7, 0.25), mp.material(0, 1e7, 0.25)]
+def materials(mp, contrast=10.0):
+    return [mp.material(0, 1e6, 0.3)] + [mp.material(0, 1e6 * contrast, 0.25)] * 2
 
 
 @pytest.mark.parametrize("elems", [(135, 135, 135), (144, 144, 144), (120, 92, 158), (131, 40, 255)],
@@ -44,25 +45,30 @@ def stiffness(mp, r, E, nu):
     return sum(b.T @ c @ b for b in r.bmat().reshape(8, 6, 24)) / (8 * r.nelem)
 
 
-def side(ne, d):
+def side(ne, d, even):
     """Coarse element, position from its first fine element and width, of every fine element of a side."""
-    at = np.array([q * ne // d for q in range(d + 1)])
+    if even and (ne % d or ne // d % 2):
+        at = np.array([2 * (q * ((ne + 1) // 2) // d) for q in range(d)] + [ne])
+    else:
+        at = np.array([q * ne // d for q in range(d + 1)])
     e = np.searchsorted(at, np.arange(ne), side="right") - 1
     return e, np.arange(ne) - at[e], (at[1:] - at[:-1])[e]
 
 
 # slabs of 14 of 17 planes of positions, of 5 of 27, and one slab
-@pytest.mark.parametrize("elems", [(85, 83, 82), (131, 131, 127), (40, 36, 31)], ids=lambda s: "x".join(map(str, s)))
-def test_coarse_inverse_of_slabs(mp, elems):
+@pytest.mark.parametrize("elems, contrast", [((85, 83, 82), 10.0), ((131, 131, 127), 10.0), ((40, 36, 31), 10.0),
+                                             ((40, 36, 31), 100.0), ((33, 35, 30), 100.0), ((85, 83, 82), 100.0)],
+                         ids=str)
+def test_coarse_inverse_of_slabs(mp, elems, contrast):
     """Against the inverse of the Galerkin matrix formed here from element matrices and hats; the bar of the small
     grids: 1e-6 of the largest entry (FP32 rounding of the entries is 6e-8 of each)."""
-    r = mp.Rve([n + 1 for n in elems], mp.MIC3D_RANDOM_SPHERES, GEO, materials(mp))
+    r = mp.Rve([n + 1 for n in elems], mp.MIC3D_RANDOM_SPHERES, GEO, materials(mp, contrast))
     dims, ainv = mp.MSolver(r, 4).coarse()
     m = [int(v) for v in dims[4:]]
     d = [v + 1 for v in m]
-    ke = [stiffness(mp, r, 1e6, 0.3), stiffness(mp, r, 1e7, 0.25), stiffness(mp, r, 1e7, 0.25)]
+    ke = [stiffness(mp, r, 1e6, 0.3)] + [stiffness(mp, r, 1e6 * contrast, 0.25)] * 2
     phase = r.elem_types().reshape(elems[::-1])
-    sides = [side(ne, n) for ne, n in zip(elems, d)]
+    sides = [side(ne, n, contrast > 30) for ne, n in zip(elems, d)]
     kinds = [sorted(set(zip(p.tolist(), w.tolist()))) for _, p, w in sides]
     sums = np.zeros((d[2] * d[1] * d[0], 24, 24))
 
