@@ -893,13 +893,17 @@ int mppd_msolver_destroy(mppd_msolver *m) {
 // is state[q & 1].  The next chunk is sized from each live field's observed
 // convergence rate (iterations still needed, + 2), so few iterations are
 // queued past the end.  *its = iterations run; *finite (may be NULL) = every
-// field's ||z|| is finite at the end (no breakdown).  *broken: the multilevel
-// preconditioner vc has shown itself not positive definite ((r, z) <= 0); the
-// CG has stopped there and X is of no use.
+// field's ||z|| is finite at the end (no breakdown).  *vstate: what became of the
+// multilevel preconditioner vc.
+enum VState {
+  kVGood,
+  kVSlow,   // max_inner iterations did not reach every field's target
+  kVBroken  // not positive definite, (r, z) <= 0: the CG has stopped there and X is of no use
+};
 static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op, const float *kinv, float *R, float *X, float *P,
                        float *AP, double *part, void *state, void *state_h, int max_inner, hipStream_t st,
                        int *its_out, bool *finite = nullptr, bool stop_on_stall = false,
-                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr, bool *broken = nullptr,
+                       const CoarseDev *coarse = nullptr, const VCycleDev *vc = nullptr, VState *vstate = nullptr,
                        long *queued_out = nullptr) {
   int queued = 0, its = 0, done = 0, its_prev = 0;
   if (vc) mixed_state_view(state_h, 0, &its, &done);  // (it may be broken at the start)
@@ -907,7 +911,7 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
   // to 13 launches each, so few are queued past the end: an iteration after it
   // costs about 50 us, a look 10.  (Rates of plateaus overshoot by far: 96
   // iterations at contrast 1000, 30^3 elements, 18.8 ms with chunks of up to 256,
-  // 7.6 with 16.)
+  // 8.0 with 16.)
   int chunk = vc ? 8 : 32;
   const int slack = vc ? 0 : 2, least = vc ? 1 : 4, most = vc ? 16 : 256;
   std::vector<double> pn_prev(K, 0.0);
@@ -950,7 +954,7 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
   }
   *its_out = its;
   if (queued_out) *queued_out += queued;
-  if (broken) *broken = mixed_state_broken(state_h, queued);
+  if (vstate) *vstate = !vc ? kVGood : mixed_state_broken(state_h, queued) ? kVBroken : its >= max_inner ? kVSlow : kVGood;
   if (finite) {
     *finite = true;
     for (int k = 0; k < K; ++k) {
@@ -966,8 +970,17 @@ static int mixed_inner(const Grid &g, int K, const float *A, const StencilOp &op
 // a_v / V of field v), then n forward fields with the macro strains eps_h,
 // then idle fields.  FP64 defect correction with FP32 inner CG until every
 // field converges; the solution is left in m->U.  A correction whose
-// preconditioner was not positive definite is dropped and solved again, and the
-// rest of the call with Jacobi.
+// preconditioner was not positive definite is dropped and solved again.  From
+// there on, and behind a pass that stopped at kVcycleMost iterations (one more
+// than max_outer allows then), the call goes on with Jacobi.
+//
+// kVcycleMost: an iteration with the multilevel preconditioner takes the time
+// of 3 to 4 with Jacobi, and where it needs so many (contrasts of 1e5, of 1e4
+// in long cells) Jacobi often needs no more of them.  40 small spheres, 8 fields
+// to 1e-8, ms with this limit / without / Jacobi alone: 5 x 89 x 90 elements,
+// contrast 1e4, 131 / 270 / 125; 30^3, 1e5, 98 / 125 / 101; 50^3, 1e6, 471 / 706
+// / 486.
+constexpr int kVcycleMost = 500;
 static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, const mppd_mixed_params *p,
                        int stats[2], std::vector<double> &pn, std::vector<double> &pn0, int *all_conv_out) {
   const Grid &g = m->r->g;
@@ -984,27 +997,27 @@ static int msolver_run(mppd_msolver *m, int nadj, int n, const double *eps_h, co
     MPP_HIP(launch_m_adj_src(g, K, nadj, m->r->bmat, m->mats_d, m->r->et, m->G, m->F, m->st));
     F = m->F;
   }
-  int outer = 0, inner_total = 0, all_conv = 0;
+  int outer = 0, inner_total = 0, all_conv = 0, most_outer = p->max_outer;
   const VCycleDev *vc = m->vc;
   pn.assign(K, 0.0);
   pn0.assign(K, 0.0);
   for (;;) {
+    const int most = vc ? std::min(p->max_inner_its, kVcycleMost) : p->max_inner_its;
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, F, m->kinv, m->R, m->X, m->P, m->part, outer == 0,
-                           p->rel_tol, p->abs_tol, p->inner_tol, p->max_inner_its, m->state, m->st));
+                           p->rel_tol, p->abs_tol, p->inner_tol, most, m->state, m->st));
     if (vc) MPP_HIP(launch_v_start(g, K, *vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
     mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
-    if (all_conv || outer >= p->max_outer) break;
-    bool broken = false;
+    if (all_conv || outer >= most_outer) break;
+    VState vstate = kVGood;
     int its = 0, rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h,
-                                  p->max_inner_its, m->st, &its, nullptr, false, nullptr, vc, &broken, &m->queued);
+                                  most, m->st, &its, nullptr, false, nullptr, vc, &vstate, &m->queued);
     if (rc) return rc;
     inner_total += its;
-    if (broken) {
-      vc = nullptr;
-      continue;
-    }
+    if (vstate != kVGood) vc = nullptr;
+    if (vstate == kVBroken) continue;
+    most_outer += vstate == kVSlow && most < p->max_inner_its;
     MPP_HIP(launch_m_accum(g, K, m->X, m->U, m->st));
     ++outer;
   }
@@ -1123,16 +1136,17 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
   std::vector<int> its(K, 0), run(K, 0), conv(K, 0), cost(K, 0), cflag(K, 0);
   std::vector<double> rn(K), rn0(K), norm0(K), pn(K), pn0(K);
   for (int k = 0; k < n; ++k) run[k] = 1;
-  int outer_total = 0, inner_total = 0;
-  const VCycleDev *vc = m->vc;  // (null once it has failed: msolver_run)
+  int outer_total = 0, inner_total = 0, most = 0;
+  const VCycleDev *vc = m->vc;  // (null once it has failed or is slow: msolver_run)
   // the residual of the current U for the fields in run, with the outer test
   // and the inner start state (first: targets from this residual)
   auto resid = [&](int first) -> int {
     MPP_HIP(hipStreamSynchronize(m->st));  // act_h may still feed an earlier copy
     for (int k = 0; k < K; ++k) m->act_h[k] = run[k];
     MPP_HIP(hipMemcpyAsync(m->act_d, m->act_h, K * sizeof(int), hipMemcpyHostToDevice, m->st));
+    most = vc ? std::min(max_inner, kVcycleMost) : max_inner;
     MPP_HIP(launch_m_resid(g, K, m->r->et, m->ke, m->U, nullptr, m->kinv, m->R, m->X, m->P, m->part, first,
-                           p->cg_rel_tol, p->cg_abs_tol, inner_tol, max_inner, m->state, m->st, m->act_d));
+                           p->cg_rel_tol, p->cg_abs_tol, inner_tol, most, m->state, m->st, m->act_d));
     if (vc) MPP_HIP(launch_v_start(g, K, *vc, m->op, m->kinv, m->R, m->P, m->AP, m->state, m->st));
     MPP_HIP(hipMemcpyAsync(m->state_h, m->state, mixed_state_bytes(), hipMemcpyDeviceToHost, m->st));
     MPP_HIP(hipStreamSynchronize(m->st));
@@ -1164,20 +1178,22 @@ int mppd_msolver_newton(mppd_msolver *m, int n, const double *eps_h, const doubl
     // current residual (the last one computed is that of the current U)
     if ((changed || !fresh) && (rc = resid(1))) return rc;
     fresh = false;
+    int most_outer = max_outer;
     for (int outer = 0;; ++outer) {
       if (outer > 0 && (rc = resid(0))) return rc;
       int all_conv = 0;
       mixed_outer_view(m->state_h, K, &all_conv, pn.data(), pn0.data());
-      if (all_conv || outer >= max_outer) break;
+      if (all_conv || outer >= most_outer) break;
       int inner = 0;
-      bool broken = false;
-      if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, max_inner,
-                            m->st, &inner, nullptr, false, nullptr, vc, &broken, &m->queued)))
+      VState vstate = kVGood;
+      if ((rc = mixed_inner(g, K, nullptr, m->op, m->kinv, m->R, m->X, m->P, m->AP, m->part, m->state, m->state_h, most,
+                            m->st, &inner, nullptr, false, nullptr, vc, &vstate, &m->queued)))
         return rc;
       inner_total += inner;
       for (int k = 0; k < n; ++k) cost[k] += run[k] ? inner : 0;
-      if (broken) {  // this outer step again, from its residual
-        vc = nullptr;
+      if (vstate != kVGood) vc = nullptr;
+      most_outer += vstate == kVSlow && most < max_inner;
+      if (vstate == kVBroken) {  // this outer step again, from its residual
         if (outer == 0 && (rc = resid(1))) return rc;
         --outer;
         continue;

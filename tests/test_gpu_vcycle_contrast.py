@@ -35,3 +35,25 @@ def test_against_jacobi(mp, monkeypatch, size, micro, contrast):
           np.abs(sig - sig_j).max() / np.abs(sig_j).max(), flush=True)
     assert ok and ok_j and np.abs(sig - sig_j).max() < 1e-5 * np.abs(sig_j).max()
     assert stats[1] < stats_j[1]
+
+
+@pytest.mark.parametrize("size, contrast", [((31, 31, 31), 1e5), ((6, 60, 61), 1e4), ((17, 14, 18), 1e6)])
+def test_passes_that_end_in_jacobi(mp, monkeypatch, size, contrast):
+    """More than 500 iterations a pass: solve, Newton and adjoint go on with Jacobi and converge with one outer pass
+    more at most, to the same sigma (as above)."""
+    mats = [mp.material(0, 1e6, 0.3)] + [mp.material(0, 1e6 * contrast, 0.25)] * 2
+    r = mp.Rve(size, mp.MIC3D_RANDOM_SPHERES, (3.0, 40.0, 0.02, 0.08), mats)
+    e = np.random.default_rng(9).uniform(-5e-3, 5e-3, (2, 6))
+    ms = mp.MSolver(r, 8)
+    monkeypatch.setenv("MPPD_COARSE", "0")
+    mj = mp.MSolver(r, 8)
+    calls = []
+    for m in (ms, mj):
+        sig, stats, rel, ok = m.solve(e, max_inner_its=8000)
+        nsig, out, nstats = m.newton(e, cg_rel_tol=1e-8, nr_rel_tol=1e-6, mixed=(1e-5, 8000, 10))
+        ctan, asig, dmat, astats, arel, aok = m.adjoint(e, max_inner_its=8000)
+        calls.append((sig, nsig, asig, ctan))
+        print(size, contrast, stats, nstats, astats, flush=True)
+        assert ok and aok and (out[:, 2] == 1).all()
+    for a, b in zip(*calls):
+        assert np.abs(a - b).max() < 1e-5 * np.abs(b).max()
