@@ -969,7 +969,7 @@ int setup(mppd_batch *B, const mppd_batch_rve *in) {
     R.nb_elem = (g.nelem + 255) / 256;
     const int nb_ke = ((R.phase_mode ? 3 : g.nelem) + kKeWaves - 1) / kKeWaves;
     R.cgrid = CGrid{};
-    if (coarse && !coarse_grid_wide(g, 2, batch_coarse_max_dofs(g), &R.cgrid)) R.cgrid = CGrid{};
+    if (coarse && !coarse_grid_additive(g, batch_coarse_max_dofs(g), &R.cgrid)) R.cgrid = CGrid{};
     const CGrid &cg = R.cgrid;
     const int counts[kS] = {R.nb_row,
                             R.nb_elem,

@@ -212,6 +212,8 @@ bool coarse_grid_cycle(const Grid &g, double contrast, CGrid *out);
 // q of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
 // divide the side, l = h + 1); false: none
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out);
+// the coarse grid beside Jacobi: at least 2 wide, or of one length on every side where the cells are long; false: none
+bool coarse_grid_additive(const Grid &g, int max_dofs, CGrid *out);
 // C (device, coarse_table_len(cg, nz) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position,
 // for nz of the coarse_table_planes(cg) planes of positions from z0 on
 // (positions of a side: those in an element h wide, in one l wide, in the last one)
