@@ -226,7 +226,8 @@ int mppd_msolver_profile(mppd_msolver *m, int iters, double *spmv_ms, double *it
  * elements per coarse element along x, y, z, interior coarse nodes along x,
  * y, z (all 0 without a coarse level).  Where a side of ne elements is no
  * multiple of its d = m + 1 coarse ones, h is the smaller of two widths, h
- * and h + 1.  With three levels and a contrast of the moduli above 30 the
+ * and h + 1.  Where the cells are at least 2.5 times as long along one side as
+ * along another the elements may have one length, not one width.  With three levels and a contrast of the moduli above 30 the
  * widths are even instead, h and h + 2, and an odd side's last one is narrower
  * by 1.  ainv_h (may be NULL): nc x nc floats,
  * the inverse of the Galerkin matrix P^T A P, P the trilinear hats of the

@@ -33,18 +33,6 @@ int pick_side(int ne, int dmax) {
   return 0;
 }
 
-// Contrast above which the multilevel preconditioner's coarse nodes have even
-// fine indices, i.e. are nodes of its second level.  A coarse hat with its peak
-// between two of them is no sum of its hats, and its Galerkin matrix says
-// nothing about the energy of what the second level makes of it: beside a stiff
-// element too little by up to the contrast.  Solves of 8 fields to 1e-8, ms, at
-// even indices / at floor(q ne / d): 30^3 elements, 40 small spheres, contrast
-// 10 1.85 / 1.84, 300 7.4 / 8.4, 1e4 39 / 86, 1e5 153 / 796; 50^3, a layer, 300
-// 3.4 / 4.0, 1e4 3.7 / 14.9, 1e-5 3.5 / 36.  Over 45 RVEs, to 1e-10, even
-// indices take 1.01 of the time at contrast 3, 1.00 at 10, 0.99 at 30, 0.97 at
-// 100 and 0.93 at 300.
-constexpr double kEvenContrast = 30.0;
-
 // Positions of a fine element along a side: 0 .. h - 1 in a coarse element h
 // wide, then those in one l wide and in the last one (t wide), as far as these
 // widths differ.  The first position in an element w wide, and all of them:
@@ -541,11 +529,21 @@ bool coarse_grid_by_two(const Grid &g, CGrid *out) {
 // costs 0.1 ms more): 30^3 elements 29 iterations to 1e-10 become 25, 29 x 37 x
 // 23 38 become 33, sigma and ctan 9% sooner.  2187 DOFs (30^3 at h = 3, 40^3 at h
 // = 4: 19 MB read an iteration and 0.7 ms more set-up) cost more than they save.
+// Above kHighContrast the multilevel preconditioner's coarse nodes have even
+// fine indices, i.e. are nodes of its second level.  A coarse hat with its peak
+// between two of them is no sum of its hats, and its Galerkin matrix says
+// nothing about the energy of what the second level makes of it: beside a stiff
+// element too little by up to the contrast.  Solves of 8 fields to 1e-8, ms, at
+// even indices / at floor(q ne / d): 30^3 elements, 40 small spheres, contrast
+// 10 1.85 / 1.84, 300 7.4 / 8.4, 1e4 39 / 86, 1e5 153 / 796; 50^3, a layer, 300
+// 3.4 / 4.0, 1e4 3.7 / 14.9, 1e-5 3.5 / 36.  Over 45 RVEs, to 1e-10, even
+// indices take 1.01 of the time at contrast 3, 1.00 at 10, 0.99 at 30, 0.97 at
+// 100 and 0.93 at 300.
 bool coarse_grid_cycle(const Grid &g, double contrast, CGrid *out) {
   const bool narrow = coarse_grid_wide(g, 4, 1100, out) &&
                       std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= 4;
   if (!narrow && !coarse_grid_wide(g, 5, kCoarseMaxDofs, out)) return false;
-  if (contrast <= kEvenContrast) return true;
+  if (contrast <= kHighContrast) return true;
   const int ne[3] = {g.nex, g.ney, g.nez}, m[3] = {out->mx, out->my, out->mz};
   int h[3] = {out->hx, out->hy, out->hz}, l[3] = {out->lx, out->ly, out->lz}, even = 0;
   for (int a = 0; a < 3; ++a) {
@@ -592,8 +590,13 @@ bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out) {
 // one length leaves fewer coarse DOFs (9 x 13 x 11 34 / 19 / 19, contrast 1000
 // and spheres 165 / 80 / 114).
 bool coarse_grid_additive(const Grid &g, int max_dofs, CGrid *out) {
+  return cell_aspect(g) < 2 ? coarse_grid_wide(g, 2, max_dofs, out) : coarse_grid_long(g, max_dofs, out);
+}
+
+double cell_aspect(const Grid &g) { return std::max({g.dx, g.dy, g.dz}) / std::min({g.dx, g.dy, g.dz}); }
+
+bool coarse_grid_long(const Grid &g, int max_dofs, CGrid *out) {
   const double len[3] = {g.dx, g.dy, g.dz}, least = std::min({g.dx, g.dy, g.dz});
-  if (std::max({g.dx, g.dy, g.dz}) < 2 * least) return coarse_grid_wide(g, 2, max_dofs, out);
   if (g.nex < 4 || g.ney < 4 || g.nez < 4) return false;
   if (g.nx > kCoarseMaxLine || g.ny > kCoarseMaxLine || g.nz > kCoarseMaxLine) return false;
   const int ne[3] = {g.nex, g.ney, g.nez};

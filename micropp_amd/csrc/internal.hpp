@@ -168,6 +168,7 @@ struct CoarseDev {
 constexpr int kCoarseSplit = 16;    // column splits of the coarse solve (one partial each)
 constexpr int kCoarseMaxLine = 256;  // nodes per side a coarse level allows
 constexpr int kCoarseMaxDofs = 2200;  // coarse DOFs of a multi-RHS solver (3 x 9^3 = 2187: 10^3 coarse elements)
+constexpr double kHighContrast = 30.0;  // of the moduli: beyond it, coarse grids of the multilevel form made for it
 constexpr int kCoarseMaxPos = 4096;   // positions of a fine element that the set-up's table holds at once (57 MB)
 // Trilinear hats along one side at one fine index: the interior coarse nodes
 // below and above it, as offsets into the coarse vectors, and their weights
@@ -212,7 +213,11 @@ bool coarse_grid_cycle(const Grid &g, double contrast, CGrid *out);
 // q of a side of ne elements and d = m + 1 coarse ones at fine index floor(q ne / d) (widths h and, where d does not
 // divide the side, l = h + 1); false: none
 bool coarse_grid_wide(const Grid &g, int least, int max_dofs, CGrid *out);
-// the coarse grid beside Jacobi: at least 2 wide, or of one length on every side where the cells are long; false: none
+// the longest cell side over the shortest, and a coarse grid of elements of one length on every side (a side's own
+// elements where those are longer), as short as max_dofs coarse DOFs allow; false: none
+double cell_aspect(const Grid &g);
+bool coarse_grid_long(const Grid &g, int max_dofs, CGrid *out);
+// the coarse grid beside Jacobi: elements at least 2 wide, or of one length where the cells are long; false: none
 bool coarse_grid_additive(const Grid &g, int max_dofs, CGrid *out);
 // C (device, coarse_table_len(cg, nz) doubles) = the Galerkin contributions P_e^T Ke P_e per phase and position,
 // for nz of the coarse_table_planes(cg) planes of positions from z0 on

@@ -895,7 +895,21 @@ constexpr float kDamp = 1.65f;
 // 20 and 47 to 54 at 22 to 26, with as many iterations (22 to 27; 33 at 24).
 // Above, the inverse's set-up (2.1 ms at 2187 DOFs against 1.4) costs more than
 // the iterations gain.
-bool coarse_grid_two_level(const Grid &g, CGrid *out) {
+// Cells kLongCells times as long along one side as along another have it with
+// coarse elements of one length, where that is at most two of the long cells:
+// twice the spacing on every side loses what the smoother leaves along the
+// long ones.  Three levels and this, inner iterations to 1e-8 and ms (contrast
+// 10, spheres, eight fields, nodes): 6 x 60 x 61 141, 7.2 and 44, 2.6; 13 x 60 x
+// 60 72, 6.2 and 57, 4.1; 17 x 41 x 41 38, 3.2 and 38, 2.5; 9 x 10 x 41 65, 3.3
+// and 28, 1.7; at 2.4 long cells (23 x 91 x 91) 64, 10.2 and 72, 9.8; at 3.3 (31
+// x 91 x 91) 52, 10.4 and 72, 11.8.  With the 2200 DOFs that stiff phases are
+// worth instead of 1536 the set-up takes 0.6 ms more (9 x 61 x 62, contrast 1e4:
+// 12.4 ms become 6.9; 10: 3.4 become 3.2).
+constexpr double kLongCells = 2.5;
+bool coarse_grid_two_level(const Grid &g, double contrast, CGrid *out) {
+  if (cell_aspect(g) >= kLongCells && coarse_grid_long(g, contrast > kHighContrast ? kCoarseMaxDofs : 1536, out) &&
+      std::max({out->lx * g.dx, out->ly * g.dy, out->lz * g.dz}) <= 2.001 * std::max({g.dx, g.dy, g.dz}))
+    return true;
   for (int width = 2; width <= 3; ++width)
     if (coarse_grid_wide(g, width, width == 2 ? kCoarseMaxDofs : 1536, out) &&
         std::max({out->hx, out->lx, out->hy, out->ly, out->hz, out->lz}) <= width)
@@ -933,7 +947,7 @@ int vcycle_setup(const Grid &g, int K, double contrast, const int *et_d, const d
   *out = nullptr;
   CGrid cg, mid;
   if (!coarse_enabled()) return MPPD_OK;
-  const bool two = coarse_grid_two_level(g, &cg);
+  const bool two = coarse_grid_two_level(g, contrast, &cg);
   if (two)
     mid = CGrid{};
   else if (!coarse_grid_cycle(g, contrast, &cg) || !coarse_grid_by_two(g, &mid))

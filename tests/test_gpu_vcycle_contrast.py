@@ -37,7 +37,7 @@ def test_against_jacobi(mp, monkeypatch, size, micro, contrast):
     assert stats[1] < stats_j[1]
 
 
-@pytest.mark.parametrize("size, contrast", [((31, 31, 31), 1e5), ((6, 60, 61), 1e4), ((17, 14, 18), 1e6)])
+@pytest.mark.parametrize("size, contrast", [((31, 31, 31), 1e5), ((17, 14, 18), 1e6)])
 def test_passes_that_end_in_jacobi(mp, monkeypatch, size, contrast):
     """More than 500 iterations a pass: solve, Newton and adjoint go on with Jacobi and converge with one outer pass
     more at most, to the same sigma (as above)."""

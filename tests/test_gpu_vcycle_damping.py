@@ -70,7 +70,7 @@ def test_one_stiff_element_of_the_second_level(mp, ne, contrast):
 # two levels (the first), three, thin cells; even sides
 @pytest.mark.parametrize("size, geo, contrast", [
     ((5, 7, 5), (7.0, 4.0, 0.1, 0.2), 10.0), ((31, 29, 33), (10.0, 8.0, 0.05, 0.15), 10.0),
-    ((31, 31, 31), (12.0, 60.0, 0.01, 0.04), 300.0), ((61, 63, 9), (13.0, 8.0, 0.05, 0.2), 100.0)])
+    ((31, 31, 31), (12.0, 60.0, 0.01, 0.04), 300.0), ((61, 63, 26), (13.0, 8.0, 0.05, 0.2), 100.0)])
 def test_spheres(mp, size, geo, contrast):
     mats = [mp.material(0, 1e6, 0.3), mp.material(0, 1e6 * contrast, 0.25), mp.material(0, 1e6, 0.3)]
     r = mp.Rve(size, mp.MIC3D_RANDOM_SPHERES, geo, mats)
