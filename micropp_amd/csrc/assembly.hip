@@ -55,9 +55,18 @@ __global__ void __launch_bounds__(256) k_elem_ke(Grid g, const double *bmat, con
   elem_ke_body(g, blockIdx.x, bmat, mats, et, u, vars, phase_mode, ke);
 }
 
-__global__ void __launch_bounds__(256) k_gather_vals(Grid g, const int *et, const double *ke, int phase_mode,
-                                                     double *vals) {
-  gather_vals_slice(g, blockIdx.x, et, ke, phase_mode, vals);
+__global__ void __launch_bounds__(256) k_gather_vals(Grid g, const int *et, const double *ke, double *vals) {
+  gather_vals_slice(g, blockIdx.x, et, ke, 0, vals);
+}
+
+__global__ void __launch_bounds__(256) k_gather_vals_rows(Grid g, const int *et, const double *ke, double *vals) {
+  const int row = blockIdx.x * 256 + threadIdx.x;
+  if (blockIdx.y == 0)
+    gather_vals_row<0>(g, row, et, ke, vals);
+  else if (blockIdx.y == 1)
+    gather_vals_row<1>(g, row, et, ke, vals);
+  else
+    gather_vals_row<2>(g, row, et, ke, vals);
 }
 
 __global__ void __launch_bounds__(256) k_elem_be(Grid g, const double *bmat, const material_base *mats, const int *et,
@@ -128,7 +137,10 @@ hipError_t launch_elem_ke(const Grid &g, const double *bmat, const material_base
 
 hipError_t launch_gather_vals(const Grid &g, const int *et, const double *ke, int phase_mode, double *vals,
                               hipStream_t st) {
-  hipLaunchKernelGGL(k_gather_vals, dim3(g.nrow_pad / 64), dim3(256), 0, st, g, et, ke, phase_mode, vals);
+  if (phase_mode)
+    hipLaunchKernelGGL(k_gather_vals_rows, dim3(nblk(g.nrow_pad, 256), 3), dim3(256), 0, st, g, et, ke, vals);
+  else
+    hipLaunchKernelGGL(k_gather_vals, dim3(g.nrow_pad / 64), dim3(256), 0, st, g, et, ke, vals);
   return hipGetLastError();
 }
 

@@ -308,6 +308,45 @@ __device__ __forceinline__ void gather_vals_slice(const Grid &g, int slice, cons
   for (int t = threadIdx.x; t < kSlots * 64; t += 256) out[t] = acc[(t >> 6) * kGatherPitch + (t & 63)];
 }
 
+// A third (neighbours of plane Z) of one row of an all-elastic RVE's matrix (ke:
+// its phases' element stiffness, in the caches) by one thread, the same sums.
+// Bound: the stores alone.  A call, us, with slices made in LDS / a thread per
+// row / per third: 11^3 nodes 18 / 23 / 17, 31^3 32 / 36 / 29, 41^3 52 / 47 / 46,
+// 51^3 85 / 70 / 69, 71^3 217 / 215 / 189.
+template <int Z>
+__device__ __forceinline__ void gather_vals_row(const Grid &g, int row, const int *et, const double *ke,
+                                                double *vals) {
+#pragma clang fp contract(off)
+  if (row >= g.nrow_pad) return;
+  double *out = vals + (size_t)(row >> 6) * kSlots * 64 + (row & 63);
+  const int node = row / 3, fi = row % 3;
+  const int i = node % g.nx, j = (node / g.nx) % g.ny, k = node / (g.nx * g.ny);
+  if (row >= g.nrow || on_boundary(g, i, j, k)) {
+    for (int s = 27 * Z; s < 27 * Z + 27; ++s) out[s * 64] = row < g.nrow && s == 13 * 3 + fi ? 1.0 : 0.0;
+    return;
+  }
+  const double *s[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {  // reference order (a, b, c) = (x, y, z)
+    const int a = q >> 2, b = (q >> 1) & 1, c = q & 1;
+    const int e = ((k - 1 + c) * g.ney + j - 1 + b) * g.nex + i - 1 + a;
+    s[q] = ke + (size_t)et[e] * 576 + (local_node(1 - a, 1 - b, 1 - c) * 3 + fi) * 24;
+  }
+#pragma unroll
+  for (int n = 9 * Z; n < 9 * Z + 9; ++n) {
+    double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int px = n % 3 - (q >> 2), py = (n / 3) % 3 - ((q >> 1) & 1), pz = n / 9 - (q & 1);
+      if (px < 0 || px > 1 || py < 0 || py > 1 || pz < 0 || pz > 1) continue;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[d] += s[q][local_node(px, py, pz) * 3 + d];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) out[(n * 3 + d) * 64] = acc[d];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // The Gauss-point kernels: a thread per Gauss point (8 lanes an element), so
 // that an RVE of a few hundred elements is not a handful of waves that each
